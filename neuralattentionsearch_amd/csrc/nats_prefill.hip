@@ -9,7 +9,9 @@
 //   prefill_split_merge_kernel combines those partial results
 //   prefill_mfma_wide_kernel   bf16 MFMA kernel for head dim 256: four wavefronts with the whole register file, whole
 //                              tiles masked row by row
-//   prefill_simple_kernel      fp32 (or bf16) FMA kernel, one query row per lane; the fp32 parity path
+//   prefill_f32_kernel         fp32 on the fp32 matrix instruction (nats_prefill_f32.hip)
+//   prefill_simple_kernel      fp32 (or bf16) FMA kernel, one query row per lane: what the others do not take (head dim
+//                              16, fp32 at head dim 256, rows that are not 16-byte aligned)
 //
 // Mask semantics (components/masks/utils.py:89-94, components/cache/nats_chunk_layer_cache.py:462-511, 603-616):
 // the queries are tokens [r_begin, r_end) of the open-chunk region, which starts at key row `base`; every key
@@ -19,51 +21,9 @@
 // A prefill from an empty cache is the case base = 0, r_begin = 0.
 #include <stdlib.h>
 
-#include "nats_common.h"
+#include "nats_prefill.h"
 
 namespace nats {
-
-struct PrefillArgs {
-  const void* q;
-  const void* k;
-  const void* v;
-  void* o;
-  const int32_t* tok_lim;  // [B*Hkv, N], then one entry holding -1
-  const int2* tile_lim;    // [B*Hkv, Tk] {max, min}
-  const int2* gran_lim;    // [B*Hkv, Tk * 4] {max, min} of every 16 key rows
-  int64_t qs_b, qs_h, qs_l;
-  int64_t ks_b, ks_h, ks_l;
-  int64_t vs_b, vs_h, vs_l;
-  int64_t os_b, os_h, os_l;
-  int B, Hq, Hkv, n_rep;
-  int N, Tk;             // key rows and 64-row key tiles
-  int base;              // first key row of the region
-  int r_begin, r_end;    // region tokens that are queries; query i of q / o is token r_begin + i
-  int qt_first, qt_last; // 64-token region tiles that hold queries
-  int hpw;       // q heads of one kv head handled by one workgroup (mfma kernel)
-  int qpw;       // 64-row query tiles handled by one workgroup (mfma kernel)
-  int n_hg;      // head groups per kv head = n_rep / hpw
-  int n_qg;      // query tile groups = ceil(n query tiles / qpw)
-  int xcd_mode;  // 1: workgroups of one kv stream share an XCD (needs B*Hkv % 8 == 0)
-  // The query groups with the fewest visible keys (the last pool_ranks ranks of every stream) are not bound to a
-  // workgroup: a few workgroups at the end of the grid draw them from counters, one queue per XCD (heaviest first),
-  // for as long as there are any, so that an XCD that reaches its last workgroups earlier takes more of them.
-  int pool_ranks;    // 0: every workgroup has its fixed query group
-  int32_t* ticket;   // one counter per XCD, kTicketStride entries apart, zero at launch
-  float scale;   // softmax scale
-  // few query tiles over many key rows: n_split workgroups share the tile list of one (kv stream, head group,
-  // query group) and leave partial results, which prefill_split_merge_kernel combines
-  int n_split;      // 1: no split
-  float* part_acc;  // [workgroup, split, wavefront, 32 rows, D]
-  float* part_ml;   // [workgroup, split, wavefront, 32 rows, 2] running maximum (base-2 exponent) and row sum
-  // packed tiles of chunks shorter than a granule: rows more than t_long tokens behind a query group come from the
-  // lists of long-lived rows (long_rows_kernel), gathered row by row; NULL = every row is walked granule by granule
-  const int32_t* long_rows;    // [streams, 2, long_cap]: list A (rows every later query sees), list B (rows with a last query)
-  const int32_t* long_lim;     // [streams, 2, long_cap]
-  const int32_t* long_before;  // [streams, 2, n_gran + 1] entries of A / of B before every granule
-  const int32_t* long_alive;   // [streams, n_rtile] first entry of B that a query of the 64-token region tile may see
-  int long_cap, n_gran, n_rtile, t_long;
-};
 
 // workgroup index -> (kv stream, head group, rank of the query group; heavy query groups come first)
 __device__ __forceinline__ void map_workgroup(const PrefillArgs& a, int bid, int& ks, int& hg, int& rank) {
@@ -1619,7 +1579,7 @@ static int launch_prefill_mfma(const PrefillArgs& a, int64_t n_wg, hipStream_t s
   return NATS_OK;
 }
 
-static int device_cu_count() {
+int device_cu_count() {
   static int cached[kMaxDevices] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
@@ -1745,7 +1705,10 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
     }
   }
 
-  // fp32, and bf16 at the head dim the MFMA kernels do not take (16): the plain kernel
+  // fp32 on the matrix cores
+  if (dtype == NATS_DTYPE_F32 && prefill_f32_takes(a, (int)g.D)) return launch_prefill_f32(a, (int)g.D, st);
+
+  // what the matrix kernels do not take (head dim 16, fp32 at head dim 256, unaligned rows): the plain kernel
   if (dtype == NATS_DTYPE_F32 || (g.D != 32 && g.D != 64 && g.D != 128)) {
     NATS_REQUIRE(g.B * g.H_q <= 65535, NATS_ERR_BAD_SHAPE, "%s: B*H_q too large for the plain kernel", who);
     dim3 grid((unsigned)n_qt, (unsigned)(g.B * g.H_q));
