@@ -13,6 +13,7 @@
 
 #include "nats_common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace nats {
@@ -36,6 +37,7 @@ struct DecodeArgs {
   int2* head_table;  // [B*Hkv] {first partial slot, number of partials}
   int n_wg;          // workgroups along x
   int share_first;   // 1/256ths of the tiles that go to the first half of the workgroups (128: equal shares)
+  int fixed_split;   // workgroups per head of the fixed schedule
 };
 
 __device__ __forceinline__ float exp2_guard(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -58,13 +60,15 @@ constexpr int kDecTile = 32;
 
 constexpr int kMaxBalancedHeads = 1024;  // (b, kv head) streams whose tile prefix sums fit in LDS
 
-template <int D, int NREP>
-struct DecodeSmem {
+template <int D, int NREP, int WAVES>
+struct DecodeTiles {
   // [wave][buffer]; after a head's tile loop the wavefront's own buffers hold its accumulators
   // (NREP * D floats <= 2 * kDecTile * D bf16 for NREP <= 16)
-  uint16_t v[4][2][kDecTile * D];
-  float wm[4][NREP];
-  float wl[4][NREP];
+  uint16_t v[WAVES][2][kDecTile * D];
+  float wm[WAVES][NREP];
+  float wl[WAVES][NREP];
+};
+struct DecodeSchedule {
   int tile_prefix[kMaxBalancedHeads + 1];  // exclusive prefix of 32-row tiles per (b, kv head)
   int slot_prefix[kMaxBalancedHeads + 1];  // exclusive prefix of partial results per (b, kv head)
   int scan_tmp[256];
@@ -110,8 +114,17 @@ __device__ __forceinline__ void block_exclusive_scan(int* dst, int n, int* tmp) 
 // or larger ones for the first half of the workgroups, see decode_share_first); a workgroup works through its
 // range head by head and emits one partial (m, l, acc) per head it touches.  All finish together, whatever the
 // per-head lengths are.
-template <int D, int NREP>
-__global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
+//
+// Fixed schedule (FIXED > 0: that many wavefronts per workgroup): workgroup (x, y) is number x of the `fixed_split`
+// workgroups of head y, and the head's tiles go round its wavefronts.  For calls in which a wavefront has a tile or
+// two, the time is the chain of dependent trips to memory before the first of them: here one (the head's end; then
+// valid bytes, K, V and Q are requested together) instead of the schedule's scans, the head's end again and the valid
+// bytes; and partial results lie where the merge kernel knows them (or nowhere: with one workgroup per head it writes
+// the output itself).  See fixed_schedule for where the line lies.
+template <int D, int NREP, int FIXED>
+__global__ __launch_bounds__(FIXED ? FIXED * kWave : 256) void decode_split_mfma_kernel(DecodeArgs a) {
+  constexpr int WAVES = FIXED ? FIXED : 4;
+  constexpr int THREADS = WAVES * kWave;
   constexpr int STEPS = D / 32;      // k-steps of the score MFMA
   constexpr int OCT = D / 8;         // 16-byte chunks per row
   constexpr int NDMA = kDecTile * OCT / kWave;  // 1 KiB transfers per V tile
@@ -121,7 +134,8 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
   auto v_swz = [](int row) { return OCT >= 8 ? (row & 3) << 1 : (row >> 2) & 3; };
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  DecodeSmem<D, NREP>& sm = *reinterpret_cast<DecodeSmem<D, NREP>*>(smem_raw);
+  DecodeTiles<D, NREP, WAVES>& sm = *reinterpret_cast<DecodeTiles<D, NREP, WAVES>*>(smem_raw);
+  DecodeSchedule& sched = *reinterpret_cast<DecodeSchedule*>(smem_raw + sizeof(DecodeTiles<D, NREP, WAVES>));  // (balanced only)
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -135,39 +149,44 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
   const int tail_tiles = (a.n_rows - ts + kDecTile - 1) / kDecTile;
 
   // ---- schedule: tiles per head, their prefix sums, this workgroup's range ----------------------------
-  for (int h = tid; h < n_heads; h += 256) {
-    int e = a.row_end ? (int)min((long long)a.row_end[h], (long long)ts) : a.n_rows;
-    sm.tile_prefix[h] = (e + kDecTile - 1) / kDecTile + tail_tiles;
-  }
-  __syncthreads();
-  block_exclusive_scan(sm.tile_prefix, n_heads, sm.scan_tmp);
-  const int total = sm.tile_prefix[n_heads];
-  // Tiles per workgroup: tpw_a for the first n_first workgroups (tiles [0, split)), tpw_b for the others.
-  const int n_first = a.share_first == 128 ? a.n_wg : a.n_wg / 2;
-  const int tpw_a = a.share_first == 128 ? (total + a.n_wg - 1) / a.n_wg
-                                         : max(1, (int)(((int64_t)total * a.share_first / 256 + n_first - 1) / n_first));
-  const int split = min(total, n_first * tpw_a);
-  const int tpw_b = max(1, (total - split + (a.n_wg - n_first) - 1) / max(1, a.n_wg - n_first));
+  int pos = 0, pos_end = 0, ks = 0, n_first = 0, tpw_a = 1, tpw_b = 1, split = 0;
   auto wg_of = [&](int p) { return p < split ? p / tpw_a : n_first + (p - split) / tpw_b; };
-  for (int h = tid; h < n_heads; h += 256) {
-    int p0 = sm.tile_prefix[h], p1 = sm.tile_prefix[h + 1];
-    sm.slot_prefix[h] = p1 > p0 ? wg_of(p1 - 1) - wg_of(p0) + 1 : 0;
-  }
-  __syncthreads();
-  block_exclusive_scan(sm.slot_prefix, n_heads, sm.scan_tmp);
-  if (wg == 0 && grp == 0) {
+  if constexpr (FIXED) {
+    ks = blockIdx.y;
+  } else {
     for (int h = tid; h < n_heads; h += 256) {
-      a.head_table[h] = make_int2(sm.slot_prefix[h], sm.slot_prefix[h + 1] - sm.slot_prefix[h]);
+      int e = a.row_end ? (int)min((long long)a.row_end[h], (long long)ts) : a.n_rows;
+      sched.tile_prefix[h] = (e + kDecTile - 1) / kDecTile + tail_tiles;
     }
+    __syncthreads();
+    block_exclusive_scan(sched.tile_prefix, n_heads, sched.scan_tmp);
+    const int total = sched.tile_prefix[n_heads];
+    // Tiles per workgroup: tpw_a for the first n_first workgroups (tiles [0, split)), tpw_b for the others.
+    n_first = a.share_first == 128 ? a.n_wg : a.n_wg / 2;
+    tpw_a = a.share_first == 128 ? (total + a.n_wg - 1) / a.n_wg
+                                           : max(1, (int)(((int64_t)total * a.share_first / 256 + n_first - 1) / n_first));
+    split = min(total, n_first * tpw_a);
+    tpw_b = max(1, (total - split + (a.n_wg - n_first) - 1) / max(1, a.n_wg - n_first));
+    for (int h = tid; h < n_heads; h += 256) {
+      int p0 = sched.tile_prefix[h], p1 = sched.tile_prefix[h + 1];
+      sched.slot_prefix[h] = p1 > p0 ? wg_of(p1 - 1) - wg_of(p0) + 1 : 0;
+    }
+    __syncthreads();
+    block_exclusive_scan(sched.slot_prefix, n_heads, sched.scan_tmp);
+    if (wg == 0 && grp == 0) {
+      for (int h = tid; h < n_heads; h += 256) {
+        a.head_table[h] = make_int2(sched.slot_prefix[h], sched.slot_prefix[h + 1] - sched.slot_prefix[h]);
+      }
+    }
+    pos = wg < n_first ? wg * tpw_a : split + (wg - n_first) * tpw_b;
+    pos_end = wg < n_first ? min(pos + tpw_a, split) : min(pos + tpw_b, total);
+    if (pos >= pos_end) return;
+    for (int h = tid; h < n_heads; h += 256) {
+      if (sched.tile_prefix[h] <= pos && pos < sched.tile_prefix[h + 1]) sched.first_head = h;
+    }
+    __syncthreads();
+    ks = sched.first_head;  // b * Hkv + hkv
   }
-  int pos = wg < n_first ? wg * tpw_a : split + (wg - n_first) * tpw_b;
-  const int pos_end = wg < n_first ? min(pos + tpw_a, split) : min(pos + tpw_b, total);
-  if (pos >= pos_end) return;
-  for (int h = tid; h < n_heads; h += 256) {
-    if (sm.tile_prefix[h] <= pos && pos < sm.tile_prefix[h + 1]) sm.first_head = h;
-  }
-  __syncthreads();
-  int ks = sm.first_head;  // b * Hkv + hkv
   const float c = a.scale * 1.4426950408889634f;
 
   const int nr = min(NREP, a.n_rep - grp * NREP);  // q heads of this group (the last group may hold fewer)
@@ -228,12 +247,18 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
   // Moves on to the head that holds tile `pos` of the list (`ks` is that head or an empty one before it): its
   // pointers and ranges, Q, and the requests for this wavefront's first tile, into LDS buffer `buf`.  Returns the
   // end of the workgroup's tiles in that head, as a list position.
+  const int tstep = FIXED ? WAVES * a.fixed_split : WAVES;  // a wavefront's next tile
   auto begin_head = [&](int buf) -> int {
-    while (sm.tile_prefix[ks + 1] == sm.tile_prefix[ks]) ++ks;  // heads without tiles (pos < total: one with tiles follows)
-    const int p0 = sm.tile_prefix[ks], p1 = sm.tile_prefix[ks + 1];
-    const int seg_end = min(pos_end, p1);
-    t_end = seg_end - p0;
-    slot = sm.slot_prefix[ks] + (wg - wg_of(p0));
+    int p0 = 0, seg_end = 0;
+    if constexpr (FIXED) {
+      slot = ks * a.fixed_split + wg;
+    } else {
+      while (sched.tile_prefix[ks + 1] == sched.tile_prefix[ks]) ++ks;  // heads without tiles (pos < total: one with tiles follows)
+      p0 = sched.tile_prefix[ks];
+      seg_end = min(pos_end, sched.tile_prefix[ks + 1]);
+      t_end = seg_end - p0;
+      slot = sched.slot_prefix[ks] + (wg - wg_of(p0));
+    }
     const int b = ks / a.Hkv, hkv = ks % a.Hkv;
     const int hq0 = hkv * a.n_rep + grp * NREP;
     kp = static_cast<const uint16_t*>(a.k) + b * a.ks_b + hkv * a.ks_h;
@@ -241,6 +266,7 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
     valp = a.valid + b * a.vs_b + hkv * a.vs_h;
     e = a.row_end ? (int)min((long long)a.row_end[ks], (long long)ts) : a.n_rows;
     nA = (e + kDecTile - 1) / kDecTile;
+    if constexpr (FIXED) t_end = nA + tail_tiles;
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + ((int64_t)b * a.Hq + hq0 + (l16 < nr ? l16 : 0)) * D;
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
@@ -248,14 +274,38 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
       if (l16 >= nr) raw = make_uint4(0, 0, 0, 0);
       qreg[s] = __builtin_bit_cast(bf16x8, raw);
     }
-    t = pos - p0 + wave;
     cur = buf;
-    vm = (uint32_t)__ballot(load_valid(t) != 0);
-    if (vm) {
-      issue_k(tile_row0(t), vm);
-      issue_v(tile_row0(t), vm, cur);
+    if constexpr (FIXED) {
+      // the first tile's rows are requested together with their valid bytes: rows that turn out not to be valid are
+      // masked in the scores and set to zero in the V tile
+      t = wg * WAVES + wave;
+      const uint32_t vb = load_valid(t);
+      uint32_t rows = 0;
+      if (t < t_end) {
+        const int n = tile_row1(t) - tile_row0(t);
+        rows = n >= 32 ? 0xffffffffu : (1u << n) - 1;
+        issue_k(tile_row0(t), rows);
+        issue_v(tile_row0(t), rows, cur);
+      }
+      vb_next = load_valid(t + tstep);
+      __builtin_amdgcn_s_waitcnt(0);
+      vm = (uint32_t)__ballot(vb != 0);
+      if (vm != rows) {
+#pragma unroll
+        for (int j = 0; j < NDMA; ++j) {
+          const int q = j * kWave + lane;
+          if (!((vm >> (q / OCT)) & 1)) *reinterpret_cast<uint4*>(&sm.v[wave][cur][q * 8]) = make_uint4(0, 0, 0, 0);
+        }
+      }
+    } else {
+      t = pos - p0 + wave;
+      vm = (uint32_t)__ballot(load_valid(t) != 0);
+      if (vm) {
+        issue_k(tile_row0(t), vm);
+        issue_v(tile_row0(t), vm, cur);
+      }
+      vb_next = load_valid(t + tstep);
     }
-    vb_next = load_valid(t + 4);
     return seg_end;
   };
 
@@ -291,10 +341,10 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
       }
       // requests for the next tile go out before this tile's softmax and PV
       if (vmn) {
-        issue_k(tile_row0(t + 4), vmn);
-        issue_v(tile_row0(t + 4), vmn, cur ^ 1);
+        issue_k(tile_row0(t + tstep), vmn);
+        issue_v(tile_row0(t + tstep), vmn, cur ^ 1);
       }
-      vb_next = load_valid(t + 8);
+      vb_next = load_valid(t + 2 * tstep);
 
       if (vm) {
         mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -341,7 +391,7 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
           oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pfrag, oacc[db], 0, 0, 0);
         }
       }
-      t += 4;
+      t += tstep;
       vm = vmn;
       cur ^= 1;
     }
@@ -366,23 +416,30 @@ __global__ __launch_bounds__(256) void decode_split_mfma_kernel(DecodeArgs a) {
     }
     const int slot_done = slot;
     pos = seg_end;
-    const bool more = pos < pos_end;  // (the same for every wavefront of the workgroup)
+    const bool more = !FIXED && pos < pos_end;  // (the same for every wavefront of the workgroup)
     if (more) {
       ++ks;
       seg_end = begin_head(1);
     }
     __syncthreads();
-    for (int idx = tid; idx < nr * D; idx += 256) {
+    for (int idx = tid; idx < nr * D; idx += THREADS) {
       int h = idx / D, d = idx % D;
-      float M = fmaxf(fmaxf(sm.wm[0][h], sm.wm[1][h]), fmaxf(sm.wm[2][h], sm.wm[3][h]));
+      float M = sm.wm[0][h];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) M = fmaxf(M, sm.wm[w][h]);
       float sum = 0.f, lsum = 0.f;
       if (M != -INFINITY) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < WAVES; ++w) {
           float f = exp2_guard(sm.wm[w][h] - M);
           sum += reinterpret_cast<const float*>(&sm.v[w][0][0])[h * D + d] * f;
           lsum += sm.wl[w][h] * f;
         }
+      }
+      if (FIXED && a.fixed_split == 1) {  // the whole head: the output itself
+        const int64_t head = (int64_t)(ks / a.Hkv) * a.Hq + (ks % a.Hkv) * a.n_rep + grp * NREP + h;
+        static_cast<uint16_t*>(a.o)[head * D + d] = f32_to_bf16_bits(lsum > 0.f ? sum / lsum : 0.f);
+        continue;
       }
       const int64_t prt = (int64_t)slot_done * a.n_rep + grp * NREP + h;  // partial of (slot, q head in the kv group)
       a.ws_acc[prt * D + d] = sum;
@@ -467,6 +524,47 @@ __global__ void decode_merge_balanced_kernel(const float* __restrict__ ws_acc, c
     for (int k = 1; k < G; ++k) sum += part[k * D + d];
   } else if (g != 0) {
     return;
+  }
+  o[(int64_t)head * D + d] = f32_to_bf16_bits(lsum > 0.f ? sum / lsum : 0.f);
+}
+
+// merge the partials of one q head of the fixed schedule: grid = B*Hq, block = G * D threads.  The n <= 64 partials of a head
+// lie side by side, so everything is requested at once: every wavefront reads the maxima and row sums of all of them (lane s
+// those of partial s, no barrier), thread (g, d) the accumulators of the partials g, g + G, ...  (at most kFixedPerGroup).
+constexpr int kFixedPerGroup = 8;
+constexpr int kFixedMaxSplit = 64;
+__global__ void decode_merge_fixed_kernel(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
+                                          uint16_t* __restrict__ o, int Hq, int Hkv, int D, int n) {
+  extern __shared__ float part[];  // [G][D]
+  const int head = blockIdx.x;  // b * Hq + hq
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int n_rep = Hq / Hkv;
+  const int64_t first = (int64_t)(head / n_rep) * n * n_rep + head % n_rep;  // (head / n_rep = b * Hkv + hkv)
+  const int G = blockDim.x / D, g = tid / D, d = tid % D;
+  float2 ml = make_float2(-INFINITY, 0.f);
+  if (lane < n) ml = *reinterpret_cast<const float2*>(ws_ml + (first + (int64_t)lane * n_rep) * 2);
+  float acc[kFixedPerGroup];
+#pragma unroll
+  for (int j = 0; j < kFixedPerGroup; ++j) {
+    const int s = g + j * G;
+    acc[j] = s < n ? ws_acc[(first + (int64_t)s * n_rep) * D + d] : 0.f;
+  }
+  float M = ml.x;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
+  const float f = ml.x == -INFINITY ? 0.f : exp2_guard(ml.x - M);
+  float lsum = ml.y * f;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) lsum += __shfl_xor(lsum, off);
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < kFixedPerGroup; ++j) sum = fmaf(acc[j], __shfl(f, min(g + j * G, kWave - 1)), sum);
+  if (G > 1) {
+    part[g * D + d] = sum;
+    __syncthreads();
+    if (g != 0) return;
+    sum = part[d];
+    for (int k = 1; k < G; ++k) sum += part[k * D + d];
   }
   o[(int64_t)head * D + d] = f32_to_bf16_bits(lsum > 0.f ? sum / lsum : 0.f);
 }
@@ -631,21 +729,76 @@ static int decode_share_first(int n_wg, int groups) {
 
 static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-template <int D, int NREP>
-static int launch_mfma(const DecodeArgs& a, int groups, hipStream_t st) {
+template <int D, int NREP, int FIXED>
+static int launch_mfma_as(const DecodeArgs& a, int groups, hipStream_t st) {
   static bool configured[64] = {};  // per instantiation; the LDS attribute is set once per device
-  const size_t smem = sizeof(DecodeSmem<D, NREP>);
+  const size_t smem = sizeof(DecodeTiles<D, NREP, FIXED ? FIXED : 4>) + (FIXED ? 0 : sizeof(DecodeSchedule));
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(NATS_ERR_LAUNCH, "decode: no current device");
   if (!configured[dev]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_split_mfma_kernel<D, NREP>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_split_mfma_kernel<D, NREP, FIXED>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return fail(NATS_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS): %s", smem, hipGetErrorString(e));
     configured[dev] = true;
   }
-  dim3 grid((unsigned)a.n_wg, 1u, (unsigned)groups);
-  hipLaunchKernelGGL((decode_split_mfma_kernel<D, NREP>), grid, dim3(256), smem, st, a);
+  const dim3 grid = FIXED ? dim3((unsigned)a.fixed_split, (unsigned)(a.B * a.Hkv), (unsigned)groups) : dim3((unsigned)a.n_wg, 1u, (unsigned)groups);
+  hipLaunchKernelGGL((decode_split_mfma_kernel<D, NREP, FIXED>), grid, dim3(FIXED ? FIXED * kWave : 256), smem, st, a);
   return NATS_OK;
+}
+// waves: 0 = the balanced schedule, else the fixed one with that many wavefronts per workgroup
+template <int D, int NREP>
+static int launch_mfma(const DecodeArgs& a, int groups, int waves, hipStream_t st) {
+  if (waves == 0) return launch_mfma_as<D, NREP, 0>(a, groups, st);
+  if constexpr (D < 256) {  // (the V tiles of eight wavefronts at head dim 256 do not fit LDS)
+    if (waves == 8) return launch_mfma_as<D, NREP, 8>(a, groups, st);
+  }
+  return launch_mfma_as<D, NREP, 4>(a, groups, st);
+}
+template <int D>
+static int launch_mfma_by_rep(const DecodeArgs& a, int nrep_k, int groups, int waves, hipStream_t st) {
+  switch (nrep_k) {
+    case 8: return launch_mfma<D, 8>(a, groups, waves, st);
+    case 4: return launch_mfma<D, 4>(a, groups, waves, st);
+    case 2: return launch_mfma<D, 2>(a, groups, waves, st);
+    default: return launch_mfma<D, 1>(a, groups, waves, st);
+  }
+}
+static int launch_mfma_by_dim(const DecodeArgs& a, int64_t D, int nrep_k, int groups, int waves, hipStream_t st) {
+  switch (D) {
+    case 128: return launch_mfma_by_rep<128>(a, nrep_k, groups, waves, st);
+    case 256: return launch_mfma_by_rep<256>(a, nrep_k, groups, waves, st);
+    case 32: return launch_mfma_by_rep<32>(a, nrep_k, groups, waves, st);
+    default: return launch_mfma_by_rep<64>(a, nrep_k, groups, waves, st);
+  }
+}
+
+// q heads of a kv head share the key / value rows of one pass, up to eight at a time (columns of the MFMA); a group
+// size that is no power of two runs the next wider kernel with its spare columns zero
+static int decode_rep_columns(int64_t n_rep) { return n_rep >= 5 ? 8 : n_rep >= 3 ? 4 : (int)n_rep; }
+
+// The fixed schedule: workgroups per head and wavefronts per workgroup (0: the balanced schedule).  Figures: GPU time of
+// the whole op, 8 kv heads of 4 q heads, head dim 128, heads that have kept 10-30 % of the context, balanced / fixed.
+//   * up to four tiles per wavefront of the longest head: two workgroups per compute unit, four wavefronts each, and the
+//     merge kernel (batch 1, contexts 2k / 16k / 64k: 13.3 / 8.1, 15.9 / 11.5, 21.7 / 19.4 us; batch 4 at 8k 18.8 / 15.4;
+//     batch 16 at 2k 19.4 / 16.0).  With more tiles the heads' unequal lengths decide, which the balanced schedule evens
+//     out, and the two meet (batch 1 at 128k 29.3 / 28.7, batch 8 at 16k 29.0 / 29.5).
+//   * one workgroup of eight wavefronts per head, which writes the output itself, when that fills at least half of the
+//     compute units and a wavefront has four tiles at most (two, for half of the units): batch 32 at contexts 512 / 2k 20.8 /
+//     12.0, 25.3 / 21.0 us (16.2 and 24.0 with four wavefronts and the merge kernel), batch 16 at 512 15.8 / 11.0.
+struct FixedSchedule {
+  int split, waves;
+};
+static FixedSchedule fixed_schedule(int64_t B, int64_t H_kv, int64_t n_rep, int64_t D, int64_t n_rows) {
+  const int64_t nrep_k = decode_rep_columns(n_rep);
+  const int64_t heads = B * H_kv * ((n_rep + nrep_k - 1) / nrep_k);
+  const int64_t tiles = (n_rows + kDecTile - 1) / kDecTile + 1;  // of one head, at most
+  const int64_t n_cu = compute_units_of_current_device();
+  if (D < 256 && heads <= n_cu && heads * 2 >= n_cu && tiles * n_cu <= 32 * heads) return {1, 8};
+  int64_t split = (D == 256 ? 1 : 2) * n_cu / heads;  // (the V tiles of a workgroup at head dim 256 are 128 KB of LDS)
+  split = std::min<int64_t>({split, (tiles + 3) / 4, kFixedMaxSplit, kFixedPerGroup * (1024 / D)});
+  if (split < 1) split = 1;
+  if (tiles > 4 * 4 * split) return {0, 0};
+  return {(int)split, 4};
 }
 
 }  // namespace nats
@@ -658,6 +811,8 @@ extern "C" size_t nats_decode_workspace_bytes(int64_t B, int64_t H_q, int64_t H_
   decode_split_geometry(B, H_kv, n_rows, &rps, &ns);
   size_t split_layout = (size_t)B * H_q * ns * (D + 2) * sizeof(float);  // fp32 kernel: [q head][split]
   size_t slots = (size_t)decode_balanced_workgroups(B, H_kv, n_rows) + (size_t)(B * H_kv);
+  const FixedSchedule fixed = fixed_schedule(B, H_kv, H_q / H_kv, D, n_rows);
+  if (fixed.split) slots = (size_t)(B * H_kv) * fixed.split;
   size_t balanced_layout = align256((size_t)(B * H_kv) * sizeof(int2)) + slots * (H_q / H_kv) * (D + 2) * sizeof(float);
   return split_layout > balanced_layout ? split_layout : balanced_layout;
 }
@@ -712,6 +867,7 @@ static int decode_fwd_impl(const void* q, const void* cache_k, const void* cache
   decode_split_geometry(B, H_kv, n_rows, &a.rows_per_split, &a.nsplit);
   a.scale = sm_scale;
   a.head_table = nullptr;
+  a.fixed_split = 0;
   a.n_wg = 0;
   a.share_first = 128;
   a.ws_acc = static_cast<float*>(workspace);
@@ -752,14 +908,28 @@ static int decode_fwd_impl(const void* q, const void* cache_k, const void* cache
   NATS_REQUIRE(H_kv <= kMaxBalancedHeads, NATS_ERR_UNSUPPORTED,
                "nats_decode_fwd: %lld kv heads, the bf16 kernel schedules at most %d per sequence", (long long)H_kv,
                kMaxBalancedHeads);
+  const int n_rep = a.n_rep;
+  const int nrep_k = decode_rep_columns(n_rep);
+  const int groups = (n_rep + nrep_k - 1) / nrep_k;
+  const FixedSchedule fixed = fixed_schedule(B, H_kv, n_rep, D, n_rows);
+  if (fixed.split) {
+    a.fixed_split = fixed.split;
+    a.ws_ml = a.ws_acc + (size_t)(B * H_q) * fixed.split * D;
+    if (int rc = launch_mfma_by_dim(a, D, nrep_k, groups, fixed.waves, st)) return rc;
+    NATS_CHECK_LAUNCH("decode_split_mfma_kernel");
+    if (fixed.split > 1) {
+      const int merge_groups = (fixed.split + kFixedPerGroup - 1) / kFixedPerGroup;
+      // (fixed_schedule keeps G * D within 1024 threads)
+      hipLaunchKernelGGL(decode_merge_fixed_kernel, dim3((unsigned)(B * H_q)), dim3((unsigned)(merge_groups * D)),
+                         merge_groups * D * sizeof(float), st, a.ws_acc, a.ws_ml, static_cast<uint16_t*>(o), (int)H_q, (int)H_kv, (int)D,
+                         fixed.split);
+      NATS_CHECK_LAUNCH("decode_merge_fixed_kernel");
+    }
+    return NATS_OK;
+  }
   // One launch pair schedules at most kMaxBalancedHeads (b, kv head) streams (their prefix sums live in LDS); a
   // larger batch goes in groups of whole sequences, one after the other on the stream, over the same workspace.
   const int64_t b_step = kMaxBalancedHeads / H_kv;
-  const int n_rep = a.n_rep;
-  // q heads of a kv head share the key / value rows of one pass, up to eight at a time (columns of the MFMA);
-  // a group size that is no power of two runs the next wider kernel with its spare columns zero
-  const int nrep_k = n_rep >= 5 ? 8 : n_rep >= 3 ? 4 : n_rep;
-  const int groups = (n_rep + nrep_k - 1) / nrep_k;
   for (int64_t b0 = 0; b0 < B; b0 += b_step) {
     const int64_t nb = B - b0 < b_step ? B - b0 : b_step;
     DecodeArgs c = a;
@@ -774,42 +944,11 @@ static int decode_fwd_impl(const void* q, const void* cache_k, const void* cache
     // (rows of 512 bytes: a workgroup's V buffers take 128 KB of LDS, so one workgroup fits a compute unit at a time; one
     // round of workgroups with equal shares measures 1 % faster than two)
     if (D == 256) c.n_wg = std::min(c.n_wg, compute_units_of_current_device());
-    c.share_first = decode_share_first(c.n_wg, groups);
+    c.share_first = D == 256 ? 128 : decode_share_first(c.n_wg, groups);
     c.head_table = static_cast<int2*>(workspace);
     c.ws_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256((size_t)(nb * H_kv) * sizeof(int2)));
     c.ws_ml = c.ws_acc + ((size_t)c.n_wg + (size_t)(nb * H_kv)) * (size_t)n_rep * D;
-    int rc;
-    if (D == 128) {
-      switch (nrep_k) {
-        case 8: rc = launch_mfma<128, 8>(c, groups, st); break;
-        case 4: rc = launch_mfma<128, 4>(c, groups, st); break;
-        case 2: rc = launch_mfma<128, 2>(c, groups, st); break;
-        default: rc = launch_mfma<128, 1>(c, groups, st); break;
-      }
-    } else if (D == 256) {
-      c.share_first = 128;
-      switch (nrep_k) {
-        case 8: rc = launch_mfma<256, 8>(c, groups, st); break;
-        case 4: rc = launch_mfma<256, 4>(c, groups, st); break;
-        case 2: rc = launch_mfma<256, 2>(c, groups, st); break;
-        default: rc = launch_mfma<256, 1>(c, groups, st); break;
-      }
-    } else if (D == 32) {
-      switch (nrep_k) {
-        case 8: rc = launch_mfma<32, 8>(c, groups, st); break;
-        case 4: rc = launch_mfma<32, 4>(c, groups, st); break;
-        case 2: rc = launch_mfma<32, 2>(c, groups, st); break;
-        default: rc = launch_mfma<32, 1>(c, groups, st); break;
-      }
-    } else {
-      switch (nrep_k) {
-        case 8: rc = launch_mfma<64, 8>(c, groups, st); break;
-        case 4: rc = launch_mfma<64, 4>(c, groups, st); break;
-        case 2: rc = launch_mfma<64, 2>(c, groups, st); break;
-        default: rc = launch_mfma<64, 1>(c, groups, st); break;
-      }
-    }
-    if (rc) return rc;
+    if (int rc = launch_mfma_by_dim(c, D, nrep_k, groups, 0, st)) return rc;
     NATS_CHECK_LAUNCH("decode_split_mfma_kernel");
     // (a head has at most one partial per workgroup plus one)
     // groups of the merge kernel's block: about four partials per group and head
