@@ -51,8 +51,10 @@ struct AddNormArgs {
   float eps, chunk;
 };
 
-// One workgroup of 256 threads per row; the row is kept in registers between the two passes.  VEC consecutive
-// columns per thread and step: 8 (16-byte loads of bf16, two 16-byte loads of fp32) when dim % 8 == 0, else 1.
+// One workgroup per row; the row is kept in registers between the two passes.  VEC consecutive columns per thread and
+// step: 8 (16-byte loads of bf16, two 16-byte loads of fp32) when dim % 8 == 0, else 1.  Bound by one trip to memory and
+// the launch: a row is one step of as many threads as it takes (dim / 8), so that every load of the row leaves at once
+// (one row with delta and chunk statistic: dim 4096 7.1 -> 5.0 us, 8192 12.3 -> 6.5 us against 256 threads that walk the row).
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxDim = 8192;
 
@@ -91,28 +93,33 @@ __device__ __forceinline__ void store_vec(void* p, int64_t i, const float (&v)[V
   }
 }
 
-template <bool kBf16, int VEC>
-__global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(AddNormArgs a) {
-  constexpr int STEPS = kNormMaxDim / (kNormThreads * VEC);
-  __shared__ float part[kNormThreads / kWave];
+template <bool kBf16, int VEC, int THREADS, int STEPS>
+__global__ __launch_bounds__(THREADS) void add_rms_norm_kernel(AddNormArgs a) {
+  __shared__ float part[THREADS / kWave];
   const int64_t base = (int64_t)blockIdx.x * a.dim;
   const int tid = threadIdx.x;
-  float v[STEPS][VEC], wv[STEPS][VEC], cv[STEPS][VEC];
+  float v[STEPS][VEC], dv[STEPS][VEC], wv[STEPS][VEC], cv[STEPS][VEC];
   const bool carry_read = a.carry_mode == 2 || a.carry_mode == 4;
   float ss = 0.f;
+  // (everything a thread needs is requested before anything is stored: the stores to x may alias the loads for all the
+  // compiler knows, and a load behind one would wait for the step before it)
 #pragma unroll
   for (int j = 0; j < STEPS; ++j) {
-    const int c = (j * kNormThreads + tid) * VEC;
+    const int c = (j * THREADS + tid) * VEC;
     if (c < a.dim) {
       load_vec<kBf16, VEC>(a.x, base + c, v[j]);
-      // (what the second pass needs is requested now, so that it does not wait for memory again)
+      if (a.delta) load_vec<kBf16, VEC>(a.delta, base + c, dv[j]);
       load_vec<kBf16, VEC>(a.weight, c, wv[j]);
       if (carry_read) load_vec<kBf16, VEC>(a.carry, base + c, cv[j]);
-      if (a.delta) {
-        float d[VEC];
-        load_vec<kBf16, VEC>(a.delta, base + c, d);
+    }
+  }
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) v[j][e] = g_round<kBf16>(v[j][e] + d[e]);
+  for (int j = 0; j < STEPS; ++j) {
+    const int c = (j * THREADS + tid) * VEC;
+    if (c < a.dim) {
+      if (a.delta) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[j][e] = g_round<kBf16>(v[j][e] + dv[j][e]);
         store_vec<kBf16, VEC>(a.x, base + c, v[j]);
       }
 #pragma unroll
@@ -125,11 +132,11 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(AddNormArgs 
   __syncthreads();
   float tot = 0.f;
 #pragma unroll
-  for (int w = 0; w < kNormThreads / kWave; ++w) tot += part[w];
+  for (int w = 0; w < THREADS / kWave; ++w) tot += part[w];
   const float r = rsqrtf(tot / (float)a.dim + a.eps);
 #pragma unroll
   for (int j = 0; j < STEPS; ++j) {
-    const int c = (j * kNormThreads + tid) * VEC;
+    const int c = (j * THREADS + tid) * VEC;
     if (c < a.dim) {
       float h[VEC];
 #pragma unroll
@@ -435,20 +442,25 @@ extern "C" int nats_add_rms_norm(void* x, const void* delta, const void* weight,
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto aligned16 = [](const void* p) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = dim % 8 == 0 && aligned16(x) && aligned16(delta) && aligned16(weight) && aligned16(out) && aligned16(carry);
-  const dim3 grid((unsigned)rows), block(kNormThreads);
-  if (dtype == NATS_DTYPE_BF16) {
-    if (vec) {
-      hipLaunchKernelGGL((add_rms_norm_kernel<true, 8>), grid, block, 0, st, a);
-    } else {
-      hipLaunchKernelGGL((add_rms_norm_kernel<true, 1>), grid, block, 0, st, a);
-    }
-  } else {
-    if (vec) {
-      hipLaunchKernelGGL((add_rms_norm_kernel<false, 8>), grid, block, 0, st, a);
-    } else {
-      hipLaunchKernelGGL((add_rms_norm_kernel<false, 1>), grid, block, 0, st, a);
-    }
+  const dim3 grid((unsigned)rows);
+#define NATS_NORM(BF, VEC, THREADS, STEPS) hipLaunchKernelGGL((add_rms_norm_kernel<BF, VEC, THREADS, STEPS>), grid, dim3(THREADS), 0, st, a)
+#define NATS_NORM_DIM(BF)                                       \
+  if (!vec) {                                                   \
+    NATS_NORM(BF, 1, kNormThreads, kNormMaxDim / kNormThreads); \
+  } else if (dim <= 2048) {                                     \
+    NATS_NORM(BF, 8, 256, 1);                                   \
+  } else if (dim <= 4096) {                                     \
+    NATS_NORM(BF, 8, 512, 1);                                   \
+  } else {                                                      \
+    NATS_NORM(BF, 8, 1024, 1);                                  \
   }
+  if (dtype == NATS_DTYPE_BF16) {
+    NATS_NORM_DIM(true)
+  } else {
+    NATS_NORM_DIM(false)
+  }
+#undef NATS_NORM_DIM
+#undef NATS_NORM
   NATS_CHECK_LAUNCH("add_rms_norm_kernel");
   return NATS_OK;
 }
