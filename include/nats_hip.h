@@ -395,6 +395,23 @@ int nats_silu_mul(const void* gate_up, void* out, int64_t rows, int64_t inter, i
 int nats_matvec(const void* w, const void* x, void* y, int64_t x_rows, int64_t n_out, int64_t k, int64_t w_stride,
                 int64_t x_stride, int64_t y_stride, int gate, int dtype, void* stream);
 
+/* What a one-token step of an attention module needs from its hidden states, in one launch
+ * (models/transformer/attention/base_attention.py:139-151, nats_chunk_attention.py:64-95, nats_attention.py:96-109,
+ * components/cache/dyn_cache.py:98-171), for 1..4 rows of x:
+ *   y [x_rows, y_stride]: the products of x with n_mats (1..4) matrices w[i] [n_out[i], k], side by side, each as
+ *     nats_matvec computes it
+ *   the mean statistic s = carry_in + x / chunk_size (x / chunk_size without carry_in; every operation rounded to the
+ *     dtype), written to carry_out if that is given
+ *   if roles is given: the role of every (row, kv head) from s and the role matrix role_w [H_kv * 3, k] (contiguous), as
+ *     nats_roles_from_logits assigns it, at roles[(row * H_kv + head) * roles_hs]
+ *   x, carry_in, carry_out [x_rows, k] contiguous; carry_out may not be carry_in while roles are asked for
+ *   k a multiple of 16 bytes, every matrix row, x and the statistics 16-byte aligned
+ */
+int nats_step_project(const void* x, int64_t x_rows, int64_t k, int64_t n_mats, const void* const* w, const int64_t* n_out,
+                      const int64_t* w_strides, void* y, int64_t y_stride, const void* role_w, int64_t H_kv,
+                      float global_bias, int force_first_global, uint8_t* roles, int64_t roles_hs, const void* carry_in,
+                      void* carry_out, int64_t chunk_size, int dtype, void* stream);
+
 /* Rotary embedding of q and k of a multi-token segment (transformers' apply_rotary_pos_emb as called at
  * hf/llama_nats_chunk.py:227: q * cos + rotate_half(q) * sin, every product and the sum rounded to the dtype):
  *   q_out [B, H_q, x_len, D] and k_out [B, H_kv, x_len, D] contiguous

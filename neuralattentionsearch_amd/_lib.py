@@ -83,6 +83,8 @@ SIGNATURES = {
                                          ctypes.c_int, c_p]),
     "nats_silu_mul": (ctypes.c_int, [c_p, c_p, c_i64, c_i64, ctypes.c_int, c_p]),
     "nats_matvec": (ctypes.c_int, [c_p, c_p, c_p] + [c_i64] * 6 + [ctypes.c_int, ctypes.c_int, c_p]),
+    "nats_step_project": (ctypes.c_int, [c_p, c_i64, c_i64, c_i64, ctypes.POINTER(c_p), c_i64p, c_i64p, c_p, c_i64, c_p, c_i64,
+                                         ctypes.c_float, ctypes.c_int, c_p, c_i64, c_p, c_p, c_i64, ctypes.c_int, c_p]),
     "nats_rope_qk": (ctypes.c_int, [c_p] * 6 + [c_i64] * 5 + [c_i64p] * 3 + [ctypes.c_int, c_p]),
     "nats_rope_append": (ctypes.c_int, [c_p] * 10 + [c_i64] * 9 + [c_i64p] * 6 + [ctypes.c_int, c_p]),
 }

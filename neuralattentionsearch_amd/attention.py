@@ -19,7 +19,7 @@ import torch
 from torch import nn
 
 from . import ops
-from .cache import ChunkMergeType, NAtSCache
+from .cache import ChunkMergeType, NAtSCache, NAtSChunkLayerCache, NAtSLayerCache
 
 
 def rotate_half(x: torch.Tensor) -> torch.Tensor:
@@ -33,6 +33,22 @@ def apply_rotary_pos_emb(q, k, cos, sin, unsqueeze_dim: int = 1):
     cos = cos.unsqueeze(unsqueeze_dim)
     sin = sin.unsqueeze(unsqueeze_dim)
     return (q * cos) + (rotate_half(q) * sin), (k * cos) + (rotate_half(k) * sin)
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """An nn.Linear without bias that nobody has wrapped, hooked or re-parametrised: its call is one matrix product."""
+    return (type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and "forward" not in m.__dict__ and m.bias is None and type(m.weight) is nn.Parameter)
+
+
+def _plain_execution(x: torch.Tensor, weights) -> bool:
+    """Whether a call may be replaced by kernels on raw addresses: nothing records, transforms or traces the torch ops that
+    would run in their place (autograd, forward-mode, vmap, autocast, dispatch and function modes, global module hooks)."""
+    return (type(x) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and not (torch.is_grad_enabled() and (x.requires_grad or any(w.requires_grad for w in weights)))
+            and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled("cuda")
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not torch.compiler.is_compiling() and not nn.modules.module._has_any_global_hook())
 
 
 class AttentionLayer(nn.Module):
@@ -64,11 +80,18 @@ class AttentionLayer(nn.Module):
     def repeat_kv_values(self, keys, values):
         return keys, values
 
+    def _one_token_step(self, x: torch.Tensor, pos_emb, start_pos: int, cache):
+        """The whole forward of one token over a filled cache in a few launches, or None when `forward` has to take its
+        general way."""
+        return None
+
     def forward(self, x: torch.Tensor, pos_emb, mask, start_pos: int = 0, cache: NAtSCache | None = None, **kwargs):
         """[B, L, dim] -> [B, L, dim] (base_attention.py:259-283)."""
         if self.training:
             raise NotImplementedError("only the inference path is built; call module.eval()")
         bsz, seqlen, _ = x.shape
+        if seqlen == 1 and (step := self._one_token_step(x, pos_emb, start_pos, cache)) is not None:
+            return step
         xq, xk, xv, mha_kwargs = self.prepare_x_values(x, bsz=bsz, seqlen=seqlen, pos_emb=pos_emb, start_pos=start_pos,
                                                        cache=cache)
         keys, values = self.prepare_kv(xq, xk, xv, start_pos, cache=cache, kwargs=mha_kwargs)
@@ -169,6 +192,87 @@ class BaseNAtSAttentionLayer(AttentionLayer):
         self._post_update(cache, x_len)
         return output
 
+    def _overridden(self) -> bool:
+        """Whether a subclass or an instance replaces one of the methods `_one_token_step` stands in for."""
+        cls, own, chunked = type(self), self.__dict__, BaseNAtSChunkAttentionLayer
+        sample = cls._sample_for_token_info_values_inference
+        return (cls.prepare_x_values is not BaseNAtSAttentionLayer.prepare_x_values
+                or cls.add_rotary_emb is not AttentionLayer.add_rotary_emb
+                or cls.prepare_kv is not BaseNAtSAttentionLayer.prepare_kv
+                or cls.repeat_kv_values is not AttentionLayer.repeat_kv_values
+                or cls.multi_head_attention is not BaseNAtSAttentionLayer.multi_head_attention
+                or cls.role_logits is not BaseNAtSAttentionLayer.role_logits
+                or (sample is not BaseNAtSAttentionLayer._sample_for_token_info_values_inference
+                    and sample is not chunked._sample_for_token_info_values_inference)
+                or not own.keys().isdisjoint(_STEP_METHODS))
+
+    def _one_token_step(self, x, pos_emb, start_pos, cache):
+        """One token per sequence over a filled cache: projections, chunk statistic and roles in one launch, the rotary
+        embedding with the cache append in a second, then the decode kernel and the output projection.  (The torch ops of
+        the general way are about thirty launches, and a token waits for each of them.)  The results are the same ops with
+        the same rounding points; only the order of the fp32 sums inside the products differs."""
+        layer_id = self.layer_id
+        if type(cache) is not NAtSCache or pos_emb is None or len(cache.cache_model) <= layer_id:
+            return None
+        layer = cache.cache_model[layer_id]
+        chunked = type(layer) is NAtSChunkLayerCache
+        if not (chunked or type(layer) is NAtSLayerCache) or self._overridden():
+            return None
+        C = cache.chunk_size
+        is_chunk_module = isinstance(self, BaseNAtSChunkAttentionLayer)
+        if is_chunk_module:
+            if self.chunk_size != C or (C > 1 and self.chunk_merge_method is not ChunkMergeType.MEAN):
+                return None
+        elif C != 1:
+            return None
+        linears = (self.wq, self.wk, self.wv, self.wo, self.proj_layer)
+        if not all(_plain_linear(m) for m in linears):
+            return None
+        wq, wk, wv, wo, wr = (m.weight for m in linears)
+        cos, sin = pos_emb
+        B, _, dim = x.shape
+        Hq, Hkv, D = self.n_local_heads, self.n_local_kv_heads, self.head_dim
+        if (not _plain_execution(x, (wq, wk, wv, wo, wr)) or type(cos) is not torch.Tensor or type(sin) is not torch.Tensor
+                or not ops.step_project_ok(x, (wq, wk, wv, wr)) or not ops.matvec_weight_ok(wo, x.dtype, Hq * D)
+                or not wr.is_contiguous() or wr.shape[0] != 3 * Hkv
+                or cos.shape != (B, 1, D) or sin.shape != cos.shape or cos.dtype != x.dtype or sin.dtype != x.dtype
+                or not cos.is_cuda or not sin.is_cuda or cos.stride(-1) != 1 or sin.stride(-1) != 1 or D > 256 or D % 2):
+            return None
+        if self._cache_is_till_updating is not None:  # nats_attention.py:122-123
+            self._cache_is_till_updating.result()
+            self._cache_is_till_updating = None
+        if layer.bsz != B or layer.get_seq_length() <= 0 or not layer.takes_rotated_rows(x.dtype, D):
+            return None
+        pre_fill = cache.get_nats_chunk_fill_size(layer_id)
+        carry_in = None
+        if pre_fill:
+            carry_in = cache.get_nats_cached_x_in_chunk(layer_id)
+            if (carry_in is None or carry_in.shape != x.shape or carry_in.dtype != x.dtype or carry_in.device != x.device
+                    or not carry_in.is_contiguous() or carry_in.data_ptr() % 16):
+                return None
+        roles = None
+        if pre_fill + 1 >= C:
+            if not chunked:
+                roles = layer.role_destination(1)
+            if roles is None:
+                roles = torch.empty(B, Hkv, 1, dtype=torch.uint8, device=x.device)
+        qkv, carry = ops.launch_step_project(x, (wq, wk, wv), C, carry_in, roles is None, wr, roles,
+                                             self.global_token_enhanced_value, start_pos < C)
+        if is_chunk_module:
+            cache._update_cache_x(carry, layer_id)
+        if layer_id == 0:
+            cache.cache_model[-1].settle()  # (as `NAtSCache.update` does)
+        qkv = qkv.view(B, 1, Hq + 2 * Hkv, D).transpose(1, 2)
+        q, keys, values = layer.append_rotated(qkv[:, :Hq], qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:], cos, sin, None, roles)
+        row_end, tail_start = layer.decode_hint()
+        output = ops.decode_attention(q, keys, values, layer.valid_tokens, keys.shape[2], self.sm_scale, row_end=row_end,
+                                      tail_start=tail_start)
+        self._post_update(cache, 1)
+        return ops.matvec(output.view(B, 1, Hq * D), wo)
+
+
+_STEP_METHODS = frozenset(("prepare_x_values", "add_rotary_emb", "prepare_kv", "repeat_kv_values", "multi_head_attention",
+                           "role_logits", "_sample_for_token_info_values_inference"))
 
 
 class BaseNAtSChunkAttentionLayer(BaseNAtSAttentionLayer):

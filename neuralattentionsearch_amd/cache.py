@@ -423,6 +423,11 @@ class NAtSChunkLayerCache:
             self._buf_pos[:, :, start:end] = torch.arange(self._seen_tokens, self._seen_tokens + end - start,
                                                           dtype=torch.int32, device=self.device)
 
+    def takes_rotated_rows(self, dtype: torch.dtype, head_dim: int) -> bool:
+        """Whether `append_rotated` can take rows of this type: the cache holds rows of the same."""
+        have = self._buf_k if self._pending is None else self._pending[0]
+        return have is not None and have.dtype == dtype and have.shape[3] == head_dim
+
     def append_rotated(self, q: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor, cos: torch.Tensor,
                        sin: torch.Tensor, token_states_info: torch.Tensor | None = None,
                        roles: torch.Tensor | None = None):

@@ -214,37 +214,21 @@ __device__ __forceinline__ void unpack_piece(const uint4& u, float (&v)[8]) {
   }
 }
 
-template <bool kBf16, int XR, int WR, bool kGate>
-__global__ __launch_bounds__(kMatvecWaves * kWave) void matvec_kernel(MatvecArgs a) {
-  constexpr int E = kBf16 ? 8 : 4;       // elements per 16-byte piece
-  constexpr int NW = kGate ? 2 * WR : WR;  // weight rows per wavefront
-  constexpr int ES = kBf16 ? 2 : 4;      // bytes per element
-  const int lane = lane_id();
-  const int n0 = (blockIdx.x * kMatvecWaves + (threadIdx.x >> 6)) * WR;
-  if (n0 >= a.n_out) return;
-  const unsigned char* wrow[NW];
-#pragma unroll
-  for (int j = 0; j < NW; ++j) {
-    // columns past the end repeat the last one (their results are not written)
-    const int col = min(n0 + (j % WR), a.n_out - 1);
-    const int64_t row = (kGate && j >= WR) ? (int64_t)a.n_out + col : col;
-    wrow[j] = static_cast<const unsigned char*>(a.w) + row * a.w_stride * ES;
-  }
-  const unsigned char* xp = static_cast<const unsigned char*>(a.x);
-  float acc[NW][XR];
+// A wavefront's products of NW weight rows with XR rows of x: lanes walk k in 16-byte pieces, batches of kMatvecUnroll
+// pieces per weight row, then one of half that, then single pieces.  load_x(r, p, v) unpacks piece p of row r.
+template <bool kBf16, int XR, int NW, typename LoadX>
+__device__ __forceinline__ void matvec_sums(const unsigned char* const (&wrow)[NW], int k, int lane, LoadX load_x,
+                                            float (&acc)[NW][XR]) {
+  constexpr int E = kBf16 ? 8 : 4;  // elements per 16-byte piece
 #pragma unroll
   for (int j = 0; j < NW; ++j)
 #pragma unroll
     for (int r = 0; r < XR; ++r) acc[j][r] = 0.f;
-
-  const int pieces = a.k / E;
+  const int pieces = k / E;
   auto step = [&](int p, const uint4 (&wv)[NW]) {
     float xv[XR][8];
 #pragma unroll
-    for (int r = 0; r < XR; ++r) {
-      const uint4 u = *reinterpret_cast<const uint4*>(xp + (r * a.x_stride + (int64_t)p * E) * ES);
-      unpack_piece<kBf16>(u, xv[r]);
-    }
+    for (int r = 0; r < XR; ++r) load_x(r, p, xv[r]);
 #pragma unroll
     for (int j = 0; j < NW; ++j) {
       float wf[8];
@@ -256,7 +240,6 @@ __global__ __launch_bounds__(kMatvecWaves * kWave) void matvec_kernel(MatvecArgs
     }
   };
   int p = lane;
-  // batches of kMatvecUnroll pieces per weight row, then one of half that, then single pieces
   auto batch = [&](auto n_const) {
     constexpr int N = decltype(n_const)::value;
     uint4 wv[N][NW];
@@ -282,6 +265,27 @@ __global__ __launch_bounds__(kMatvecWaves * kWave) void matvec_kernel(MatvecArgs
     for (int r = 0; r < XR; ++r)
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) acc[j][r] += __shfl_xor(acc[j][r], o);
+}
+
+// columns [n0, n0 + WR) of one product
+template <bool kBf16, int XR, int WR, bool kGate>
+__device__ __forceinline__ void matvec_columns(const MatvecArgs& a, int n0, int lane) {
+  constexpr int E = kBf16 ? 8 : 4;
+  constexpr int NW = kGate ? 2 * WR : WR;  // weight rows per wavefront
+  constexpr int ES = kBf16 ? 2 : 4;        // bytes per element
+  const unsigned char* wrow[NW];
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    // columns past the end repeat the last one (their results are not written)
+    const int col = min(n0 + (j % WR), a.n_out - 1);
+    const int64_t row = (kGate && j >= WR) ? (int64_t)a.n_out + col : col;
+    wrow[j] = static_cast<const unsigned char*>(a.w) + row * a.w_stride * ES;
+  }
+  const unsigned char* xp = static_cast<const unsigned char*>(a.x);
+  float acc[NW][XR];
+  matvec_sums<kBf16, XR, NW>(wrow, a.k, lane, [&](int r, int p, float (&v)[8]) {
+    unpack_piece<kBf16>(*reinterpret_cast<const uint4*>(xp + (r * a.x_stride + (int64_t)p * E) * ES), v);
+  }, acc);
   if (lane == 0) {
 #pragma unroll
     for (int j = 0; j < WR; ++j) {
@@ -296,6 +300,121 @@ __global__ __launch_bounds__(kMatvecWaves * kWave) void matvec_kernel(MatvecArgs
         g_store<kBf16>(a.y, r * a.y_stride + n0 + j, v);
       }
     }
+  }
+}
+
+template <bool kBf16, int XR, int WR, bool kGate>
+__global__ __launch_bounds__(kMatvecWaves * kWave) void matvec_kernel(MatvecArgs a) {
+  const int n0 = (blockIdx.x * kMatvecWaves + (threadIdx.x >> 6)) * WR;
+  if (n0 >= a.n_out) return;
+  matvec_columns<kBf16, XR, WR, kGate>(a, n0, lane_id());
+}
+
+// ---- everything a one-token step of an attention module needs from its hidden states, in one launch --------------
+// The products with up to four matrices (q, k and v projections that lie apart in memory), the running chunk statistic
+// and, for a step that completes a chunk, the roles: the workgroups are dealt to these parts in that order.  A step
+// is bound by the launches it consists of and by the latency of each, not by bytes: side by side the parts cost what
+// the longest of them costs.  (dim 4096, 32 / 8 heads, one row: 10.4 us
+// with the statistic, where three library products and the torch ops of the statistic took 46 us of kernel time in seven
+// launches; a module call of one token 265 -> 100 us of host and device time.)
+// Roles: a wavefront computes the three logits of one kv head from the statistic (built on the fly) and takes their
+// argmax with the rounding points of roles_kernel: statistic, logits and the biased logit each rounded to the dtype.
+constexpr int kMaxProjections = 4;
+struct StepProjectArgs {
+  const void* x;  // [rows, k] contiguous
+  void* y;        // [rows, y_stride]: the products side by side
+  const void* w[kMaxProjections];
+  int64_t w_stride[kMaxProjections];
+  int n_out[kMaxProjections], col0[kMaxProjections];
+  int block0[kMaxProjections + 2];  // first workgroup of each product, then of the roles, then of the statistic
+  int64_t y_stride;
+  int n_mats, k;
+  const void* role_w;  // [H * 3, k] or null
+  uint8_t* roles;      // role of (row, head) at (row * H + head) * roles_hs
+  int64_t roles_hs;
+  int H, force_first;
+  float bias;
+  const void* carry_in;  // [rows, k] or null
+  void* carry_out;       // [rows, k] or null
+  float inv_chunk;       // (the library's division by a number is this product)
+};
+
+template <bool kBf16, int XR>
+__global__ __launch_bounds__(kMatvecWaves * kWave) void step_project_kernel(StepProjectArgs a) {
+#pragma clang fp contract(off)  // (the statistic's product and sum round separately; the dot products call fmaf)
+  constexpr int E = kBf16 ? 8 : 4, ES = kBf16 ? 2 : 4;
+  const int lane = lane_id(), wave = threadIdx.x >> 6;
+  const int bid = blockIdx.x;
+  const unsigned char* xp = static_cast<const unsigned char*>(a.x);
+  const unsigned char* cp = static_cast<const unsigned char*>(a.carry_in);
+  auto load_stat = [&](int64_t byte, float (&v)[8]) {  // the chunk statistic with this token in it
+    unpack_piece<kBf16>(*reinterpret_cast<const uint4*>(xp + byte), v);
+    float c[8];
+    if (cp) unpack_piece<kBf16>(*reinterpret_cast<const uint4*>(cp + byte), c);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      v[e] = g_round<kBf16>(v[e] * a.inv_chunk);
+      if (cp) v[e] = g_round<kBf16>(c[e] + v[e]);
+    }
+  };
+  if (bid < a.block0[kMaxProjections]) {
+    int m = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxProjections; ++i) m = bid >= a.block0[i] ? i : m;
+    MatvecArgs p;
+    p.w = a.w[0]; p.w_stride = a.w_stride[0]; p.n_out = a.n_out[0];
+    int col0 = a.col0[0], block0 = a.block0[0];
+#pragma unroll
+    for (int i = 1; i < kMaxProjections; ++i) {
+      if (m == i) {
+        p.w = a.w[i]; p.w_stride = a.w_stride[i]; p.n_out = a.n_out[i];
+        col0 = a.col0[i];
+        block0 = a.block0[i];
+      }
+    }
+    p.x = a.x; p.x_stride = a.k; p.k = a.k;
+    p.y = static_cast<unsigned char*>(a.y) + (int64_t)col0 * ES;
+    p.y_stride = a.y_stride;
+    const int n0 = (bid - block0) * kMatvecWaves + wave;
+    if (n0 < p.n_out) matvec_columns<kBf16, XR, 1, false>(p, n0, lane);
+    return;
+  }
+  if (bid < a.block0[kMaxProjections + 1]) {
+    const int h = (bid - a.block0[kMaxProjections]) * kMatvecWaves + wave;
+    if (h >= a.H) return;
+    const unsigned char* wrow[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) wrow[j] = static_cast<const unsigned char*>(a.role_w) + (int64_t)(h * 3 + j) * a.k * ES;
+    float acc[3][XR];
+    matvec_sums<kBf16, XR, 3>(wrow, a.k, lane, [&](int r, int p, float (&v)[8]) {
+      load_stat(((int64_t)r * a.k + (int64_t)p * E) * ES, v);
+    }, acc);
+    if (lane == 0) {
+#pragma unroll
+      for (int r = 0; r < XR; ++r) {
+        const float x0 = g_round<kBf16>(g_round<kBf16>(acc[0][r]) + a.bias);
+        const float x1 = g_round<kBf16>(acc[1][r]), x2 = g_round<kBf16>(acc[2][r]);
+        int arg = NATS_ROLE_GLOBAL;
+        float best = x0;
+        if (x1 > best) {
+          best = x1;
+          arg = NATS_ROLE_LOCAL;
+        }
+        if (x2 > best) arg = NATS_ROLE_SW;
+        if (a.force_first) arg = NATS_ROLE_GLOBAL;
+        a.roles[((int64_t)r * a.H + h) * a.roles_hs] = uint8_t(arg);
+      }
+    }
+    return;
+  }
+  const int64_t piece = (int64_t)(bid - a.block0[kMaxProjections + 1]) * (kMatvecWaves * kWave) + threadIdx.x;
+  if (piece * E >= (int64_t)XR * a.k) return;
+  float v[8];
+  load_stat(piece * 16, v);
+  if (kBf16) {
+    store_vec<true, 8>(a.carry_out, piece * 8, v);
+  } else {
+    *reinterpret_cast<float4*>(static_cast<float*>(a.carry_out) + piece * 4) = make_float4(v[0], v[1], v[2], v[3]);
   }
 }
 
@@ -539,6 +658,76 @@ extern "C" int nats_matvec(const void* w, const void* x, void* y, int64_t x_rows
     if (gate) launch_matvec_rows<false, true>(a, (int)x_rows, st); else launch_matvec_rows<false, false>(a, (int)x_rows, st);
   }
   NATS_CHECK_LAUNCH("matvec_kernel");
+  return NATS_OK;
+}
+
+extern "C" int nats_step_project(const void* x, int64_t x_rows, int64_t k, int64_t n_mats, const void* const* w,
+                                 const int64_t* n_out, const int64_t* w_strides, void* y, int64_t y_stride,
+                                 const void* role_w, int64_t H_kv, float global_bias, int force_first_global, uint8_t* roles,
+                                 int64_t roles_hs, const void* carry_in, void* carry_out, int64_t chunk_size, int dtype,
+                                 void* stream) {
+  const char* who = "nats_step_project";
+  NATS_REQUIRE(x && y && w && n_out && w_strides, NATS_ERR_NULL_POINTER, "%s: NULL pointer", who);
+  NATS_REQUIRE(dtype == NATS_DTYPE_BF16 || dtype == NATS_DTYPE_F32, NATS_ERR_BAD_DTYPE, "%s: dtype %d", who, dtype);
+  const int64_t e = dtype == NATS_DTYPE_BF16 ? 8 : 4;
+  NATS_REQUIRE(x_rows >= 1 && x_rows <= 4, NATS_ERR_UNSUPPORTED, "%s: %lld rows of x (1..4)", who, (long long)x_rows);
+  NATS_REQUIRE(n_mats >= 1 && n_mats <= kMaxProjections, NATS_ERR_UNSUPPORTED, "%s: %lld matrices (1..%d)", who,
+               (long long)n_mats, kMaxProjections);
+  NATS_REQUIRE(k > 0 && k <= 0x3fffffff && k % e == 0 && chunk_size > 0, NATS_ERR_BAD_SHAPE, "%s: k=%lld chunk_size=%lld", who,
+               (long long)k, (long long)chunk_size);
+  auto aligned16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  NATS_REQUIRE(aligned16(x) && aligned16(carry_in) && aligned16(carry_out) && aligned16(role_w), NATS_ERR_BAD_SHAPE,
+               "%s: x, the statistic and the role matrix must be 16-byte aligned", who);
+  NATS_REQUIRE(!(roles && carry_out && carry_out == carry_in), NATS_ERR_BAD_SHAPE,
+               "%s: the statistic may not be updated in place while roles are computed from it", who);
+  StepProjectArgs a{};
+  a.x = x; a.y = y; a.y_stride = y_stride;
+  a.n_mats = (int)n_mats; a.k = (int)k;
+  int64_t cols = 0, blocks = 0;
+  for (int i = 0; i < kMaxProjections; ++i) {
+    a.block0[i] = (int)blocks;
+    if (i >= n_mats) {
+      a.block0[i] = 0x7fffffff;  // (no workgroup reaches it)
+      continue;
+    }
+    NATS_REQUIRE(w[i] && aligned16(w[i]) && n_out[i] > 0 && n_out[i] <= 0xfffffff && w_strides[i] >= k && w_strides[i] % e == 0,
+                 NATS_ERR_BAD_SHAPE, "%s: matrix %d: n_out=%lld row stride %lld (rows of 16-byte pieces, 16-byte aligned)", who, i,
+                 (long long)n_out[i], (long long)w_strides[i]);
+    a.w[i] = w[i]; a.w_stride[i] = w_strides[i];
+    a.n_out[i] = (int)n_out[i]; a.col0[i] = (int)cols;
+    cols += n_out[i];
+    blocks += (n_out[i] + kMatvecWaves - 1) / kMatvecWaves;
+  }
+  NATS_REQUIRE(y_stride >= cols, NATS_ERR_BAD_SHAPE, "%s: y_stride=%lld < %lld columns", who, (long long)y_stride, (long long)cols);
+  a.block0[kMaxProjections] = (int)blocks;
+  a.inv_chunk = 1.f / (float)chunk_size;
+  a.carry_in = carry_in; a.carry_out = carry_out;
+  if (roles) {
+    NATS_REQUIRE(role_w && H_kv > 0 && H_kv <= 65535 && roles_hs >= 1, NATS_ERR_BAD_SHAPE, "%s: H_kv=%lld roles_hs=%lld", who,
+                 (long long)H_kv, (long long)roles_hs);
+    a.role_w = role_w; a.roles = roles; a.roles_hs = roles_hs; a.H = (int)H_kv;
+    a.bias = global_bias; a.force_first = force_first_global;
+    blocks += (H_kv + kMatvecWaves - 1) / kMatvecWaves;
+  }
+  a.block0[kMaxProjections + 1] = (int)blocks;
+  if (carry_out) blocks += (x_rows * k / e + kMatvecWaves * kWave - 1) / (kMatvecWaves * kWave);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+#define NATS_STEP(BF, XR) hipLaunchKernelGGL((step_project_kernel<BF, XR>), dim3((unsigned)blocks), dim3(kMatvecWaves * kWave), 0, st, a)
+#define NATS_STEP_ROWS(BF)                \
+  switch (x_rows) {                       \
+    case 1: NATS_STEP(BF, 1); break;      \
+    case 2: NATS_STEP(BF, 2); break;      \
+    case 3: NATS_STEP(BF, 3); break;      \
+    default: NATS_STEP(BF, 4); break;     \
+  }
+  if (dtype == NATS_DTYPE_BF16) {
+    NATS_STEP_ROWS(true)
+  } else {
+    NATS_STEP_ROWS(false)
+  }
+#undef NATS_STEP_ROWS
+#undef NATS_STEP
+  NATS_CHECK_LAUNCH("step_project_kernel");
   return NATS_OK;
 }
 

@@ -832,6 +832,56 @@ class MatvecPlan:
         return y
 
 
+def step_project_ok(x: torch.Tensor, weights) -> bool:
+    """Whether `step_project` takes these tensors: one to four rows of x, 16-byte pieces along k everywhere."""
+    k = x.shape[-1]
+    return (x.is_cuda and x.is_contiguous() and 1 <= x.numel() // k <= MATVEC_MAX_ROWS and x.data_ptr() % 16 == 0
+            and all(_matvec_weight_ok(w) and w.dtype == x.dtype and w.shape[1] == k for w in weights))
+
+
+def matvec_weight_ok(weight: torch.Tensor, dtype: torch.dtype, k: int) -> bool:
+    """Whether `matvec` takes this matrix for rows of k entries of this dtype."""
+    return _matvec_weight_ok(weight) and weight.dtype == dtype and weight.shape[1] == k
+
+
+def step_project(x: torch.Tensor, weights, chunk_size: int = 1, carry_in: torch.Tensor | None = None, with_carry: bool = False,
+                 role_weight: torch.Tensor | None = None, roles_out: torch.Tensor | None = None, global_bias: float = 0.1,
+                 force_first_global: bool = False):
+    """The products of up to four rows of x [B, 1, k] with one to four matrices [n_i, k], side by side in one tensor
+    [B, 1, sum n_i]; with `with_carry` also the chunk statistic carry_in + x / chunk_size, [B, 1, k]; with `roles_out`
+    (uint8 [B, H_kv, 1], laid out as `role_destination` and `torch.empty` make it) the roles from that statistic and
+    `role_weight` [H_kv * 3, k].  Returns (products, statistic or None)."""
+    B, k = x.numel() // x.shape[-1], x.shape[-1]
+    if not step_project_ok(x, weights) or not 1 <= len(weights) <= 4:
+        raise ValueError("step_project: x [<= 4 rows, k] contiguous and 1..4 matrices [n, k] of its dtype, k a multiple of 16 bytes")
+    if carry_in is not None and (carry_in.numel() != x.numel() or carry_in.dtype != x.dtype or not carry_in.is_contiguous()
+                                 or not carry_in.is_cuda):
+        raise ValueError("step_project: the chunk statistic must be a contiguous tensor of x's size and dtype")
+    if roles_out is not None:
+        H = role_weight.shape[0] // 3
+        if (role_weight.dtype != x.dtype or tuple(role_weight.shape) != (H * 3, k) or not role_weight.is_contiguous()
+                or not role_weight.is_cuda or roles_out.dtype != torch.uint8 or tuple(roles_out.shape) != (B, H, 1)
+                or not roles_out.is_cuda or (B > 1 and roles_out.stride(0) != H * roles_out.stride(1))):
+            raise ValueError("step_project: role_weight [H_kv * 3, k] of x's dtype and roles_out uint8 [B, H_kv, 1]")
+    return launch_step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global)
+
+
+def launch_step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global):
+    """`step_project` for a caller that has made its checks."""
+    B, k = x.numel() // x.shape[-1], x.shape[-1]
+    n = [w.shape[0] for w in weights]
+    total = sum(n)
+    y = torch.empty(B, 1, total, dtype=x.dtype, device=x.device)
+    carry = torch.empty(B, 1, k, dtype=x.dtype, device=x.device) if with_carry else None
+    ptrs = (ctypes.c_void_p * len(n))(*[w.data_ptr() for w in weights])
+    H, hs = (0, 0) if roles_out is None else (roles_out.shape[1], roles_out.stride(1))
+    check(_lib.load().nats_step_project(x.data_ptr(), B, k, len(n), ptrs, i64_array(n), i64_array([w.stride(0) for w in weights]),
+                                        y.data_ptr(), total, _ptr(role_weight), H, float(global_bias), int(force_first_global),
+                                        _ptr(roles_out), hs, _ptr(carry_in), _ptr(carry), int(chunk_size), _dtype_code(x),
+                                        _stream(x)))
+    return y, carry
+
+
 def rope_qk_ok(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
     """Whether `rope_qk` takes these tensors (16-byte rows everywhere)."""
     e = 16 // q.element_size()

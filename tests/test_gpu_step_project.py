@@ -1,0 +1,117 @@
+"""GPU: the one-launch projections, chunk statistic and roles of a one-token step, and the attention modules' one-token
+path that is built on them, against the separate torch ops."""
+import pytest
+import torch
+
+from tests.gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,k,ns,H,C,hs", [(1, 4096, (4096, 1024, 1024), 8, 64, 1), (4, 512, (129, 3, 70, 1), 5, 12, 16),
+                                              (3, 8, (1,), 1, 1, 16), (2, 2056, (4, 5), 2, 16, 1)])
+def test_step_project(dtype, rows, k, ns, H, C, hs):
+    from neuralattentionsearch_amd import ops
+    say("step_project", dtype, rows, k, ns, H, C, hs)
+    g = torch.Generator().manual_seed(rows * k)
+    x = torch.randn(rows, 1, k, generator=g).to(dtype).cuda()
+    w = [(torch.randn(n, k, generator=g) / k ** 0.5).to(dtype).cuda() for n in ns]
+    wr = (torch.randn(3 * H, k, generator=g) * (C / k) ** 0.5).to(dtype).cuda()
+    carry = torch.randn(rows, 1, k, generator=g).to(dtype).cuda()
+    for c_in in (None, carry):
+        buf = torch.full((rows, H, hs), 7, dtype=torch.uint8, device="cuda")
+        y, stat = ops.step_project(x, w, C, c_in, with_carry=True, role_weight=wr, roles_out=buf[:, :, :1])
+        # elementwise steps equal the torch ops bit for bit (components/cache/dyn_cache.py:101-104)
+        want = x / C if c_in is None else c_in + x / C
+        assert torch.equal(stat, want)
+        # products: fp32 sums in another order, one rounding (2^-8 of the value in bf16) at the end
+        exact = torch.cat([x.double() @ m.double().T for m in w], dim=-1)
+        err = ((y.double() - exact).abs() / exact.abs().clamp_min(1.0)).max().item()
+        assert err <= (2.0 ** -8 if dtype == torch.bfloat16 else 2e-6), err
+        # roles: the argmax of the rounded logits, wherever no logit of the sums in 64 bits is that close to another
+        lg = (want.double() @ wr.double().T).view(rows, H, 3)
+        ulp = (lg.abs().max().item() + 0.2) * (2.0 ** -7 if dtype == torch.bfloat16 else 2e-6)
+        lg[..., 0] += 0.1
+        top = lg.topk(2, dim=-1).values
+        sure = top[..., 0] - top[..., 1] > 2 * ulp
+        assert torch.equal(buf[:, :, 0][sure], lg.argmax(-1).to(torch.uint8)[sure])
+        assert bool((buf[:, :, 1:] == 7).all())
+    roles = torch.empty(rows, H, 1, dtype=torch.uint8, device="cuda")
+    y2, none = ops.step_project(x, w, C, role_weight=wr, roles_out=roles, force_first_global=True)
+    assert none is None and torch.equal(y2, y) and not roles.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,C,W,lens", [(1, 16, 32, [50] + [1] * 40 + [20] + [1] * 20), (4, 1, 32, [40] + [1] * 40 + [7] + [1] * 9),
+                                        (2, 12, 36, [5] + [1] * 30), (3, 1, 16, [1] * 40)])
+def test_module_step_equals_the_general_way(dtype, B, C, W, lens):
+    """The fast step and the general forward (forced by a hook) on the same hidden states: the same roles and rows."""
+    from neuralattentionsearch_amd.attention import LlamaNAtSAttentionLayer, LlamaNAtSChunkAttentionLayer
+    from neuralattentionsearch_amd.cache import NAtSCache
+    from neuralattentionsearch_amd.llama import rotary_tables
+    say("module step", dtype, B, C, W)
+    torch.manual_seed(3)
+    kw = dict(dim=512, n_heads=8, n_kv_heads=4, layer_id=0, local_seq_max_length=W)
+    mod = LlamaNAtSAttentionLayer(**kw) if C == 1 else LlamaNAtSChunkAttentionLayer(chunk_size=C, **kw)
+    mod = mod.cuda().to(dtype).eval().requires_grad_(False)
+    mod.proj_layer.weight.mul_(8.0)
+    fast, slow = NAtSCache(W, C), NAtSCache(W, C)
+    taken = []
+    general = type(mod)._one_token_step
+    at = 0
+    tol = 4 * 2.0 ** -8 if dtype == torch.bfloat16 else 2e-5
+    with torch.no_grad():
+        for n in lens:
+            x = torch.randn(B, n, 512, device="cuda").to(dtype)
+            pos = torch.arange(at, at + n, device="cuda")[None].expand(B, -1)
+            emb = rotary_tables(pos, 64, 10000.0, dtype)
+            if n == 1:
+                taken.append(general(mod, x, emb, at, None) is None)  # (no cache: the general way)
+            got = mod(x, emb, None, start_pos=at, cache=fast)
+            hook = mod.wv.register_forward_hook(lambda m, i, o: None)
+            want = mod(x, emb, None, start_pos=at, cache=slow)
+            hook.remove()
+            at += n
+            err = ((got - want).float().norm() / want.float().norm()).item()
+            assert err <= tol, (at, err)
+            a, b = fast.cache_model[0], slow.cache_model[0]
+            assert a.n_ctx_data == b.n_ctx_data and torch.equal(a.valid_tokens, b.valid_tokens), at
+            assert torch.equal(a.size_global_kv, b.size_global_kv) and torch.equal(a.size_local_kv, b.size_local_kv), at
+    assert all(taken)
+
+
+def test_module_step_leaves_watched_modules_to_the_general_way():
+    """Hooks, wrapped projections, autograd and overridden methods see every call."""
+    from neuralattentionsearch_amd.attention import LlamaNAtSChunkAttentionLayer
+    from neuralattentionsearch_amd.cache import NAtSCache
+    from neuralattentionsearch_amd.llama import rotary_tables
+
+    class Scaled(LlamaNAtSChunkAttentionLayer):
+        calls = 0
+
+        def add_rotary_emb(self, xq, xk, pos_emb):
+            Scaled.calls += 1
+            return super().add_rotary_emb(xq, xk, pos_emb)
+
+    kw = dict(dim=256, n_heads=4, n_kv_heads=2, layer_id=0, local_seq_max_length=16, chunk_size=8)
+    x = torch.randn(1, 1, 256, device="cuda")
+
+    def step(mod):
+        cache = NAtSCache(16, 8)
+        with torch.no_grad():
+            emb = rotary_tables(torch.arange(20, device="cuda")[None], 64, 10000.0, torch.float32)
+            mod(torch.randn(1, 20, 256, device="cuda"), emb, None, start_pos=0, cache=cache)
+        emb = rotary_tables(torch.full((1, 1), 20, device="cuda"), 64, 10000.0, torch.float32)
+        return mod._one_token_step(x, emb, 20, cache), cache, emb
+
+    mod = LlamaNAtSChunkAttentionLayer(**kw).cuda().eval()
+    assert step(mod)[0] is None  # (autograd records the projections)
+    mod.requires_grad_(False)
+    out, cache, emb = step(mod)
+    assert out is not None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert mod._one_token_step(x, emb, 21, cache) is None
+    assert step(Scaled(**kw).cuda().eval().requires_grad_(False))[0] is None
+    mod.wo.register_forward_hook(lambda m, i, o: o)
+    assert step(mod)[0] is None
