@@ -1015,16 +1015,68 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   }
 }
 
+// A launch of a few rounds of workgroups per compute unit whose streams differ in how much of them is visible (heads keep
+// different shares of a context, and the whole share of a stream lies on one XCD in the plain map): the heavy streams'
+// query groups come first, over all XCDs, so that no long workgroup starts in the last round.  Every workgroup counts the
+// streams' key tiles that the middle query sees (one trip to L2), takes those above half of the largest count as the heavy
+// ones and finds its own item; streams within 1.5 times their mean keep the plain map and with it one stream's tiles per L2.
+// Measured at 32 / 8 heads, head dim 128, chunk 64, segments of 4096 tokens whose first head keeps three to nine times what
+// the others keep: 82 / 143 / 167 / 184 -> 75 / 98 / 127 / 140 us for the first to the fourth segment; with streams alike
+// 53.9 / 53.7 us (4096 tokens from empty).  What bounds it then is the longest single query group.
+constexpr int kBalanceStreams = 64;   // one per lane
+constexpr int kBalanceTiles = 8192;   // tile summaries a workgroup may read for it
+__device__ __forceinline__ void map_balanced(const PrefillArgs& a, int* counts, int bid, int& ks, int& hg, int& rank) {
+  const int ns = a.B * a.Hkv;
+  const int lane = threadIdx.x & 63;
+  const int r_mid = a.r_begin + (a.r_end - a.r_begin) / 2;
+  const int n_t = min((a.base + r_mid) / kTile + 1, a.Tk);
+  for (int s = threadIdx.x >> 6; s < ns; s += kPrefillWaves) {
+    const int2* tl = a.tile_lim + (int64_t)s * a.Tk;
+    int n = 0;
+    for (int t0 = 0; t0 < n_t; t0 += 4 * kWave) {
+      int lim[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) lim[u] = tl[min(t0 + u * kWave + lane, n_t - 1)].x;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) n += __popcll(__ballot(t0 + u * kWave + lane < n_t && lim[u] >= r_mid));
+    }
+    if (lane == 0) counts[s] = n;
+  }
+  __syncthreads();
+  const int mine = lane < ns ? counts[lane] : 0;
+  __syncthreads();  // (the caller's tiles go where the counts were)
+  int most = mine, sum = mine;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    most = max(most, __shfl_xor(most, o));
+    sum += __shfl_xor(sum, o);
+  }
+  most = __builtin_amdgcn_readfirstlane(most);  // (the same in every lane; as scalars they keep the map and the item scalar)
+  sum = __builtin_amdgcn_readfirstlane(sum);
+  if (2 * most * ns < 3 * sum) {
+    map_workgroup(a, bid, ks, hg, rank);
+    return;
+  }
+  balanced_item(__ballot(2 * mine > most), ns, a.n_hg, a.n_qg, bid, ks, hg, rank);
+}
+
 // One (kv stream, head group, query group) per workgroup.  The workgroups at the end of the grid (two per compute
 // unit) have no query group of their own: they draw the pooled ones (the lightest of every stream) from counters for
 // as long as there are any.  XCDs do not finish their fixed share at the same time (streams differ in how many keys
 // their roles keep visible, and the XCDs of one device differ in speed by a few percent): those that get to the pool
 // earlier take more of it.  The tile loop exists twice in the code, once for each kind of workgroup, so that the
 // loop around the pooled one costs the other nothing.
-template <int D, bool kUniform, int kMode = 0>
+// (kBalance: an instantiation of its own, since the map's code before the tile loop costs the loop 5 % in the plain one)
+template <int D, bool kUniform, int kMode, bool kBalance>
 __global__ __launch_bounds__(kPrefillWaves * kWave) void prefill_mfma_kernel(PrefillArgs args) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   int bid = blockIdx.x;
+  if constexpr (kBalance) {
+    int ks, hg, rank;
+    map_balanced(args, reinterpret_cast<int*>(smem_raw), bid, ks, hg, rank);
+    prefill_mfma_item<D, kUniform, kMode>(args, smem_raw, bid, 0, ks, hg, rank);
+    return;
+  }
   int split = 0;  // which share of the tile list (n_split > 1)
   if (args.n_split > 1) {
     split = bid % args.n_split;
@@ -1562,19 +1614,19 @@ static int launch_prefill_wide(const PrefillArgs& a, int64_t n_wg, hipStream_t s
   return NATS_OK;
 }
 
-template <int D, bool kUniform, int kMode = 0>
+template <int D, bool kUniform, int kMode, bool kBalance = false>
 static int launch_prefill_mfma(const PrefillArgs& a, int64_t n_wg, hipStream_t st) {
   static bool configured[kMaxDevices] = {};  // per instantiation; the attribute is set once per device
   const size_t smem = sizeof(PrefillSmem<D>);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return fail(NATS_ERR_LAUNCH, "prefill: no current device");
   if (!configured[dev]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma_kernel<D, kUniform, kMode>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma_kernel<D, kUniform, kMode, kBalance>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return fail(NATS_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS): %s", smem, hipGetErrorString(e));
     configured[dev] = true;
   }
-  hipLaunchKernelGGL((prefill_mfma_kernel<D, kUniform, kMode>), dim3((unsigned)n_wg), dim3(kPrefillWaves * kWave), smem, st, a);
+  hipLaunchKernelGGL((prefill_mfma_kernel<D, kUniform, kMode, kBalance>), dim3((unsigned)n_wg), dim3(kPrefillWaves * kWave), smem, st, a);
   NATS_CHECK_LAUNCH("prefill_mfma_kernel");
   return NATS_OK;
 }
@@ -1794,6 +1846,18 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
     }
     NATS_CHECK_LAUNCH("prefill_split_merge_kernel");
     return NATS_OK;
+  }
+  // One to four rounds of workgroups per compute unit: see map_balanced.  (Below that every workgroup starts at once, above
+  // it the drawn query groups even the XCDs out.  Packed tiles from empty, where streams differ by their new roles only, keep
+  // the plain map: alike, they pay 1 us of 52 for the look.)
+  if (const int64_t n_cu = device_cu_count(), ns = g.B * g.H_kv;
+      hpw == 4 && n_cu > 0 && n_wg > n_cu && n_wg < 4 * n_cu && ns > 1 && ns <= kBalanceStreams && ns * a.Tk <= kBalanceTiles && (!packed || g.base > 0)) {
+#define NATS_PREFILL_BALANCED(MODE)                                                                  \
+  (g.D == 32 ? launch_prefill_mfma<32, true, MODE, true>(a, n_wg, st)                                \
+             : g.D == 64 ? launch_prefill_mfma<64, true, MODE, true>(a, n_wg, st) : launch_prefill_mfma<128, true, MODE, true>(a, n_wg, st))
+    if (!packed) return NATS_PREFILL_BALANCED(0);
+    return a.long_rows ? NATS_PREFILL_BALANCED(2) : NATS_PREFILL_BALANCED(1);
+#undef NATS_PREFILL_BALANCED
   }
   // A launch of several rounds of workgroups per compute unit draws its lightest query groups from the counter
   // (NATS_PREFILL_POOL = eighths of the query groups that are drawn, 0 = none).
