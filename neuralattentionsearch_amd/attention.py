@@ -37,8 +37,9 @@ def apply_rotary_pos_emb(q, k, cos, sin, unsqueeze_dim: int = 1):
 
 def _plain_linear(m: nn.Module) -> bool:
     """An nn.Linear without bias that nobody has wrapped, hooked or re-parametrised: its call is one matrix product."""
-    return (type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-            and "forward" not in m.__dict__ and m.bias is None and type(m.weight) is nn.Parameter)
+    d = m.__dict__
+    return (type(m) is nn.Linear and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"])
+            and "forward" not in d and d["_parameters"].get("bias") is None and type(d["_parameters"].get("weight")) is nn.Parameter)
 
 
 def _plain_execution(x: torch.Tensor, weights) -> bool:
@@ -225,17 +226,17 @@ class BaseNAtSAttentionLayer(AttentionLayer):
                 return None
         elif C != 1:
             return None
-        linears = (self.wq, self.wk, self.wv, self.wo, self.proj_layer)
-        if not all(_plain_linear(m) for m in linears):
+        mods = self._modules
+        linears = (mods.get("wq"), mods.get("wk"), mods.get("wv"), mods.get("wo"), mods.get("proj_layer"))
+        if not all(map(_plain_linear, linears)):
             return None
-        wq, wk, wv, wo, wr = (m.weight for m in linears)
+        wq, wk, wv, wo, wr = (m._parameters["weight"] for m in linears)
         cos, sin = pos_emb
         B, _, dim = x.shape
         Hq, Hkv, D = self.n_local_heads, self.n_local_kv_heads, self.head_dim
         if (not _plain_execution(x, (wq, wk, wv, wo, wr)) or type(cos) is not torch.Tensor or type(sin) is not torch.Tensor
-                or not ops.step_project_ok(x, (wq, wk, wv, wr)) or not ops.matvec_weight_ok(wo, x.dtype, Hq * D)
-                or not wr.is_contiguous() or wr.shape[0] != 3 * Hkv
-                or cos.shape != (B, 1, D) or sin.shape != cos.shape or cos.dtype != x.dtype or sin.dtype != x.dtype
+                or not ops.matvec_takes(x, wo, Hq * D) or not ops.matvec_takes(x, wr, dim) or wr.shape[0] != 3 * Hkv
+                or wq.shape[0] != Hq * D or wk.shape[0] != Hkv * D or wv.shape[0] != Hkv * D or cos.shape != (B, 1, D) or sin.shape != cos.shape or cos.dtype != x.dtype or sin.dtype != x.dtype
                 or not cos.is_cuda or not sin.is_cuda or cos.stride(-1) != 1 or sin.stride(-1) != 1 or D > 256 or D % 2):
             return None
         if self._cache_is_till_updating is not None:  # nats_attention.py:122-123
@@ -256,17 +257,17 @@ class BaseNAtSAttentionLayer(AttentionLayer):
                 roles = layer.role_destination(1)
             if roles is None:
                 roles = torch.empty(B, Hkv, 1, dtype=torch.uint8, device=x.device)
-        qkv, carry = ops.launch_step_project(x, (wq, wk, wv), C, carry_in, roles is None, wr, roles,
-                                             self.global_token_enhanced_value, start_pos < C)
+        projected = ops.try_step_project(x, (wq, wk, wv), C, carry_in, roles is None, wr, roles, self.global_token_enhanced_value,
+                                         start_pos < C)
+        if projected is None:
+            return None
+        qkv, carry = projected
         if is_chunk_module:
             cache._update_cache_x(carry, layer_id)
         if layer_id == 0:
             cache.cache_model[-1].settle()  # (as `NAtSCache.update` does)
         qkv = qkv.view(B, 1, Hq + 2 * Hkv, D).transpose(1, 2)
-        q, keys, values = layer.append_rotated(qkv[:, :Hq], qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:], cos, sin, None, roles)
-        row_end, tail_start = layer.decode_hint()
-        output = ops.decode_attention(q, keys, values, layer.valid_tokens, keys.shape[2], self.sm_scale, row_end=row_end,
-                                      tail_start=tail_start)
+        output = layer.step_attention(qkv[:, :Hq], qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:], cos, sin, None, roles, self.sm_scale)
         self._post_update(cache, 1)
         return ops.matvec(output.view(B, 1, Hq * D), wo)
 

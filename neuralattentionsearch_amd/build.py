@@ -1,12 +1,15 @@
-"""Builds libnats_hip.so (gfx950) in-tree with hipcc.  Usage: python -m neuralattentionsearch_amd.build"""
+"""Builds libnats_hip.so (gfx950) in-tree with hipcc, and _nats_host.so (the native front) with the host compiler.  Usage: python -m neuralattentionsearch_amd.build"""
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libnats_hip.so")
+HOST_SOURCE = os.path.join(CSRC, "nats_host.cpp")  # the native front of the step-wise operators: a Python extension, no GPU code
+HOST_PATH = os.path.join(PKG_DIR, "_nats_host.so")
 SOURCES = ["nats_roles.hip", "nats_rolestep.hip", "nats_prefill.hip", "nats_prefill_f32.hip", "nats_decode.hip", "nats_evict.hip", "nats_glue.hip"]
 
 HIPCC_FLAGS = [
@@ -45,7 +48,21 @@ def build(verbose: bool = True) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
+    build_host(verbose)
     return LIB_PATH
+
+
+def build_host(verbose: bool = True) -> str:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", os.path.join(root, "include"),
+           "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I", sysconfig.get_paths()["include"], "-I", INCLUDE,
+           HOST_SOURCE, "-L", os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python", "-o", HOST_PATH]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    return HOST_PATH
 
 
 if __name__ == "__main__":

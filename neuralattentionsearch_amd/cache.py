@@ -434,6 +434,17 @@ class NAtSChunkLayerCache:
         """`update` for a cache that already holds rows, with the rotary embedding of q and k applied on the way
         (one kernel: hf/llama_nats_chunk.py:227 + nats_chunk_layer_cache.py:243-256).  q / k / v are the projections
         before the rotary embedding; returns (rotated q, keys, values)."""
+        q_rot, end = self._append_rotated(q, key_states, value_states, cos, sin, token_states_info, roles)
+        return q_rot, self._buf_k[:, :, :end], self._buf_v[:, :, :end]
+
+    def step_attention(self, q, key_states, value_states, cos, sin, token_states_info, roles, sm_scale: float):
+        """`append_rotated` of one token per sequence and its attention over the cache: [B, H_q, 1, D]."""
+        q_rot, end = self._append_rotated(q, key_states, value_states, cos, sin, token_states_info, roles)
+        row_end, tail_start = self.decode_hint()
+        # (the buffers as they lie: rows behind `end` are not looked at)
+        return ops.decode_attention(q_rot, self._buf_k, self._buf_v, self._buf_valid, end, sm_scale, row_end=row_end, tail_start=tail_start)
+
+    def _append_rotated(self, q, key_states, value_states, cos, sin, token_states_info, roles):
         if self._buf_k is None and self._pending is None:
             raise ValueError("append_rotated needs a cache that holds rows; the first segment goes through update")
         x_len = key_states.shape[2]
@@ -446,9 +457,8 @@ class NAtSChunkLayerCache:
         start = self.n_ctx_data
         end = start + x_len
         self._grow(math.ceil(end / self.chunk_size) * self.chunk_size)
-        q_rot = ops.rope_append(q, key_states, value_states, cos, sin, self._buf_k, self._buf_v, self._buf_valid,
-                                self._buf_pos, start, self._seen_tokens)
-        return q_rot, self._buf_k[:, :, :end], self._buf_v[:, :, :end]
+        return ops.rope_append(q, key_states, value_states, cos, sin, self._buf_k, self._buf_v, self._buf_valid, self._buf_pos, start,
+                               self._seen_tokens), end
 
     # -- masks (nats_chunk_layer_cache.py:156-163, 444-460, 622-632) ------------------------------
     def generate_mask(self, x_len: int):
@@ -692,8 +702,7 @@ class NAtSLayerCache(NAtSChunkLayerCache):
         self._write_rows(key_states, value_states, start, end)
         return self._buf_k[:, :, :end], self._buf_v[:, :, :end]
 
-    def append_rotated(self, q, key_states, value_states, cos, sin, token_states_info=None, roles=None):
-        """`update` for a cache that already holds rows, with the rotary embedding of q and k applied on the way."""
+    def _append_rotated(self, q, key_states, value_states, cos, sin, token_states_info, roles):
         if self._buf_k is None and self._pending is None:
             raise ValueError("append_rotated needs a cache that holds rows; the first segment goes through update")
         if token_states_info is None and roles is None:
@@ -706,9 +715,8 @@ class NAtSLayerCache(NAtSChunkLayerCache):
         end = start + x_len
         self._grow(end)
         clear, self._clear_slot = self._clear_slot, None
-        q_rot = ops.rope_append(q, key_states, value_states, cos, sin, self._buf_k, self._buf_v, self._buf_valid,
-                                self._buf_pos, start, self._seen_tokens, -1 if clear is None else clear)
-        return q_rot, self._buf_k[:, :, :end], self._buf_v[:, :, :end]
+        return ops.rope_append(q, key_states, value_states, cos, sin, self._buf_k, self._buf_v, self._buf_valid, self._buf_pos, start,
+                               self._seen_tokens, -1 if clear is None else clear), end
 
     # -- masks (nats_layer_cache.py:155-162, 469-554) ------------------------------------------------
     def generate_mask(self, x_len: int):

@@ -206,10 +206,7 @@ class NAtSLlamaAttention(nn.Module):
             roles, tsi = ops.roles_from_logits(logit, 0.0, force_first_global=start_pos < C, force_last_global=pad != 0)
         layer = past_key_value.cache_model[idx]
         cos, sin = position_embeddings
-        q, keys, values = layer.append_rotated(q, k, v, cos, sin, tsi, roles)
-        row_end, tail_start = layer.decode_hint()
-        out = ops.decode_attention(q, keys, values, layer.valid_tokens, keys.shape[2], 1.0 / math.sqrt(D),
-                                   row_end=row_end, tail_start=tail_start)
+        out = layer.step_attention(q, k, v, cos, sin, tsi, roles, 1.0 / math.sqrt(D))
         past_key_value.post_update(layer_idx=idx, x_len=1)
         return step_linear(out.transpose(1, 2).reshape(bsz, 1, -1), self.o_proj)
 

@@ -84,6 +84,30 @@ def workspace(device, key: str, nbytes: int) -> torch.Tensor:
     return buf
 
 
+class _NativeFront:
+    """The functions of _nats_host.so, bound to the loaded library at the first call.  Those that stand for an operator
+    below take its plain form and answer None to everything else, for which the operator goes its general way; the others
+    take addresses and sizes their callers have checked and return the library's error code."""
+
+    def __getattr__(self, name):
+        try:
+            from . import _nats_host
+        except ImportError as e:
+            raise ImportError("_nats_host.so is missing or does not fit this torch: build it with `python -m "
+                              f"neuralattentionsearch_amd.build` ({e})") from e
+        lib = _lib.load()
+        names = [n for n in _lib.SIGNATURES if n not in ("nats_abi_version", "nats_last_error")]
+        raw = _raw_stream or (lambda i: torch.cuda.current_stream(i).cuda_stream)
+        _nats_host.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, _workspaces, workspace, raw)
+        for n in dir(_nats_host):
+            if not n.startswith("_") and n != "bind":
+                self.__dict__[n] = getattr(_nats_host, n)
+        return self.__dict__[name]
+
+
+_front = _NativeFront()
+
+
 # ------------------------------------------------------------------------------------------------
 # roles
 # ------------------------------------------------------------------------------------------------
@@ -92,6 +116,11 @@ def roles_from_logits(logits: torch.Tensor, global_bias: float = 0.1, force_firs
     """logits [B, S, H_kv, 3] -> (roles uint8 [B, H_kv, S], token_states_info [B, H_kv, S, 3] or None).
 
     models/transformer/attention/nats_attention.py:96-109."""
+    pair = _front.roles_from_logits(logits, global_bias, force_first_global, force_last_global, with_one_hot)
+    if pair is not None:
+        if pair[1] is not None:
+            _attach_roles(pair[1], pair[0])
+        return pair
     _require_cuda(logits)
     lib = _lib.load()
     if logits.dim() != 4 or logits.shape[-1] != 3:
@@ -251,6 +280,8 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, roles: 
 
     q [B, H_q, L, D], k / v [B, H_kv, L, D] (any strides with a contiguous last dimension), roles uint8
     [B, H_kv, ceil(L / chunk_size)].  Returns [B, H_q, L, D] (or fills `out`, which may be strided)."""
+    if out is None and (done := _front.prefill(q, k, v, roles, chunk_size, window, sm_scale)) is not None:
+        return done
     _require_cuda(q, k, v, roles)
     lib = _lib.load()
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
@@ -439,6 +470,9 @@ def decode_attention(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tens
     Attends to rows i < n_rows with valid[b, h, i]; returns [B, H_q, 1, D].
     Optional hint: `row_end` int64 [B, H_kv] and `tail_start` state that rows [row_end, tail_start) of a head
     hold nothing valid (size_global_kv + size_local_kv and the start of the open chunk); they are skipped."""
+    done = _front.decode(q, cache_k, cache_v, valid, n_rows, sm_scale, row_end, tail_start)
+    if done is not None:
+        return done
     _require_cuda(q, cache_k, cache_v, valid)
     lib = _lib.load()
     if q.dim() != 4 or cache_k.dim() != 4 or valid.dim() != 3:
@@ -624,12 +658,10 @@ class CacheAppendCall:
         e = 16 // cache_k.element_size()
         fix = lambda t: tuple(st if n != 1 else e for st, n in zip(t.stride()[:3], t.shape[:3]))
         B, H, x_len, D = k.shape
-        self.fn = _lib.load().nats_cache_append
-        self.fn_plan = _lib.load().nats_cache_append_plan
         self.head = (_ptr(cache_k), _ptr(cache_v), _ptr(valid), _ptr(pos), B, H, x_len, D)
         self.n_rows = min(cache_k.shape[2], valid.shape[2])
-        self.tail = (i64_array(fix(k)), i64_array(fix(v)), i64_array(fix(cache_k)), i64_array(valid.stride()[:2]),
-                     cache_k.element_size())
+        self.strides = [i64_array(s) for s in (fix(k), fix(v), fix(cache_k), valid.stride()[:2])]
+        self.tail = (*(ctypes.addressof(s) for s in self.strides), cache_k.element_size())
 
     def matches(self, k, v, cache_k, cache_v, valid, pos) -> bool:
         b = self.bufs
@@ -644,11 +676,11 @@ class CacheAppendCall:
         if not self.ok or (pk | pv) & 15:
             return False
         if plan is None:
-            check(self.fn(pk, pv, *self.head, row0, self.n_rows, pos0, *self.tail, _stream(k)))
+            check(_front.cache_append(pk, pv, *self.head, row0, self.n_rows, pos0, *self.tail, _stream(k)))
         else:
             params.seq = plan.buffers.next_seq()
-            check(self.fn_plan(pk, pv, *self.head, row0, self.n_rows, pos0, *self.tail, roles.data_ptr(), *plan.sizes,
-                               ctypes.byref(params), *plan.plan_tail, _stream(k)))
+            check(_front.cache_append(pk, pv, *self.head, row0, self.n_rows, pos0, *self.tail, roles.data_ptr(), *plan.sizes,
+                                      ctypes.addressof(params), *plan.plan_tail, _stream(k)))
         return True
 
 
@@ -669,12 +701,11 @@ class EvictInplaceCall:
         self.buffers = buffers
         ws = buffers.workspace(lib.nats_evict_workspace_bytes(B, H_kv, S))
         self.ws = ws
-        self.plan, self.apply = lib.nats_evict_plan, lib.nats_evict_apply_inplace
         self.sizes = (_ptr(size_global), _ptr(size_local))
         self.plan_tail = (_ptr(ws), ws.numel(), _ptr(buffers.result), _ptr(buffers.mirror))
         self.apply_head = (_ptr(cache_k), _ptr(cache_v), _ptr(v8), _ptr(pos))
-        self.apply_tail = (i64_array(cache_k.stride()[:3]), i64_array(v8.stride()[:2]), cache_k.element_size(), _ptr(ws),
-                           _ptr(buffers.result))
+        self.strides = [i64_array(cache_k.stride()[:3]), i64_array(v8.stride()[:2])]
+        self.apply_tail = (*(ctypes.addressof(s) for s in self.strides), cache_k.element_size(), _ptr(ws), _ptr(buffers.result))
 
     def matches(self, cache_k, cache_v, valid, pos, S) -> bool:
         b = self.bufs
@@ -687,14 +718,15 @@ class EvictInplaceCall:
         if not roles.is_cuda or roles.dtype != torch.uint8 or not roles.is_contiguous():
             raise ValueError("roles must be a contiguous uint8 GPU tensor")
         params.seq = self.buffers.next_seq()
-        pr, ref, st = roles.data_ptr(), ctypes.byref(params), _stream(roles)
-        check(self.plan(pr, *self.sizes, ref, *self.plan_tail, st))
-        check(self.apply(*self.apply_head, pr, *self.sizes, ref, *self.apply_tail, st))
+        pr, ref, st = roles.data_ptr(), ctypes.addressof(params), _stream(roles)
+        check(_front.evict_plan(pr, *self.sizes, ref, *self.plan_tail, st))
+        check(_front.evict_apply_inplace(*self.apply_head, pr, *self.sizes, ref, *self.apply_tail, st))
 
     def apply_planned(self, roles: torch.Tensor, params: EvictParams):
         """The apply step alone, for an eviction whose plan rode with the append (`CacheAppendCall(..., plan=self)`):
         `params` are the ones that launch was given, sequence number included."""
-        check(self.apply(*self.apply_head, roles.data_ptr(), *self.sizes, ctypes.byref(params), *self.apply_tail, _stream(roles)))
+        check(_front.evict_apply_inplace(*self.apply_head, roles.data_ptr(), *self.sizes, ctypes.addressof(params), *self.apply_tail,
+                                         _stream(roles)))
 
 
 def evict_apply_inplace(cache_k, cache_v, valid, pos, roles, size_global, size_local, params: EvictParams, ws, result):
@@ -787,6 +819,9 @@ def matvec_ok(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def matvec(x: torch.Tensor, weight: torch.Tensor, gate: bool = False) -> torch.Tensor:
     """nn.functional.linear(x, weight) for up to four rows of x: [..., K] x [N, K] -> [..., N].
     gate=True: weight is [2 * I, K] (gate rows, then up rows) and the result is silu(x W_g^T) * (x W_u^T), [..., I]."""
+    done = _front.matvec(x, weight, gate)
+    if done is not None:
+        return done
     _require_cuda(x, weight)
     if not matvec_ok(x, weight):
         raise ValueError("matvec: x [<= 4 rows, K] contiguous and weight [N, K] of the same dtype, K a multiple of 16 bytes")
@@ -825,6 +860,9 @@ class MatvecPlan:
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         """x must satisfy `takes(x)`."""
+        weight = self.weight()
+        if weight is not None and (done := _front.matvec(x, weight, self.gate)) is not None:
+            return done
         k, n = self.k, self.n
         y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
         check(self.fn(self.w_ptr, x.data_ptr(), y.data_ptr(), x.numel() // k, n, k, self.w_stride, k, n, self.gate,
@@ -839,11 +877,6 @@ def step_project_ok(x: torch.Tensor, weights) -> bool:
             and all(_matvec_weight_ok(w) and w.dtype == x.dtype and w.shape[1] == k for w in weights))
 
 
-def matvec_weight_ok(weight: torch.Tensor, dtype: torch.dtype, k: int) -> bool:
-    """Whether `matvec` takes this matrix for rows of k entries of this dtype."""
-    return _matvec_weight_ok(weight) and weight.dtype == dtype and weight.shape[1] == k
-
-
 def step_project(x: torch.Tensor, weights, chunk_size: int = 1, carry_in: torch.Tensor | None = None, with_carry: bool = False,
                  role_weight: torch.Tensor | None = None, roles_out: torch.Tensor | None = None, global_bias: float = 0.1,
                  force_first_global: bool = False):
@@ -851,6 +884,9 @@ def step_project(x: torch.Tensor, weights, chunk_size: int = 1, carry_in: torch.
     [B, 1, sum n_i]; with `with_carry` also the chunk statistic carry_in + x / chunk_size, [B, 1, k]; with `roles_out`
     (uint8 [B, H_kv, 1], laid out as `role_destination` and `torch.empty` make it) the roles from that statistic and
     `role_weight` [H_kv * 3, k].  Returns (products, statistic or None)."""
+    done = try_step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global)
+    if done is not None:
+        return done
     B, k = x.numel() // x.shape[-1], x.shape[-1]
     if not step_project_ok(x, weights) or not 1 <= len(weights) <= 4:
         raise ValueError("step_project: x [<= 4 rows, k] contiguous and 1..4 matrices [n, k] of its dtype, k a multiple of 16 bytes")
@@ -863,12 +899,6 @@ def step_project(x: torch.Tensor, weights, chunk_size: int = 1, carry_in: torch.
                 or not role_weight.is_cuda or roles_out.dtype != torch.uint8 or tuple(roles_out.shape) != (B, H, 1)
                 or not roles_out.is_cuda or (B > 1 and roles_out.stride(0) != H * roles_out.stride(1))):
             raise ValueError("step_project: role_weight [H_kv * 3, k] of x's dtype and roles_out uint8 [B, H_kv, 1]")
-    return launch_step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global)
-
-
-def launch_step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global):
-    """`step_project` for a caller that has made its checks."""
-    B, k = x.numel() // x.shape[-1], x.shape[-1]
     n = [w.shape[0] for w in weights]
     total = sum(n)
     y = torch.empty(B, 1, total, dtype=x.dtype, device=x.device)
@@ -880,6 +910,16 @@ def launch_step_project(x, weights, chunk_size, carry_in, with_carry, role_weigh
                                         _ptr(roles_out), hs, _ptr(carry_in), _ptr(carry), int(chunk_size), _dtype_code(x),
                                         _stream(x)))
     return y, carry
+
+
+def try_step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global):
+    """`step_project`, or None (and nothing done) for tensors it does not take."""
+    return _front.step_project(x, weights, chunk_size, carry_in, with_carry, role_weight, roles_out, global_bias, force_first_global)
+
+
+def matvec_takes(x: torch.Tensor, weight: torch.Tensor, k: int) -> bool:
+    """Whether `matvec` takes this matrix for rows of k entries of x's type on x's device."""
+    return _front.matvec_takes(x, weight, k)
 
 
 def rope_qk_ok(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
@@ -915,6 +955,9 @@ def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Te
     bytes (and stream positions).  q [B, H_q, x_len, D], k / v [B, H_kv, x_len, D] (any strides, last dimension
     contiguous), cos / sin [B, x_len, D].  `clear_row` >= 0: the valid byte of that row (below row0) is set to 0 in
     every head.  Returns the rotated q, contiguous."""
+    done = _front.rope_append(q, k, v, cos, sin, cache_k, cache_v, valid, pos, row0, pos0, clear_row)
+    if done is not None:
+        return done
     _require_cuda(q, k, v, cos, sin, cache_k, cache_v, valid, pos)
     B, Hq, x_len, D = q.shape
     Hkv = k.shape[1]

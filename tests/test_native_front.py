@@ -1,0 +1,105 @@
+"""The native front of the step-wise operators: it answers None to every form it does not take, and what it takes comes
+out as on the general way, bit for bit."""
+import pytest
+import torch
+
+from neuralattentionsearch_amd import ops
+from tests.gpu_util import say
+
+
+class NoFront:
+    """The general way: every operator of the front declines."""
+
+    def __init__(self, front):
+        self.front = front
+
+    def __getattr__(self, name):
+        if name in ("cache_append", "evict_plan", "evict_apply_inplace", "matvec_takes"):
+            return getattr(self.front, name)
+        return lambda *a: None
+
+
+def test_declines_what_is_not_plain():
+    t = torch.zeros(1, 2, 1, 32)  # (not on a GPU)
+    v = torch.zeros(1, 2, 8, dtype=torch.uint8)
+    f = ops._front
+    assert f.decode(t, t, t, v, 1, None, None, None) is None
+    assert f.decode(None, 1, "x", t, 1.5, None, None, None) is None
+    assert f.decode(t) is None
+    assert f.prefill(t, t, t, v, 8, 8, None) is None
+    assert f.roles_from_logits(t, 0.1, True, False, True) is None
+    assert f.rope_append(*[t] * 7, v, None, 0, 0, -1) is None
+    assert f.matvec(t, t, False) is None
+    assert f.matvec_takes(t, t, 32) is False
+    assert f.step_project(t, (t,), 1, None, True, None, None, 0.1, False) is None
+    assert f.step_project(t, [t], 1, None, True, None, None, 0.1, False) is None
+    assert f.add_rms_norm(t, None, t, 1e-5, None, 0, 1) is None
+    with pytest.raises(TypeError):
+        f.cache_append(1, 2)
+    with pytest.raises(ValueError):  # (and the operator says why)
+        ops.decode_attention(t, t, t, v, 1)
+
+
+def both(monkeypatch, call):
+    got = call()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_front", NoFront(ops._front))
+        want = call()
+    return got, want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("layout", ["plain", "strided", "single"])
+def test_equals_the_general_way(dtype, layout, monkeypatch):
+    say("native front", dtype, layout)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    B, Hq, Hkv, D, N = (1, 4, 1, 64, 300) if layout == "single" else (3, 8, 4, 64, 300)
+    taken = []
+    real = ops._front.decode
+
+    # decode: caches that are slices of larger buffers, bool and uint8 valid rows, q that is a transposed view
+    k, v = (rn(B, Hkv, N + 84, D)[:, :, :N + 20] if layout == "strided" else rn(B, Hkv, N, D) for _ in range(2))
+    valid = torch.rand(B, Hkv, k.shape[2], generator=g, device="cuda") < 0.7
+    q = rn(B, 1, Hq, D).transpose(1, 2) if layout == "strided" else rn(B, Hq, 1, D)
+    end = torch.full((B, Hkv), 200, device="cuda")
+    for args in ((q, k, v, valid, N), (q, k, v, valid.to(torch.uint8), N - 7, 0.3), (q, k, v, valid, N, None, end, 290),
+                 (q, k, v, valid, N, None, end.t().contiguous().t(), 290)):
+        a, b = both(monkeypatch, lambda: ops.decode_attention(*args))
+        assert a.shape == b.shape == (B, Hq, 1, D) and torch.equal(a, b)
+    # prefill and roles
+    L, C, W = 77, 16, 32
+    logits = rn(B, -(-L // C), Hkv, 3)
+    if layout == "strided":
+        logits = rn(B, Hkv, -(-L // C), 3).transpose(1, 2)
+    (r1, h1), (r2, h2) = both(monkeypatch, lambda: ops.roles_from_logits(logits, 0.1, True, True))
+    assert torch.equal(r1, r2) and torch.equal(h1, h2) and ops.roles_from_one_hot(h1) is r1
+    pq, pk, pv = ((rn(B, L, h, D).transpose(1, 2) if layout == "strided" else rn(B, h, L, D)) for h in (Hq, Hkv, Hkv))
+    a, b = both(monkeypatch, lambda: ops.prefill_attention(pq, pk, pv, r1, C, W, 0.2))
+    assert torch.equal(a, b)
+    # rotary embedding with the append
+    cos, sin = rn(B, 1, D), rn(B, 1, D)
+    qkv = rn(B, 1, Hq + 2 * Hkv, D).transpose(1, 2)
+
+    def append():
+        ck, cv = torch.zeros(B, Hkv, 16, D, dtype=dtype, device="cuda"), torch.zeros(B, Hkv, 16, D, dtype=dtype, device="cuda")
+        val, pos = torch.ones(B, Hkv, 16, dtype=torch.uint8, device="cuda"), torch.zeros(B, Hkv, 16, dtype=torch.int32, device="cuda")
+        out = ops.rope_append(qkv[:, :Hq], qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:], cos, sin, ck, cv, val, pos, 5, 9, 2)
+        return torch.cat([t.flatten().double() for t in (out, ck, cv, val, pos)])
+
+    a, b = both(monkeypatch, append)
+    assert torch.equal(a, b)
+    # rows and matrices
+    x, w = rn(B, 1, 256), torch.nn.Parameter(rn(64, 256), requires_grad=False)
+    for gate in (False, True):
+        a, b = both(monkeypatch, lambda: ops.matvec(x, w, gate))
+        assert torch.equal(a, b)
+    a, b = both(monkeypatch, lambda: ops.add_rms_norm(x.clone(), x, rn(256) * 0 + 1, 1e-5))
+    assert torch.equal(a, b)
+
+    # a call with new scratch needs takes the operator's own table
+    monkeypatch.setattr(ops._front, "decode", lambda *a: taken.append(real(*a)) or taken[-1], raising=False)
+    ops._workspaces.clear()
+    ops.decode_attention(rn(B, Hq, 1, D), k, v, valid, N)
+    assert taken[-1] is not None and len(ops._workspaces) == 1
