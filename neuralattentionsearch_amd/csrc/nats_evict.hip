@@ -24,6 +24,8 @@
 
 #include <stddef.h>
 
+#include <algorithm>
+
 namespace nats {
 
 struct HeadPlan {
@@ -122,8 +124,8 @@ __device__ __forceinline__ void plan_one_head(const uint8_t* __restrict__ roles,
   } else {
     // pass 1: counts and the last complete global slot
     int n_glob_all = 0, n_sw = 0, n_loc = 0, last_g = -1;
+    int rb[kSlotsPerLane];
     for (int base = 0; base < S; base += kSlotsPerBlock) {
-      int rb[kSlotsPerLane];
       load_roles(r, S, base, lane, rb);
 #pragma unroll
       for (int j = 0; j < kSlotsPerLane; ++j) {
@@ -141,8 +143,7 @@ __device__ __forceinline__ void plan_one_head(const uint8_t* __restrict__ roles,
     // pass 2: kept slots in order, destination rank by prefix sum (stream compaction of slot ids)
     int count = 0, later_local = 0;
     for (int base = 0; base < S; base += kSlotsPerBlock) {
-      int rb[kSlotsPerLane];
-      load_roles(r, S, base, lane, rb);
+      if (S > kSlotsPerBlock) load_roles(r, S, base, lane, rb);  // (else the first pass has left them in the registers)
       unsigned kept_bits = 0;
       int loc_after = 0;
 #pragma unroll
@@ -282,6 +283,7 @@ __device__ __forceinline__ void plan_finalize(const int64_t* __restrict__ size_g
   w.max_tot_new = 0; w.max_tot_old = 0; w.max_tot_alllocal = 0;
   w.min_sg_new = 0x7fffffffffffffffLL; w.min_sg_old = 0x7fffffffffffffffLL; w.sum_keep = 0;
   for (int h = tid; h < n_heads; h += 256) {
+    if (tid >= 256) break;
     HeadPlan hp;
     if (kCoherent) {  // plans written by other workgroups of this launch
       uint64_t w[sizeof(HeadPlan) / 8];
@@ -301,9 +303,10 @@ __device__ __forceinline__ void plan_finalize(const int64_t* __restrict__ size_g
     x.min_sg_new = hp.sg_new; x.min_sg_old = sg; x.sum_keep = hp.count;
     fold(w, x);
   }
-  agg[tid] = w;
+  if (tid < 256) agg[tid] = w;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
+    if (o >= n_heads) continue;  // (entries from n_heads on are neutral)
     if (tid < o) fold(agg[tid], agg[tid + o]);
     __syncthreads();
   }
@@ -345,7 +348,7 @@ __device__ __forceinline__ void plan_finalize(const int64_t* __restrict__ size_g
   __syncthreads();
   if (all_local_flag) {
     // every slot local: nothing moves and only the local size grows (:747-749, :356)
-    for (int h = tid; h < n_heads; h += 256) {
+    for (int h = tid; h < n_heads && tid < 256; h += 256) {
       plans[h].sg_new = old_size_global(p, size_global, h);
       plans[h].sl_new = old_size_local(p, size_local, h) + (long long)n_done * C;
     }
@@ -361,6 +364,20 @@ __global__ __launch_bounds__(256) void evict_plan_small_kernel(const uint8_t* __
                                                                nats_evict_brief* __restrict__ result_mirror) {
   const int n_heads = (int)(p.B * p.H_kv);
   for (int head = threadIdx.x; head < n_heads; head += 256) plan_one_head_serial(roles, size_global, size_local, p, ws, head);
+  __syncthreads();  // (global writes of this workgroup are visible to it after the barrier)
+  plan_finalize(size_global, size_local, p, ws, result, result_mirror);
+}
+
+// The heads of one sequence or two: a wavefront per head, all in one workgroup of up to 16, which folds them itself (no
+// ticket, no plans past the caches: 64 slots of 8 heads 9.9 -> 7.7 us).
+constexpr int kPlanOneHeads = 16;
+__global__ __launch_bounds__(kPlanOneHeads * kWave) void evict_plan_one_kernel(const uint8_t* __restrict__ roles,
+                                                                               const int64_t* __restrict__ size_global,
+                                                                               const int64_t* __restrict__ size_local, nats_evict_params p,
+                                                                               char* __restrict__ ws, nats_evict_result* __restrict__ result,
+                                                                               nats_evict_brief* __restrict__ result_mirror) {
+  const int head = threadIdx.x >> 6;
+  if (head < (int)(p.B * p.H_kv)) plan_one_head(roles, size_global, size_local, p, ws, head, threadIdx.x & 63);
   __syncthreads();  // (global writes of this workgroup are visible to it after the barrier)
   plan_finalize(size_global, size_local, p, ws, result, result_mirror);
 }
@@ -421,7 +438,9 @@ struct TensorView {
 };
 
 constexpr int kFirstUnr = 4;  // 16-byte units a thread of the out-of-place kernel has in flight
-constexpr int kUnr = 4;  // moves per wavefront and batch
+// entries per wavefront and batch: what a segment moves in one batch, or few registers for a step of a stream, whose many
+// workgroups wait for each other's bandwidth rather than for a second batch
+constexpr int kUnrMany = 8, kUnrFew = 2;
 constexpr int kNu = 2;   // units per lane and chunk slice (a slice holds at most 128 units)
 
 template <typename U>
@@ -431,7 +450,7 @@ __device__ __forceinline__ uint4 zero_unit<uint4>() { return make_uint4(0, 0, 0,
 template <>
 __device__ __forceinline__ int32_t zero_unit<int32_t>() { return -1; }  // "no token" in the position shadow
 
-template <typename U>
+template <int kUnr, typename U>
 __device__ void apply_inplace_body(const ApplyArgs& a, TensorView<U> t, int head, int slice, bool owns_valid) {
   const nats_evict_params& p = a.p;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -441,92 +460,101 @@ __device__ void apply_inplace_body(const ApplyArgs& a, TensorView<U> t, int head
   const int wc = (int)(p.W / p.C);
   const int64_t off = p.n_ctx_data / p.C;
   const int n_heads = (int)(p.B * p.H_kv);
-  const nats_evict_result res = *a.result;
-  const HeadPlan hp = reinterpret_cast<const HeadPlan*>(a.ws + kPlanHeaderBytes)[head];
   const int32_t* keep = reinterpret_cast<const int32_t*>(a.ws + plan_lists_offset(n_heads)) + (int64_t)head * S;
   const uint8_t* r = a.roles + (int64_t)head * S;
   const int units = a.rs * t.upr;  // per chunk slice
   const int row0 = slice * a.rs;
+  const int n_ring = n_done < wc ? n_done : wc;
 
   auto unit_ptr = [&](int64_t chunk, int u) -> U* {
     return t.base + (chunk * C + row0 + u / t.upr) * t.row_stride + (u % t.upr);
   };
 
-  // 1. ring insert (:391-437)
+  // One ordered list of copies: the ring inserts (:391-437), then the chunk moves.  Wavefront w takes entries w, w + 4, ...
+  // of a batch; the batch is read completely before it is written.  Ring inserts may stand in front: their sources are
+  // rows that moves can only overwrite later, their destinations are nobody's source.
+  // What an entry needs to know (the role of a ring slot, the chunk a move takes) is one load per lane for the whole batch,
+  // requested for the first batch beside the plan itself: the kernel is a chain of trips to memory, here plan -> rows.
+  auto load_meta = [&](int b0) -> int {
+    const int i = b0 + (lane & (kUnr - 1)) * 4 + wave;
+    if (i < n_ring) return r[n_done - n_ring + i];
+    return i - n_ring < S ? keep[i - n_ring] : 0;
+  };
+  int meta = load_meta(0);
+  const nats_evict_result res = *a.result;
+  const HeadPlan hp = reinterpret_cast<const HeadPlan*>(a.ws + kPlanHeaderBytes)[head];
+
   const bool token = p.update_chunk != 0;
-  const int n_ring = n_done < wc ? n_done : wc;
   // the chunked cache's tail is the next slot to write, the per-token cache's the slot written last; its one-step
   // branch writes one slot further on (nats_layer_cache.py:340-345: slot 1 for the first token ever, else tail + 2,
   // while the tail itself advances by one), unless every head's token is sliding-window (:316-317)
   const int skip = token && one_step_scatter(p) && !res.all_sw ? 1 : 0;
   const int start_chunk = p.first ? skip : token ? (int)((p.tail + 1 + skip) % p.W) : (int)(p.tail / p.C);
-  for (int j = wave; j < n_ring; j += 4) {
-    int slot = n_done - n_ring + j;
-    bool is_sw = r[slot] == NATS_ROLE_SW;
-    int rc = (start_chunk + j) % wc;
-    for (int u = lane; u < units; u += kWave) {
-      U val = (is_sw || token) ? *unit_ptr(off + slot, u) : zero_unit<U>();  // (nats_layer_cache.py:451-454 copies all)
-      *unit_ptr(rc, u) = val;
-    }
-    if (owns_valid && lane < a.rs) {
-      a.valid[(int64_t)(head / p.H_kv) * a.vs_b + (int64_t)(head % p.H_kv) * a.vs_h + (int64_t)rc * C + row0 + lane] = is_sw;
-    }
-  }
-  if (res.all_sw) return;
-  __syncthreads();
-
-  // 2. ordered chunk moves, each batch read completely before it is written
-  int n_moves;
-  bool tail_move = false;
-  if (one_step_scatter(p)) {
-    n_moves = 1;
-  } else if (res.all_local) {
+  int n_moves = 0;
+  if (res.all_sw || (res.all_local && !one_step_scatter(p))) {
     n_moves = 0;
+  } else if (one_step_scatter(p)) {
+    n_moves = 1;
   } else {
-    tail_move = partial && res.max_keep < S - 1;
-    n_moves = hp.count + (tail_move ? 1 : 0);
+    n_moves = hp.count + (partial && res.max_keep < S - 1 ? 1 : 0);
   }
-  for (int b0 = 0; b0 < n_moves; b0 += 4 * kUnr) {
+  const int n_entries = n_ring + n_moves;
+  for (int b0 = 0; b0 < n_entries; b0 += 4 * kUnr) {
     U regs[kUnr][kNu];
     int64_t dsts[kUnr];
 #pragma unroll
     for (int k = 0; k < kUnr; ++k) {
-      int mv = b0 + wave * kUnr + k;
+      const int i = b0 + k * 4 + wave;
+      const int m = __builtin_amdgcn_readlane(meta, k);
       dsts[k] = -1;
-      if (mv < n_moves) {
+#pragma unroll
+      for (int e = 0; e < kNu; ++e) regs[k][e] = zero_unit<U>();
+      if (i < n_entries) {
         int64_t src, dst;
-        if (mv < hp.count) {
-          src = off + keep[mv];
-          dst = hp.dst_base + mv;
+        bool copy = true;
+        if (i < n_ring) {
+          src = off + n_done - n_ring + i;
+          dst = (start_chunk + i) % wc;
+          copy = m == NATS_ROLE_SW || token;  // (nats_layer_cache.py:451-454 copies all)
+          if (owns_valid && lane < a.rs)
+            a.valid[(int64_t)(head / p.H_kv) * a.vs_b + (int64_t)(head % p.H_kv) * a.vs_h + dst * C + row0 + lane] = m == NATS_ROLE_SW;
+        } else if (i - n_ring < hp.count) {
+          src = off + m;
+          dst = hp.dst_base + (i - n_ring);
         } else {
           src = off + S - 1;
           dst = res.max_end;
         }
         if (src != dst) {
           dsts[k] = dst;
+          if (copy) {
 #pragma unroll
-          for (int e = 0; e < kNu; ++e) {
-            int u = lane + e * kWave;
-            if (u < units) regs[k][e] = *unit_ptr(src, u);
+            for (int e = 0; e < kNu; ++e) {
+              const int u = lane + e * kWave;
+              if (u < units) regs[k][e] = *unit_ptr(src, u);
+            }
           }
         }
       }
     }
+    if (b0 + 4 * kUnr < n_entries) meta = load_meta(b0 + 4 * kUnr);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kUnr; ++k) {
       if (dsts[k] >= 0) {
 #pragma unroll
         for (int e = 0; e < kNu; ++e) {
-          int u = lane + e * kWave;
-          if (u < units) *unit_ptr(dsts[k], u) = regs[k][e];
+          const int u = lane + e * kWave;
+          // (rows from n_ctx_data on are to be zero, see below: whoever writes them writes that)
+          if (u < units) *unit_ptr(dsts[k], u) = !token && dsts[k] * C + row0 + u / t.upr >= res.n_ctx_data ? zero_unit<U>() : regs[k][e];
         }
       }
     }
   }
-  __syncthreads();
+  if (res.all_sw) return;
 
-  // 3. rows >= n_ctx_data are zeroed (:360-362); the per-token cache leaves them as they are
+  // rows >= n_ctx_data are zeroed (:360-362); the per-token cache leaves them as they are.  (Every source has been read:
+  // the last batch's barrier is behind.)
   const int64_t n_chunks_alloc = token ? 0 : p.n_alloc / C;
   for (int64_t ci = res.n_ctx_data / C + wave; ci < n_chunks_alloc; ci += 4) {
     for (int u = lane; u < units; u += kWave) {
@@ -536,7 +564,7 @@ __device__ void apply_inplace_body(const ApplyArgs& a, TensorView<U> t, int head
   }
 
   if (owns_valid) {
-    // 4. valid_tokens rewrite with the minimum global size from before this call (:634-656)
+    // valid_tokens rewrite with the minimum global size from before this call (:634-656)
     const long long sg_new = hp.sg_new, sl_new = hp.sl_new;
     if (res.n_ctx_data != p.gmin) {
       uint8_t* vrow = a.valid + (int64_t)(head / p.H_kv) * a.vs_b + (int64_t)(head % p.H_kv) * a.vs_h;
@@ -553,6 +581,8 @@ __device__ void apply_inplace_body(const ApplyArgs& a, TensorView<U> t, int head
   }
 }
 
+// (16 sequences of 8 heads, one chunk of 64 rows each: 11.6 -> 10.3 us; one sequence, a segment of 64 chunks, 17.7 -> 14.9 us)
+template <int kUnr>
 __global__ __launch_bounds__(256) void evict_apply_inplace_kernel(ApplyArgs a) {
   const int slice = blockIdx.x;
   const int head = blockIdx.y;
@@ -564,13 +594,13 @@ __global__ __launch_bounds__(256) void evict_apply_inplace_kernel(ApplyArgs a) {
     t.base = reinterpret_cast<uint4*>(static_cast<char*>(a.tensor[which]) + (b * a.ks_b + h * a.ks_h) * a.elem_bytes);
     t.row_stride = a.ks_r * a.elem_bytes / 16;
     t.upr = row_units;
-    apply_inplace_body<uint4>(a, t, head, slice, which == 0);
+    apply_inplace_body<kUnr, uint4>(a, t, head, slice, which == 0);
   } else {
     TensorView<int32_t> t;
     t.base = static_cast<int32_t*>(a.tensor[2]) + b * a.vs_b + h * a.vs_h;
     t.row_stride = 1;
     t.upr = 1;
-    apply_inplace_body<int32_t>(a, t, head, slice, false);
+    apply_inplace_body<kUnr, int32_t>(a, t, head, slice, false);
   }
 }
 
@@ -810,6 +840,13 @@ extern "C" int nats_evict_plan(const uint8_t* roles, const int64_t* size_global,
     NATS_CHECK_LAUNCH("evict_plan_small_kernel");
     return NATS_OK;
   }
+  if (params->B * params->H_kv <= kPlanOneHeads) {
+    const unsigned threads = (unsigned)std::max<int64_t>(256, params->B * params->H_kv * kWave);  // (the fold takes 256)
+    hipLaunchKernelGGL(evict_plan_one_kernel, dim3(1), dim3(threads), 0, st, roles, size_global, size_local, *params,
+                       static_cast<char*>(workspace), result, result_mirror);
+    NATS_CHECK_LAUNCH("evict_plan_one_kernel");
+    return NATS_OK;
+  }
   hipLaunchKernelGGL(evict_plan_heads_kernel, dim3(n_wg), dim3(256), 0, st, roles, size_global, size_local, *params,
                      static_cast<char*>(workspace), result, result_mirror);
   NATS_CHECK_LAUNCH("evict_plan_heads_kernel");
@@ -824,6 +861,8 @@ static int slice_geometry(const char* who, const nats_evict_params* p, int elem_
   int64_t r = 1;
   while (r * 2 <= p->C && r * 2 * row_bytes <= 2048 && p->C % (r * 2) == 0) r *= 2;
   NATS_REQUIRE(p->C % r == 0, NATS_ERR_UNSUPPORTED, "%s: chunk size %lld", who, (long long)p->C);
+  // a few heads: slices of 1 KiB (one 16-byte unit per lane), so that more compute units take part
+  while (r > 1 && p->B * p->H_kv * 2 * (p->C / r) < 512 && r * row_bytes > 1024) r /= 2;
   if (r > 128) r = 128;  // the position shadow moves one 4-byte unit per row
   *rs = (int)r;
   *n_slices = (int)(p->C / r);
@@ -857,7 +896,12 @@ extern "C" int nats_evict_apply_inplace(void* cache_k, void* cache_v, uint8_t* v
   a.vs_b = valid_strides[0]; a.vs_h = valid_strides[1];
   a.elem_bytes = elem_bytes;
   dim3 grid((unsigned)a.n_slices, (unsigned)(params->B * params->H_kv), pos ? 3u : 2u);
-  hipLaunchKernelGGL(evict_apply_inplace_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  const int64_t n_done = params->fill / params->C;
+  if (std::min(n_done, params->W / params->C) + params->S <= 4 * kUnrFew) {  // ring inserts and moves of a head, at most
+    hipLaunchKernelGGL(evict_apply_inplace_kernel<kUnrFew>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  } else {
+    hipLaunchKernelGGL(evict_apply_inplace_kernel<kUnrMany>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  }
   NATS_CHECK_LAUNCH("evict_apply_inplace_kernel");
   return NATS_OK;
 }
