@@ -10,7 +10,7 @@ INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libnats_hip.so")
 HOST_SOURCE = os.path.join(CSRC, "nats_host.cpp")  # the native front of the step-wise operators: a Python extension, no GPU code
 HOST_PATH = os.path.join(PKG_DIR, "_nats_host.so")
-SOURCES = ["nats_roles.hip", "nats_rolestep.hip", "nats_prefill.hip", "nats_prefill_f32.hip", "nats_decode.hip", "nats_evict.hip", "nats_glue.hip"]
+SOURCES = ["nats_roles.hip", "nats_rolestep.hip", "nats_prefill.hip", "nats_prefill_f32.hip", "nats_prefill_short.hip", "nats_decode.hip", "nats_evict.hip", "nats_glue.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",

@@ -9,6 +9,7 @@
 //   prefill_split_merge_kernel combines those partial results
 //   prefill_mfma_wide_kernel   bf16 MFMA kernel for head dim 256: four wavefronts with the whole register file, whole
 //                              tiles masked row by row
+//   prefill_short_kernel       bf16, short prompts from an empty cache in one launch (nats_prefill_short.hip)
 //   prefill_f32_kernel         fp32 on the fp32 matrix instruction (nats_prefill_f32.hip)
 //   prefill_simple_kernel      fp32 (or bf16) FMA kernel, one query row per lane: what the others do not take (head dim
 //                              16, fp32 at head dim 256, rows that are not 16-byte aligned)
@@ -1928,6 +1929,8 @@ extern "C" int nats_prefill_fwd(const void* q, const void* k, const void* v, con
   PrefillWorkspace w = carve_prefill_workspace(workspace, B * H_kv, S, L);
   NATS_REQUIRE(workspace_bytes >= w.bytes, NATS_ERR_WORKSPACE, "%s: workspace %zu bytes < %zu", who, workspace_bytes, w.bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (prefill_short_takes(B, H_q, D, L, dtype))
+    return launch_prefill_short(q, k, v, roles, o, B, H_q, H_kv, L, D, C, W, q_strides, k_strides, v_strides, o_strides, sm_scale, st);
   if (int rc = prepare_key_limits(roles, B, H_kv, S, L, C, W, nullptr, w, st)) return rc;
   return launch_segment(who, g, q, k, v, o, q_strides, k_strides, v_strides, o_strides, sm_scale, dtype, w,
                         static_cast<char*>(workspace) + w.bytes, workspace_bytes - w.bytes, st);
