@@ -1650,13 +1650,30 @@ static bool use_split() {
   const char* e = getenv("NATS_PREFILL_SPLIT");
   return !(e && e[0] == '0');
 }
-static int choose_split(int64_t n_wg, int64_t Tk) {
+static int most_split(int64_t n_wg, int64_t Tk) {
   const int n_cu = device_cu_count();
   if (!use_split() || n_cu <= 0 || n_wg * 2 > n_cu) return 1;
   int64_t n = n_cu / n_wg;
   if (n > kMaxSplit) n = kMaxSplit;
   if (n > Tk / 4) n = Tk / 4;  // at least four key tiles per share
   return n < 2 ? 1 : (int)n;
+}
+// How many of them pay: what a share saves is its part of the visible tiles (1.8 us each at head dim 128; cached rows are
+// mostly visible, of the region's own tiles a quarter is a guess), what the split costs is the merge launch (4 us) and the
+// partial results, 131 KB out and back per workgroup (0.066 us at the rate such a launch reaches).  32 / 8 heads of 128, one
+// workgroup per list / split as far as the device goes: 1024 tokens from empty 24.4 / 35.4 us, 700 tokens over 492 rows
+// 29.5 / 37.3, 1024 over 1024 rows 40.3 / 45.5; 1024 over 1728 rows 60.5 / 57.8, 40 over 1728 rows 57 / 28, 301 over 6656
+// rows 180 / 58.
+static int choose_split(int64_t n_wg, int64_t Tk, int64_t base) {
+  const int most = most_split(n_wg, Tk);
+  const double visible = (double)(base / kTile) + 0.25 * (double)(Tk - base / kTile);
+  int best = 1;
+  double gain = 0.0;
+  for (int n = 2; n <= most; ++n) {
+    const double g = 1.8 * visible * (n - 1) / n - 4.0 - 0.066 * (double)n_wg * n;
+    if (g > gain) gain = g, best = n;
+  }
+  return best;
 }
 static size_t split_partial_bytes(int64_t n_wg, int n_split, int64_t D) {
   return n_split <= 1 ? 0 : (size_t)n_wg * n_split * kPrefillWaves * (kTile / 2) * (D + 2) * sizeof(float);
@@ -1822,7 +1839,7 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   };
   a.n_split = 1;
   if (hpw == 4 || packed) {  // the kernels in which every wavefront walks the whole tile list
-    const int ns = choose_split(n_wg, a.Tk);
+    const int ns = choose_split(n_wg, a.Tk, a.base);
     if (ns > 1 && extra && extra_bytes >= split_partial_bytes(n_wg, ns, g.D)) {
       a.n_split = ns;
       a.part_acc = static_cast<float*>(extra);
@@ -1907,7 +1924,7 @@ extern "C" size_t nats_prefill_sched_workspace_bytes(int64_t B, int64_t H_q, int
   // turns out to be: room for that many partial results whenever a launch of this size may be split)
   const int64_t n_qg_min = (n_qt > 1 ? n_qt - 1 : 1) + 4 / hpw - 1;
   const int64_t n_wg_min = B * H_kv * (n_rep / hpw > 0 ? n_rep / hpw : 1) * (n_qg_min / (4 / hpw));
-  return choose_split(n_wg_min, Tk) > 1 ? split_partial_bytes(device_cu_count(), 2, 128) / 2 : 0;
+  return most_split(n_wg_min, Tk) > 1 ? split_partial_bytes(device_cu_count(), 2, 128) / 2 : 0;
 }
 
 extern "C" size_t nats_prefill_past_workspace_bytes(int64_t B, int64_t H_kv, int64_t n_rows, int64_t S) {
