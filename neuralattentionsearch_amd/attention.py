@@ -75,6 +75,12 @@ class AttentionLayer(nn.Module):
     def add_rotary_emb(self, xq, xk, pos_emb):
         if pos_emb is not None:
             cos, sin = pos_emb
+            B, _, L, D = xq.shape
+            # (one kernel with the rounding points of the torch ops, where nothing watches those)
+            if (all(type(t) is torch.Tensor for t in (xk, cos, sin)) and _plain_execution(xq, (xk, cos, sin))
+                    and cos.shape == sin.shape == (B, L, D) and xk.shape == (B, xk.shape[1], L, D) and D <= 256
+                    and ops.rope_qk_ok(xq, xk, cos, sin)):
+                return ops.rope_qk(xq, xk, cos, sin)
             xq, xk = apply_rotary_pos_emb(xq, xk, cos, sin)
         return xq, xk
 
