@@ -336,6 +336,14 @@ int nats_evict_apply_first(const void* src_k, const void* src_v, void* cache_k, 
                            const int64_t* valid_strides, int elem_bytes, const void* workspace,
                            const nats_evict_result* result, void* stream);
 
+/* A cache's rows into larger buffers, the new rows empty (zeros, not valid, position -1), in one launch:
+ *   the first old_rows rows of old_k / old_v [heads, old_pitch, row] and their valid / pos, new_k / new_v [heads, new_rows, row], valid / pos [heads, rows]: contiguous, rows of
+ *   row_bytes (a multiple of 16), 16-byte aligned; old_pos and new_pos both NULL or both given
+ */
+int nats_cache_widen(const void* old_k, const void* old_v, const uint8_t* old_valid, const int32_t* old_pos, void* new_k, void* new_v,
+                     uint8_t* new_valid, int32_t* new_pos, int64_t heads, int64_t old_pitch, int64_t old_rows, int64_t new_rows,
+                     int64_t row_bytes, void* stream);
+
 /* The row write of the cache update for a cache that already holds rows (NAtSChunkLayerCache.update,
  * components/cache/nats_chunk_layer_cache.py:243-256; NAtSLayerCache.update, nats_layer_cache.py:279-284) in one launch:
  *   cache_k / cache_v[b, h, row0 + l] = k / v[b, h, l],  valid[b, h, row0 + l] = 1,  pos[b, h, row0 + l] = pos0 + l

@@ -75,6 +75,7 @@ SIGNATURES = {
                                                 c_i64p, ctypes.c_int, c_p, c_p, c_p]),
     "nats_evict_apply_first": (ctypes.c_int, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_p, ctypes.POINTER(EvictParams),
                                               c_i64p, c_i64p, c_i64p, ctypes.c_int, c_p, c_p, c_p]),
+    "nats_cache_widen": (ctypes.c_int, [c_p] * 8 + [c_i64] * 5 + [c_p]),
     "nats_cache_append": (ctypes.c_int, [c_p] * 6 + [c_i64] * 7 + [c_i64p] * 4 + [ctypes.c_int, c_p]),
     "nats_cache_append_plan": (ctypes.c_int, [c_p] * 6 + [c_i64] * 7 + [c_i64p] * 4 + [ctypes.c_int, c_p, c_p, c_p,
                                                                                         ctypes.POINTER(EvictParams), c_p,

@@ -302,15 +302,23 @@ class NAtSChunkLayerCache:
 
     def _grow(self, rows: int):
         cap = self._buf_k.shape[2]
+        if rows > cap:
+            # (a quarter more than asked for, so that the next segment of a prompt, over a few more kept rows, fits as well)
+            new_cap = max(rows + rows // 4, cap + max(cap // 2, 4 * self.chunk_size))
+            new_cap = math.ceil(new_cap / self.chunk_size) * self.chunk_size
+            # (spare rows that hold nothing yet need not be initialised to be copied)
+            wide = ops.cache_widen(self._buf_k, self._buf_v, self._buf_valid, self._buf_pos, new_cap, self._clean)
+            if wide is not None:
+                self._clean = None
+                self._buf_k, self._buf_v, self._buf_valid, self._buf_pos = wide
+                self._rows = max(self._rows, rows)
+                return
         if self._clean is not None and rows > self._clean:
             # the cache extends into spare rows: the ones it takes now (all of them before the buffers are copied)
             hi = cap if rows >= cap else rows
             self._init_rows(self._clean, hi)
             self._clean = hi if hi < cap else None
         if rows > cap:
-            new_cap = max(rows, cap + max(cap // 2, 4 * self.chunk_size))
-            new_cap = math.ceil(new_cap / self.chunk_size) * self.chunk_size
-
             def widen(t, fill):
                 shape = list(t.shape)
                 shape[2] = new_cap

@@ -644,6 +644,23 @@ def cache_append(k: torch.Tensor, v: torch.Tensor, cache_k: torch.Tensor, cache_
                                         cache_k.element_size(), _stream(k)))
 
 
+def cache_widen(k: torch.Tensor, v: torch.Tensor, valid: torch.Tensor, pos: torch.Tensor | None, rows: int,
+                keep: int | None = None):
+    """The buffers of a cache (k / v [B, H, rows, D], valid uint8 and pos int32 [B, H, rows], contiguous) with `rows` rows: the
+    old ones (the first `keep` of them), then empty ones.  Returns the four new tensors, or None if these cannot take the kernel."""
+    B, H, have, D = k.shape
+    row_bytes = D * k.element_size()
+    old = (k, v, valid) if pos is None else (k, v, valid, pos)
+    if row_bytes % 16 or row_bytes > 65536 or not 0 < B * H <= 65535 or not have or not all(t.is_contiguous() for t in old) \
+            or (k.data_ptr() | v.data_ptr()) % 16:
+        return None
+    new = [torch.empty(*t.shape[:2], rows, *t.shape[3:], dtype=t.dtype, device=t.device) for t in old]
+    check(_lib.load().nats_cache_widen(_ptr(k), _ptr(v), _ptr(valid), _ptr(pos), _ptr(new[0]), _ptr(new[1]), _ptr(new[2]),
+                                       None if pos is None else _ptr(new[3]), B * H, have, have if keep is None else keep, rows, row_bytes,
+                                       _stream(k)))
+    return new if pos is not None else [*new, None]
+
+
 class CacheAppendCall:
     """`cache_append` for one pair of layouts (the new rows' and the cache's), with the checks made and the stride
     arrays and buffer addresses prepared once: a caller that appends step after step into the same buffers pays one
