@@ -1878,10 +1878,15 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
 #undef NATS_PREFILL_BALANCED
   }
   // A launch of several rounds of workgroups per compute unit draws its lightest query groups from the counter
-  // (NATS_PREFILL_POOL = eighths of the query groups that are drawn, 0 = none).
+  // (NATS_PREFILL_POOL = eighths of the query groups that are drawn, 0 = none).  How many (32 / 8 heads of 128, us with 2 / 3
+  // / 8 eighths): with one to three streams per XCD, whose sums differ from XCD to XCD, three (8192 tokens 125.6 / 121.3 / 120.0,
+  // 12000 215.7 / 195.9 / 190.5, 16000 with even roles 747 / 724 / 731, 32768 700.6 / 700.8 / 712.0; packed tiles, 12000 at chunk
+  // 16 163.4 / 164.4 / 165.8, stay at two); with four and more all (batch 4, 4096 tokens 205 / 205 / 196, 32 kv heads, 8192
+  // tokens 158.8 / 156.5 / 146.6, batch 4, 3001 tokens at chunk 32 141.1 / 142.7 / 137.3); gathered rows all (16384 tokens at
+  // chunk 1 290.6 / 289.3 / 283.7).
   {
     const char* e = getenv("NATS_PREFILL_POOL");
-    const int eighths = e ? atoi(e) : 2;
+    const int eighths = e ? atoi(e) : (a.long_rows || g.B * g.H_kv >= 32) ? 8 : packed ? 2 : 3;
     const int n_cu = device_cu_count();
     if (eighths > 0 && eighths <= 8 && w.ticket && n_cu > 0 && n_wg >= 4 * (int64_t)n_cu) {
       a.pool_ranks = (int)((int64_t)a.n_qg * eighths / 8);
