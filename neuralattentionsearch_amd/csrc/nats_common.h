@@ -70,7 +70,7 @@ struct PastView {
 };
 
 struct KeyLimArgs {
-  const uint8_t* roles;         // [streams, S]; if set, the kernel derives the slot-level limits itself (no past only)
+  const uint8_t* roles;         // [streams, S]; if set, the kernel derives the slot-level limits and the first global slot itself
   const int32_t* vis_lim;       // [streams, S] slot-level limits of the segment's roles (used when roles is NULL)
   const int32_t* first_global;  // [streams] first global slot of the segment
   const uint8_t* valid;

@@ -171,11 +171,23 @@ __global__ __launch_bounds__(256) void key_lim_kernel(KeyLimArgs a) {
   int32_t v_inline = 0;
   // (x / C for x >= 0; a shift when the chunk size is a power of two)
   auto slot_of = [&](int x) { return a.c_shift >= 0 ? x >> a.c_shift : x / a.C; };
-  if (!kPast && a.roles) {
+  int first_g = 0;  // first global slot of the segment, for the cached local rows
+  if (a.roles) {
     const uint8_t* r = a.roles + (int64_t)stream * a.S;
-    const bool in = row < a.N;
-    const int slot = in ? slot_of(row) : 0;
-    const int s0 = slot_of(tile * kTile);  // slot of lane 0 (the tile starts inside N)
+    const int base = kPast ? a.base : 0;
+    const bool in = row < a.N && row >= base;
+    const int slot = in ? slot_of(row - base) : 0;
+    const int s0 = slot_of(max(tile * kTile, base) - base);  // slot of the tile's first region row (the tile starts inside N)
+    if (kPast && tile * kTile < base) {
+      for (int blk = 0; blk < a.S; blk += kWave) {
+        const int n = blk + lane;
+        const uint64_t bits = __ballot(n < a.S && (r[n] == NATS_ROLE_GLOBAL || n == a.S - 1));
+        if (bits) {
+          first_g = blk + __builtin_ctzll(bits);
+          break;
+        }
+      }
+    }
     const uint8_t role = in ? r[slot] : uint8_t(NATS_ROLE_GLOBAL);
     const bool want = in && role == NATS_ROLE_LOCAL;
     int g = -1;
@@ -196,13 +208,14 @@ __global__ __launch_bounds__(256) void key_lim_kernel(KeyLimArgs a) {
   }
   if (row < a.N) {
     if (!kPast || row >= a.base) {
-      int32_t v = (!kPast && a.roles) ? v_inline : a.vis_lim[(int64_t)stream * a.S + slot_of(row - a.base)];
+      int32_t v = a.roles ? v_inline : a.vis_lim[(int64_t)stream * a.S + slot_of(row - a.base)];
       int64_t t = (int64_t(v) + 1) * a.C - 1;
       lim = (v == kLimGlobal || t >= kLimGlobal) ? kLimGlobal : int32_t(t);
     } else {
       const int b = stream / a.Hkv, h = stream % a.Hkv;
       const bool val = a.valid[b * a.valid_s_b + h * a.valid_s_h + row] != 0;
       const int C = a.C;
+      const int fg = a.roles ? first_g : a.first_global[stream];
       if (a.token_mode) {
         // The per-token cache (components/cache/nats_layer_cache.py:469-517, 603-649).  Its limits count the
         // queries of this call (i = r - old_fill), hence the + old_fill.
@@ -224,7 +237,7 @@ __global__ __launch_bounds__(256) void key_lim_kernel(KeyLimArgs a) {
           if (row >= sg + sl) {
             lim = -1;
           } else if (row >= sg) {
-            lim = a.first_global[stream] + a.old_fill;
+            lim = fg + a.old_fill;
           } else {
             lim = kLimGlobal;
           }
@@ -254,7 +267,7 @@ __global__ __launch_bounds__(256) void key_lim_kernel(KeyLimArgs a) {
           } else if (cc < lo) {
             lim = kLimGlobal;
           } else {
-            lim = (a.first_global[stream] + 1) * C - 1;  // query slot <= first global slot of the segment (:480-494)
+            lim = (fg + 1) * C - 1;  // query slot <= first global slot of the segment (:480-494)
           }
         }
       }
@@ -518,10 +531,10 @@ int prepare_key_limits(const uint8_t* roles, int64_t B, int64_t H_kv, int64_t S,
                        const PastView* past, const PrefillWorkspace& w, hipStream_t st) {
   const int64_t n_streams = B * H_kv;
   KeyLimArgs a{};
-  // A prefill from an empty cache needs the scan's result only inside the key-limit kernel, which then searches the
-  // roles itself (one launch less); streams so long that a run of local slots could make that search slow, and
-  // segments over a filled cache (which also need the first global slot), take the scan kernel.
-  const bool inline_scan = past == nullptr && S <= 8192;
+  // The scan's result is needed only inside the key-limit kernel, which searches the roles itself (one launch less: a
+  // segment's limits 4.1 + 1 + 4.2 -> 5.1 us); streams so long that a run of local slots could make that search slow take the scan
+  // kernel.
+  const bool inline_scan = S <= 8192;
   if (inline_scan) {
     a.roles = roles;
   } else if (int rc = launch_role_scan(roles, n_streams, S, W, C, nullptr, w.vis_lim, w.first_global, st)) {
