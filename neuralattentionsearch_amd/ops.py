@@ -102,6 +102,8 @@ class _NativeFront:
         for n in dir(_nats_host):
             if not n.startswith("_") and n != "bind":
                 self.__dict__[n] = getattr(_nats_host, n)
+        if name not in self.__dict__:
+            raise AttributeError(name)
         return self.__dict__[name]
 
 
