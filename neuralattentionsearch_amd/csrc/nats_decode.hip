@@ -531,6 +531,7 @@ __global__ void decode_merge_balanced_kernel(const float* __restrict__ ws_acc, c
 // merge the partials of one q head of the fixed schedule: grid = B*Hq, block = G * D threads.  The n <= 64 partials of a head
 // lie side by side, so everything is requested at once: every wavefront reads the maxima and row sums of all of them (lane s
 // those of partial s, no barrier), thread (g, d) the accumulators of the partials g, g + G, ...  (at most kFixedPerGroup).
+// The block is whole wavefronts: the shuffles reach all 64 lanes (head dim 32 takes an even G; a group without partials adds 0).
 constexpr int kFixedPerGroup = 8;
 constexpr int kFixedMaxSplit = 64;
 __global__ void decode_merge_fixed_kernel(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
@@ -918,7 +919,8 @@ static int decode_fwd_impl(const void* q, const void* cache_k, const void* cache
     if (int rc = launch_mfma_by_dim(a, D, nrep_k, groups, fixed.waves, st)) return rc;
     NATS_CHECK_LAUNCH("decode_split_mfma_kernel");
     if (fixed.split > 1) {
-      const int merge_groups = (fixed.split + kFixedPerGroup - 1) / kFixedPerGroup;
+      int merge_groups = (fixed.split + kFixedPerGroup - 1) / kFixedPerGroup;
+      if (merge_groups * D % kWave) ++merge_groups;  // (whole wavefronts, see the kernel)
       // (fixed_schedule keeps G * D within 1024 threads)
       hipLaunchKernelGGL(decode_merge_fixed_kernel, dim3((unsigned)(B * H_q)), dim3((unsigned)(merge_groups * D)),
                          merge_groups * D * sizeof(float), st, a.ws_acc, a.ws_ml, static_cast<uint16_t*>(o), (int)H_q, (int)H_kv, (int)D,

@@ -40,14 +40,18 @@ def ragged_cache(seed, B, Hkv, D, W, C, n_max_chunks, dtype, frac=(0.1, 1.0), fi
     return k, v, vt, n_rows
 
 
-def run_case(B, Hq, Hkv, D, W, C, n_max_chunks, dtype, seed=0, frac=(0.1, 1.0), fill=0, q_scale=1.0):
+def run_case(B, Hq, Hkv, D, W, C, n_max_chunks, dtype, seed=0, frac=(0.1, 1.0), fill=0, q_scale=1.0, shift=None):
     """`q_scale` > 1 makes the scores peaked (their standard deviation in nats is q_scale): a row's output is then
-    carried by a few keys and is of the size of v, and the error is held against the row's own magnitude."""
+    carried by a few keys and is of the size of v, and the error is held against the row's own magnitude.
+    `shift`: the first dimension gives every score about that many nats."""
     from neuralattentionsearch_amd import ops
-    say("decode", B, Hq, Hkv, D, W, C, n_max_chunks, dtype, seed, frac, fill, q_scale)
+    say("decode", B, Hq, Hkv, D, W, C, n_max_chunks, dtype, seed, frac, fill, q_scale, shift)
     k, v, valid, n_rows = ragged_cache(seed, B, Hkv, D, W, C, n_max_chunks, dtype, frac, fill)
     g = torch.Generator().manual_seed(seed + 100)
     q = (torch.randn(B, Hq, 1, D, generator=g) * q_scale).to(dtype)
+    if shift is not None:
+        k[..., 0] = torch.where(k[..., 0].isnan(), k[..., 0], 8.0)
+        q[..., 0] = shift * math.sqrt(D) / 8.0
     want = orc.decode_attention(q, k, v, valid, n_rows).float()
     rms = want.pow(2).mean(-1, keepdim=True).sqrt()
     bound = TOL[dtype] * (torch.maximum(rms, want.abs()) if q_scale > 1 else 1.0) + (2e-3 if q_scale > 1 else 0.0)
