@@ -1658,19 +1658,23 @@ static int most_split(int64_t n_wg, int64_t Tk) {
   if (n > Tk / 4) n = Tk / 4;  // at least four key tiles per share
   return n < 2 ? 1 : (int)n;
 }
-// How many of them pay: what a share saves is its part of the visible tiles (1.8 us each at head dim 128; cached rows are
-// mostly visible, of the region's own tiles a quarter is a guess), what the split costs is the merge launch (4 us) and the
-// partial results, 131 KB out and back per workgroup (0.066 us at the rate such a launch reaches).  32 / 8 heads of 128, one
-// workgroup per list / split as far as the device goes: 1024 tokens from empty 24.4 / 35.4 us, 700 tokens over 492 rows
-// 29.5 / 37.3, 1024 over 1024 rows 40.3 / 45.5; 1024 over 1728 rows 60.5 / 57.8, 40 over 1728 rows 57 / 28, 301 over 6656
-// rows 180 / 58.
-static int choose_split(int64_t n_wg, int64_t Tk, int64_t base) {
+// How many of them pay: what a share saves is its part of the visible tiles, what the split costs is the merge launch (4 us) and
+// the partial results, 32 rows of D floats per wavefront out and back.  A tile takes 1.6 / 1.25 / 1.1 us at head dims 128 / 64 / 32
+// (300 tokens over 25000 visible rows, no split: 615 / 490 / 425 us).  Cached rows are taken as visible, of the region's own tiles
+// half (the heaviest list of unequal heads ends the launch), a share's partial results as 0.045 us per workgroup at head dim 128:
+// the two that lose least over 1278 launches (256 to 7000 tokens from empty and over 300 to 65536 tokens, 4 to 32 heads, chunks 1
+// to 64), where this rule takes 1.02 times the best number of shares, never splitting 1.1 and more, always as far as the device
+// goes 1.03 and up to 1.5.  32 / 8 heads of 128, one workgroup per list / split as far as the device goes: 1024 tokens from empty
+// 24.4 / 35.4 us, 700 tokens over 492 rows 29.5 / 37.3; 40 over 1728 rows 57 / 28, 301 over 6656 rows 180 / 58.  8 heads of 32, 3000
+// tokens from empty 40.4 / 32.4; of 64 50.6 / 42.3; 1024 tokens at chunk 16 over 348 rows of 32 24.2 / 18.7.
+static int choose_split(int64_t n_wg, int64_t Tk, int64_t base, int64_t D) {
   const int most = most_split(n_wg, Tk);
-  const double visible = (double)(base / kTile) + 0.25 * (double)(Tk - base / kTile);
+  const double visible = (double)(base / kTile) + 0.5 * (double)(Tk - base / kTile);
+  const double tile = D == 128 ? 1.6 : D == 64 ? 1.25 : 1.1;
   int best = 1;
   double gain = 0.0;
   for (int n = 2; n <= most; ++n) {
-    const double g = 1.8 * visible * (n - 1) / n - 4.0 - 0.066 * (double)n_wg * n;
+    const double g = tile * visible * (n - 1) / n - 4.0 - 0.045 * (double)D / 128.0 * (double)n_wg * n;
     if (g > gain) gain = g, best = n;
   }
   return best;
@@ -1839,7 +1843,7 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   };
   a.n_split = 1;
   if (hpw == 4 || packed) {  // the kernels in which every wavefront walks the whole tile list
-    const int ns = choose_split(n_wg, a.Tk, a.base);
+    const int ns = choose_split(n_wg, a.Tk, a.base, g.D);
     if (ns > 1 && extra && extra_bytes >= split_partial_bytes(n_wg, ns, g.D)) {
       a.n_split = ns;
       a.part_acc = static_cast<float*>(extra);

@@ -235,6 +235,23 @@ def test_short_segments_over_a_long_cache_split_their_tile_lists(split_lists, C,
         assert (x - y).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("Hq,Hkv,L,D,C", [(8, 8, 3000, 32, 64), (8, 2, 3001, 32, 64), (8, 4, 2999, 64, 64), (4, 4, 2500, 64, 1)])
+def test_prompts_of_few_workgroups_split_their_tile_lists(split_lists, Hq, Hkv, L, D, C):
+    """Prompts whose lists go to a few workgroups each, at the head dims below 128."""
+    from neuralattentionsearch_amd import ops
+    say("prefill split lists, from empty", Hq, Hkv, L, D, C)
+    g = torch.Generator().manual_seed(L + D)
+    roles = to_dev(draw_roles(L, 1, Hkv, math.ceil(L / C), p=(0.37, 0.315, 0.315)))
+    q, k, v = (torch.randn(1, h, L, D, generator=g).bfloat16().cuda() for h in (Hq, Hkv, Hkv))
+    outs = []
+    for on in (False, True):
+        split_lists(on)
+        outs.append(ops.prefill_attention(q, k, v, roles, C, 256).float())
+    assert torch.isfinite(outs[1]).all()
+    assert not torch.equal(*outs), "the lists were not split"
+    assert (outs[0] - outs[1]).abs().max().item() <= 2e-2
+
+
 @pytest.fixture
 def packed_tiles(monkeypatch):
     def switch(on: bool):
