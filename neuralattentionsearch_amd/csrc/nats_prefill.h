@@ -31,6 +31,7 @@ struct PrefillArgs {
   // workgroup: a few workgroups at the end of the grid draw them from counters, one queue per XCD (heaviest first),
   // for as long as there are any, so that an XCD that reaches its last workgroups earlier takes more of them.
   int pool_ranks;    // 0: every workgroup has its fixed query group
+  int heavy_first;   // launches with the balanced map: how far above the mean the largest stream has to be, in hundredths
   int32_t* ticket;   // one counter per XCD, kTicketStride entries apart, zero at launch
   float scale;   // softmax scale
   // few query tiles over many key rows: n_split workgroups share the tile list of one (kv stream, head group,

@@ -1020,10 +1020,10 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
 // different shares of a context, and the whole share of a stream lies on one XCD in the plain map): the heavy streams'
 // query groups come first, over all XCDs, so that no long workgroup starts in the last round.  Every workgroup counts the
 // streams' key tiles that the middle query sees (one trip to L2), takes those above half of the largest count as the heavy
-// ones and finds its own item; streams within 1.5 times their mean keep the plain map and with it one stream's tiles per L2.
-// Measured at 32 / 8 heads, head dim 128, chunk 64, segments of 4096 tokens whose first head keeps three to nine times what
-// the others keep: 82 / 143 / 167 / 184 -> 75 / 98 / 127 / 140 us for the first to the fourth segment; with streams alike
-// 53.9 / 53.7 us (4096 tokens from empty).  What bounds it then is the longest single query group.
+// ones and finds its own item; streams among which the largest is not far enough above their mean keep the plain map and with
+// it one stream's tiles per L2.  Measured at 32 / 8 heads, head dim 128, chunk 64, segments of 4096 tokens whose first head keeps
+// three to nine times what the others keep: 82 / 143 / 167 / 184 -> 75 / 98 / 127 / 140 us for the first to the fourth segment.
+// What bounds it then is the longest single query group.  See balance_threshold for what the look costs and where it pays.
 constexpr int kBalanceStreams = 64;   // one per lane
 constexpr int kBalanceTiles = 8192;   // tile summaries a workgroup may read for it
 __device__ __forceinline__ void map_balanced(const PrefillArgs& a, int* counts, int bid, int& ks, int& hg, int& rank) {
@@ -1054,7 +1054,7 @@ __device__ __forceinline__ void map_balanced(const PrefillArgs& a, int* counts, 
   }
   most = __builtin_amdgcn_readfirstlane(most);  // (the same in every lane; as scalars they keep the map and the item scalar)
   sum = __builtin_amdgcn_readfirstlane(sum);
-  if (2 * most * ns < 3 * sum) {
+  if (100 * most * ns < a.heavy_first * sum) {
     map_workgroup(a, bid, ks, hg, rank);
     return;
   }
@@ -1679,6 +1679,29 @@ static int choose_split(int64_t n_wg, int64_t Tk, int64_t base, int64_t D) {
   }
   return best;
 }
+// Where the balanced map is taken, and from which ratio of the largest stream to the mean on the heavy streams come first
+// (hundredths; 0: the plain map).  The look at the streams is 1 to 2 us of every workgroup, and heavy streams first is worse than
+// the plain map when they are not much heavier.  Speed against the plain map at chunk 64 over 715 launches of 1400 to 7000 tokens,
+// streams alike / one head of several times the others' share:
+//   * over cached rows, whole multiples of 8 streams: head dim 128 1.00 to 1.03 / 1.04 to 2.05, 64 over 1k rows 0.98 / 1.35, over
+//     4k and 20k 1.01 to 1.04 / 1.5 to 2.1, 32 over 1k 0.96 / 1.35, over 4k and 20k 0.99 / 1.5 to 2.05.  So there, from a number of
+//     cached rows on, with a threshold of 1.5.
+//   * over cached rows, other numbers of streams (whose plain map is rank by rank over all XCDs already): 4 streams 1.14 to 1.7
+//     where they differ; 6 streams down to 0.86 at 1.5, at a threshold of 2 0.97 and more.
+//   * from empty: head dim 128 at 8 and 16 streams 1.00 to 1.04 / 1.23 to 1.3; 64 at 8 streams and two rounds of workgroups 1.01 /
+//     1.12 to 1.24 at a threshold of 2.  Not otherwise: head dim 32 0.93 to 0.98, 64 at 16 streams 0.95 to 0.98, 32 streams 0.89 to
+//     0.97, 4 streams of 128, 7000 tokens 0.84, packed tiles 0.98.
+// (NATS_PREFILL_BALANCE=0 / 1 in the environment: nowhere / everywhere, for comparison.)
+static int balance_threshold(int64_t D, int64_t ns, int64_t base, int64_t x_len, int64_t n_wg, int64_t n_cu, bool packed) {
+  if (const char* e = getenv("NATS_PREFILL_BALANCE"); e && e[0]) return e[0] == '0' ? 0 : 150;
+  if (base > 0) {
+    const int64_t part = D == 128 && !packed ? 8 : D == 32 ? 2 : 4;
+    return base * part < x_len ? 0 : ns % 8 == 0 ? 150 : 200;
+  }
+  if (packed || ns % 8 != 0) return 0;
+  if (D == 128) return ns <= 16 ? 150 : 0;
+  return D == 64 && ns == 8 && n_wg >= 2 * n_cu ? 200 : 0;
+}
 static size_t split_partial_bytes(int64_t n_wg, int n_split, int64_t D) {
   return n_split <= 1 ? 0 : (size_t)n_wg * n_split * kPrefillWaves * (kTile / 2) * (D + 2) * sizeof(float);
 }
@@ -1870,10 +1893,10 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
     return NATS_OK;
   }
   // One to four rounds of workgroups per compute unit: see map_balanced.  (Below that every workgroup starts at once, above
-  // it the drawn query groups even the XCDs out.  Packed tiles from empty, where streams differ by their new roles only, keep
-  // the plain map: alike, they pay 1 us of 52 for the look.)
+  // it the drawn query groups even the XCDs out.)
   if (const int64_t n_cu = device_cu_count(), ns = g.B * g.H_kv;
-      hpw == 4 && n_cu > 0 && n_wg > n_cu && n_wg < 4 * n_cu && ns > 1 && ns <= kBalanceStreams && ns * a.Tk <= kBalanceTiles && (!packed || g.base > 0)) {
+      hpw == 4 && n_cu > 0 && n_wg > n_cu && n_wg < 4 * n_cu && ns > 1 && ns <= kBalanceStreams && ns * a.Tk <= kBalanceTiles &&
+      (a.heavy_first = balance_threshold(g.D, ns, g.base, g.x_len, n_wg, n_cu, packed)) > 0) {
 #define NATS_PREFILL_BALANCED(MODE)                                                                  \
   (g.D == 32 ? launch_prefill_mfma<32, true, MODE, true>(a, n_wg, st)                                \
              : g.D == 64 ? launch_prefill_mfma<64, true, MODE, true>(a, n_wg, st) : launch_prefill_mfma<128, true, MODE, true>(a, n_wg, st))

@@ -12,6 +12,14 @@ from tests.gpu_util import draw_roles, say
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(params=["1", None], ids=["looks", "rule"])
+def balance(request, monkeypatch):
+    """The look at the streams in every launch of such a size, and where the rule has it."""
+    if request.param:
+        monkeypatch.setenv("NATS_PREFILL_BALANCE", request.param)
+        monkeypatch.setenv("NATS_PREFILL_SPLIT", "0")
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,L,C,W,heavy", [
     (1, 32, 8, 128, 2100, 64, 128, [0]),          # one heavy stream of eight, 33 query tiles
     (2, 32, 4, 128, 2050, 64, 128, [5]),          # two head groups per kv head
@@ -19,8 +27,9 @@ pytestmark = pytest.mark.gpu
     (1, 4, 1, 32, 20000, 64, 64, [0]),            # a single stream: the plain map
     (2, 32, 8, 64, 1100, 64, 64, []),             # no heavy stream
     (2, 32, 8, 64, 1100, 64, 64, list(range(16))),
+    (1, 32, 8, 64, 4200, 64, 64, [3]),            # head dim 64: from two rounds of workgroups on
 ])
-def test_prefill_with_streams_of_unequal_weight(B, Hq, Hkv, D, L, C, W, heavy):
+def test_prefill_with_streams_of_unequal_weight(balance, B, Hq, Hkv, D, L, C, W, heavy):
     from neuralattentionsearch_amd import ops
     say("balance", B, Hq, Hkv, D, L, C, W, heavy)
     S = math.ceil(L / C)
@@ -66,8 +75,9 @@ def orc_rows(roles, L, C, W, lo, hi):
     (32, 8, 64, 1000, 2112, 16, 64, [7, 3]),  # packed tiles
     (32, 8, 32, 600, 2070, 4, 32, [1]),       # gathered rows
     (12, 3, 64, 300, 6000, 32, 64, [2]),      # three streams on eight XCDs
+    (12, 3, 64, 1500, 6000, 64, 64, [2]),     # over enough rows: a stream twice as heavy as the mean
 ])
-def test_segment_with_streams_of_unequal_weight(Hq, Hkv, D, first, L, C, W, heavy):
+def test_segment_with_streams_of_unequal_weight(balance, Hq, Hkv, D, first, L, C, W, heavy):
     from neuralattentionsearch_amd.cache import NAtSChunkLayerCache
     say("balance, filled cache", Hq, Hkv, D, first, L, C, W, heavy)
     roles = draw_roles(L, 1, Hkv, -(-(first + L) // C) + 1, p=(0.02, 0.05, 0.93))
