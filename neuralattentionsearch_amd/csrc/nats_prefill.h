@@ -85,7 +85,7 @@ __host__ __device__ inline void balanced_item(uint64_t heavy, int ns, int n_hg, 
 bool prefill_f32_takes(const PrefillArgs& a, int D);
 int launch_prefill_f32(const PrefillArgs& a, int D, hipStream_t st);
 // short prompts from an empty cache in one launch (nats_prefill_short.hip)
-bool prefill_short_takes(int64_t B, int64_t H_q, int64_t D, int64_t L, int dtype);
+bool prefill_short_takes(int64_t B, int64_t H_q, int64_t H_kv, int64_t D, int64_t L, int64_t C, int dtype);
 int launch_prefill_short(const void* q, const void* k, const void* v, const uint8_t* roles, void* o, int64_t B, int64_t H_q, int64_t H_kv,
                          int64_t L, int64_t D, int64_t C, int64_t W, const int64_t* q_strides, const int64_t* k_strides,
                          const int64_t* v_strides, const int64_t* o_strides, float sm_scale, hipStream_t st);

@@ -1978,7 +1978,7 @@ extern "C" int nats_prefill_fwd(const void* q, const void* k, const void* v, con
   PrefillWorkspace w = carve_prefill_workspace(workspace, B * H_kv, S, L);
   NATS_REQUIRE(workspace_bytes >= w.bytes, NATS_ERR_WORKSPACE, "%s: workspace %zu bytes < %zu", who, workspace_bytes, w.bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (prefill_short_takes(B, H_q, D, L, dtype))
+  if (prefill_short_takes(B, H_q, H_kv, D, L, C, dtype))
     return launch_prefill_short(q, k, v, roles, o, B, H_q, H_kv, L, D, C, W, q_strides, k_strides, v_strides, o_strides, sm_scale, st);
   if (int rc = prepare_key_limits(roles, B, H_kv, S, L, C, W, nullptr, w, st)) return rc;
   return launch_segment(who, g, q, k, v, o, q_strides, k_strides, v_strides, o_strides, sm_scale, dtype, w,

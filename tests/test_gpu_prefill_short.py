@@ -31,6 +31,23 @@ def test_short_prompts(D, L, C, W):
         assert err <= 2e-2, (p, err)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,C,lens", [
+    (16, 4, 64, 64, (1536, 1537)), (16, 16, 64, 64, (2048,)),  # three / four workgroups per compute unit
+    (8, 8, 128, 64, (2047, 2049)), (12, 4, 128, 64, (1344, 1345)),
+    (8, 8, 64, 1, (1792, 1793)), (8, 8, 128, 3, (1792, 1793)), (8, 8, 128, 4, (1793,)),  # chunks of a few tokens
+])
+def test_both_sides_of_the_line(Hq, Hkv, D, C, lens):
+    from neuralattentionsearch_amd import ops
+    for L in lens:
+        say("short, line", Hq, Hkv, D, C, L)
+        g = torch.Generator().manual_seed(L)
+        roles = draw_roles(L, 1, Hkv, math.ceil(L / C), p=(0.05, 0.15, 0.8))
+        q, k, v = (torch.randn(1, h, L, D, generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
+        want = orc.masked_attention(q.float(), k.float(), v.float(), orc.prefill_mask(roles, L, C, 192 // C * C))
+        got = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), to_dev(roles), C, 192 // C * C).cpu().float()
+        assert (got - want).abs().max().item() <= 2e-2, L  # (as above)
+
+
 def test_short_prompt_into_strided_output_at_other_scales():
     from neuralattentionsearch_amd import ops
     g = torch.Generator().manual_seed(9)
