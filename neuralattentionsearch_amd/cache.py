@@ -445,8 +445,19 @@ class NAtSChunkLayerCache:
         q_rot, end = self._append_rotated(q, key_states, value_states, cos, sin, token_states_info, roles)
         return q_rot, self._buf_k[:, :, :end], self._buf_v[:, :, :end]
 
+    def _step_as_defined(self) -> bool:
+        """Whether nobody has replaced what `step_attention` stands in for (in a subclass, on the class or on the object)."""
+        cls = type(self)
+        return (cls.append_rotated is _APPEND_ROTATED and cls.valid_tokens in _VALID_TOKENS
+                and "append_rotated" not in self.__dict__)
+
     def step_attention(self, q, key_states, value_states, cos, sin, token_states_info, roles, sm_scale: float):
         """`append_rotated` of one token per sequence and its attention over the cache: [B, H_q, 1, D]."""
+        if not self._step_as_defined():
+            q_rot, keys, values = self.append_rotated(q, key_states, value_states, cos, sin, token_states_info, roles)
+            row_end, tail_start = self.decode_hint()
+            return ops.decode_attention(q_rot, keys, values, self.valid_tokens, keys.shape[2], sm_scale, row_end=row_end,
+                                        tail_start=tail_start)
         q_rot, end = self._append_rotated(q, key_states, value_states, cos, sin, token_states_info, roles)
         row_end, tail_start = self.decode_hint()
         # (the buffers as they lie: rows behind `end` are not looked at)
@@ -836,6 +847,11 @@ try:  # the reference's container is a transformers cache (dyn_cache.py:66): HF 
     from transformers.cache_utils import DynamicCache as _CacheBase
 except Exception:  # transformers absent or unusable: a plain class with the same surface
     _CacheBase = object
+
+
+# (as this module defines them)
+_APPEND_ROTATED = NAtSChunkLayerCache.append_rotated
+_VALID_TOKENS = (NAtSChunkLayerCache.valid_tokens, NAtSLayerCache.valid_tokens)
 
 
 class NAtSCache(_CacheBase):
