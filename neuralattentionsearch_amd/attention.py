@@ -35,6 +35,9 @@ def apply_rotary_pos_emb(q, k, cos, sin, unsqueeze_dim: int = 1):
     return (q * cos) + (rotate_half(q) * sin), (k * cos) + (rotate_half(k) * sin)
 
 
+_ROTARY = (rotate_half, apply_rotary_pos_emb)  # (as this module defines them)
+
+
 def _plain_linear(m: nn.Module) -> bool:
     """An nn.Linear without bias that nobody has wrapped, hooked or re-parametrised: its call is one matrix product."""
     d = m.__dict__
@@ -76,9 +79,9 @@ class AttentionLayer(nn.Module):
         if pos_emb is not None:
             cos, sin = pos_emb
             B, _, L, D = xq.shape
-            # (one kernel with the rounding points of the torch ops, where nothing watches those)
-            if (all(type(t) is torch.Tensor for t in (xk, cos, sin)) and _plain_execution(xq, (xk, cos, sin))
-                    and cos.shape == sin.shape == (B, L, D) and xk.shape == (B, xk.shape[1], L, D) and D <= 256
+            # (one kernel with the rounding points of the torch ops, where nothing watches or replaces those)
+            if (rotate_half is _ROTARY[0] and apply_rotary_pos_emb is _ROTARY[1]
+                    and all(type(t) is torch.Tensor for t in (xk, cos, sin)) and _plain_execution(xq, (xk, cos, sin)) and cos.shape == sin.shape == (B, L, D) and xk.shape == (B, xk.shape[1], L, D) and D <= 256
                     and ops.rope_qk_ok(xq, xk, cos, sin)):
                 return ops.rope_qk(xq, xk, cos, sin)
             xq, xk = apply_rotary_pos_emb(xq, xk, cos, sin)

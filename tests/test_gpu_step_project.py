@@ -160,3 +160,19 @@ def test_model_step_calls_a_replaced_append(C, where, monkeypatch):
     got = run(replace)
     assert len(calls) == (8 if where == "class" else 4)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("name", ["rotate_half", "apply_rotary_pos_emb"])
+def test_segment_calls_a_replaced_rotary_embedding(name, monkeypatch):
+    """The rotary functions of the module, replaced by a program, rotate a segment of several tokens."""
+    from neuralattentionsearch_amd import attention
+    from neuralattentionsearch_amd.llama import rotary_tables
+    say("segment, replaced rotary embedding", name)
+    mod = attention.LlamaNAtSAttentionLayer(dim=256, n_heads=4, n_kv_heads=2).cuda().eval().requires_grad_(False)
+    q, k = torch.randn(1, 4, 20, 64, device="cuda"), torch.randn(1, 2, 20, 64, device="cuda")
+    emb = rotary_tables(torch.arange(20, device="cuda")[None], 64, 10000.0, torch.float32)
+    want = mod.add_rotary_emb(q, k, emb)
+    calls, old = [], getattr(attention, name)
+    monkeypatch.setattr(attention, name, lambda *a, **kw: calls.append(1) or old(*a, **kw))
+    got = mod.add_rotary_emb(q, k, emb)
+    assert calls and all(torch.equal(a, b) for a, b in zip(got, want))
