@@ -78,11 +78,11 @@ class AttentionLayer(nn.Module):
     def add_rotary_emb(self, xq, xk, pos_emb):
         if pos_emb is not None:
             cos, sin = pos_emb
-            B, _, L, D = xq.shape
             # (one kernel with the rounding points of the torch ops, where nothing watches or replaces those)
             if (rotate_half is _ROTARY[0] and apply_rotary_pos_emb is _ROTARY[1]
-                    and all(type(t) is torch.Tensor for t in (xk, cos, sin)) and _plain_execution(xq, (xk, cos, sin)) and cos.shape == sin.shape == (B, L, D) and xk.shape == (B, xk.shape[1], L, D) and D <= 256
-                    and ops.rope_qk_ok(xq, xk, cos, sin)):
+                    and all(type(t) is torch.Tensor for t in (xk, cos, sin)) and _plain_execution(xq, (xk, cos, sin))
+                    and xq.dim() == xk.dim() == 4 and cos.shape == sin.shape == (xq.shape[0], *xq.shape[2:])
+                    and (xk.shape[0], *xk.shape[2:]) == cos.shape and xq.shape[3] <= 256 and ops.rope_qk_ok(xq, xk, cos, sin)):
                 return ops.rope_qk(xq, xk, cos, sin)
             xq, xk = apply_rotary_pos_emb(xq, xk, cos, sin)
         return xq, xk

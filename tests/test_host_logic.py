@@ -48,3 +48,14 @@ def test_the_bench_role_logit_biases_give_the_configured_shares():
     off = chunk_pairs.sum() - 2 * 3 * 40
     assert flops == 4.0 * 64 * 4 * (off * C * C + 2 * 3 * 40 * (C * (C + 1) // 2))
     assert dense == 4.0 * 64 * 4 * 2 * 3 * (L * (L + 1) // 2)
+
+
+def test_rotary_embedding_of_tensors_without_a_head_dimension():
+    """add_rotary_emb takes whatever broadcasts against cos / sin, as apply_rotary_pos_emb does."""
+    from neuralattentionsearch_amd.attention import AttentionLayer, apply_rotary_pos_emb
+    layer = AttentionLayer(dim=32, n_heads=4).eval()
+    q, k = torch.randn(3, 5, 8), torch.randn(2, 5, 8)
+    emb = torch.randn(1, 5, 8), torch.randn(1, 5, 8)
+    with torch.no_grad():
+        for a, b in zip(layer.add_rotary_emb(q, k, emb), apply_rotary_pos_emb(q, k, *emb)):
+            assert torch.equal(a, b)
