@@ -202,19 +202,24 @@ class BaseNAtSAttentionLayer(AttentionLayer):
         self._post_update(cache, x_len)
         return output
 
-    def _overridden(self) -> bool:
-        """Whether a subclass or an instance replaces one of the methods `_one_token_step` stands in for."""
-        cls, own, chunked = type(self), self.__dict__, BaseNAtSChunkAttentionLayer
-        sample = cls._sample_for_token_info_values_inference
-        return (cls.prepare_x_values is not BaseNAtSAttentionLayer.prepare_x_values
-                or cls.add_rotary_emb is not AttentionLayer.add_rotary_emb
-                or cls.prepare_kv is not BaseNAtSAttentionLayer.prepare_kv
-                or cls.repeat_kv_values is not AttentionLayer.repeat_kv_values
-                or cls.multi_head_attention is not BaseNAtSAttentionLayer.multi_head_attention
-                or cls.role_logits is not BaseNAtSAttentionLayer.role_logits
-                or (sample is not BaseNAtSAttentionLayer._sample_for_token_info_values_inference
-                    and sample is not chunked._sample_for_token_info_values_inference)
-                or not own.keys().isdisjoint(_STEP_METHODS))
+    def _step_as_defined(self, cache, layer) -> bool:
+        """Whether everything `_one_token_step` stands in for is what this package (and torch) defines: nothing of it replaced
+        in a subclass, on a class, on an object or in a module."""
+        cls, kind, d = type(self), type(layer), _DEFINED
+        return (cls.prepare_x_values is d.prepare_x_values and cls.add_rotary_emb is d.add_rotary_emb
+                and cls.prepare_kv is d.prepare_kv and cls.repeat_kv_values is d.repeat_kv_values
+                and cls.multi_head_attention is d.multi_head_attention and cls.role_logits is d.role_logits
+                and cls._sample_for_token_info_values_inference in d.sample
+                and BaseNAtSAttentionLayer._sample_for_token_info_values_inference is d.sample[0]
+                and apply_rotary_pos_emb is _ROTARY[1] and rotate_half is _ROTARY[0]
+                and ops.roles_from_logits is d.roles_from_logits and ops.roles_from_one_hot is d.roles_from_one_hot
+                and NAtSCache.update is d.cache_update and NAtSCache.merge_new_x_values_in_chunk is d.merge
+                and NAtSCache.update_nats_cached_x_in_chunk is d.in_chunk
+                and NAtSCache.update_nats_cached_x_across_chunk is d.across_chunk
+                and kind.update in d.layer_update and kind.valid_tokens in d.valid_tokens
+                and nn.Linear.forward is d.linear_forward and nn.functional.linear is d.linear and nn.Module.__call__ is d.call
+                and self.__dict__.keys().isdisjoint(_STEP_METHODS) and cache.__dict__.keys().isdisjoint(_CACHE_METHODS)
+                and "update" not in layer.__dict__)
 
     def _one_token_step(self, x, pos_emb, start_pos, cache):
         """One token per sequence over a filled cache: projections, chunk statistic and roles in one launch, the rotary
@@ -226,7 +231,7 @@ class BaseNAtSAttentionLayer(AttentionLayer):
             return None
         layer = cache.cache_model[layer_id]
         chunked = type(layer) is NAtSChunkLayerCache
-        if not (chunked or type(layer) is NAtSLayerCache) or self._overridden():
+        if not (chunked or type(layer) is NAtSLayerCache) or not self._step_as_defined(cache, layer):
             return None
         C = cache.chunk_size
         is_chunk_module = isinstance(self, BaseNAtSChunkAttentionLayer)
@@ -283,6 +288,7 @@ class BaseNAtSAttentionLayer(AttentionLayer):
 
 _STEP_METHODS = frozenset(("prepare_x_values", "add_rotary_emb", "prepare_kv", "repeat_kv_values", "multi_head_attention",
                            "role_logits", "_sample_for_token_info_values_inference"))
+_CACHE_METHODS = frozenset(("update", "merge_new_x_values_in_chunk", "update_nats_cached_x_in_chunk", "update_nats_cached_x_across_chunk"))
 
 
 class BaseNAtSChunkAttentionLayer(BaseNAtSAttentionLayer):
@@ -335,3 +341,24 @@ class GPTNAtSChunkAttentionLayer(BaseNAtSChunkAttentionLayer):
 
 class LlamaNAtSChunkAttentionLayer(BaseNAtSChunkAttentionLayer):
     pass
+
+
+class _DEFINED:
+    """What `_one_token_step` stands in for, as it was when this module was loaded."""
+    prepare_x_values = BaseNAtSAttentionLayer.prepare_x_values
+    add_rotary_emb = AttentionLayer.add_rotary_emb
+    prepare_kv = BaseNAtSAttentionLayer.prepare_kv
+    repeat_kv_values = AttentionLayer.repeat_kv_values
+    multi_head_attention = BaseNAtSAttentionLayer.multi_head_attention
+    role_logits = BaseNAtSAttentionLayer.role_logits
+    sample = (BaseNAtSAttentionLayer._sample_for_token_info_values_inference,
+              BaseNAtSChunkAttentionLayer._sample_for_token_info_values_inference)
+    roles_from_logits = staticmethod(ops.roles_from_logits)
+    roles_from_one_hot = staticmethod(ops.roles_from_one_hot)
+    cache_update = NAtSCache.update
+    merge = staticmethod(NAtSCache.merge_new_x_values_in_chunk)
+    in_chunk = NAtSCache.update_nats_cached_x_in_chunk
+    across_chunk = NAtSCache.update_nats_cached_x_across_chunk
+    layer_update = (NAtSChunkLayerCache.update, NAtSLayerCache.update)
+    valid_tokens = (NAtSChunkLayerCache.valid_tokens, NAtSLayerCache.valid_tokens)
+    linear_forward, linear, call = nn.Linear.forward, staticmethod(nn.functional.linear), nn.Module.__call__

@@ -176,3 +176,64 @@ def test_segment_calls_a_replaced_rotary_embedding(name, monkeypatch):
     monkeypatch.setattr(attention, name, lambda *a, **kw: calls.append(1) or old(*a, **kw))
     got = mod.add_rotary_emb(q, k, emb)
     assert calls and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _targets():
+    from neuralattentionsearch_amd import attention, cache, ops
+    base, chunk = attention.BaseNAtSAttentionLayer, attention.BaseNAtSChunkAttentionLayer
+    return {"prepare_x_values": base, "prepare_kv": base, "multi_head_attention": base, "role_logits": base,
+            "_sample_for_token_info_values_inference": chunk, "add_rotary_emb": attention.AttentionLayer,
+            "repeat_kv_values": attention.AttentionLayer, "apply_rotary_pos_emb": attention, "rotate_half": attention,
+            "NAtSCache.update": cache.NAtSCache, "update_nats_cached_x_in_chunk": cache.NAtSCache,
+            "update_nats_cached_x_across_chunk": cache.NAtSCache, "merge_new_x_values_in_chunk": cache.NAtSCache,
+            "NAtSChunkLayerCache.update": cache.NAtSChunkLayerCache, "valid_tokens": cache.NAtSChunkLayerCache,
+            "roles_from_logits": ops, "roles_from_one_hot": ops, "Linear.forward": torch.nn.Linear,
+            "linear": torch.nn.functional, "Module.__call__": torch.nn.Module}
+
+
+def _counted(owner, name, monkeypatch):
+    """Replaces owner.name by one that counts its calls."""
+    calls = []
+    name = name.split(".")[-1]
+    old = owner.__dict__[name] if isinstance(owner, type) else getattr(owner, name)
+    if isinstance(old, property):
+        new = property(lambda self: calls.append(1) or old.fget(self))
+    elif isinstance(old, staticmethod):
+        new = staticmethod(lambda *a, **kw: calls.append(1) or old.__func__(*a, **kw))
+    else:
+        def new(*a, **kw):
+            calls.append(1)
+            return old(*a, **kw)
+    monkeypatch.setattr(owner, name, new)
+    return calls
+
+
+@pytest.mark.parametrize("name", list(_targets()))
+@pytest.mark.parametrize("where", ["class", "instance"])
+def test_module_step_calls_what_was_replaced(name, where, monkeypatch):
+    """A method, a function or a cache update that a program replaces is called by one-token steps as by any other."""
+    from neuralattentionsearch_amd.attention import LlamaNAtSChunkAttentionLayer
+    from neuralattentionsearch_amd.cache import NAtSCache
+    from neuralattentionsearch_amd.llama import rotary_tables
+    say("module step, replaced", name, where)
+    owner = _targets()[name]
+    kw = dict(dim=256, n_heads=4, n_kv_heads=2, layer_id=0, local_seq_max_length=16, chunk_size=8)
+    mod = LlamaNAtSChunkAttentionLayer(**kw).cuda().eval().requires_grad_(False)
+    cache = NAtSCache(16, 8)
+    calls, at = None, 0
+    for n in [20] + [1] * 9:  # (through the open chunk and the step that completes it)
+        if n == 1 and calls is None:
+            if where == "instance":
+                short = name.split(".")[-1]
+                owner = next((o for o in (mod, cache, cache.cache_model[0]) if isinstance(owner, type) and isinstance(o, owner)), None)
+                if owner is None or short in ("valid_tokens", "__call__", "forward", "merge_new_x_values_in_chunk"):
+                    pytest.skip("nothing that an instance can replace")
+                calls, old = [], getattr(owner, short)
+                monkeypatch.setattr(owner, short, lambda *a, _old=old, **kws: calls.append(1) or _old(*a, **kws), raising=False)
+            else:
+                calls = _counted(owner, name, monkeypatch)
+        emb = rotary_tables(torch.arange(at, at + n, device="cuda")[None], 64, 10000.0, torch.float32)
+        with torch.no_grad():
+            mod(torch.randn(1, n, 256, device="cuda"), emb, None, start_pos=at, cache=cache)
+        at += n
+    assert len(calls) > (9 if name == "Module.__call__" else 0), name  # (9: the module itself)
