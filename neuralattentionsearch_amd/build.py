@@ -56,7 +56,7 @@ def build_host(verbose: bool = True) -> str:
     import torch
     root = os.path.dirname(torch.__file__)
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", os.path.join(root, "include"),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DNATS_TORCH_VERSION="{torch.__version__}"', "-I", os.path.join(root, "include"),
            "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I", sysconfig.get_paths()["include"], "-I", INCLUDE,
            HOST_SOURCE, "-L", os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python", "-o", HOST_PATH]
     if verbose:

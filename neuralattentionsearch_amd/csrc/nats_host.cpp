@@ -539,5 +539,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_nats_host", "native front of the
 PyMODINIT_FUNC PyInit__nats_host(void) {
   g_key_prefill = PyUnicode_InternFromString("prefill");
   g_key_decode = PyUnicode_InternFromString("decode");
-  return PyModule_Create(&kModule);
+  PyObject* m = PyModule_Create(&kModule);
+  // (the functions read tensors through this torch's classes; ops.py binds them under no other)
+  if (m && PyModule_AddStringConstant(m, "built_for", NATS_TORCH_VERSION)) Py_CLEAR(m);
+  return m;
 }

@@ -10,6 +10,7 @@ import collections
 import ctypes
 import math
 import time
+import warnings
 import weakref
 
 import torch
@@ -84,27 +85,60 @@ def workspace(device, key: str, nbytes: int) -> torch.Tensor:
     return buf
 
 
+def _by_address(lib, name: str):
+    """The library's function `name` with every pointer argument taken as a plain address."""
+    restype, argtypes = _lib.SIGNATURES[name]
+    numbers = (ctypes.c_int, ctypes.c_int64, ctypes.c_size_t, ctypes.c_float)
+    proto = ctypes.CFUNCTYPE(restype, *(t if t in numbers else ctypes.c_void_p for t in argtypes))
+    return proto(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+
+
 class _NativeFront:
     """The functions of _nats_host.so, bound to the loaded library at the first call.  Those that stand for an operator
     below take its plain form and answer None to everything else, for which the operator goes its general way; the others
-    take addresses and sizes their callers have checked and return the library's error code."""
+    take addresses and sizes their callers have checked and return the library's error code.  Where _nats_host.so is missing
+    or was built for another torch, every operator goes its general way, with a warning once."""
+
+    _OPERATORS = ("decode", "prefill", "roles_from_logits", "rope_append", "matvec", "step_project")
 
     def __getattr__(self, name):
+        if self.__dict__:  # (bound)
+            raise AttributeError(name)
+        try:
+            lib = _lib.load()
+        except ImportError:
+            if name in self._OPERATORS:
+                return lambda *a: None  # (the operator's general way checks its arguments and then raises it)
+            raise
         try:
             from . import _nats_host
+            if _nats_host.built_for != torch.__version__:
+                raise ImportError(f"built for torch {_nats_host.built_for}, this is {torch.__version__}")
         except ImportError as e:
-            raise ImportError("_nats_host.so is missing or does not fit this torch: build it with `python -m "
-                              f"neuralattentionsearch_amd.build` ({e})") from e
-        lib = _lib.load()
-        names = [n for n in _lib.SIGNATURES if n not in ("nats_abi_version", "nats_last_error")]
-        raw = _raw_stream or (lambda i: torch.cuda.current_stream(i).cuda_stream)
-        _nats_host.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, _workspaces, workspace, raw)
-        for n in dir(_nats_host):
-            if not n.startswith("_") and n != "bind":
-                self.__dict__[n] = getattr(_nats_host, n)
+            warnings.warn("the native front _nats_host.so is not used, calls spend more time on the host: build it with `python -m "
+                          f"neuralattentionsearch_amd.build` ({e})", RuntimeWarning, stacklevel=3)
+            self.__dict__.update(self._general(lib))
+        else:
+            names = [n for n in _lib.SIGNATURES if n not in ("nats_abi_version", "nats_last_error")]
+            raw = _raw_stream or (lambda i: torch.cuda.current_stream(i).cuda_stream)
+            _nats_host.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, _workspaces, workspace, raw)
+            for n in dir(_nats_host):
+                if not n.startswith("_") and n not in ("bind", "built_for"):
+                    self.__dict__[n] = getattr(_nats_host, n)
         if name not in self.__dict__:
             raise AttributeError(name)
         return self.__dict__[name]
+
+    @staticmethod
+    def _general(lib):
+        append, append_plan = _by_address(lib, "nats_cache_append"), _by_address(lib, "nats_cache_append_plan")
+        front = dict.fromkeys(_NativeFront._OPERATORS, lambda *a: None)
+        front["matvec_takes"] = lambda x, w, k: (x.is_cuda and x.device == w.device and x.dtype == w.dtype and _matvec_weight_ok(w)
+                                                 and w.shape[0] > 0 and w.shape[1] == k)
+        front["cache_append"] = lambda *a: append(*a) if len(a) == 19 else append_plan(*a)
+        front["evict_plan"] = _by_address(lib, "nats_evict_plan")
+        front["evict_apply_inplace"] = _by_address(lib, "nats_evict_apply_inplace")
+        return front
 
 
 _front = _NativeFront()

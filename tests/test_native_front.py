@@ -1,8 +1,11 @@
 """The native front of the step-wise operators: it answers None to every form it does not take, and what it takes comes
 out as on the general way, bit for bit."""
+import sys
+
 import pytest
 import torch
 
+import neuralattentionsearch_amd
 from neuralattentionsearch_amd import ops
 from tests.gpu_util import say
 
@@ -103,3 +106,85 @@ def test_equals_the_general_way(dtype, layout, monkeypatch):
     ops._workspaces.clear()
     ops.decode_attention(rn(B, Hq, 1, D), k, v, valid, N)
     assert taken[-1] is not None and len(ops._workspaces) == 1
+
+
+@pytest.fixture
+def without(monkeypatch):
+    """The package as it is where _nats_host.so has not been built, or was built for another torch."""
+    def take_away(how):
+        if how == "missing":
+            monkeypatch.delattr(neuralattentionsearch_amd, "_nats_host", raising=False)
+            monkeypatch.setitem(sys.modules, "neuralattentionsearch_amd._nats_host", None)
+        else:
+            from neuralattentionsearch_amd import _nats_host
+            monkeypatch.setattr(_nats_host, "built_for", "0.0")
+        monkeypatch.setattr(ops, "_front", ops._NativeFront())
+    return take_away
+
+
+@pytest.mark.parametrize("how", ["missing", "other torch"])
+def test_without_the_native_front_operators_go_the_general_way(without, how):
+    without(how)
+    t, v = torch.zeros(1, 2, 1, 32), torch.zeros(1, 2, 8, dtype=torch.uint8)
+    with pytest.warns(RuntimeWarning, match="native front"):
+        assert ops._front.decode(t, t, t, v, 1, None, None, None) is None
+    with pytest.raises(ValueError, match="CPU tensor"):
+        ops.decode_attention(t, t, t, v, 1)
+    with pytest.raises(ValueError, match="CPU tensor"):
+        ops.prefill_attention(t, t, t, v, 8, 8)
+    assert ops.matvec_takes(t, t[0, 0], 32) is False
+    assert ops._front.cache_append(*[None] * 6, *[0] * 7, *[None] * 4, 0, None) < 0  # (the library's error code)
+    assert ops._front.cache_append(*[None] * 6, *[0] * 7, *[None] * 4, 0, *[None] * 5, 0, None, None, None) < 0
+    assert ops._front.evict_plan(*[None] * 5, 0, None, None, None) < 0
+    assert ops._front.evict_apply_inplace(*[None] * 10, 0, None, None, None) < 0
+    with pytest.raises(AttributeError):
+        ops._front.no_such_function
+
+
+def test_without_the_library_arguments_are_checked_first(monkeypatch):
+    from neuralattentionsearch_amd import _lib
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libnats_hip.so")
+    monkeypatch.setattr(ops, "_front", ops._NativeFront())
+    t, v = torch.zeros(1, 2, 1, 32), torch.zeros(1, 2, 8, dtype=torch.uint8)
+    with pytest.raises(ValueError, match="CPU tensor"):
+        ops.decode_attention(t, t, t, v, 1)
+    with pytest.raises(ImportError, match="build it"):
+        ops._front.cache_append()
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:the native front")
+def test_without_the_native_front_everything_runs(without):
+    """A layer's conversation (prompt, one-token steps, segment, streamed evictions) and a cache filled piece by piece."""
+    from neuralattentionsearch_amd.attention import LlamaNAtSChunkAttentionLayer
+    from neuralattentionsearch_amd.cache import NAtSCache, NAtSChunkLayerCache
+    from neuralattentionsearch_amd.llama import rotary_tables
+    say("without the native front")
+    torch.manual_seed(5)
+    mod = LlamaNAtSChunkAttentionLayer(dim=256, n_heads=4, n_kv_heads=2, chunk_size=8, local_seq_max_length=16)
+    mod = mod.cuda().bfloat16().eval().requires_grad_(False)
+    x = torch.randn(1, 60, 256, device="cuda").bfloat16()
+    k, v = (torch.randn(2, 4, 96, 64, device="cuda").bfloat16() for _ in range(2))
+    roles = torch.randint(0, 3, (2, 4, 12), device="cuda", dtype=torch.uint8)
+    roles[:, :, 0] = 0
+
+    def run():
+        outs, at, cache = [], 0, NAtSCache(16, 8)
+        for n in [20] + [1] * 18 + [13] + [1] * 9:
+            emb = rotary_tables(torch.arange(at, at + n, device="cuda")[None], 64, 10000.0, torch.bfloat16)
+            with torch.no_grad():
+                outs.append(mod(x[:, at:at + n], emb, None, start_pos=at, cache=cache))
+            at += n
+        layer = NAtSChunkLayerCache(2, 4, 16, chunk_size=8, device="cuda", track_positions=True)
+        for i in range(12):
+            layer.update(k[:, :, 8 * i:8 * i + 8], v[:, :, 8 * i:8 * i + 8], None, roles=roles[:, :, i:i + 1])
+            layer.post_update(8)
+        return torch.cat(outs, dim=1), [layer.cache_k, layer.cache_v, layer.valid_tokens, layer.token_positions]
+
+    want, rows = run()
+    without("missing")
+    got, got_rows = run()
+    # (the products of a one-token step sum in another order: one rounding to bf16, carried through the layer)
+    assert ((got - want).float().norm() / want.float().norm()).item() <= 4 * 2.0 ** -8
+    assert all(torch.equal(a, b) for a, b in zip(got_rows, rows))
