@@ -20,7 +20,7 @@
 namespace {
 
 // entry points of the library the Python side has loaded, in the order of `kNames`
-enum Fn { kRoles, kPrefillWs, kPrefill, kDecodeWs, kDecode, kRopeAppend, kMatvec, kStepProject, kAppend, kAppendPlan, kApplyInplace, kPlan, kAddNorm, kFns };
+enum Fn { kRoles, kPrefillWs, kPrefill, kDecodeWs, kDecode, kRopeAppend, kMatvec, kStepProject, kAppend, kAppendPlan, kApplyInplace, kPlan, kFns };
 void* g_fn[kFns];
 PyObject *g_workspaces, *g_workspace, *g_raw_stream, *g_move_to_end;  // ops._workspaces, ops.workspace, torch's raw stream of a device
 
@@ -468,40 +468,9 @@ PyObject* evict_apply_inplace(PyObject*, PyObject* const* arg, Py_ssize_t n) {
   return PyLong_FromLong(NATS_CALL(kApplyInplace, nats_evict_apply_inplace, ck, cv, valid, pos, roles, sg, sl, params, ks, vs, es, ws, result, st));
 }
 
-// add_rms_norm(x, delta, weight, eps, carry, carry_mode, chunk_size) -> out
-PyObject* add_rms_norm(PyObject*, PyObject* const* arg, Py_ssize_t n) {
-  TRY
-  if (n != 7) return none();
-  const at::Tensor *x = plain(arg[0]), *w = plain(arg[2]);
-  const at::Tensor* delta = arg[1] == Py_None ? nullptr : plain(arg[1]);
-  const at::Tensor* carry = arg[4] == Py_None ? nullptr : plain(arg[4]);
-  int64_t mode, chunk;
-  float eps;
-  if (!x || !w || (arg[1] != Py_None && !delta) || (arg[4] != Py_None && !carry) || arg[3] == Py_None || !as_scale(arg[3], 0.0, &eps) ||
-      !as_i64(arg[5], &mode) || !as_i64(arg[6], &chunk))
-    return none();
-  const int code = code_of(*x);
-  if (code < 0 || x->dim() < 1 || x->numel() == 0 || !x->is_contiguous()) return none();
-  const int64_t dim = x->size(-1);
-  if (w->dim() != 1 || w->size(0) != dim || w->scalar_type() != x->scalar_type() || !w->is_contiguous() || !same_place(*w, *x)) return none();
-  if (delta && (!delta->is_contiguous() || delta->sizes() != x->sizes() || delta->scalar_type() != x->scalar_type() || !same_place(*delta, *x)))
-    return none();
-  if ((mode != 0 && !carry) || (carry && (carry->numel() != x->numel() || !carry->is_contiguous() || carry->scalar_type() != x->scalar_type() ||
-                                          !same_place(*carry, *x))))
-    return none();
-  void* st;
-  if (!stream_of(*x, &st)) return declined();
-  at::Tensor out = at::empty(x->sizes(), x->options());
-  if (NATS_CALL(kAddNorm, nats_add_rms_norm, x->data_ptr(), delta ? delta->data_ptr() : nullptr, w->data_ptr(), out.data_ptr(),
-                                                 carry ? carry->data_ptr() : nullptr, x->numel() / dim, dim, eps, (int)mode, chunk, code, st))
-    return none();
-  return THPVariable_Wrap(std::move(out));
-  CATCH
-}
-
 const char* const kNames[kFns] = {"nats_roles_from_logits", "nats_prefill_workspace_bytes", "nats_prefill_fwd", "nats_decode_workspace_bytes",
                                   "nats_decode_fwd", "nats_rope_append", "nats_matvec", "nats_step_project", "nats_cache_append",
-                                  "nats_cache_append_plan", "nats_evict_apply_inplace", "nats_evict_plan", "nats_add_rms_norm"};
+                                  "nats_cache_append_plan", "nats_evict_apply_inplace", "nats_evict_plan"};
 
 // bind({name: address}, workspaces, workspace, raw_stream)
 PyObject* bind(PyObject*, PyObject* const* arg, Py_ssize_t n) {
@@ -531,7 +500,7 @@ PyObject* bind(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {METHOD(bind),         METHOD(decode),       METHOD(prefill),    METHOD(roles_from_logits),   METHOD(rope_append),
                           METHOD(matvec),       METHOD(matvec_takes), METHOD(step_project), METHOD(cache_append), METHOD(evict_plan),
-                          METHOD(evict_apply_inplace), METHOD(add_rms_norm), {nullptr, nullptr, 0, nullptr}};
+                          METHOD(evict_apply_inplace), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_nats_host", "native front of the step-wise operators", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
