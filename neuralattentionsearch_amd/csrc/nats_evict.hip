@@ -368,9 +368,12 @@ __global__ __launch_bounds__(256) void evict_plan_small_kernel(const uint8_t* __
   plan_finalize(size_global, size_local, p, ws, result, result_mirror);
 }
 
-// The heads of one sequence or two: a wavefront per head, all in one workgroup of up to 16, which folds them itself (no
-// ticket, no plans past the caches: 64 slots of 8 heads 9.9 -> 7.7 us).
-constexpr int kPlanOneHeads = 16;
+// A few heads: a wavefront per head, all in one workgroup, which folds them itself (no ticket, no plans past the caches: 64 slots
+// of 8 heads in an eviction 9.9 -> 7.7 us).  The wavefronts share one compute unit, so that the line against the kernel below lies
+// where its four heads per workgroup take over (plan alone, 64 / 1024 / 5000 slots, this kernel against that one: 1 head 5.4 / 6.4,
+// 5.6 / 6.7, 16.5 / 17.1 us; 4 heads 5.9 / 7.0, 6.6 / 7.7, 20.7 / 21.8; 8 heads 6.6 / 7.0, 8.0 / 7.8, 24.2 / 22.3; 16 heads 8.3 /
+// 7.3, 10.3 / 8.4, 43.8 / 22.9): four heads, or eight of up to 512 slots.
+constexpr int kPlanOneHeads = 8, kPlanOneAnySlots = 4, kPlanOneSlots = 512;
 __global__ __launch_bounds__(kPlanOneHeads * kWave) void evict_plan_one_kernel(const uint8_t* __restrict__ roles,
                                                                                const int64_t* __restrict__ size_global,
                                                                                const int64_t* __restrict__ size_local, nats_evict_params p,
@@ -880,7 +883,8 @@ extern "C" int nats_evict_plan(const uint8_t* roles, const int64_t* size_global,
     NATS_CHECK_LAUNCH("evict_plan_small_kernel");
     return NATS_OK;
   }
-  if (params->B * params->H_kv <= kPlanOneHeads) {
+  if (const int64_t heads = params->B * params->H_kv;
+      heads <= kPlanOneAnySlots || (heads <= kPlanOneHeads && params->S <= kPlanOneSlots)) {
     const unsigned threads = (unsigned)std::max<int64_t>(256, params->B * params->H_kv * kWave);  // (the fold takes 256)
     hipLaunchKernelGGL(evict_plan_one_kernel, dim3(1), dim3(threads), 0, st, roles, size_global, size_local, *params,
                        static_cast<char*>(workspace), result, result_mirror);

@@ -365,3 +365,16 @@ def test_the_container_takes_its_layers_up_again_after_a_reset():
     gc.collect()
     assert any(m is mirror for m in ops._mirror_pool)
     assert ops.EvictBuffers("cuda").mirror is not None
+
+
+@pytest.mark.parametrize("H,S", [(1, 1025), (4, 513), (5, 512), (5, 513), (8, 512), (8, 513), (9, 33), (16, 64), (16, 1025)])
+def test_plans_of_a_few_heads(H, S):
+    """Both sides of the lines between the plan kernels (heads in one workgroup, heads over the device), a partial chunk too."""
+    rng = np.random.default_rng(S + H)
+    C, W = 8, 16
+    for pad in (0, 3):
+        roles = rng.choice(3, size=(1, H, S), p=(0.05, 0.15, 0.8)).astype(np.uint8)
+        roles[:, :, 0] = 0
+        if pad:
+            roles[:, :, -1] = 0
+        drive(f"plan {H} heads, {S} slots, {pad} short", 1, H, 64, C, W, [(S * C - pad, roles)], torch.bfloat16, seed=S, check_masks=False)
