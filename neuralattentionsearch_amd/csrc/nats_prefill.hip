@@ -1905,15 +1905,22 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
 #undef NATS_PREFILL_BALANCED
   }
   // A launch of several rounds of workgroups per compute unit draws its lightest query groups from the counter
-  // (NATS_PREFILL_POOL = eighths of the query groups that are drawn, 0 = none).  How many (32 / 8 heads of 128, us with 2 / 3
-  // / 8 eighths): with one to three streams per XCD, whose sums differ from XCD to XCD, three (8192 tokens 125.6 / 121.3 / 120.0,
-  // 12000 215.7 / 195.9 / 190.5, 16000 with even roles 747 / 724 / 731, 32768 700.6 / 700.8 / 712.0; packed tiles, 12000 at chunk
-  // 16 163.4 / 164.4 / 165.8, stay at two); with four and more all (batch 4, 4096 tokens 205 / 205 / 196, 32 kv heads, 8192
-  // tokens 158.8 / 156.5 / 146.6, batch 4, 3001 tokens at chunk 32 141.1 / 142.7 / 137.3); gathered rows all (16384 tokens at
-  // chunk 1 290.6 / 289.3 / 283.7).
+  // (NATS_PREFILL_POOL = eighths of the query groups that are drawn, 0 = none).  How many (speed against two eighths, sparse and
+  // even roles, 1400 to 16000 tokens, and us with 2 / 3 / 8 eighths at 32 / 8 heads of 128):
+  //   * all, where the streams of an XCD are a power of two from four on, so that its 64 resident workgroups hold the same
+  //     ranks of all of them again and again: 32 streams 1.02 to 1.10 at every head dim (batch 4, 4096 tokens 205 / 205 / 196, batch
+  //     4, 3001 tokens at chunk 32 141 / 143 / 137), 64 streams 1.02 to 1.08 at 64 and 32 (1.00 at 128).  Others lose: 40 to 56
+  //     streams of 128 0.97 to 0.99, 7 x 1663 tokens 115.7 / 118.1 / 124.1.
+  //   * gathered rows: all at head dims 128 and 32 (1.02 to 1.05, 1.00 to 1.02; 16384 tokens at chunk 1 290.6 / 289.3 / 283.7),
+  //     not at 64 (0.98 to 1.00; batch 3, 16000 tokens with even roles 1788 / 1790 / 1831).
+  //   * three eighths of whole tiles with up to two streams per XCD, whose sums differ from XCD to XCD: 1.00 to 1.03 (8192 tokens
+  //     125.6 / 121.3 / 120.0, 12000 215.7 / 195.9 / 190.5, 16000 with even roles 747 / 724 / 731, 32768 700.6 / 700.8 / 712.0).
+  //   * two otherwise (packed tiles, 12000 at chunk 16 163.4 / 164.4 / 165.8; 24 streams of 128, 3001 tokens 104.6 / 104.4 / 111.4).
   {
     const char* e = getenv("NATS_PREFILL_POOL");
-    const int eighths = e ? atoi(e) : (a.long_rows || g.B * g.H_kv >= 32) ? 8 : packed ? 2 : 3;
+    const int64_t ns = g.B * g.H_kv, per_xcd = ns / 8;
+    const bool in_step = ns % 8 == 0 && per_xcd >= 4 && (per_xcd & (per_xcd - 1)) == 0 && per_xcd * g.D <= 512;
+    const int eighths = e ? atoi(e) : a.long_rows ? (g.D == 64 ? 2 : 8) : in_step ? 8 : !packed && ns <= 16 ? 3 : 2;
     const int n_cu = device_cu_count();
     if (eighths > 0 && eighths <= 8 && w.ticket && n_cu > 0 && n_wg >= 4 * (int64_t)n_cu) {
       a.pool_ranks = (int)((int64_t)a.n_qg * eighths / 8);

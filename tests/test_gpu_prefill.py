@@ -487,6 +487,8 @@ def pooled_groups(monkeypatch):
                                             (1, 64, 8, 6000, 64, 128),     # GQA groups of 8: two head groups per kv head
                                             (2, 32, 8, 9000, 64, 256),     # sixteen streams: two per XCD queue
                                             (3, 16, 8, 7000, 16, 64),      # 24 streams, packed tiles, groups of 2
+                                            (4, 32, 8, 3001, 32, 256),     # four streams per XCD: every group is drawn
+                                            (7, 32, 8, 1663, 64, 256),     # seven
                                             (1, 16, 8, 4096, 64, 256)])    # too few workgroups: nothing is pooled
 def test_pooled_query_groups_change_nothing(pooled_groups, B, Hq, Hkv, L, C, W):
     """Large launches deal their lightest query groups from a counter.  Who computes a query group does not change
