@@ -16,6 +16,8 @@
 // components/cache/nats_chunk_layer_cache.py:603-616).
 // Measured (32 / 8 heads of 128, chunk 64, attention call with its key limits): 40 / 173 / 512 tokens 11.3 -> 5.8, 14.6 -> 8.0, 28.4 -> 15.4
 // us; what is left is the launch, one trip to memory for Q, K and V, a tile or four per wavefront, and the merge.
+#include <stdlib.h>
+
 #include "nats_prefill.h"
 
 namespace nats {
@@ -295,8 +297,10 @@ __global__ __launch_bounds__(kShortWaves * kWave, 2) void prefill_short_kernel(S
 //   * chunks of one to three tokens, whose old rows the other kernel gathers one by one: up to 1792 tokens.  Chunk 1, 1024 / 1536 /
 //     1792 / 2048 tokens: 8 heads of 128 38.2 / 24.0, 38.0 / 35.6, 39.9 / 38.5, 40.3 / 44.9; 8 heads of 64 33.3 / 19.6, 33.6 / 26.1,
 //     31.1 / 29.4, 31.7 / 33.4.  (Chunk 4, 2048 tokens: 41.2 / 30.8, 31.9 / 23.2; chunk 8 41.6 / 28.2, 32.1 / 21.3.)
+// (NATS_PREFILL_SHORT=0 in the environment: nowhere, for comparison.)
 bool prefill_short_takes(int64_t B, int64_t H_q, int64_t H_kv, int64_t D, int64_t L, int64_t C, int dtype) {
   if (dtype != NATS_DTYPE_BF16 || (D != 32 && D != 64 && D != 128) || L > kShortMaxLen) return false;
+  if (const char* e = getenv("NATS_PREFILL_SHORT"); e && e[0] == '0') return false;
   if (C < 4 && D >= 64 && L > 1792) return false;
   const int64_t n_wg = B * H_q * ((L + kShortRows - 1) / kShortRows);
   const int64_t n_cu = device_cu_count();

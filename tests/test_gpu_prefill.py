@@ -13,6 +13,18 @@ pytestmark = pytest.mark.gpu
 TOL = {torch.float32: 1e-5, torch.bfloat16: 2e-2}
 
 
+@pytest.fixture
+def kernels(request, monkeypatch):
+    if request.param == "long":
+        monkeypatch.setenv("NATS_PREFILL_SHORT", "0")
+
+
+def both_kernels(test):
+    """Prompts of a length that the one-launch kernel of short prompts may take: on the kernels of long ones, and as the rule
+    deals them."""
+    return pytest.mark.usefixtures("kernels")(pytest.mark.parametrize("kernels", ["long", "rule"], indirect=True)(test))
+
+
 def run_case(B, Hq, Hkv, L, D, C, W, dtype, seed=0, p=(0.2, 0.3, 0.5), scale_inputs=1.0):
     from neuralattentionsearch_amd import ops
     say("prefill", B, Hq, Hkv, L, D, C, W, dtype, seed)
@@ -40,12 +52,14 @@ def test_fp32_ragged_lengths_and_chunk_sizes(L, C, W, D):
     run_case(2, 4, 2, L, D, C, W, torch.float32, seed=L)
 
 
+@both_kernels
 @pytest.mark.parametrize("n_rep", [1, 2, 3, 4, 6, 7, 8, 12])
 def test_bf16_gqa_group_sizes(n_rep):
     run_case(1, 2 * n_rep, 2, 1024, 128, 64, 256, torch.bfloat16, seed=n_rep)
     run_case(1, 2 * n_rep, 2, 1100, 128, 16, 64, torch.bfloat16, seed=n_rep)  # packed tiles
 
 
+@both_kernels
 @pytest.mark.parametrize("L,C,W,D", [(1000, 64, 256, 128), (777, 32, 64, 128), (512, 16, 64, 64), (2048, 64, 128, 64),
                                      (1536, 128, 256, 128), (200, 8, 16, 128), (63, 64, 64, 128), (65, 64, 64, 128),
                                      (900, 1, 64, 128), (333, 2, 8, 64)])  # per-token roles (chunk size 1) included
@@ -53,6 +67,7 @@ def test_bf16_shapes(L, C, W, D):
     run_case(2, 8, 2, L, D, C, W, torch.bfloat16, seed=L + C)
 
 
+@both_kernels
 @pytest.mark.parametrize("L,C,W,D,dtype", [(700, 3, 12, 128, torch.bfloat16), (900, 6, 24, 64, torch.bfloat16),
                                            (1000, 12, 36, 128, torch.bfloat16), (1300, 24, 48, 128, torch.bfloat16),
                                            (1500, 48, 96, 128, torch.bfloat16), (2000, 96, 192, 128, torch.bfloat16),
@@ -63,6 +78,7 @@ def test_chunk_sizes_that_are_no_power_of_two(L, C, W, D, dtype):
     run_case(2, 8, 2, L, D, C, W, dtype, seed=L + C)
 
 
+@both_kernels
 @pytest.mark.parametrize("Hq,Hkv,L,C,W", [(8, 2, 1000, 64, 128), (8, 2, 777, 32, 64), (4, 4, 900, 16, 32), (4, 2, 650, 1, 16),
                                           (8, 2, 2100, 128, 256)])
 def test_head_dim_32_on_the_matrix_kernels(Hq, Hkv, L, C, W):
@@ -87,11 +103,13 @@ def test_other_head_dims(D, dtype):
     run_case(1, 2, 2, 200, D, 64, 128, dtype, seed=D + 1)
 
 
+@both_kernels
 def test_bf16_llama_head_shape_8_streams():
     # 32 q / 8 kv heads as in Llama-3-8B: exercises the XCD-aware workgroup mapping (B * H_kv % 8 == 0)
     run_case(1, 32, 8, 2048, 128, 64, 256, torch.bfloat16, seed=5, p=(0.05, 0.15, 0.8), scale_inputs=1 / math.sqrt(128) ** 0.5)
 
 
+@both_kernels
 def test_bf16_all_global_equals_causal_attention():
     from neuralattentionsearch_amd import ops
     say("prefill all-global == causal")
@@ -188,6 +206,7 @@ def test_packed_tiles_full_size_sampled_rows(Hq, Hkv, L, C, W):
 def split_lists(monkeypatch):
     def switch(on: bool):
         monkeypatch.setenv("NATS_PREFILL_SPLIT", "1" if on else "0")
+        monkeypatch.setenv("NATS_PREFILL_SHORT", "0")
     yield switch
     monkeypatch.delenv("NATS_PREFILL_SPLIT", raising=False)
 
@@ -256,6 +275,7 @@ def test_prompts_of_few_workgroups_split_their_tile_lists(split_lists, Hq, Hkv, 
 def packed_tiles(monkeypatch):
     def switch(on: bool):
         monkeypatch.setenv("NATS_PREFILL_PACKED", "1" if on else "0")
+        monkeypatch.setenv("NATS_PREFILL_SHORT", "0")
     yield switch
     monkeypatch.delenv("NATS_PREFILL_PACKED", raising=False)
 
@@ -288,6 +308,7 @@ def test_packed_tiles_agree_with_whole_tiles(packed_tiles, B, Hq, Hkv, L, D, C, 
     packed_tiles(True)
     packed = ops.prefill_attention(q, k, v, roles, C, W).float()
     assert torch.isfinite(packed).all()
+    assert p[0] == 1.0 or not torch.equal(packed, whole), "both ways took one kernel"
     assert (packed - whole).abs().max().item() <= 2e-2
 
 
@@ -327,6 +348,7 @@ def test_packed_tiles_on_segments_over_a_filled_cache(packed_tiles):
 def far_rows(monkeypatch):
     def switch(on: bool):
         monkeypatch.setenv("NATS_PREFILL_FAR", "1" if on else "0")
+        monkeypatch.setenv("NATS_PREFILL_SHORT", "0")
     yield switch
     monkeypatch.delenv("NATS_PREFILL_FAR", raising=False)
 
@@ -342,6 +364,7 @@ def test_long_lived_rows_full_size_sampled_rows(Hq, Hkv, L, C, W, p):
     check_sampled_rows(1, Hq, Hkv, L, 128, C, W, n_samples=64, p=p)
 
 
+@both_kernels
 @pytest.mark.parametrize("B,Hq,Hkv,L,D,C,W,p", [
     (2, 8, 2, 1500, 128, 1, 4, (0.1, 0.3, 0.6)),
     (1, 8, 2, 1100, 64, 2, 8, (0.05, 0.5, 0.45)),
@@ -355,6 +378,7 @@ def test_long_lived_rows_against_the_oracle(B, Hq, Hkv, L, D, C, W, p):
     run_case(B, Hq, Hkv, L, D, C, W, torch.bfloat16, seed=L, p=p)
 
 
+@both_kernels
 @pytest.mark.parametrize("L", [1, 2, 15, 16, 17, 31, 63, 64, 65, 129])
 @pytest.mark.parametrize("C,W", [(1, 1), (1, 4), (2, 4), (8, 8), (3, 6)])
 def test_short_sequences_with_short_chunks(L, C, W):
@@ -420,6 +444,7 @@ def check_rising(B, Hq, Hkv, L, D, C, W, p, step_rows=48, step_nats=7.0, seed=0)
     assert not bad.any(), (int(bad.sum()), (got - want).abs().max().item())
 
 
+@both_kernels
 @pytest.mark.parametrize("Hq,Hkv,L,D,C,W,p", [
     (8, 2, 1500, 128, 64, 256, (1.0, 0.0, 0.0)),   # whole tiles, dense
     (8, 2, 1500, 128, 64, 128, (0.2, 0.3, 0.5)),   # whole tiles, mixed roles
