@@ -35,7 +35,7 @@ def apply_rotary_pos_emb(q, k, cos, sin, unsqueeze_dim: int = 1):
     return (q * cos) + (rotate_half(q) * sin), (k * cos) + (rotate_half(k) * sin)
 
 
-_ROTARY = (rotate_half, apply_rotary_pos_emb)  # (as this module defines them)
+_ROTATE_HALF, _APPLY_ROTARY = rotate_half, apply_rotary_pos_emb  # (as this module defines them)
 
 
 def _plain_linear(m: nn.Module) -> bool:
@@ -79,7 +79,7 @@ class AttentionLayer(nn.Module):
         if pos_emb is not None:
             cos, sin = pos_emb
             # (one kernel with the rounding points of the torch ops, where nothing watches or replaces those)
-            if (rotate_half is _ROTARY[0] and apply_rotary_pos_emb is _ROTARY[1]
+            if (rotate_half is _ROTATE_HALF and apply_rotary_pos_emb is _APPLY_ROTARY
                     and all(type(t) is torch.Tensor for t in (xk, cos, sin)) and _plain_execution(xq, (xk, cos, sin))
                     and xq.dim() == xk.dim() == 4 and cos.shape == sin.shape == (xq.shape[0], *xq.shape[2:])
                     and (xk.shape[0], *xk.shape[2:]) == cos.shape and xq.shape[3] <= 256 and ops.rope_qk_ok(xq, xk, cos, sin)):
@@ -205,19 +205,18 @@ class BaseNAtSAttentionLayer(AttentionLayer):
     def _step_as_defined(self, cache, layer) -> bool:
         """Whether everything `_one_token_step` stands in for is what this package (and torch) defines: nothing of it replaced
         in a subclass, on a class, on an object or in a module."""
-        cls, kind, d = type(self), type(layer), _DEFINED
-        return (cls.prepare_x_values is d.prepare_x_values and cls.add_rotary_emb is d.add_rotary_emb
-                and cls.prepare_kv is d.prepare_kv and cls.repeat_kv_values is d.repeat_kv_values
-                and cls.multi_head_attention is d.multi_head_attention and cls.role_logits is d.role_logits
-                and cls._sample_for_token_info_values_inference in d.sample
-                and BaseNAtSAttentionLayer._sample_for_token_info_values_inference is d.sample[0]
-                and apply_rotary_pos_emb is _ROTARY[1] and rotate_half is _ROTARY[0]
-                and ops.roles_from_logits is d.roles_from_logits and ops.roles_from_one_hot is d.roles_from_one_hot
-                and NAtSCache.update is d.cache_update and NAtSCache.merge_new_x_values_in_chunk is d.merge
-                and NAtSCache.update_nats_cached_x_in_chunk is d.in_chunk
-                and NAtSCache.update_nats_cached_x_across_chunk is d.across_chunk
-                and kind.update in d.layer_update and kind.valid_tokens in d.valid_tokens
-                and nn.Linear.forward is d.linear_forward and nn.functional.linear is d.linear and nn.Module.__call__ is d.call
+        cls, kind = type(self), type(layer)
+        return (cls.prepare_x_values is _PREPARE_X and cls.add_rotary_emb is _ADD_ROTARY and cls.prepare_kv is _PREPARE_KV
+                and cls.repeat_kv_values is _REPEAT_KV and cls.multi_head_attention is _ATTENTION and cls.role_logits is _ROLE_LOGITS
+                and cls._sample_for_token_info_values_inference in _SAMPLES
+                and BaseNAtSAttentionLayer._sample_for_token_info_values_inference is _SAMPLE
+                and apply_rotary_pos_emb is _APPLY_ROTARY and rotate_half is _ROTATE_HALF
+                and ops.roles_from_logits is _ROLES_FROM_LOGITS and ops.roles_from_one_hot is _ROLES_FROM_ONE_HOT
+                and NAtSCache.update is _CACHE_UPDATE and NAtSCache.merge_new_x_values_in_chunk is _MERGE
+                and NAtSCache.update_nats_cached_x_in_chunk is _IN_CHUNK
+                and NAtSCache.update_nats_cached_x_across_chunk is _ACROSS_CHUNK
+                and kind.update in _LAYER_UPDATES and kind.valid_tokens in _VALID_TOKENS
+                and nn.Linear.forward is _LINEAR_FORWARD and nn.functional.linear is _LINEAR and nn.Module.__call__ is _CALL
                 and self.__dict__.keys().isdisjoint(_STEP_METHODS) and cache.__dict__.keys().isdisjoint(_CACHE_METHODS)
                 and "update" not in layer.__dict__)
 
@@ -343,22 +342,18 @@ class LlamaNAtSChunkAttentionLayer(BaseNAtSChunkAttentionLayer):
     pass
 
 
-class _DEFINED:
-    """What `_one_token_step` stands in for, as it was when this module was loaded."""
-    prepare_x_values = BaseNAtSAttentionLayer.prepare_x_values
-    add_rotary_emb = AttentionLayer.add_rotary_emb
-    prepare_kv = BaseNAtSAttentionLayer.prepare_kv
-    repeat_kv_values = AttentionLayer.repeat_kv_values
-    multi_head_attention = BaseNAtSAttentionLayer.multi_head_attention
-    role_logits = BaseNAtSAttentionLayer.role_logits
-    sample = (BaseNAtSAttentionLayer._sample_for_token_info_values_inference,
-              BaseNAtSChunkAttentionLayer._sample_for_token_info_values_inference)
-    roles_from_logits = staticmethod(ops.roles_from_logits)
-    roles_from_one_hot = staticmethod(ops.roles_from_one_hot)
-    cache_update = NAtSCache.update
-    merge = staticmethod(NAtSCache.merge_new_x_values_in_chunk)
-    in_chunk = NAtSCache.update_nats_cached_x_in_chunk
-    across_chunk = NAtSCache.update_nats_cached_x_across_chunk
-    layer_update = (NAtSChunkLayerCache.update, NAtSLayerCache.update)
-    valid_tokens = (NAtSChunkLayerCache.valid_tokens, NAtSLayerCache.valid_tokens)
-    linear_forward, linear, call = nn.Linear.forward, staticmethod(nn.functional.linear), nn.Module.__call__
+# What `_one_token_step` stands in for, as it is when this module is loaded.
+_PREPARE_X = BaseNAtSAttentionLayer.prepare_x_values
+_ADD_ROTARY = AttentionLayer.add_rotary_emb
+_PREPARE_KV = BaseNAtSAttentionLayer.prepare_kv
+_REPEAT_KV = AttentionLayer.repeat_kv_values
+_ATTENTION = BaseNAtSAttentionLayer.multi_head_attention
+_ROLE_LOGITS = BaseNAtSAttentionLayer.role_logits
+_SAMPLE = BaseNAtSAttentionLayer._sample_for_token_info_values_inference
+_SAMPLES = (BaseNAtSChunkAttentionLayer._sample_for_token_info_values_inference, _SAMPLE)
+_ROLES_FROM_LOGITS, _ROLES_FROM_ONE_HOT = ops.roles_from_logits, ops.roles_from_one_hot
+_CACHE_UPDATE, _MERGE = NAtSCache.update, NAtSCache.merge_new_x_values_in_chunk
+_IN_CHUNK, _ACROSS_CHUNK = NAtSCache.update_nats_cached_x_in_chunk, NAtSCache.update_nats_cached_x_across_chunk
+_LAYER_UPDATES = (NAtSChunkLayerCache.update, NAtSLayerCache.update)
+_VALID_TOKENS = (NAtSChunkLayerCache.valid_tokens, NAtSLayerCache.valid_tokens)
+_LINEAR_FORWARD, _LINEAR, _CALL = nn.Linear.forward, nn.functional.linear, nn.Module.__call__
