@@ -532,9 +532,12 @@ int prepare_key_limits(const uint8_t* roles, int64_t B, int64_t H_kv, int64_t S,
   const int64_t n_streams = B * H_kv;
   KeyLimArgs a{};
   // The scan's result is needed only inside the key-limit kernel, which searches the roles itself (one launch less: a
-  // segment's limits 4.1 + 1 + 4.2 -> 5.1 us); streams so long that a run of local slots could make that search slow take the scan
-  // kernel.
-  const bool inline_scan = S <= 8192;
+  // segment's limits 4.1 + 1 + 4.2 -> 5.1 us).  The search is one trip to L2 per 64 slots up to the next global one: streams so
+  // long that a run of local slots could make it slow take the scan kernel, and so do segments over a filled cache from 512
+  // slots on, where every wavefront of cached rows looks for the segment's first global slot besides.  Attention of a segment
+  // whose only global slot is its last one, 8 heads of 64 over 1000 rows, search / scan: 512 slots 33.9 / 35.4 us, 1024 34.5 /
+  // 33.6, 2048 45.6 / 37.8 (5 % global slots: 29.7 / 32.7, 28.0 / 31.6, 32.3 / 36.2); from empty up to 8192 slots.
+  const bool inline_scan = S <= (past == nullptr ? 8192 : 512);
   if (inline_scan) {
     a.roles = roles;
   } else if (int rc = launch_role_scan(roles, n_streams, S, W, C, nullptr, w.vis_lim, w.first_global, st)) {

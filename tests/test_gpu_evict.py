@@ -378,3 +378,17 @@ def test_plans_of_a_few_heads(H, S):
         if pad:
             roles[:, :, -1] = 0
         drive(f"plan {H} heads, {S} slots, {pad} short", 1, H, 64, C, W, [(S * C - pad, roles)], torch.bfloat16, seed=S, check_masks=False)
+
+
+@pytest.mark.parametrize("S", [511, 512, 513])
+@pytest.mark.parametrize("role", [0, 1, 2])
+def test_limits_of_a_segment_on_both_sides_of_the_scan(S, role):
+    """Key limits searched in the roles and taken from the scan kernel: a segment of one role but for its last slot."""
+    C, W, H = 2, 8, 2
+    rng = np.random.default_rng(S + role)
+    first = rng.choice(3, size=(1, H, 60), p=(0.2, 0.4, 0.4)).astype(np.uint8)
+    first[:, :, 0] = 0
+    seg = np.full((1, H, S), role, dtype=np.uint8)
+    seg[:, 1, S // 3] = 0
+    seg[:, :, -1] = 0
+    drive(f"limits, {S} slots of role {role}", 1, H, 64, C, W, [(120, first), (S * C - 1, seg)], torch.bfloat16, seed=S, attend_n_rep=2)
