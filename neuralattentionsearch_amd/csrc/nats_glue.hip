@@ -55,6 +55,8 @@ struct AddNormArgs {
 // step: 8 (16-byte loads of bf16, two 16-byte loads of fp32) when dim % 8 == 0, else 1.  Bound by one trip to memory and
 // the launch: a row is one step of as many threads as it takes (dim / 8), so that every load of the row leaves at once
 // (one row with delta and chunk statistic: dim 4096 7.1 -> 5.0 us, 8192 12.3 -> 6.5 us against 256 threads that walk the row).
+// Many rows are bound by HBM, and threads without columns cost it: 8192 bf16 rows of 5120 with 256 / 640 / 1024 threads 65.3 / 66.0 /
+// 67.2 us, of 4104 60.1 / 55.5 / 60.5, of 6144 with 768 / 1024 76.4 / 77.2.
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxDim = 8192;
 
@@ -570,6 +572,10 @@ extern "C" int nats_add_rms_norm(void* x, const void* delta, const void* weight,
     NATS_NORM(BF, 8, 256, 1);                                   \
   } else if (dim <= 4096) {                                     \
     NATS_NORM(BF, 8, 512, 1);                                   \
+  } else if (dim <= 5120) {                                     \
+    NATS_NORM(BF, 8, 640, 1);                                   \
+  } else if (dim <= 6144) {                                     \
+    NATS_NORM(BF, 8, 768, 1);                                   \
   } else {                                                      \
     NATS_NORM(BF, 8, 1024, 1);                                  \
   }

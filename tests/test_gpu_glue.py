@@ -21,7 +21,8 @@ def torch_rms(x, w, eps):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,dim", [(1, 4096), (3, 512), (2, 8192), (5, 100)])
+@pytest.mark.parametrize("rows,dim", [(1, 4096), (3, 512), (2, 8192), (5, 100), (2, 2048), (3, 2056), (2, 4104), (3, 5120),
+                                      (2, 5128), (2, 6144), (1, 6152)])
 def test_add_rms_norm_and_chunk_statistic(dtype, rows, dim):
     from neuralattentionsearch_amd import ops
     say("add_rms_norm", dtype, rows, dim)
