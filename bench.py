@@ -43,7 +43,7 @@ if ROOT not in sys.path:
 # recorded with `python bench.py --record-traffic prefill=<FETCH KiB>,<WRITE KiB> ...`.
 TRAFFIC_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "bench_traffic.json")
 TRAFFIC_SOURCES = {
-    "prefill": ["nats_prefill.hip", "nats_roles.hip", "nats_common.h"],
+    "prefill": ["nats_prefill.hip", "nats_prefill.h", "nats_roles.hip", "nats_common.h"],
     "decode": ["nats_decode.hip", "nats_common.h"],
     "evict": ["nats_evict.hip", "nats_common.h"],
 }
@@ -714,7 +714,7 @@ def main():
         d = res["decode"]
         line["roofline_decode"] = {"bound": "hbm", "achieved": d["gbs"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
                                    "frac": d["frac_of_hbm_peak"],
-                                   "kernel": f"decode_split_mfma_kernel<{args.head_dim},4> + decode_merge_balanced_kernel"}
+                                   "kernel": f"decode_split_mfma_kernel<{args.head_dim}, 4, 0> + decode_merge_balanced_kernel"}
         line["roofline_decode"]["traffic"], line["roofline_decode"]["traffic_source"] = (
             measured_traffic("decode") if (args.decode_batch, args.decode_context, args.head_dim) == (32, 65536, 128)
             else (None, "not the profiled workload"))
