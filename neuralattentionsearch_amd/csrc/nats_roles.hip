@@ -178,31 +178,42 @@ __global__ __launch_bounds__(256) void key_lim_kernel(KeyLimArgs a) {
     const bool in = row < a.N && row >= base;
     const int slot = in ? slot_of(row - base) : 0;
     const int s0 = slot_of(max(tile * kTile, base) - base);  // slot of the tile's first region row (the tile starts inside N)
-    if (kPast && tile * kTile < base) {
-      for (int blk = 0; blk < a.S; blk += kWave) {
-        const int n = blk + lane;
-        const uint64_t bits = __ballot(n < a.S && (r[n] == NATS_ROLE_GLOBAL || n == a.S - 1));
-        if (bits) {
-          first_g = blk + __builtin_ctzll(bits);
-          break;
+    // The global slots of blocks of 64 from slot `from` on, until `stop(first slot of the block, their bits)`: one trip to L2
+    // for kAhead blocks (requested one by one they were the time of a stream whose next global slot is far).
+    constexpr int kAhead = 8;
+    auto global_bits = [&](int from, auto stop) {
+      for (int blk = from; blk < a.S; blk += kAhead * kWave) {
+        uint8_t v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const int n = blk + u * kWave + lane;
+          v[u] = n < a.S ? r[n] : uint8_t(NATS_ROLE_SW);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const int n = blk + u * kWave + lane;
+          if (stop(blk + u * kWave, __ballot(v[u] == NATS_ROLE_GLOBAL || n == a.S - 1))) return;
         }
       }
+    };
+    if (kPast && tile * kTile < base) {
+      global_bits(0, [&](int blk, uint64_t bits) {
+        if (bits) first_g = blk + __builtin_ctzll(bits);
+        return bits != 0;
+      });
     }
     const uint8_t role = in ? r[slot] : uint8_t(NATS_ROLE_GLOBAL);
     const bool want = in && role == NATS_ROLE_LOCAL;
     int g = -1;
     if (__ballot(want)) {
-      for (int blk = s0; blk < a.S; blk += kWave) {
-        const int n = blk + lane;
-        const bool is_g = n < a.S && (r[n] == NATS_ROLE_GLOBAL || n == a.S - 1);
-        const uint64_t bits = __ballot(is_g);
+      global_bits(s0, [&](int blk, uint64_t bits) {
         if (want && g < 0) {
           const int rel = slot - blk;  // 0 .. 63 in the first block, negative afterwards
           const uint64_t ahead = rel > 0 ? bits >> rel : bits;
           if (ahead) g = (rel > 0 ? slot : blk) + __builtin_ctzll(ahead);
         }
-        if (!__ballot(want && g < 0)) break;
-      }
+        return __ballot(want && g < 0) == 0;
+      });
     }
     v_inline = role == NATS_ROLE_GLOBAL ? kLimGlobal : role == NATS_ROLE_SW ? slot + slot_of(a.W) : g;
   }
@@ -532,12 +543,12 @@ int prepare_key_limits(const uint8_t* roles, int64_t B, int64_t H_kv, int64_t S,
   const int64_t n_streams = B * H_kv;
   KeyLimArgs a{};
   // The scan's result is needed only inside the key-limit kernel, which searches the roles itself (one launch less: a
-  // segment's limits 4.1 + 1 + 4.2 -> 5.1 us).  The search is one trip to L2 per 64 slots up to the next global one: streams so
-  // long that a run of local slots could make it slow take the scan kernel, and so do segments over a filled cache from 512
+  // segment's limits 4.1 + 1 + 4.2 -> 5.1 us).  The search is one trip to L2 per 512 slots up to the next global one: streams so
+  // long that a run of local slots could make it slow take the scan kernel, and so do segments over a filled cache from 1024
   // slots on, where every wavefront of cached rows looks for the segment's first global slot besides.  Attention of a segment
-  // whose only global slot is its last one, 8 heads of 64 over 1000 rows, search / scan: 512 slots 33.9 / 35.4 us, 1024 34.5 /
-  // 33.6, 2048 45.6 / 37.8 (5 % global slots: 29.7 / 32.7, 28.0 / 31.6, 32.3 / 36.2); from empty up to 8192 slots.
-  const bool inline_scan = S <= (past == nullptr ? 8192 : 512);
+  // whose only global slot is its last one, 8 heads of 64 over 1000 rows, search / scan: 512 slots 33.8 / 35.4 us, 1024 33.7 /
+  // 33.4, 2048 44.2 / 38.6 (5 % global slots: 30.8 / 33.0, 29.4 / 31.9, 34.7 / 36.8); from empty up to 8192 slots.
+  const bool inline_scan = S <= (past == nullptr ? 8192 : 1024);
   if (inline_scan) {
     a.roles = roles;
   } else if (int rc = launch_role_scan(roles, n_streams, S, W, C, nullptr, w.vis_lim, w.first_global, st)) {

@@ -380,7 +380,7 @@ def test_plans_of_a_few_heads(H, S):
         drive(f"plan {H} heads, {S} slots, {pad} short", 1, H, 64, C, W, [(S * C - pad, roles)], torch.bfloat16, seed=S, check_masks=False)
 
 
-@pytest.mark.parametrize("S", [511, 512, 513])
+@pytest.mark.parametrize("S", [511, 513, 1024, 1025])
 @pytest.mark.parametrize("role", [0, 1, 2])
 def test_limits_of_a_segment_on_both_sides_of_the_scan(S, role):
     """Key limits searched in the roles and taken from the scan kernel: a segment of one role but for its last slot."""
