@@ -1659,22 +1659,22 @@ static int most_split(int64_t n_wg, int64_t Tk) {
   return n < 2 ? 1 : (int)n;
 }
 // How many of them pay: what a share saves is its part of the visible tiles, what the split costs is the merge launch (4 us) and
-// the partial results, 32 rows of D floats per wavefront out and back.  A tile takes 1.6 / 1.25 / 1.1 us at head dims 128 / 64 / 32
-// (300 tokens over 25000 visible rows, no split: 615 / 490 / 425 us).  Cached rows are taken as visible, of the region's own tiles
-// half (the heaviest list of unequal heads ends the launch), a share's partial results as 0.045 us per workgroup at head dim 128:
-// the two that lose least over 1278 launches (256 to 7000 tokens from empty and over 300 to 65536 tokens, 4 to 32 heads, chunks 1
-// to 64), where this rule takes 1.02 times the best number of shares, never splitting 1.1 and more, always as far as the device
-// goes 1.03 and up to 1.5.  32 / 8 heads of 128, one workgroup per list / split as far as the device goes: 1024 tokens from empty
-// 24.4 / 35.4 us, 700 tokens over 492 rows 29.5 / 37.3; 40 over 1728 rows 57 / 28, 301 over 6656 rows 180 / 58.  8 heads of 32, 3000
-// tokens from empty 40.4 / 32.4; of 64 50.6 / 42.3; 1024 tokens at chunk 16 over 348 rows of 32 24.2 / 18.7.
+// the partial results, 32 rows of D floats per wavefront out and back (0.066 us per workgroup at head dim 128).  A tile takes 1.6 /
+// 1.25 / 1.1 us at head dims 128 / 64 / 32 (300 tokens over 25000 visible rows, no split: 615 / 490 / 425 us).  Cached rows are taken
+// as visible, of the region's own tiles three tenths: what the roles leave visible is not known here, and prompts with the roles of
+// random weights would take twice that (8 heads of 64, 2500 tokens, one workgroup per list / split: 40.6 / 31.2 us), sparse ones none
+// (2 kv heads of 128, 3000 tokens 28.9 / 36.6).  Of the constants tried over 1339 launches (256 to 7000 tokens from empty and over 300 to
+// 65536 tokens, 4 to 32 heads, chunks 1 to 64) these are within 1.2 % of the best number of shares in the mean; with head dim 128's at
+// every head dim 2 %, always as far as the device goes 3 to 15 %, never 3 to 40 %.  32 / 8 heads of 128: 1024 tokens from empty 24.4 / 35.4
+// us, 700 over 492 rows 29.5 / 37.3; 40 over 1728 rows 57 / 28, 301 over 6656 rows 180 / 58.  8 heads of 32, 3000 tokens 40.4 / 32.4.
 static int choose_split(int64_t n_wg, int64_t Tk, int64_t base, int64_t D) {
   const int most = most_split(n_wg, Tk);
-  const double visible = (double)(base / kTile) + 0.5 * (double)(Tk - base / kTile);
+  const double visible = (double)(base / kTile) + 0.3 * (double)(Tk - base / kTile);
   const double tile = D == 128 ? 1.6 : D == 64 ? 1.25 : 1.1;
   int best = 1;
   double gain = 0.0;
   for (int n = 2; n <= most; ++n) {
-    const double g = tile * visible * (n - 1) / n - 4.0 - 0.045 * (double)D / 128.0 * (double)n_wg * n;
+    const double g = tile * visible * (n - 1) / n - 4.0 - 0.066 * (double)D / 128.0 * (double)n_wg * n;
     if (g > gain) gain = g, best = n;
   }
   return best;
