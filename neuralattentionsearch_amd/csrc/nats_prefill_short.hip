@@ -291,9 +291,10 @@ __global__ __launch_bounds__(kShortWaves * kWave, 2) void prefill_short_kernel(S
 //     below.  32 / 8 heads of 128: 40 / 173 / 512 tokens 11.2 / 5.8, 14.7 / 8.0, 22.4 / 15.4, beyond that (700, 1024) 22.4 / 23.6,
 //     24.4 / 31.2; batch 4, 128 / 173 tokens 13.3 / 9.3, 15.2 / 16.1.  8 heads of 64: 2048 tokens 29.4 / 16.8, batch 2 of them 31.8 /
 //     29.3; 32 heads of 64, 1024 tokens 28.0 / 22.0, 1280 28.5 / 27.6.
-//   * three at head dim 64 (44 KB: that many fit) where groups of four q heads share a workgroup of the other kernel: 16 / 4
-//     heads, 1536 / 1792 / 2048 tokens 19.5 / 17.3, 21.8 / 22.7, 22.6 / 29.6 (chunk 16: 21.3 / 18.0, 19.4 / 21.6, 19.7 / 27.8); 32 /
-//     8 heads, 768 / 1024 tokens 18.1 / 14.2, 19.6 / 20.7.
+//   * at head dim 64 (44 KB: three fit) and with groups of four q heads, which share a workgroup of the other kernel, fewer the longer
+//     the prompt: four up to 768 tokens (300 tokens, 832 / 1024 workgroups 1.2 to 2.0 / 0.97 to 1.5 times its speed), three and a half up
+//     to 1024 (850 tokens, 864 workgroups 1.06 to 1.44; 940, 960 0.86 to 1.22), three beyond: 16 / 4 heads, 1536 / 1792 / 2048 tokens
+//     19.5 / 17.3, 21.8 / 22.7, 22.6 / 29.6 (chunk 16: 21.3 / 18.0, 19.4 / 21.6, 19.7 / 27.8).
 //   * chunks of one to three tokens, whose old rows the other kernel gathers one by one: up to 1792 tokens.  Chunk 1, 1024 / 1536 /
 //     1792 / 2048 tokens: 8 heads of 128 38.2 / 24.0, 38.0 / 35.6, 39.9 / 38.5, 40.3 / 44.9; 8 heads of 64 33.3 / 19.6, 33.6 / 26.1,
 //     31.1 / 29.4, 31.7 / 33.4.  (Chunk 4, 2048 tokens: 41.2 / 30.8, 31.9 / 23.2; chunk 8 41.6 / 28.2, 32.1 / 21.3.)
@@ -304,7 +305,8 @@ bool prefill_short_takes(int64_t B, int64_t H_q, int64_t H_kv, int64_t D, int64_
   if (C < 4 && D >= 64 && L > 1792) return false;
   const int64_t n_wg = B * H_q * ((L + kShortRows - 1) / kShortRows);
   const int64_t n_cu = device_cu_count();
-  return n_wg <= (D == 128 ? 2 : D == 64 && H_q / H_kv % 4 == 0 ? 3 : 4) * n_cu;
+  const int64_t halves = D == 128 ? 4 : D == 32 || H_q / H_kv % 4 != 0 || L <= 768 ? 8 : L <= 1024 ? 7 : 6;  // of n_cu workgroups
+  return 2 * n_wg <= halves * n_cu;
 }
 
 template <int D>
