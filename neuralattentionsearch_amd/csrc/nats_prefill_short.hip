@@ -293,8 +293,9 @@ __global__ __launch_bounds__(kShortWaves * kWave, 2) void prefill_short_kernel(S
 //     29.3; 32 heads of 64, 1024 tokens 28.0 / 22.0, 1280 28.5 / 27.6.
 //   * at head dim 64 (44 KB: three fit) and with groups of four q heads, which share a workgroup of the other kernel, fewer the longer
 //     the prompt: four up to 768 tokens (300 tokens, 832 / 1024 workgroups 1.2 to 2.0 / 0.97 to 1.5 times its speed), three and a half up
-//     to 1024 (850 tokens, 864 workgroups 1.06 to 1.44; 940, 960 0.86 to 1.22), three beyond: 16 / 4 heads, 1536 / 1792 / 2048 tokens
-//     19.5 / 17.3, 21.8 / 22.7, 22.6 / 29.6 (chunk 16: 21.3 / 18.0, 19.4 / 21.6, 19.7 / 27.8).
+//     to 1024 (850 tokens, 864 workgroups 1.06 to 1.44; 940, 960 0.86 to 1.09, chunk 1 1.22 and 1.09 to 1024 tokens: four there), three
+//     beyond: 16 / 4 heads, 1536 / 1792 / 2048 tokens 19.5 / 17.3, 21.8 / 22.7, 22.6 / 29.6 (chunk 16: 21.3 / 18.0, 19.4 / 21.6,
+//     19.7 / 27.8; chunk 1: 29.0 / 29.2, 33.5 / 29.7, 38.3 / 30.2).
 //   * chunks of one to three tokens, whose old rows the other kernel gathers one by one: up to 1792 tokens.  Chunk 1, 1024 / 1536 /
 //     1792 / 2048 tokens: 8 heads of 128 38.2 / 24.0, 38.0 / 35.6, 39.9 / 38.5, 40.3 / 44.9; 8 heads of 64 33.3 / 19.6, 33.6 / 26.1,
 //     31.1 / 29.4, 31.7 / 33.4.  (Chunk 4, 2048 tokens: 41.2 / 30.8, 31.9 / 23.2; chunk 8 41.6 / 28.2, 32.1 / 21.3.)
@@ -305,7 +306,8 @@ bool prefill_short_takes(int64_t B, int64_t H_q, int64_t H_kv, int64_t D, int64_
   if (C < 4 && D >= 64 && L > 1792) return false;
   const int64_t n_wg = B * H_q * ((L + kShortRows - 1) / kShortRows);
   const int64_t n_cu = device_cu_count();
-  const int64_t halves = D == 128 ? 4 : D == 32 || H_q / H_kv % 4 != 0 || L <= 768 ? 8 : L <= 1024 ? 7 : 6;  // of n_cu workgroups
+  int64_t halves = D == 128 ? 4 : 8;  // of n_cu workgroups
+  if (D == 64 && H_q / H_kv % 4 == 0 && L > (C < 4 ? 1024 : 768)) halves = L <= 1024 ? 7 : 6;
   return 2 * n_wg <= halves * n_cu;
 }
 

@@ -34,6 +34,7 @@ def test_short_prompts(D, L, C, W):
 @pytest.mark.parametrize("Hq,Hkv,D,C,lens", [
     (16, 4, 64, 64, (1536, 1537)), (16, 16, 64, 64, (2048,)),  # three / four workgroups per compute unit
     (40, 10, 64, 64, (768, 769)), (32, 8, 64, 64, (896, 897)), (64, 16, 64, 64, (512, 513)),
+    (32, 8, 64, 1, (1024, 1025)),
     (8, 8, 128, 64, (2047, 2049)), (12, 4, 128, 64, (1344, 1345)),
     (8, 8, 64, 1, (1792, 1793)), (8, 8, 128, 3, (1792, 1793)), (8, 8, 128, 4, (1793,)),  # chunks of a few tokens
 ])
