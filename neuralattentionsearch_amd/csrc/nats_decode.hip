@@ -782,12 +782,13 @@ static int decode_rep_columns(int64_t n_rep) { return n_rep >= 5 ? 8 : n_rep >= 
 //   * up to four tiles per wavefront of the longest head: two workgroups per compute unit, four wavefronts each, and the
 //     merge kernel (batch 1, contexts 2k / 16k / 64k: 13.3 / 8.1, 15.9 / 11.5, 21.7 / 19.4 us; batch 4 at 8k 18.8 / 15.4;
 //     batch 16 at 2k 19.4 / 16.0).  With more tiles the heads' unequal lengths decide, which the balanced schedule evens
-//     out, and the two meet (batch 1 at 128k 29.3 / 28.7, batch 8 at 16k 29.0 / 29.5).  Three tiles where the fourth loses: at
-//     head dim 256 (one workgroup per compute unit; four tiles: batch 1, 16338 rows 31.0 / 32.4, batch 36, 466 rows 38.5 / 40.6,
-//     one head six times as long as the others at batch 5, 3026 rows 20.4 / 23.4; three: batch 3, 3794 rows 27.3 / 24.3, 19.9 /
-//     19.7) and where whole workgroups per head leave an eighth of the device or more idle (192 heads of 128, 978 rows 25.1 /
-//     25.9).  Over 1 to 56 sequences of 4 to 32 heads, dims 32 to 256, even and unequal heads, nothing on this side is then slower
-//     than 0.97 times the balanced schedule (the spread), and short contexts are up to twice as fast.
+//     out, and the two meet (batch 1 at 128k 29.3 / 28.7, batch 8 at 16k 29.0 / 29.5).  Less where the last ones
+//     lose: three at head dim 256 (one workgroup per compute unit; four: batch 1, 16338 rows 31.0 / 32.4, batch 36, 466 rows 38.5 /
+//     40.6, one head six times as long as the others at batch 5, 3026 rows 20.4 / 23.4; three: batch 3, 3794 rows 27.3 / 24.3,
+//     19.9 / 19.7), and 15 per workgroup at head dim 128 where whole workgroups per head leave an eighth of the device or more
+//     idle (192 heads, 896 / 1024 rows 22.2 / 22.0, 23.0 / 24.1; with heads of 64 and 32 all 16 still win: 17.5 / 14.2, 15.0 /
+//     10.5).  Over 1 to 56 sequences of 4 to 32 heads, dims 32 to 256, even and unequal heads, nothing on this side is then
+//     slower than 0.97 times the balanced schedule (the spread), and short contexts are up to twice as fast.
 //   * one workgroup of eight wavefronts per head, which writes the output itself, when that fills at least half of the
 //     compute units and a wavefront has four tiles at most (two, for half of the units): batch 32 at contexts 512 / 2k 20.8 /
 //     12.0, 25.3 / 21.0 us (16.2 and 24.0 with four wavefronts and the merge kernel), batch 16 at 512 15.8 / 11.0.
@@ -803,8 +804,8 @@ static FixedSchedule fixed_schedule(int64_t B, int64_t H_kv, int64_t n_rep, int6
   int64_t split = (D == 256 ? 1 : 2) * n_cu / heads;  // (the V tiles of a workgroup at head dim 256 are 128 KB of LDS)
   split = std::min<int64_t>({split, (tiles + 3) / 4, kFixedMaxSplit, kFixedPerGroup * (1024 / D)});
   if (split < 1) split = 1;
-  const int64_t most = D == 256 || (split > 1 && split * heads * 8 < 14 * n_cu) ? 3 : 4;  // tiles of a wavefront
-  if (tiles > most * 4 * split) return {0, 0};
+  const int64_t most = D == 256 ? 12 : D == 128 && split > 1 && split * heads * 8 < 14 * n_cu ? 15 : 16;  // tiles of a workgroup
+  if (tiles > most * split) return {0, 0};
   return {(int)split, 4};
 }
 

@@ -22,7 +22,8 @@ pytestmark = pytest.mark.gpu
     (16, 32, 8, 256, 64, 64, 3, 9),                                     # eight wavefronts do not fit at head dim 256
     (40, 8, 8, 64, 32, 32, 9, 1),                                       # more heads than compute units: one workgroup each
     (5, 32, 8, 256, 64, 64, 33, 0), (5, 32, 8, 256, 64, 64, 38, 0),     # head dim 256: three tiles per wavefront and more
-    (24, 32, 8, 128, 64, 64, 9, 63), (24, 32, 8, 128, 64, 64, 13, 63),  # 192 heads, two workgroups each: three tiles and more
+    (24, 32, 8, 128, 64, 64, 9, 63), (24, 32, 8, 128, 64, 64, 13, 63),  # 192 heads, two workgroups each: 15 tiles and more
+    (24, 32, 8, 64, 64, 64, 12, 63), (24, 8, 8, 32, 64, 64, 14, 63),    # heads of 64 and 32: 16 tiles and more
     (130, 8, 8, 32, 64, 64, 8, 1),                                      # balanced, more streams than one launch schedules
 ])
 def test_schedules(B, Hq, Hkv, D, W, C, chunks, fill):
