@@ -2,23 +2,25 @@
 // fp32 accumulation).
 //
 // A workgroup owns 32 query rows of one q head; its wavefronts share the visible 32-key tiles among themselves (every
-// n_waves-th one each), keep their own O, row maxima and row sums, and are combined through LDS at the end.  Nothing is
-// staged: every operand is laid out so that it comes from global memory (K, V: L2) in the form the instruction takes.
+// n_waves-th one each), keep their own O, row maxima and row sums, and are combined through LDS at the end.  A wavefront brings
+// its K tile to LDS in whole rows and takes V from global memory (L2) in the form the instruction takes.
 //
-//   S^T = K Q^T   A = K, B = Q.  The contraction runs over head dimensions in any order, so a lane of half `hl` holds every
-//                 second 16-byte piece of its row of K (of Q): the two halves of a load take 32 contiguous bytes of a row.
+//   S^T = K Q^T   A = K, B = Q, both from LDS.  The contraction runs over head dimensions in any order, so a lane of half `hl`
+//                 takes every second 16-byte piece of its row of K (of Q).
 //   O^T = V^T P^T A = V, B = P.  Accumulator i of S^T holds, in half hl, key 8 * (i / 4) + 4 * hl + i % 4 of query
 //                 lane % 32, which is what the i-th step of this product takes as B when its two keys are those two; its A
 //                 operand is head dimension (lane % 32) * DT + dt of the same key, so the DT tiles of a step are one load
 //                 of DT floats per lane and a row of V arrives as one contiguous read of a half wavefront.
 //
 // Bound: the fp32 matrix rate (64 FLOP per cycle and SIMD, 157 TFLOP/s): a 32 x 32 tile at D = 64 is 64 instructions of 64
-// cycles.  K of the next tile is requested when the scores of this one are done, V of this one before they begin, so
-// both travel under matrix instructions.  Measured (8 heads, D = 64, chunk 64): all keys visible, L = 2048, batch 8 0.357 ms =
-// 96 TFLOP/s; even roles at batch 8 0.236 ms, at batch 1 (two workgroups per compute unit, of which the heaviest has 44
-// tiles and the average one 17) 0.048 ms, where the plain kernel (a query row per lane, one wavefront per workgroup)
-// takes 0.88 ms.  The ends of a workgroup (Q, the tile summaries, the first K tile, the combination) are a third of an
-// average workgroup's life there.
+// cycles.  One wavefront's tile is a chain of trips and products, so up to head dim 64 four of them share a SIMD: 128 registers
+// each, which is why K goes through LDS (one buffer per wavefront: the next tile is requested when the scores of this one are
+// done and travels under the softmax and the PV product, V of this one under the scores).  K straight from global memory in
+// operand form, 16 bytes of each of 32 rows per instruction, kept L1 busy for 64 accesses per load, two thirds of all, and left
+// registers for two wavefronts per SIMD.  Measured, the op with its two kernels in front (10 us), before / now, 8 heads, chunk 64,
+// even roles: D = 64, L = 2048 44.5 / 35.5 us (batch 2 79.1 / 63.0, batch 8 203 now), L = 800 23.2 / 21.7; D = 32 27.4 / 23.1;
+// D = 128 (one workgroup of eight wavefronts per compute unit) 75.6 / 66.9, L = 3000 133 / 116.  The plain kernel (a query row per lane)
+// takes 0.88 ms at D = 64, L = 2048.
 #include "nats_prefill.h"
 
 namespace nats {
@@ -26,15 +28,14 @@ namespace nats {
 constexpr int kF32Rows = 32;      // query rows of a workgroup, keys of a tile
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// The Q operand is in LDS (one copy per workgroup): at D = 64 a wavefront then fits 168 registers, three to a SIMD (5 to 8 %
-// faster than two with Q in registers), at D = 128 it fits 256.
+// In LDS: Q (one copy per workgroup), and per wavefront one K tile and its row limits.
 template <int D>
 struct F32Layout {
-  static constexpr bool kQInLds = D >= 64;
   static constexpr int kQPitch = D + 4;   // floats; rows of the 16-byte reads fall into different banks
   static constexpr int kOPitch = D + 1;   // floats per query row of a wavefront's partial result
+  static constexpr int kWaveFloats = kF32Rows * D + kWave;  // K tile, row limits
   static size_t smem_bytes(int n_waves) {
-    const size_t q = (kQInLds ? sizeof(float) * kF32Rows * kQPitch : 0) + sizeof(int) * n_waves * kWave;  // Q, row limits
+    const size_t q = sizeof(float) * (kF32Rows * kQPitch + n_waves * kWaveFloats);
     const size_t merge = sizeof(float) * n_waves * kF32Rows * (kOPitch + 2);
     return q > merge ? q : merge;  // (the partial results take their place)
   }
@@ -53,8 +54,37 @@ __device__ __forceinline__ float f32_part(const typename F32Vec<DT>::type& v, in
 template <>
 __device__ __forceinline__ float f32_part<1>(const float& v, int) { return v; }
 
-template <int D, int kMaxWaves>
-__global__ __launch_bounds__(kMaxWaves * kWave, kMaxWaves == 4 && D <= 64 ? 3 : 2) void prefill_f32_kernel(PrefillArgs a, int blk_first, int n_blk) {
+constexpr int kWaitLoads = 0x0f70;  // vmcnt(0), the other counters at their largest
+
+// Rows of K or V as a raw buffer of `bytes` bytes: reads beyond its end give zero, and a row is a scalar offset beside a lane's
+// own, where addresses per row (two registers each) would not fit beside the tiles.  (Its type exists in the device pass only.)
+struct RowBuffer {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __amdgpu_buffer_rsrc_t desc;
+  __device__ __forceinline__ RowBuffer(const float* base, int bytes) : desc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000)) {}
+  __device__ __forceinline__ void to_lds(float* dst, int lane_off, int row_off) const {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(desc, (void __attribute__((address_space(3)))*)dst, 16, lane_off, row_off, 0, 0);
+  }
+  template <int DT>
+  __device__ __forceinline__ typename F32Vec<DT>::type row(int lane_off, int row_off) const {
+    if constexpr (DT == 1) {
+      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(desc, lane_off, row_off, 0));
+    } else if constexpr (DT == 2) {
+      return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(desc, lane_off, row_off, 0));
+    } else {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(desc, lane_off, row_off, 0));
+    }
+  }
+#else
+  __device__ RowBuffer(const float*, int) {}
+  __device__ void to_lds(float*, int, int) const {}
+  template <int DT>
+  __device__ typename F32Vec<DT>::type row(int, int) const { return {}; }
+#endif
+};
+
+template <int D, int kWaves>
+__global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_kernel(PrefillArgs a, int blk_first, int n_blk, int paired) {
   using Lay = F32Layout<D>;
   constexpr int HD = D / 2;   // head dimensions per half wavefront
   constexpr int DT = D / 32;  // 32-row tiles of O^T
@@ -63,10 +93,14 @@ __global__ __launch_bounds__(kMaxWaves * kWave, kMaxWaves == 4 && D <= 64 ? 3 : 
 
   const int lane = threadIdx.x & 63, l32 = lane & 31, hl = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n_waves = __builtin_amdgcn_readfirstlane(blockDim.x >> 6);
-  // (q heads change fastest, so that with 8 heads and more the blocks of a head run on one XCD; heavy blocks first)
+  constexpr int n_waves = kWaves;
+  // (q heads change fastest, so that with 8 heads and more the blocks of a head run on one XCD; heavy blocks first, or,
+  // where the first `paired` ranks take every compute unit and the others join them, see launch_d, the light blocks in
+  // falling order beside the others in rising order)
   const int n_heads = a.B * a.Hq;
-  const int bh = blockIdx.x % n_heads, blk = blk_first + n_blk - 1 - (int)(blockIdx.x / n_heads);
+  const int rank = (int)(blockIdx.x / n_heads);
+  const int bh = blockIdx.x % n_heads;
+  const int blk = blk_first + (rank < paired ? n_blk - paired + rank : n_blk - 1 - rank);
   const int b = bh / a.Hq, hq = bh % a.Hq, hkv = hq / a.n_rep;
   const int stream = b * a.Hkv + hkv;
   const float* qp = static_cast<const float*>(a.q) + b * a.qs_b + hq * a.qs_h;
@@ -82,27 +116,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave, kMaxWaves == 4 && D <= 64 ? 3 : 
   const int t_last = (a.base + rlast) / kF32Rows;  // last key tile somebody may see
   const float c = a.scale * 1.4426950408889634f;
 
-  // ---- Q: the B operand of the scores ----
-  float qreg[Lay::kQInLds ? 1 : HD];
-  if (Lay::kQInLds) {
-    for (int i = threadIdx.x; i < kF32Rows * D / 4; i += blockDim.x) {
-      const int row = i / (D / 4), piece = i % (D / 4);
-      const int m = min(max(q0 + row, a.r_begin), a.r_end - 1) - a.r_begin;
-      *reinterpret_cast<f32x4*>(smem + row * Lay::kQPitch + piece * 4) =
-          *reinterpret_cast<const f32x4*>(qp + (int64_t)m * a.qs_l + piece * 4);
-    }
-    __syncthreads();
-  } else {
-    const int m = min(max(qtok, a.r_begin), a.r_end - 1) - a.r_begin;
-    const f32x4* rp = reinterpret_cast<const f32x4*>(qp + (int64_t)m * a.qs_l + hl * 4);
-#pragma unroll
-    for (int i = 0; i < HD / 4; ++i) {
-      const f32x4 x = rp[2 * i];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qreg[(i * 4 + e) % (Lay::kQInLds ? 1 : HD)] = x[e];
-    }
-  }
-  int* lim_lds = reinterpret_cast<int*>(smem + (Lay::kQInLds ? kF32Rows * Lay::kQPitch : 0)) + wave * kWave;
+  float* k_lds = smem + kF32Rows * Lay::kQPitch + wave * Lay::kWaveFloats;
+  int* lim_lds = reinterpret_cast<int*>(k_lds + kF32Rows * D);
   const float* q_lds = smem + l32 * Lay::kQPitch + hl * 4;
 
   f32x16 oacc[DT];
@@ -113,26 +128,31 @@ __global__ __launch_bounds__(kMaxWaves * kWave, kMaxWaves == 4 && D <= 64 ? 3 : 
   float m_run = -INFINITY, l_run = 0.f;
 
   // ---- iterator over this wavefront's tiles: 64 tile summaries per ballot; the bits stay in scalar registers ----
-  int w0 = -64;        // first tile of the window
+  int w0 = 0;          // first tile of the window
   uint64_t mine = 0;   // this wavefront's visible tiles of the window that are still to come
   uint64_t mixed = 0;  // tiles of the window with rows that some query does not see
   int turn = 0;        // visible tiles before the window
+  auto summary = [&](int t, int2& g0, int2& g1) {
+    g0 = g1 = make_int2(-1, -1);
+    if (t <= t_last) g0 = gl[2 * t], g1 = gl[2 * t + 1];  // (the granule table is filled up to whole 64-row tiles)
+  };
+  auto open_window = [&](const int2& g0, const int2& g1) {
+    const int t = w0 + lane;
+    const bool v = max(g0.x, g1.x) >= r0;
+    const bool mx = !(min(g0.y, g1.y) >= rlast && t * kF32Rows + kF32Rows - 1 - a.base <= r0 && (t + 1) * kF32Rows <= a.N);
+    const uint64_t vis = __ballot(v);
+    mixed = __ballot(mx);
+    const int nth = turn + __builtin_popcountll(vis & ((uint64_t(1) << lane) - 1));
+    mine = __ballot(v && (nth & (n_waves - 1)) == wave);  // (n_waves is a power of two)
+    turn += __builtin_popcountll(vis);
+  };
   auto next_tile = [&](bool& masked) -> int {
     while (mine == 0) {
       w0 += 64;
       if (w0 > t_last) return -1;
-      const int t = w0 + lane;
-      bool v = false, mx = true;
-      if (t <= t_last) {
-        const int2 g0 = gl[2 * t], g1 = gl[2 * t + 1];  // (the granule table is filled up to whole 64-row tiles)
-        v = max(g0.x, g1.x) >= r0;
-        mx = !(min(g0.y, g1.y) >= rlast && t * kF32Rows + kF32Rows - 1 - a.base <= r0 && (t + 1) * kF32Rows <= a.N);
-      }
-      const uint64_t vis = __ballot(v);
-      mixed = __ballot(mx);
-      const int nth = turn + __builtin_popcountll(vis & ((uint64_t(1) << lane) - 1));
-      mine = __ballot(v && (nth & (n_waves - 1)) == wave);  // (n_waves is a power of two)
-      turn += __builtin_popcountll(vis);
+      int2 g0, g1;
+      summary(w0 + lane, g0, g1);
+      open_window(g0, g1);
     }
     const int i = __builtin_ctzll(mine);
     mine &= mine - 1;
@@ -140,33 +160,65 @@ __global__ __launch_bounds__(kMaxWaves * kWave, kMaxWaves == 4 && D <= 64 ? 3 : 
     return w0 + i;
   };
 
-  f32x4 kreg[HD / 4];
-  // (a tile's rows at a lane offset from a uniform base; the last tile's rows past the end repeat the last row)
-  const uint32_t koff = uint32_t(l32 * a.ks_l + hl * 4), voff = uint32_t(hl * 4 * a.vs_l + l32 * DT);
-  auto load_k = [&](int t) {
-    const int k0 = t * kF32Rows;
-    const float* tb = kp + (int64_t)k0 * a.ks_l;
-    const uint32_t off = k0 + kF32Rows <= a.N ? koff : uint32_t(min(l32, a.N - 1 - k0) * a.ks_l + hl * 4);
-#pragma unroll
-    for (int i = 0; i < HD / 4; ++i) kreg[i] = *reinterpret_cast<const f32x4*>(tb + off + i * 8);
+  // K tile: global -> LDS (16 bytes per lane, whole rows per instruction).  The 16-byte chunks of a row are permuted so that the
+  // rows which a quarter wavefront reads at once fall into different banks.
+  constexpr int OCT = D / 4;                // 16-byte chunks per row
+  constexpr int kRowsPerInst = kWave / OCT;
+  auto swz = [](int row) { return D == 32 ? (row >> 1) & 7 : row & 15; };
+  // (the buffer of a tile ends with the last row; the lane id is taken afresh for every tile so that nothing derived from it lives
+  // from one to the next)
+  auto tile_buffer = [&](const float* base, int64_t row_stride, int k0) {
+    return RowBuffer(base + (int64_t)k0 * row_stride, ((min(kF32Rows, a.N - k0) - 1) * (int)row_stride + D) * 4);
   };
+  auto load_k = [&](int t) {
+    const RowBuffer buf = tile_buffer(kp, a.ks_l, t * kF32Rows);
+    int ln = lane;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(ln));
+#endif
+    const int row0 = ln / OCT;
+#pragma unroll
+    for (int j = 0; j < kF32Rows / kRowsPerInst; ++j) {
+      const int off = (row0 * (int)a.ks_l + ((ln % OCT) ^ swz(j * kRowsPerInst + row0)) * 4) * 4;
+      buf.to_lds(k_lds + j * kWave * 4, off, j * kRowsPerInst * (int)a.ks_l * 4);
+    }
+  };
+  auto k_frag = [&](int i) { return *reinterpret_cast<const f32x4*>(k_lds + l32 * D + ((2 * i + hl) ^ swz(l32)) * 4); };
+  const int voff = (hl * 4 * (int)a.vs_l + l32 * DT) * 4;  // bytes
 
+  // ---- Q goes to LDS (the B operand of the scores); the first tile summaries are requested before it and the first K tile
+  // while it is under way: three trips to memory, of which two run side by side ----
+  int2 g0, g1;
+  summary(lane, g0, g1);
+  constexpr int kQPieces = kF32Rows * D / 4, kQSteps = (kQPieces + n_waves * kWave - 1) / (n_waves * kWave);
+  f32x4 qp_reg[kQSteps];
+#pragma unroll
+  for (int j = 0; j < kQSteps; ++j) {
+    const int i = min(j * n_waves * kWave + (int)threadIdx.x, kQPieces - 1);
+    const int m = min(max(q0 + i / (D / 4), a.r_begin), a.r_end - 1) - a.r_begin;
+    qp_reg[j] = *reinterpret_cast<const f32x4*>(qp + (int64_t)m * a.qs_l + i % (D / 4) * 4);
+  }
+  open_window(g0, g1);
   bool masked = false;
   int t = next_tile(masked);
   if (t >= 0) load_k(t);
+#pragma unroll
+  for (int j = 0; j < kQSteps; ++j) {
+    const int i = min(j * n_waves * kWave + (int)threadIdx.x, kQPieces - 1);
+    *reinterpret_cast<f32x4*>(smem + i / (D / 4) * Lay::kQPitch + i % (D / 4) * 4) = qp_reg[j];
+  }
+  __syncthreads();
   while (t >= 0) {
     const int k0 = t * kF32Rows;
+    // K of this tile has landed in LDS (the compiler does not wait for transfers into LDS before it reads there)
+    __builtin_amdgcn_s_waitcnt(kWaitLoads);
+    __builtin_amdgcn_sched_barrier(0);
     // V rows of this tile (rows past the end repeat the last one: their probabilities are 0) and the row limits
     VecV vreg[16];
-    if (k0 + kF32Rows <= a.N) {
+    {
+      const RowBuffer buf = tile_buffer(vp, a.vs_l, k0);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) vreg[i] = *reinterpret_cast<const VecV*>(vp + (int64_t)(k0 + 8 * (i / 4) + i % 4) * a.vs_l + voff);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int n = min(k0 + 8 * (i / 4) + 4 * hl + i % 4, a.N - 1);
-        vreg[i] = *reinterpret_cast<const VecV*>(vp + (int64_t)n * a.vs_l + l32 * DT);
-      }
+      for (int i = 0; i < 16; ++i) vreg[i] = buf.template row<DT>(voff, (8 * (i / 4) + i % 4) * (int)a.vs_l * 4);
     }
     if (masked) lim_lds[lane] = lim[min(k0 + l32, a.N - 1)];
     __builtin_amdgcn_sched_barrier(0);
@@ -175,19 +227,18 @@ __global__ __launch_bounds__(kMaxWaves * kWave, kMaxWaves == 4 && D <= 64 ? 3 : 
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
+    f32x4 kn = k_frag(0), qn = *reinterpret_cast<const f32x4*>(q_lds);
 #pragma unroll
     for (int i = 0; i < HD / 4; ++i) {
-      f32x4 qv;
-      if (Lay::kQInLds) {
-        qv = *reinterpret_cast<const f32x4*>(q_lds + i * 8);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) qv[e] = qreg[(i * 4 + e) % (Lay::kQInLds ? 1 : HD)];
+      const f32x4 kv = kn, qv = qn;
+      if (i + 1 < HD / 4) {
+        kn = k_frag(i + 1);
+        qn = *reinterpret_cast<const f32x4*>(q_lds + (i + 1) * 8);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kreg[i][e], qv[e], s, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qv[e], s, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
     const bool was_masked = masked;
     const int t_next = next_tile(masked);
     if (t_next >= 0) load_k(t_next);
@@ -293,27 +344,35 @@ static int launch_d(const PrefillArgs& a, hipStream_t st) {
   const int blk_first = a.r_begin / kF32Rows, n_blk = (a.r_end - 1) / kF32Rows - blk_first + 1;
   const int64_t n_wg = (int64_t)a.B * a.Hq * n_blk;
   NATS_REQUIRE(n_wg < (int64_t(1) << 31), NATS_ERR_BAD_SHAPE, "prefill: grid too large");
-  // Eight wavefronts per workgroup while the launch is at most four workgroups per compute unit: the heaviest block is the
-  // end of the launch there and has to be short; above, four (three workgroups per compute unit at D = 64) waste less on the
-  // ends of a workgroup.  8 heads, L = 2048, D = 64: 0.048 against 0.057 ms at batch 1 (2 workgroups per compute unit), 0.085 /
-  // 0.088 at batch 2, 0.165 / 0.146 at batch 4.
+  // How many wavefronts share a block's tiles.  Eight (two workgroups per compute unit at head dims 32 and 64, one at 128) make
+  // the heaviest block, which ends the launch, short; four (three workgroups or more) waste less on the ends of a workgroup.
+  // 8 / 4 wavefronts, even and sparse roles, by workgroups per compute unit:
+  //   D = 64   up to 2: 27 / 28, 24 / 24 us (1.4), 36 / 38, 30 / 30 (2).  2.75: 44 / 42, 39 / 34.  3.25: 73 / 70, 54 / 50.  4: 63 / 69, 50 / 55.
+  //            5.3: 94 / 100, 67 / 69.  6.5: 126 / 127, 87 / 84.  11: 125 / 117, 107 / 101.  26: 456 / 442, 302 / 282.
+  //   D = 32   1.4: 20 / 21, 18 / 18.  2: 23 / 24, 20 / 20.  2.66: 33 / 33, 28 / 25.  4: 36 / 34, 30 / 27.  13: 150 / 139, 97 / 83.
+  //   D = 128  eight always: four are one workgroup per compute unit as well (105 / 111, 75 / 81 at 2.66).
   const int n_cu = device_cu_count();
-  const int waves = n_wg <= 4 * (int64_t)n_cu ? 8 : 4;
+  const bool few = D == 128 || n_wg <= 2 * (int64_t)n_cu || (D == 64 && 2 * n_wg > 7 * (int64_t)n_cu && n_wg <= 6 * (int64_t)n_cu);
+  // Between one and two workgroups per compute unit: workgroups i and i + n_cu share one, so the lightest blocks come last, in
+  // falling order, beside the lightest of the others, and the heaviest have a compute unit to themselves (8 heads of 64, 2048
+  // tokens 39.0 -> 35.8 us, 1400 31.6 -> 26.1, 4 heads, 3000 tokens 41.4 -> 34.0).
+  const int per_round = (int)(n_cu / ((int64_t)a.B * a.Hq));  // blocks of a head that take every compute unit once
+  const int paired = per_round > 0 && n_blk > per_round && n_blk <= 2 * per_round ? per_round : 0;
+  constexpr int kMany = D == 128 ? 8 : 4;
   if (!configured[dev]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, 4>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)F32Layout<D>::smem_bytes(4));
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)F32Layout<D>::smem_bytes(8));
     if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)F32Layout<D>::smem_bytes(8));
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, kMany>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)F32Layout<D>::smem_bytes(kMany));
     if (e != hipSuccess) return fail(NATS_ERR_LAUNCH, "prefill_f32_kernel: LDS: %s", hipGetErrorString(e));
     configured[dev] = true;
   }
-  const dim3 grid((unsigned)n_wg), block(waves * kWave);
-  const size_t smem = F32Layout<D>::smem_bytes(waves);
-  if (waves == 8) {
-    hipLaunchKernelGGL((prefill_f32_kernel<D, 8>), grid, block, smem, st, a, blk_first, n_blk);
+  const dim3 grid((unsigned)n_wg);
+  if (few) {
+    hipLaunchKernelGGL((prefill_f32_kernel<D, 8>), grid, dim3(8 * kWave), F32Layout<D>::smem_bytes(8), st, a, blk_first, n_blk, paired);
   } else {
-    hipLaunchKernelGGL((prefill_f32_kernel<D, 4>), grid, block, smem, st, a, blk_first, n_blk);
+    hipLaunchKernelGGL((prefill_f32_kernel<D, kMany>), grid, dim3(kMany * kWave), F32Layout<D>::smem_bytes(kMany), st, a, blk_first, n_blk, paired);
   }
   NATS_CHECK_LAUNCH("prefill_f32_kernel");
   return NATS_OK;

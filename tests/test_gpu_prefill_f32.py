@@ -21,6 +21,9 @@ pytestmark = pytest.mark.gpu
     (1, 2, 1, 1, 64, 64), (1, 2, 2, 31, 8, 8), (2, 3, 1, 32, 16, 16), (1, 4, 2, 33, 1, 4), (1, 2, 1, 64, 64, 128), (1, 2, 1, 97, 6, 12),
     (1, 1, 1, 2049, 64, 128),   # the second window of tile summaries
     (4, 33, 11, 300, 32, 64),   # more than four workgroups per compute unit: four wavefronts each
+    (1, 8, 8, 1030, 64, 128),   # one block of a head more than the compute units take at once: the two lightest share one
+    (1, 16, 4, 1000, 16, 32),   # two workgroups per compute unit, all in pairs
+    (2, 9, 3, 1111, 64, 64),    # between two and three and a half workgroups per compute unit
 ])
 def test_tile_edges(B, Hq, Hkv, L, C, W, D):
     run_case(B, Hq, Hkv, L, D, C, W, torch.float32, seed=L)
