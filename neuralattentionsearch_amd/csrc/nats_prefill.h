@@ -47,6 +47,66 @@ struct PrefillArgs {
   const int32_t* long_before;  // [streams, 2, n_gran + 1] entries of A / of B before every granule
   const int32_t* long_alive;   // [streams, n_rtile] first entry of B that a query of the 64-token region tile may see
   int long_cap, n_gran, n_rtile, t_long;
+  int rows64;  // a stream's rows of K or V reach beyond 32-bit byte offsets
+};
+
+// ---- transfers global memory -> LDS -------------------------------------------------------------------------
+// Lane i's bytes go to the (uniform) LDS destination + i * its size.  They are issued from assembly: for the builtins the compiler
+// waits for every transfer in flight before an LDS read that may alias one, which here are the first V fragment of every tile
+// and the row limits of every masked one, in the middle of the step that put the next tiles in flight.  Nothing else waits for them:
+// wait_transfers() and, for other wavefronts' rows, a barrier stand before the first read.  (Counted by vmcnt like any vector
+// memory load; no output registers.  The host pass of the single-source compile never runs these.)
+__device__ __forceinline__ uint32_t lds_address(const void* lds_ptr) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds_ptr);
+#else
+  return 0;
+#endif
+}
+// 16 bytes from every lane's own address
+__device__ __forceinline__ void lds_transfer16(const void* gptr, uint32_t lds_addr) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory", "m0");
+#endif
+}
+__device__ __forceinline__ void wait_transfers() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+}
+// Rows of K or V (or row limits) as a raw buffer of `bytes` bytes: reads beyond its end give zero, and a row is a scalar offset
+// beside a lane's own, where addresses per row would take two registers and vector arithmetic each.
+struct RowBuffer {
+  typedef int Words __attribute__((ext_vector_type(4)));
+  static constexpr int kFlags = 0x00027000;  // last word of a raw buffer's descriptor
+  const void* base;
+  uint32_t bytes;
+  Words desc;
+  __device__ __forceinline__ RowBuffer(const void* base, uint32_t bytes)
+      : base(base), bytes(bytes), desc{(int)(uintptr_t)base, (int)((uintptr_t)base >> 32) & 0xffff, (int)bytes, kFlags} {}
+  template <int kBytes>
+  __device__ __forceinline__ void to_lds(uint32_t lds_addr, int lane_off, uint32_t row_off) const {
+    static_assert(kBytes == 16 || kBytes == 4, "sizes a transfer can have here");
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (kBytes == 16) {
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds" ::"v"(lane_off), "s"(desc), "s"(lds_addr), "s"(row_off)
+                   : "memory", "m0");
+    } else {
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, %3 offen lds" ::"v"(lane_off), "s"(desc), "s"(lds_addr), "s"(row_off)
+                   : "memory", "m0");
+    }
+#endif
+  }
+  // two transfers of 16 bytes to consecutive KiB of LDS
+  __device__ __forceinline__ void to_lds_pair(uint32_t lds_addr, int lane_off0, int lane_off1, uint32_t row_off) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile(
+        "s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %2, %4 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %4 offen lds" ::"v"(lane_off0), "v"(lane_off1), "s"(desc), "s"(lds_addr),
+        "s"(row_off)
+        : "memory", "m0", "scc");
+#endif
+  }
 };
 
 // fp32 kernel on the fp32 matrix instruction (nats_prefill_f32.hip)

@@ -22,6 +22,9 @@
 // A prefill from an empty cache is the case base = 0, r_begin = 0.
 #include <stdlib.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "nats_prefill.h"
 
 namespace nats {
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(64) void prefill_simple_kernel(PrefillArgs a) {
 // through LDS.  With 256 registers per lane two wavefronts share a SIMD, so that the vector ALU work of
 // one (exponentials) runs under the matrix instructions of the other.
 //
-// K / V tiles travel global -> LDS without passing through registers (global_load_lds, 16 bytes per lane),
+// K / V tiles travel global -> LDS without passing through registers (16 bytes per lane),
 // double buffered, row major with 256-byte rows whose 16-byte chunks are XOR-swizzled (the lane supplies
 // the global address, so the permutation costs nothing) to keep the operand reads free of bank conflicts.
 //
@@ -282,11 +285,33 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   // ---- wavefront 0 asks for the tile summaries of the first kEarly * 64 key tiles before anything else is requested:
   // memory operations complete in the order of their issue, so the wait for these (a trip to L2) does not include
   // the Q rows (a trip to HBM), which stay in flight while the visit list is built and the first tiles are requested.
-  constexpr int kEarly = 8;
+  // Packed tiles: the same with the granule summaries, where the granules [near_g0, g_end_group] and the gathered tiles fit one
+  // early list; wavefront 1 asks for the cache rows of the first gathered tiles.
+  constexpr int kEarly = kPacked ? 4 : 8;
+  constexpr int kIdsAhead = 5;  // gathered tiles whose cache rows are known before the first step
+  const int near_g0 = near_row0 / kGranule;
+  const int g_end_group = (a.base + rlast_group) / kGranule;
+  const int n_near = g_end_group - near_g0 + 1;
+  const bool early_list = kPacked && n_near <= kEarly * kWave && (!kFar || n_far_tiles + (n_near + kGranPerTile - 1) / kGranPerTile + 1 <= kWin - 1);
+  const bool early_ids = kFar && early_list && a.n_split == 1 && n_far_tiles > 0;
   int2 tl_early[kEarly];
   if (!kPacked && wave == 0) {
 #pragma unroll
     for (int j = 0; j < kEarly; ++j) tl_early[j] = tl[min(j * kWave + lane, kt_end_group)];
+  }
+  if (early_list && wave == 0) {
+    const int2* gl = a.gran_lim + (int64_t)ks * a.Tk * kGranPerTile;
+#pragma unroll
+    for (int j = 0; j < kEarly; ++j)
+      if (j * kWave < n_near) tl_early[j] = gl[min(near_g0 + j * kWave + lane, g_end_group)];
+  }
+  // (gathered tile t of the list: its first entry in the lists of long-lived rows)
+  auto far_start = [&](int t) { return t < n_far_ta ? t * kTile : a.long_cap + b_lo + (t - n_far_ta) * kTile; };
+  int ids_early[kIdsAhead];
+  if (early_ids && wave == 1) {
+#pragma unroll
+    for (int j = 0; j < kIdsAhead; ++j)
+      if (j < n_far_tiles) ids_early[j] = lrows[far_start(j) + lane];
   }
 
   // ---- Q fragments: B operand, lane (query l32, k-group hl) --------------------------------------
@@ -315,9 +340,9 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   // = all banks) by a quarter per pair of rows.
   // (rows of 64 bytes: four rows = all banks and the four pieces of a read are one contiguous 256 bytes)
   auto v_swizzle = [](int row) { return OCT >= 16 ? (row & 3) << 2 : OCT >= 8 ? ((row >> 1) & 1) << 2 : 0; };
-  // global -> LDS, one 64-key tile of K or of V; rows beyond N repeat row N-1 (their scores are masked,
-  // so their probabilities are exactly 0 and a finite V row contributes nothing).  The lane's share of a
-  // tile sits at fixed offsets from the tile's first row, computed once.
+  // global -> LDS, one 64-key tile of K or of V as a buffer that ends with row N - 1; rows beyond are zeros (their scores are masked,
+  // so their probabilities are exactly 0 and contribute nothing).  The lane's share of a tile sits at fixed offsets (bytes) from
+  // the tile's first row, computed once.
   int koff[DMA_PER_WAVE], voff[DMA_PER_WAVE];
 #pragma unroll
   for (int j = 0; j < DMA_PER_WAVE; ++j) {
@@ -325,100 +350,64 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
     const int row = q / OCT, pos = q % OCT;
     // (packed tiles: this wavefront's 8 rows of a tile lie in one granule; the offset counts from its first row)
     const int srow = kPacked ? row % kGranule : row;
-    koff[j] = int(srow * a.ks_l + (pos ^ (row % OCT)) * 8);
-    voff[j] = int(srow * a.vs_l + (pos ^ v_swizzle(row)) * 8);
+    koff[j] = int(srow * a.ks_l + (pos ^ (row % OCT)) * 8) * 2;
+    voff[j] = int(srow * a.vs_l + (pos ^ v_swizzle(row)) * 8) * 2;
   }
-  auto issue_rows = [&](const uint16_t* base, int64_t stride, const int (&off)[DMA_PER_WAVE], uint16_t* dst, int kt,
-                        bool is_v) {
-    if (kt * kTile + kTile <= a.N) {
-      const uint16_t* tb = base + (int64_t)kt * kTile * stride;  // uniform
+  const uint32_t lds0 = lds_address(smem_raw);
+  constexpr uint32_t kTileBytes = kTile * D * 2, kVOff = 4 * kTileBytes;
+  constexpr uint32_t kLimOff = __builtin_offsetof(PrefillSmem<D>, limk), kPosOff = __builtin_offsetof(PrefillSmem<D>, posk);
+  static_assert(__builtin_offsetof(PrefillSmem<D>, k) == 0 && __builtin_offsetof(PrefillSmem<D>, v) == kVOff, "tile buffers come first");
+  const uint32_t lds_wave = lds0 + wave * DMA_PER_WAVE * kWave * 16;  // this wavefront's share of tile buffer 0
+  const RowBuffer kbuf(kp, (uint32_t)((int64_t)(a.N - 1) * a.ks_l + D) * 2), vbuf(vp, (uint32_t)((int64_t)(a.N - 1) * a.vs_l + D) * 2);
+  // This wavefront's share of the tile whose rows begin at row0 (a granule: of its own rows), to the tile buffer at byte `tile`.
+  // A step's transfers stand in front of its matrix instructions, so they are kept short: one offset from the stream's first
+  // row (where a stream's rows do not reach beyond 32 bits of it) and the LDS address, both scalar.
+  auto issue_rows = [&](const RowBuffer& buf, int64_t stride, const int (&off)[DMA_PER_WAVE], uint32_t tile, int row0) {
+    if (N_INST < kPrefillWaves && wave >= N_INST) return;
+    uint32_t row_off = (uint32_t)row0 * ((uint32_t)stride * 2);
+    if (!kFar && __builtin_expect(a.rows64, 0)) {
+      const RowBuffer near(static_cast<const uint16_t*>(buf.base) + (int64_t)row0 * stride, ((min(kTile, a.N - row0) - 1) * (int)stride + D) * 2);
 #pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) {
-        const int inst = wave * DMA_PER_WAVE + j;
-        if (inst < N_INST)
-          __builtin_amdgcn_global_load_lds(tb + (int)off[j], (uint32_t __attribute__((address_space(3)))*)(dst + inst * kWave * 8), 16, 0, 0);
-      }
+      for (int j = 0; j < DMA_PER_WAVE; ++j) near.template to_lds<16>(lds_wave + tile + j * kWave * 16, off[j], 0);
+    } else if (DMA_PER_WAVE == 2) {
+      buf.to_lds_pair(lds_wave + tile, off[0], off[DMA_PER_WAVE - 1], row_off);
     } else {
-#pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) {
-        const int inst = wave * DMA_PER_WAVE + j;  // uniform
-        const int q = inst * kWave + lane;
-        const int row = q / OCT, pos = q % OCT;
-        const int n = min(kt * kTile + row, a.N - 1);
-        const int chunk = is_v ? pos ^ v_swizzle(row) : pos ^ (row % OCT);
-        if (inst < N_INST)
-          __builtin_amdgcn_global_load_lds(base + (int64_t)n * stride + chunk * 8,
-                                           (uint32_t __attribute__((address_space(3)))*)(dst + inst * kWave * 8), 16, 0, 0);
-      }
+      buf.template to_lds<16>(lds_wave + tile, off[0], row_off);
     }
   };
+  static_assert(DMA_PER_WAVE <= 2, "two transfers of a wavefront at most");
   // K tile and the visibility limits of its rows; the limits go to slot (list index & 7)
-  auto issue_k = [&](int kt, int buf, int slot, bool need_lim) {
-    issue_rows(kp, a.ks_l, koff, sm.k[buf], kt, false);
-    // (asynchronous like the tile itself; rows beyond N are later than every query, which masks them whatever
-    // limit they get, so their address is clamped)
-    if (need_lim && wave == 0)
-      __builtin_amdgcn_global_load_lds(lim + min(kt * kTile + lane, a.N - 1),
-                                       (uint32_t __attribute__((address_space(3)))*)(&sm.limk[slot][0]), 4, 0, 0);
-  };
-  auto issue_v = [&](int kt, int buf) { issue_rows(vp, a.vs_l, voff, sm.v[buf], kt, true); };
-  // packed tiles: the wavefront's 8 rows of the tile come from granule (wave / 2) of the list entry; a missing
-  // granule (padding) repeats granule 0, whose rows the limit -1 masks
-  auto issue_rows_p = [&](const uint16_t* base, int64_t stride, const int (&off)[DMA_PER_WAVE], uint16_t* dst, int gid,
-                          bool is_v) {
-    if (gid < 0) gid = 0;
-    if ((gid + 1) * kGranule <= a.N) {
-      const uint16_t* tb = base + (int64_t)gid * kGranule * stride;  // uniform
-#pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) {
-        const int inst = wave * DMA_PER_WAVE + j;
-        if (inst < N_INST)
-          __builtin_amdgcn_global_load_lds(tb + (int)off[j], (uint32_t __attribute__((address_space(3)))*)(dst + inst * kWave * 8), 16, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) {
-        const int inst = wave * DMA_PER_WAVE + j;  // uniform
-        const int q = inst * kWave + lane;
-        const int row = q / OCT, pos = q % OCT;
-        const int n = min(gid * kGranule + row % kGranule, a.N - 1);
-        const int chunk = is_v ? pos ^ v_swizzle(row) : pos ^ (row % OCT);
-        if (inst < N_INST)
-          __builtin_amdgcn_global_load_lds(base + (int64_t)n * stride + chunk * 8,
-                                           (uint32_t __attribute__((address_space(3)))*)(dst + inst * kWave * 8), 16, 0, 0);
-      }
-    }
+  auto issue_k = [&](int kt, uint32_t tile, int slot, bool need_lim) {
+    issue_rows(kbuf, a.ks_l, koff, tile, kt * kTile);
+    // (rows beyond N are later than every query, which masks them whatever limit they get)
+    if (need_lim && wave == 0) RowBuffer(lim, (uint32_t)a.N * 4).template to_lds<4>(lds0 + kLimOff + slot * kTile * 4, lane * 4, (uint32_t)kt * kTile * 4);
   };
   // a tile of the list of long-lived rows: the cache row of every tile row is in posk[slot] (requested a step ahead)
-  auto issue_rows_far = [&](const uint16_t* base, int64_t stride, uint16_t* dst, int slot, bool is_v) {
+  auto issue_rows_far = [&](const RowBuffer& buf, int64_t stride, uint32_t tile, int slot, bool is_v) {
+    if (N_INST < kPrefillWaves && wave >= N_INST) return;
 #pragma unroll
     for (int j = 0; j < DMA_PER_WAVE; ++j) {
-      const int inst = wave * DMA_PER_WAVE + j;  // uniform
-      const int q = inst * kWave + lane;
+      int ln = lane;
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(ln));
+#endif
+      const int q = (wave * DMA_PER_WAVE + j) * kWave + ln;
       const int row = q / OCT, pos = q % OCT;
-      const int n = max(0, min(sm.posk[slot][row & (kTile - 1)], a.N - 1));  // (padding entries hold INT_MAX and the limit -1)
+      const int n = max(0, min(sm.posk[slot][row], a.N - 1));  // (padding entries hold INT_MAX and the limit -1)
       const int chunk = is_v ? pos ^ v_swizzle(row) : pos ^ (row % OCT);
-      if (inst < N_INST)
-        __builtin_amdgcn_global_load_lds(base + (int64_t)n * stride + chunk * 8,
-                                         (uint32_t __attribute__((address_space(3)))*)(dst + inst * kWave * 8), 16, 0, 0);
+      const uint32_t dst = lds_wave + tile + j * kWave * 16;
+      buf.template to_lds<16>(dst, (int)((uint32_t)n * ((uint32_t)stride * 2) + chunk * 16), 0);
     }
   };
-  // (id0: the first field of the list entry, with its flags; mine: this wavefront's granule of the tile, or the first
-  // list entry of a gathered tile; idx: the entry's place in the list)
-  auto issue_k_p = [&](int id0, int mine, int idx, int buf, int slot) {
+  // (packed tiles; id0: the first field of the list entry, with its flags; mine: this wavefront's granule of the tile -- its eight
+  // rows of a tile lie in one -- or the first list entry of a gathered tile; idx: the entry's place in the list.  A missing
+  // granule (padding) repeats granule 0, whose rows the mask excludes.)
+  auto issue_k_p = [&](int id0, int mine, int idx, uint32_t tile, int slot) {
     if (kFar && (id0 & kFarTileFlag)) {
-      issue_rows_far(kp, a.ks_l, sm.k[buf], slot, false);
-      if ((id0 & kPackedMaskFlag) && wave == 0) {
-        int ln = lane;
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("" : "+v"(ln));
-#endif
-        __builtin_amdgcn_global_load_lds(llim + mine + ln,
-                                         (uint32_t __attribute__((address_space(3)))*)(&sm.limk[slot][0]), 4, 0, 0);
-      }
-      return;
+      issue_rows_far(kbuf, a.ks_l, tile, slot, false);
+    } else {
+      issue_rows(kbuf, a.ks_l, koff, tile, max(mine, 0) * kGranule);
     }
-    issue_rows_p(kp, a.ks_l, koff, sm.k[buf], mine, false);
     if ((id0 & kPackedMaskFlag) && wave == 0) {
       // limits and region tokens of the 64 rows, for the element mask (asynchronous like the tile itself).
       // (The lane id is taken afresh so that nothing derived from it has to live across the tile loop.)
@@ -426,48 +415,62 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
 #if defined(__HIP_DEVICE_COMPILE__)
       asm volatile("" : "+v"(ln));
 #endif
-      int gid = reinterpret_cast<const int*>(&sm.vlist[idx])[ln >> 4];
-      if ((ln >> 4) == 0) gid &= ~kPackedMaskFlag;
-      const int row = gid * kGranule + (ln & (kGranule - 1));
-      const bool real = gid >= 0 && row < a.N;
-      const int32_t* src = real ? lim + row : a.tok_lim + (int64_t)a.B * a.Hkv * a.N;  // (the entry that holds -1)
-      __builtin_amdgcn_global_load_lds(src, (uint32_t __attribute__((address_space(3)))*)(&sm.limk[slot][0]), 4, 0, 0);
-      sm.posk[slot][ln] = real ? row - a.base : 0x7fffffff;
+      const uint32_t lim_dst = lds0 + kLimOff + slot * kTile * 4;
+      if (kFar && (id0 & kFarTileFlag)) {
+        RowBuffer(llim + mine, kTile * 4).template to_lds<4>(lim_dst, ln * 4, 0);
+      } else {
+        int gid = reinterpret_cast<const int*>(&sm.vlist[idx])[ln >> 4];
+        if ((ln >> 4) == 0) gid &= ~kPackedMaskFlag;
+        const int row = gid * kGranule + (ln & (kGranule - 1));
+        const bool real = gid >= 0 && row < a.N;
+        // (rows that are not there: beyond the buffer, and their region token excludes every query)
+        RowBuffer(lim, (uint32_t)a.N * 4).template to_lds<4>(lim_dst, real ? row * 4 : -4, 0);
+        sm.posk[slot][ln] = real ? row - a.base : 0x7fffffff;
+      }
     }
   };
-  auto issue_v_p = [&](int id0, int mine, int buf, int slot) {
+  auto issue_v_p = [&](int id0, int mine, uint32_t tile, int slot) {
     if (kFar && (id0 & kFarTileFlag)) {
-      issue_rows_far(vp, a.vs_l, sm.v[buf], slot, true);
-      return;
+      issue_rows_far(vbuf, a.vs_l, kVOff + tile, slot, true);
+    } else {
+      issue_rows(vbuf, a.vs_l, voff, kVOff + tile, max(mine, 0) * kGranule);
     }
-    issue_rows_p(vp, a.vs_l, voff, sm.v[buf], mine, true);
   };
 
-  auto k_frag = [&](const uint16_t* Kt, int kb, int s) {
-    const int row = kb * 32 + l32;
-    const int chunk = (s * 2 + hl) ^ (row % OCT);
-    return *reinterpret_cast<const bf16x8*>(Kt + row * D + chunk * 8);
+  // K fragments: row kb * 32 + l32 of the tile, 16-byte chunk s * 2 + hl at its permuted place.  One LDS address per s (the row's
+  // permutation is the same for both halves of the tile); the tile buffer, a constant in every step, and the half are offsets of
+  // the instruction.
+  uint32_t k_addr[DSTEPS], v_addr[DT];
+#pragma unroll
+  for (int s = 0; s < DSTEPS; ++s) k_addr[s] = lds0 + l32 * (D * 2) + (((s * 2 + hl) ^ (l32 % OCT)) * 16);
+  auto k_frag = [&](uint32_t tile, int kb, int s) {
+    return *(const __attribute__((address_space(3))) bf16x8*)(uintptr_t)(k_addr[s] + (tile + kb * 32 * (D * 2)));
   };
   // ds_read_b64_tr_b16: within 16 lanes, lane r reads 4 dims of key (K0 + r / 4) starting at dim
-  // D0 + 4 * (r % 4) and receives keys K0 .. K0 + 3 of dim D0 + r.
-  const int r16 = lane & 15;
-  const int dsel = (lane >> 4) & 1;
-  auto v_frag = [&](const uint16_t* Vt, int t, int dt) {
-    const int chunk0 = dt * 4 + dsel * 2 + ((r16 & 3) >> 1);
-    const int half4 = (r16 & 1) * 4;
-    const int row_lo = t * 16 + hl * 4 + (r16 >> 2);
-    const int row_hi = row_lo + 8;
-    const uint16_t* pl = Vt + row_lo * D + ((chunk0 ^ v_swizzle(row_lo)) * 8) + half4;
-    const uint16_t* ph = Vt + row_hi * D + ((chunk0 ^ v_swizzle(row_hi)) * 8) + half4;
-    bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 __attribute__((address_space(3)))*)pl);
-    bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 __attribute__((address_space(3)))*)ph);
+  // D0 + 4 * (r % 4) and receives keys K0 .. K0 + 3 of dim D0 + r.  (The permutation of V rows is the same for rows 4 apart.)
+  {
+    const int r16 = lane & 15, dsel = (lane >> 4) & 1, row = hl * 4 + (r16 >> 2);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      v_addr[dt] = lds0 + kVOff + row * (D * 2) + ((dt * 4 + dsel * 2 + ((r16 & 3) >> 1)) ^ v_swizzle(row)) * 16 + (r16 & 1) * 8;
+  }
+#if defined(__HIP_DEVICE_COMPILE__)
+  // (kept as they are: recomputed from one another they would cost an instruction per fragment)
+#pragma unroll
+  for (int s = 0; s < DSTEPS; ++s) asm volatile("" : "+v"(k_addr[s]));
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) asm volatile("" : "+v"(v_addr[dt]));
+#endif
+  auto v_frag = [&](uint32_t tile, int t, int dt) {
+    const uint32_t at = v_addr[dt] + (tile + t * 16 * (D * 2));
+    bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 __attribute__((address_space(3)))*)(uintptr_t)at);
+    bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((bf16x4 __attribute__((address_space(3)))*)(uintptr_t)(at + 8 * (D * 2)));
     bf16x8 va = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return va;
   };
 
   // ---- S^T = K Q^T -----------------------------------------------------------------------------------
-  auto qk_tile = [&](int buf, f32x16 (&sacc)[2]) {
-    const uint16_t* Kt = sm.k[buf];
+  auto qk_tile = [&](uint32_t Kt, f32x16 (&sacc)[2]) {
 #pragma unroll
     for (int s = 0; s < DSTEPS; ++s) {
 #pragma unroll
@@ -484,8 +487,7 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   };
   // The scores of the first tile of a list have nothing to run under: every K fragment is requested before the first
   // matrix instruction, so that the LDS latency is paid once and not once per pair of instructions.
-  auto qk_tile_first = [&](int buf, f32x16 (&sacc)[2]) {
-    const uint16_t* Kt = sm.k[buf];
+  auto qk_tile_first = [&](uint32_t Kt, f32x16 (&sacc)[2]) {
     constexpr int N_QK = 2 * DSTEPS;
     constexpr int AHEAD = N_QK < 8 ? N_QK : 8;  // fragments in flight
     bf16x8 kf[AHEAD];
@@ -573,8 +575,7 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
     pb[t][i] = (__bf16)p;
   };
   // ---- plain step: probabilities, then O^T += V^T P^T ------------------------------------------------
-  auto finish_tile = [&](int vbuf, const f32x16 (&sv)[2]) {
-    const uint16_t* Vt = sm.v[vbuf];
+  auto finish_tile = [&](uint32_t Vt, const f32x16 (&sv)[2]) {
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
     float rs = 0.f;
     bf16x8 pb[4];
@@ -593,9 +594,7 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   //   phase A  score MFMAs of the next tile   + probabilities of keys  0..31 of this tile
   //   phase B  O += P V for keys 0..31        + probabilities of keys 32..63
   //   phase C  O += P V for keys 32..63
-  auto fused_step = [&](int kbuf_next, int vbuf, const f32x16 (&sv)[2], f32x16 (&sacc)[2]) {
-    const uint16_t* Kt = sm.k[kbuf_next];
-    const uint16_t* Vt = sm.v[vbuf];
+  auto fused_step = [&](uint32_t Kt, uint32_t Vt, const f32x16 (&sv)[2], f32x16 (&sacc)[2]) {
     constexpr int N_QK = 2 * DSTEPS;         // score MFMAs
     constexpr int N_PV = 4 * DT;             // PV MFMAs
     constexpr int VA = 16 / N_QK > 0 ? 16 / N_QK : 1;  // probabilities per slot in phase A
@@ -657,10 +656,12 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   // Visit list of a window of whole tiles: wavefront 0 compacts the tiles some query of the group sees.  (The first
   // window is built ahead of the window loop, from the summaries requested at the top of the kernel, so that those do
   // not stay in registers through the tile loop.)
+  // (the element mask is only evaluated on diagonal tiles and on tiles with mixed visibility)
+  auto needs_lim = [&](int t, int emin) { return t * kTile + kTile - 1 - a.base > r0_group || emin < rlast_group; };
   auto compact_round = [&](int t, int2 val, int& count) {
     const bool v = t <= kt_end_group && val.x >= r0_group;
     const uint64_t bits = __ballot(v);
-    if (v) sm.vlist[count + __builtin_popcountll(bits & ((uint64_t(1) << lane) - 1))] = make_int4(t, val.x, val.y, 0);
+    if (v) sm.vlist[count + __builtin_popcountll(bits & ((uint64_t(1) << lane) - 1))] = make_int4(kUniform && needs_lim(t, val.y) ? t | kPackedMaskFlag : t, val.x, val.y, 0);
     count += __builtin_popcountll(bits);
   };
   auto build_list = [&](int w0, bool first) {
@@ -682,6 +683,71 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
       if (w0 + j * kWave <= kt_end_group) compact_round(w0 + j * kWave + lane, vals[j], count);
     if (lane == 0) sm.vcount = count;
   };
+  // Packed tiles: a granule joins the list of its kind (staged in the tile buffers, which are idle here) ...
+  auto sort_granule = [&](int g, bool in_range, const int2& v, int& n_plain, int& n_mask) {
+    int* plain_ids = reinterpret_cast<int*>(&sm.k[0][0]);
+    int* mask_ids = reinterpret_cast<int*>(&sm.v[0][0]);
+    const bool vis = in_range && v.x >= r0_group;
+    const int last_pos = g * kGranule + kGranule - 1 - a.base;
+    const bool plain = vis && v.y >= rlast_group && last_pos <= r0_group && (g + 1) * kGranule <= a.N;
+    const bool masked = vis && !plain;
+    const uint64_t bp = __ballot(plain), bm = __ballot(masked);
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    if (plain) plain_ids[n_plain + __builtin_popcountll(bp & below)] = g;
+    if (masked) mask_ids[n_mask + __builtin_popcountll(bm & below)] = g;
+    n_plain += __builtin_popcountll(bp);
+    n_mask += __builtin_popcountll(bm);
+  };
+  // ... and the two kinds become tiles of four, behind `head` gathered ones
+  auto list_granules = [&](int head, int n_plain, int n_mask) {
+    int* plain_ids = reinterpret_cast<int*>(&sm.k[0][0]);
+    int* mask_ids = reinterpret_cast<int*>(&sm.v[0][0]);
+    wave_lds_sync();
+    const int n_pt = n_plain / kGranPerTile;
+    const int left = n_plain - n_pt * kGranPerTile;  // these join the masked kind
+    if (lane < left) mask_ids[n_mask + lane] = plain_ids[n_pt * kGranPerTile + lane];
+    n_mask += left;
+    wave_lds_sync();
+    const int n_mt = (n_mask + kGranPerTile - 1) / kGranPerTile;
+    for (int i = lane; i < n_pt + n_mt; i += kWave) {
+      int4 d;
+      if (i < n_pt) {
+        const int* p = plain_ids + i * kGranPerTile;
+        d = make_int4(p[0], p[1], p[2], p[3]);
+      } else {
+        const int o = (i - n_pt) * kGranPerTile;
+        d.x = mask_ids[o] | kPackedMaskFlag;
+        d.y = o + 1 < n_mask ? mask_ids[o + 1] : -1;
+        d.z = o + 2 < n_mask ? mask_ids[o + 2] : -1;
+        d.w = o + 3 < n_mask ? mask_ids[o + 3] : -1;
+      }
+      sm.vlist[head + i] = d;
+    }
+    if (lane == 0) sm.vcount = head + n_pt + n_mt;
+  };
+  // gathered tiles [first, first + count) at the head of the list: whole tiles of list A need no mask (every query sees their
+  // rows, and they lie below near_row0); the last one of A and the tiles of B go through it
+  auto list_far = [&](int first, int count) {
+    for (int i = lane; i < count; i += kWave) {
+      const int t = first + i;
+      sm.vlist[i] = make_int4(kFarTileFlag | ((t + 1) * kTile <= n_far_a ? 0 : kPackedMaskFlag), far_start(t), 0, 0);
+    }
+  };
+  if (early_list && wave == 0) {
+    // (one trip to memory between the start of the workgroup and its list; in the windows below two, one after the other, and both
+    // behind the Q rows)
+    if (kFar) list_far(0, n_far_tiles);
+    int n_plain = 0, n_mask = 0;
+#pragma unroll
+    for (int j = 0; j < kEarly; ++j)
+      if (j * kWave < n_near) sort_granule(near_g0 + j * kWave + lane, j * kWave + lane < n_near, tl_early[j], n_plain, n_mask);
+    list_granules(kFar ? n_far_tiles : 0, n_plain, n_mask);
+  }
+  if (early_ids && wave == 1) {
+#pragma unroll
+    for (int j = 0; j < kIdsAhead; ++j)
+      if (j < n_far_tiles) sm.posk[j][lane] = ids_early[j];
+  }
   if (!kPacked && wave == 0) {
     if (kt_end_group < kEarly * kWave) {
       // every tile summary the list needs was requested at the top: nothing else is loaded here, and the wait for
@@ -697,12 +763,11 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   }
 
   // (packed tiles: the window counts granules, and leaves room for the one tile the packing can add)
-  const int g_end_group = (a.base + rlast_group) / kGranule;
   const int win_last = kPacked ? g_end_group : kt_end_group;
   constexpr int kWinStep = kPacked ? (kWin - 1) * kGranPerTile : kWin;
   int f0 = 0;                                // first tile of the long-lived rows in this window
   bool far_win = far_mode && n_far_tiles > 0;  // windows of gathered tiles come first, then the granule walk
-  for (int w0 = far_mode ? near_row0 / kGranule : 0; w0 <= win_last;) {
+  for (int w0 = kPacked ? near_g0 : 0; w0 <= win_last;) {
     // ---- visit list of this window: wavefront 0 compacts the tiles some query tile of the group sees ----
     // far_cnt gathered tiles at the head of the list; the granule walk joins the window that holds the last of them
     // when its tiles fit behind (the usual case: one pass of the tile pipeline per workgroup)
@@ -710,31 +775,16 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
     bool with_near = !far_win;
     if (kFar && far_win) {
       far_cnt = min(kWin - 1, n_far_tiles - f0);
-      const int n_near = g_end_group - w0 + 1;  // granules of the walk
       with_near = f0 + far_cnt == n_far_tiles && n_near <= kWinStep &&
                   far_cnt + (n_near + kGranPerTile - 1) / kGranPerTile + 1 <= kWin - 1;
     }
-    if (kFar && far_win && wave == 0) {
-      // gathered tiles [f0, f0 + count): whole tiles of list A need no mask (every query sees their rows, and they
-      // lie below near_row0); the last one of A and the tiles of B go through it
-      const int cnt = far_cnt;
-      for (int i = lane; i < cnt; i += kWave) {
-        const int t = f0 + i;
-        int4 d;
-        if (t < n_far_ta) {
-          d = make_int4(kFarTileFlag | ((t + 1) * kTile <= n_far_a ? 0 : kPackedMaskFlag), t * kTile, 0, 0);
-        } else {
-          d = make_int4(kFarTileFlag | kPackedMaskFlag, a.long_cap + b_lo + (t - n_far_ta) * kTile, 0, 0);
-        }
-        sm.vlist[i] = d;
-      }
-      if (lane == 0 && !with_near) sm.vcount = cnt;
+    if (kFar && far_win && wave == 0 && !early_list) {
+      list_far(f0, far_cnt);
+      if (lane == 0 && !with_near) sm.vcount = far_cnt;
     }
-    if (kPacked && with_near && wave == 0) {
+    if (kPacked && with_near && wave == 0 && !early_list) {
       // granules seen without a mask and granules that need one, each kind in its own list (staged in the tile
       // buffers, which are idle here), then four ids per tile
-      int* plain_ids = reinterpret_cast<int*>(&sm.k[0][0]);
-      int* mask_ids = reinterpret_cast<int*>(&sm.v[0][0]);
       const int2* gl = a.gran_lim + (int64_t)ks * a.Tk * kGranPerTile;
       const int g_hi = min(w0 + kWinStep - 1, g_end_group);
       int n_plain = 0, n_mask = 0;
@@ -766,40 +816,10 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
 #pragma unroll
         for (int u = 0; u < kGranPerTile; ++u) {
           const int g = t * kGranPerTile + u;
-          const bool vis = t >= 0 && g >= w0 && g <= g_hi && vals[u].x >= r0_group;
-          const int last_pos = g * kGranule + kGranule - 1 - a.base;
-          const bool plain = vis && vals[u].y >= rlast_group && last_pos <= r0_group && (g + 1) * kGranule <= a.N;
-          const bool masked = vis && !plain;
-          const uint64_t bp = __ballot(plain), bm = __ballot(masked);
-          const uint64_t below = (uint64_t(1) << lane) - 1;
-          if (plain) plain_ids[n_plain + __builtin_popcountll(bp & below)] = g;
-          if (masked) mask_ids[n_mask + __builtin_popcountll(bm & below)] = g;
-          n_plain += __builtin_popcountll(bp);
-          n_mask += __builtin_popcountll(bm);
+          sort_granule(g, t >= 0 && g >= w0 && g <= g_hi, vals[u], n_plain, n_mask);
         }
       }
-      wave_lds_sync();
-      const int n_pt = n_plain / kGranPerTile;
-      const int left = n_plain - n_pt * kGranPerTile;  // these join the masked kind
-      if (lane < left) mask_ids[n_mask + lane] = plain_ids[n_pt * kGranPerTile + lane];
-      n_mask += left;
-      wave_lds_sync();
-      const int n_mt = (n_mask + kGranPerTile - 1) / kGranPerTile;
-      for (int i = lane; i < n_pt + n_mt; i += kWave) {
-        int4 d;
-        if (i < n_pt) {
-          const int* p = plain_ids + i * kGranPerTile;
-          d = make_int4(p[0], p[1], p[2], p[3]);
-        } else {
-          const int o = (i - n_pt) * kGranPerTile;
-          d.x = mask_ids[o] | kPackedMaskFlag;
-          d.y = o + 1 < n_mask ? mask_ids[o + 1] : -1;
-          d.z = o + 2 < n_mask ? mask_ids[o + 2] : -1;
-          d.w = o + 3 < n_mask ? mask_ids[o + 3] : -1;
-        }
-        sm.vlist[far_cnt + i] = d;
-      }
-      if (lane == 0) sm.vcount = far_cnt + n_pt + n_mt;
+      list_granules(far_cnt, n_plain, n_mask);
     }
     if (!kPacked && wave == 0 && w0 > 0) build_list(w0, false);
     __syncthreads();
@@ -811,69 +831,66 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
       n_vis = max(0, min(per, n_vis - j0));
     }
     if (n_vis > 0) {
-      // The list entries are the same for every lane: they are kept in scalar registers.
       // Tile j of the list: the matrix pipe computes the scores of tile j+1 while the vector ALU turns those of
       // tile j into probabilities; then O += P V for tile j.  Buffers: K tile j in k[j & 3], V tile j in
       // v[j & 3], row limits of tile j in limk[j & 7].
-      auto entry = [&](int j, int& kt, int& emax, int& emin) {
-        const int4 e = sm.vlist[j0 + j];
-        kt = __builtin_amdgcn_readfirstlane(e.x);
-        emax = __builtin_amdgcn_readfirstlane(e.y);
-        emin = __builtin_amdgcn_readfirstlane(e.z);
-      };
-      // the element mask is only evaluated on diagonal tiles and on tiles with mixed visibility
-      auto group_needs_lim = [&](int kt, int emin) { return kt * kTile + kTile - 1 - a.base > r0_group || emin < rlast_group; };
       auto visits = [&](int kt, int emax) { return kUniform || (wave_live && kt <= my_kt_end && emax >= tile_r0); };
 
       // One step handles two tiles of the list (2s, 2s + 1) between two workgroup barriers.  At its start the
       // K tiles 2s + 1, 2s + 2 and the V tiles 2s, 2s + 1 are in LDS and the scores of tile 2s in registers; the
       // step puts K tiles 2s + 3, 2s + 4 and V tiles 2s + 2, 2s + 3 in flight.
-      // (packed tiles: kt is the entry's first field with its flags, emax this wavefront's granule of the tile -- or
-      // the first list entry of a gathered tile -- and emin the entry's place in the list)
+      // The entries of the list are the same for every lane: lane l holds entry l of a group of 64, and a step takes its two
+      // from there into scalar registers.
+      // (whole tiles: the tile with the mask flag, and its limits where wavefronts walk on their own; packed tiles: the entry's
+      // first field with its flags, and this wavefront's granule of the tile -- or the first list entry of a gathered tile)
       struct Entry {
         int kt, emax, emin;
       };
-      auto read_entry = [&](int j) {
-        Entry r = {0, 0, 0};
-        if (j < n_vis) {
-          if (kPacked) {
-            const int* ep = reinterpret_cast<const int*>(&sm.vlist[j0 + j]);
-            r.kt = __builtin_amdgcn_readfirstlane(ep[0]);
-            // (this wavefront's granule: the one its first transferred row lies in; a wavefront without transfers
-            // reads the last one and does not use it)
-            const int my_gran = min(wave * DMA_PER_WAVE * kRowsPerInst / kGranule, kGranPerTile - 1);
-            const int sel = (kFar && (r.kt & kFarTileFlag)) ? 1 : my_gran;
-            const int mine = __builtin_amdgcn_readfirstlane(ep[sel]);
-            r.emax = sel == 0 ? mine & ~kPackedMaskFlag : mine;
-            r.emin = j0 + j;
-          } else {
-            int kt, emax, emin;
-            entry(j, kt, emax, emin);
-            r.kt = kt; r.emax = emax; r.emin = emin;
-          }
+      int ent0 = 0, ent1 = 0, ent2 = 0;
+      auto open_entries = [&](int first) {
+        const int* ep = reinterpret_cast<const int*>(&sm.vlist[min(j0 + first + lane, kWin - 1)]);
+        ent0 = ep[0];
+        if (kPacked) {
+          // (the granule of the wavefront's first transferred row; a wavefront without transfers reads the last one and does
+          // not use it)
+          const int my_gran = min(wave * DMA_PER_WAVE * kRowsPerInst / kGranule, kGranPerTile - 1);
+          ent1 = ep[(kFar && (ent0 & kFarTileFlag)) ? 1 : my_gran];
+          if (my_gran == 0 && !(kFar && (ent0 & kFarTileFlag))) ent1 &= ~kPackedMaskFlag;
+        } else if (!kUniform) {
+          ent1 = ep[1];
+          ent2 = ep[2];
         }
+      };
+      auto read_entry = [&](int j) {
+        Entry r;
+        r.kt = __builtin_amdgcn_readlane(ent0, j & 63);
+        r.emax = kPacked || !kUniform ? __builtin_amdgcn_readlane(ent1, j & 63) : 0;
+        r.emin = !kPacked && !kUniform ? __builtin_amdgcn_readlane(ent2, j & 63) : 0;
         return r;
       };
-      auto load_k = [&](int j, const Entry& e) {
+      // (tile: the tile buffer's place, a constant)
+      auto load_k = [&](int j, const Entry& e, uint32_t tile) {
         if (j < n_vis) {
           if (kPacked) {
-            issue_k_p(e.kt, e.emax, e.emin, j & 3, j & 7);
+            issue_k_p(e.kt, e.emax, j0 + j, tile, j & 7);
+          } else if (kUniform) {
+            issue_k(e.kt & ~kPackedMaskFlag, tile, j & 7, (e.kt & kPackedMaskFlag) != 0);
           } else {
-            issue_k(e.kt, j & 3, j & 7, group_needs_lim(e.kt, e.emin));
+            issue_k(e.kt, tile, j & 7, needs_lim(e.kt, e.emin));
           }
         }
       };
-      auto load_v = [&](int j, const Entry& e) {
+      auto load_v = [&](int j, const Entry& e, uint32_t tile) {
         if (j < n_vis) {
           if (kPacked) {
-            issue_v_p(e.kt, e.emax, j & 3, j & 7);
+            issue_v_p(e.kt, e.emax, tile, j & 7);
           } else {
-            issue_v(e.kt, j & 3);
+            issue_rows(vbuf, a.vs_l, voff, kVOff + tile, (e.kt & ~kPackedMaskFlag) * kTile);
           }
         }
       };
       // tile t: its scores (in sacc) become probabilities while the scores of tile t + 1 are computed, then O += P V
-      auto process_tile = [&](int t, const Entry& ec, const Entry& en) {
+      auto process_tile = [&](int t, const Entry& ec, const Entry& en, uint32_t k_next, uint32_t v_this) {
         const bool vis_c = visits(ec.kt, ec.emax);
         // (uniform case: the last tile computes scores of a stale tile that nobody reads, which keeps the step
         // free of branches around the matrix instructions)
@@ -881,26 +898,25 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
         if (vis_c) {
           f32x16 sv[2] = {sacc[0], sacc[1]};
           // no masked score: every key row is at or before the first query and visible to the last one
-          const bool full = kPacked ? !(ec.kt & kPackedMaskFlag)
-                                    : (ec.kt * kTile + kTile - 1 - a.base <= my_r0 && ec.emin >= my_rlast);
+          const bool full = kUniform ? !(ec.kt & kPackedMaskFlag) : (ec.kt * kTile + kTile - 1 - a.base <= my_r0 && ec.emin >= my_rlast);
           if (!full) {
             if (kPacked) {
               mask_scores_p(t & 7, sv, kFar && (ec.kt & kFarTileFlag) != 0);
             } else {
-              mask_scores(ec.kt, t & 7, sv);
+              mask_scores(ec.kt & ~kPackedMaskFlag, t & 7, sv);
             }
           }
           const float mx = row_max(sv);
           if (__ballot(mx > m_run + kRescaleSlack)) rescale(mx);
           if (kUniform) {
-            fused_step((t + 1) & 3, t & 3, sv, sacc);
+            fused_step(k_next, v_this, sv, sacc);
           } else {
             // wavefronts with different query tiles: the same pipeline, its two halves one after the other
-            finish_tile(t & 3, sv);
-            if (vis_n) qk_tile((t + 1) & 3, sacc);
+            finish_tile(v_this, sv);
+            if (vis_n) qk_tile(k_next, sacc);
           }
         } else if (vis_n) {
-          qk_tile((t + 1) & 3, sacc);
+          qk_tile(k_next, sacc);
         }
       };
 
@@ -912,41 +928,57 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
 #if defined(__HIP_DEVICE_COMPILE__)
           asm volatile("" : "+v"(ln));
 #endif
-          const int start = __builtin_amdgcn_readfirstlane(sm.vlist[j0 + j].y);
-          __builtin_amdgcn_global_load_lds(lrows + start + ln,
-                                           (uint32_t __attribute__((address_space(3)))*)(&sm.posk[j & 7][0]), 4, 0, 0);
+          RowBuffer(lrows + far_start(f0 + j0 + j), kTile * 4).template to_lds<4>(lds0 + kPosOff + (j & 7) * kTile * 4, ln * 4, 0);
         }
       };
-      if (kFar && j0 < far_cnt) {
+      if (kFar && j0 < far_cnt && !early_ids) {
 #pragma unroll
-        for (int j = 0; j < 5; ++j) load_ids(j);
-        __builtin_amdgcn_s_waitcnt(0);
+        for (int j = 0; j < kIdsAhead; ++j) load_ids(j);
+        wait_transfers();
         __syncthreads();
       }
+      open_entries(0);
       Entry e0 = read_entry(0), e1 = read_entry(1), e2 = read_entry(2);
-      load_k(0, e0);
-      load_v(0, e0);
-      load_k(1, e1);
-      load_v(1, e1);
-      load_k(2, e2);
-      __builtin_amdgcn_s_waitcnt(0);
+      load_k(0, e0, 0);
+      load_v(0, e0, 0);
+      load_k(1, e1, kTileBytes);
+      load_v(1, e1, kTileBytes);
+      load_k(2, e2, 2 * kTileBytes);
+      wait_transfers();
       __syncthreads();
       if (visits(e0.kt, e0.emax)) qk_tile_first(0, sacc);
       __syncthreads();  // k[0] is overwritten by the first step
 
-      for (int t = 0; t < n_vis; t += 2) {
-        const Entry e3 = read_entry(t + 3), e4 = read_entry(t + 4);
-        load_k(t + 3, e3);
-        load_k(t + 4, e4);
-        load_v(t + 2, e2);
-        load_v(t + 3, e3);
+      // (The step exists twice, for the two places in the rings of buffers at which it may start, so that the LDS addresses of its
+      // fragments and transfers are constants of the instructions.  Two wavefronts share a SIMD and either issues one instruction in
+      // four cycles at most, scalar ones among them, so a step's time follows its instructions: with run-time buffer numbers, generic
+      // pointers, a branch for the last tile's rows and entries read from LDS one by one it had 266 scalar and 25 vector
+      // instructions more than the matrix instructions and the softmax need, now 155 and none.  32768 tokens at chunk 64, 32 / 8 heads of 128
+      // 762 -> 721 us, 4 x 3001 at chunk 32 150.7 -> 148.1, 8192 at chunk 1 137.5 -> 128.4.  A second copy of the transfers for
+      // steps far from the list's end, without their conditions, was slower: its scalars did not fit the registers.)
+      auto step = [&](int t, auto phase) {
+        constexpr uint32_t P = decltype(phase)::value;  // t & 3
+        constexpr uint32_t b0 = P * kTileBytes, b1 = (P + 1) * kTileBytes, b2 = ((P + 2) & 3) * kTileBytes, b3 = ((P + 3) & 3) * kTileBytes;
+        const Entry e3 = read_entry(t + 3);
+        if (P == 0 && ((t + 4) & 63) == 0) open_entries(t + 4);
+        const Entry e4 = read_entry(t + 4);
+        load_k(t + 3, e3, b3);
+        load_k(t + 4, e4, b0);
+        load_v(t + 2, e2, b2);
+        load_v(t + 3, e3, b3);
         load_ids(t + 5);
         load_ids(t + 6);
-        process_tile(t, e0, e1);
-        if (t + 1 < n_vis) process_tile(t + 1, e1, e2);
+        process_tile(t, e0, e1, b1, b0);
+        if (t + 1 < n_vis) process_tile(t + 1, e1, e2, b2, b1);
         e0 = e2; e1 = e3; e2 = e4;
-        __builtin_amdgcn_s_waitcnt(0);  // the tiles in flight have landed in LDS
-        __syncthreads();                // ... for every wavefront, and the tiles of this step are no longer read
+        wait_transfers();  // the tiles in flight have landed in LDS
+        __syncthreads();   // ... for every wavefront, and the tiles of this step are no longer read
+      };
+      for (int t = 0;;) {
+        step(t, std::integral_constant<int, 0>{});
+        if ((t += 2) >= n_vis) break;
+        step(t, std::integral_constant<int, 2>{});
+        if ((t += 2) >= n_vis) break;
       }
     } else if (!with_near || w0 + kWinStep <= win_last) {
       __syncthreads();  // (nobody may still be reading this window's count when wavefront 0 starts the next list)
@@ -1221,28 +1253,6 @@ struct WideSmem {
   int limk[4][kTile];          // row limits of tile j in limk[j & 3]
 };
 
-// One global -> LDS transfer: lane i moves kBytes from its own global address to LDS address (uniform) + i * kBytes.
-// Counted by vmcnt like any vector memory load.  (The host pass of the single-source compile never runs this.)
-template <int kBytes>
-__device__ __forceinline__ void lds_transfer(const void* gptr, const void* lds_ptr) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t lds_addr =
-      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds_ptr);
-  if (kBytes == 16) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory", "m0");
-  } else {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr), "s"(lds_addr) : "memory", "m0");
-  }
-#endif
-}
-// The LDS address of an object as a number: taken from the pointer once, it is plain scalar arithmetic from then on.
-__device__ __forceinline__ uint32_t lds_address(const void* lds_ptr) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds_ptr);
-#else
-  return 0;
-#endif
-}
 // A 16-byte transfer with the global address as a uniform base (scalar registers) plus a byte offset per lane (no 64-bit
 // vector arithmetic) and the LDS address as a number.
 __device__ __forceinline__ void lds_transfer16_base(const void* base, uint32_t byte_off, uint32_t lds_addr) {
@@ -1251,12 +1261,6 @@ __device__ __forceinline__ void lds_transfer16_base(const void* base, uint32_t b
                : "memory", "m0");
 #endif
 }
-__device__ __forceinline__ void wait_transfers() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#endif
-}
-
 constexpr int kWideWaves = 4;
 
 __global__ __launch_bounds__(kWideWaves * kWave) void prefill_mfma_wide_kernel(PrefillArgs a) {
@@ -1368,12 +1372,12 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_mfma_wide_kernel(P
         const int row = wave * (2 * DMA_PER_WAVE) + 2 * j + hl;
         const int chunk = is_v ? l32 ^ v_swizzle(row) : l32 ^ (row % OCT);
         const int n = min(kt * kTile + row, a.N - 1);
-        lds_transfer<16>(base + (int64_t)n * stride + chunk * 8, dst + (wave * DMA_PER_WAVE + j) * kWave * 8);
+        lds_transfer16(base + (int64_t)n * stride + chunk * 8, lds_address(dst + (wave * DMA_PER_WAVE + j) * kWave * 8));
       }
     }
   };
   auto issue_lim = [&](int kt, int slot) {
-    if (wave == 0) lds_transfer<4>(lim + min(kt * kTile + lane, a.N - 1), &sm.limk[slot][0]);
+    if (wave == 0) RowBuffer(lim + kt * kTile, min(kTile, a.N - kt * kTile) * 4).to_lds<4>(lds_address(&sm.limk[slot][0]), lane * 4, 0);
   };
   auto issue_k = [&](int kt, int buf, int slot) {
     issue_rows(kp, a.ks_l, sm.k[buf], kt, false);
@@ -1779,6 +1783,7 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   a.qt_first = a.r_begin / kTile; a.qt_last = (a.r_end - 1) / kTile;
   const int64_t n_qt = a.qt_last - a.qt_first + 1;
   a.scale = sm_scale;
+  a.rows64 = ((g.N - 1) * std::max(a.ks_l, a.vs_l) + g.D) * 2 >= (int64_t(1) << 32);
   a.hpw = 1; a.qpw = 1; a.n_hg = 1; a.n_qg = (int)n_qt; a.xcd_mode = 0;
 
   // bf16 at head dim 256 (rows that 16-byte transfers can take; other layouts go to the plain kernel)
@@ -1850,7 +1855,7 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   // long-lived rows instead, row by row (NATS_PREFILL_FAR=0 in the environment walks every granule, for comparison).
   // (Chunks of a granule and more: a visible granule is visible as a whole there, and its transfer from one base
   // address is cheaper than a gathered one; measured 10 % slower at chunk 32.)
-  if (packed && g.C < kGranule && use_far_rows()) {
+  if (packed && g.C < kGranule && use_far_rows() && !a.rows64) {
     a.t_long = (int)long_row_threshold(g.W);
     if (int rc = launch_long_rows(w, g.B * g.H_kv, g.N, g.base, g.W, st)) return rc;
     a.long_rows = w.long_rows; a.long_lim = w.long_lim; a.long_before = w.long_before; a.long_alive = w.long_alive;

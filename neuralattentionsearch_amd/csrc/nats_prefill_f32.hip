@@ -54,34 +54,21 @@ __device__ __forceinline__ float f32_part(const typename F32Vec<DT>::type& v, in
 template <>
 __device__ __forceinline__ float f32_part<1>(const float& v, int) { return v; }
 
-constexpr int kWaitLoads = 0x0f70;  // vmcnt(0), the other counters at their largest
-
-// Rows of K or V as a raw buffer of `bytes` bytes: reads beyond its end give zero, and a row is a scalar offset beside a lane's
-// own, where addresses per row (two registers each) would not fit beside the tiles.  (Its type exists in the device pass only.)
-struct RowBuffer {
+template <int DT>
+__device__ __forceinline__ typename F32Vec<DT>::type row_part(const RowBuffer& buf, int lane_off, int row_off) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __amdgpu_buffer_rsrc_t desc;
-  __device__ __forceinline__ RowBuffer(const float* base, int bytes) : desc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000)) {}
-  __device__ __forceinline__ void to_lds(float* dst, int lane_off, int row_off) const {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(desc, (void __attribute__((address_space(3)))*)dst, 16, lane_off, row_off, 0, 0);
-  }
-  template <int DT>
-  __device__ __forceinline__ typename F32Vec<DT>::type row(int lane_off, int row_off) const {
-    if constexpr (DT == 1) {
-      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(desc, lane_off, row_off, 0));
-    } else if constexpr (DT == 2) {
-      return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(desc, lane_off, row_off, 0));
-    } else {
-      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(desc, lane_off, row_off, 0));
-    }
+  const __amdgpu_buffer_rsrc_t desc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(buf.base), 0, (int)buf.bytes, RowBuffer::kFlags);
+  if constexpr (DT == 1) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(desc, lane_off, row_off, 0));
+  } else if constexpr (DT == 2) {
+    return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(desc, lane_off, row_off, 0));
+  } else {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(desc, lane_off, row_off, 0));
   }
 #else
-  __device__ RowBuffer(const float*, int) {}
-  __device__ void to_lds(float*, int, int) const {}
-  template <int DT>
-  __device__ typename F32Vec<DT>::type row(int, int) const { return {}; }
+  return {};
 #endif
-};
+}
 
 template <int D, int kWaves>
 __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_kernel(PrefillArgs a, int blk_first, int n_blk, int paired) {
@@ -118,6 +105,7 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
 
   float* k_lds = smem + kF32Rows * Lay::kQPitch + wave * Lay::kWaveFloats;
   int* lim_lds = reinterpret_cast<int*>(k_lds + kF32Rows * D);
+  const uint32_t k_addr = lds_address(k_lds);
   const float* q_lds = smem + l32 * Lay::kQPitch + hl * 4;
 
   f32x16 oacc[DT];
@@ -180,7 +168,7 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
 #pragma unroll
     for (int j = 0; j < kF32Rows / kRowsPerInst; ++j) {
       const int off = (row0 * (int)a.ks_l + ((ln % OCT) ^ swz(j * kRowsPerInst + row0)) * 4) * 4;
-      buf.to_lds(k_lds + j * kWave * 4, off, j * kRowsPerInst * (int)a.ks_l * 4);
+      buf.to_lds<16>(k_addr + j * kWave * 16, off, j * kRowsPerInst * (int)a.ks_l * 4);
     }
   };
   auto k_frag = [&](int i) { return *reinterpret_cast<const f32x4*>(k_lds + l32 * D + ((2 * i + hl) ^ swz(l32)) * 4); };
@@ -210,15 +198,14 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
   __syncthreads();
   while (t >= 0) {
     const int k0 = t * kF32Rows;
-    // K of this tile has landed in LDS (the compiler does not wait for transfers into LDS before it reads there)
-    __builtin_amdgcn_s_waitcnt(kWaitLoads);
+    wait_transfers();  // K of this tile has landed in LDS
     __builtin_amdgcn_sched_barrier(0);
     // V rows of this tile (rows past the end repeat the last one: their probabilities are 0) and the row limits
     VecV vreg[16];
     {
       const RowBuffer buf = tile_buffer(vp, a.vs_l, k0);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) vreg[i] = buf.template row<DT>(voff, (8 * (i / 4) + i % 4) * (int)a.vs_l * 4);
+      for (int i = 0; i < 16; ++i) vreg[i] = row_part<DT>(buf, voff, (8 * (i / 4) + i % 4) * (int)a.vs_l * 4);
     }
     if (masked) lim_lds[lane] = lim[min(k0 + l32, a.N - 1)];
     __builtin_amdgcn_sched_barrier(0);

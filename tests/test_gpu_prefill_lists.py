@@ -1,0 +1,51 @@
+"""Visit lists of the bf16 prefill at the edges of how they are read and built (entries are held 64 at a time, granules of up to
+4096 rows are listed in one trip) and streams whose rows reach beyond 32-bit byte offsets, against the oracle and each other.
+
+Tolerance 2e-2 as for every bf16 prefill; the two layouts of one input hold the same rows, so their outputs are the same bytes."""
+import math
+
+import pytest
+import torch
+
+from tests.gpu_util import draw_roles, say, to_dev
+from tests.test_gpu_prefill import run_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L,D,C,W,p", [
+    (4095, 128, 64, 256, (0.96, 0.02, 0.02)),   # 64 entries, of which a step opens the second group for nothing
+    (4161, 128, 64, 256, (0.96, 0.02, 0.02)),   # 66
+    (8300, 64, 64, 128, (0.97, 0.01, 0.02)),    # three groups
+    (4096, 128, 32, 256, (0.4, 0.3, 0.3)),      # the last query group walks 256 granules: the early list
+    (4112, 128, 32, 256, (0.4, 0.3, 0.3)),      # 257: tile summaries first
+    (4300, 32, 16, 32, (0.9, 0.05, 0.05)),      # four groups of packed entries
+    (4200, 128, 1, 16, (0.5, 0.25, 0.25)),      # gathered tiles, more than the five known ahead
+    (700, 128, 1, 256, (0.1, 0.5, 0.4)),        # fewer
+])
+@pytest.mark.parametrize("heads", [(4, 1), (1, 1)])
+def test_list_edges(monkeypatch, heads, L, D, C, W, p):
+    monkeypatch.setenv("NATS_PREFILL_SPLIT", "0")  # one workgroup walks a whole list
+    run_case(1, heads[0], heads[1], L, D, C, W, torch.bfloat16, seed=L, p=p)
+
+
+@pytest.mark.parametrize("C", [64, 32, 1])
+def test_rows_beyond_32_bit_offsets(C):
+    """K and V as every 720000th element group of a 4.3 GB buffer: row 2983 on lies beyond 2^32 bytes."""
+    from neuralattentionsearch_amd import ops
+    say("rows beyond 32-bit offsets", C)
+    L, D, W, stride = 3100, 128, 256, 720000
+    g = torch.Generator(device="cuda").manual_seed(C)
+    q = torch.randn(1, 4, L, D, generator=g, device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.randn(1, 1, L, D, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    roles = to_dev(draw_roles(C, 1, 1, math.ceil(L / C)))
+    want = ops.prefill_attention(q, k, v, roles, C, W)
+    wide = torch.empty(L * stride, device="cuda", dtype=torch.bfloat16)
+    spread = []
+    for i, x in enumerate((k, v)):
+        view = wide.as_strided((1, 1, L, D), (L * stride, L * stride, stride, 1), storage_offset=i * D)
+        view.copy_(x)
+        spread.append(view)
+    got = ops.prefill_attention(q, spread[0], spread[1], roles, C, W)
+    # (a role per token: the far rows are walked by granules there, in another order)
+    assert torch.equal(got, want) if C > 1 else (got.float() - want.float()).abs().max().item() <= 2e-2
