@@ -55,8 +55,8 @@ __device__ __forceinline__ float exp2_guard(float x) { return __builtin_amdgcn_e
 // ---------------------------------------------------------------------------------------------------
 constexpr float kDecodeRescaleSlack = 8.0f;
 // K and V rows are read once per step: their loads carry the streaming hint (no retention in the caches)
-constexpr int kAuxStream = 2;  // the "nt" bit of a global_load_lds
 constexpr int kDecTile = 32;
+constexpr int kAuxStream = 2;  // ... as the "nt" bit of a global_load_lds
 
 constexpr int kMaxBalancedHeads = 1024;  // (b, kv head) streams whose tile prefix sums fit in LDS
 
@@ -231,17 +231,25 @@ __global__ __launch_bounds__(FIXED ? FIXED * kWave : 256) void decode_split_mfma
       }
     }
   };
+  const uint32_t v_lds = lds_address(&sm.v[__builtin_amdgcn_readfirstlane(wave)][0][0]);
   auto issue_v = [&](int r0, uint32_t m, int buf) {
     const int fv = __builtin_ctz(m);
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(v_lds + buf * kDecTile * D * 2);
 #pragma unroll
     for (int j = 0; j < NDMA; ++j) {
       const int q = j * kWave + lane;  // chunk slot in the LDS tile
       const int row = q / OCT, cpos = q % OCT;
       const int src_row = ((m >> row) & 1) ? row : fv;
       const int chunk = cpos ^ v_swz(row);
-      __builtin_amdgcn_global_load_lds(vp + (int64_t)(r0 + src_row) * a.ks_r + chunk * 8,
-                                       (uint32_t __attribute__((address_space(3)))*)(&sm.v[wave][buf][j * kWave * 8]), 16, 0,
-                                       kAuxStream);
+      const uint16_t* src = vp + (int64_t)(r0 + src_row) * a.ks_r + chunk * 8;
+      // (The builtin's transfers are waited for before this tile's first V fragment, next tile's and all: many tiles per wavefront lose
+      // by it (batch 32, context 65536 271.0 -> 269.0 us without), the one or two of the fixed schedule by the assembly's order:
+      // batch 1, context 16384 11.65 / 11.88.)
+      if constexpr (FIXED) {
+        __builtin_amdgcn_global_load_lds(src, (uint32_t __attribute__((address_space(3)))*)(&sm.v[wave][buf][j * kWave * 8]), 16, 0, kAuxStream);
+      } else {
+        lds_transfer16<true>(src, dst + j * kWave * 16);
+      }
     }
   };
   // Moves on to the head that holds tile `pos` of the list (`ks` is that head or an empty one before it): its
@@ -288,7 +296,7 @@ __global__ __launch_bounds__(FIXED ? FIXED * kWave : 256) void decode_split_mfma
         issue_v(tile_row0(t), rows, cur);
       }
       vb_next = load_valid(t + tstep);
-      __builtin_amdgcn_s_waitcnt(0);
+      wait_transfers();
       vm = (uint32_t)__ballot(vb != 0);
       if (vm != rows) {
 #pragma unroll
@@ -317,7 +325,7 @@ __global__ __launch_bounds__(FIXED ? FIXED * kWave : 256) void decode_split_mfma
     float m_run = -INFINITY, l_run = 0.f;  // of q head l16 (meaningful for l16 < nr)
 
     while (t < t_end) {
-      __builtin_amdgcn_s_waitcnt(0);  // K(t) in registers, V(t) in LDS, valid bytes of the next tile loaded
+      wait_transfers();  // K(t) in registers, V(t) in LDS, valid bytes of the next tile loaded
       const uint32_t vmn = (uint32_t)__ballot(vb_next != 0);
       float sc[2][4];
       float mx = -INFINITY;
@@ -395,7 +403,7 @@ __global__ __launch_bounds__(FIXED ? FIXED * kWave : 256) void decode_split_mfma
       vm = vmn;
       cur ^= 1;
     }
-    __builtin_amdgcn_s_waitcnt(0);
+    wait_transfers();
 
     // ---- merge the wavefronts of the workgroup, emit this head's partial ------------------------------
     // The accumulators are staged in the wavefront's LDS buffer 0 (its tiles are consumed); the first tile of the

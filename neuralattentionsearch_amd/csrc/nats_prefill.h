@@ -50,30 +50,6 @@ struct PrefillArgs {
   int rows64;  // a stream's rows of K or V reach beyond 32-bit byte offsets
 };
 
-// ---- transfers global memory -> LDS -------------------------------------------------------------------------
-// Lane i's bytes go to the (uniform) LDS destination + i * its size.  They are issued from assembly: for the builtins the compiler
-// waits for every transfer in flight before an LDS read that may alias one, which here are the first V fragment of every tile
-// and the row limits of every masked one, in the middle of the step that put the next tiles in flight.  Nothing else waits for them:
-// wait_transfers() and, for other wavefronts' rows, a barrier stand before the first read.  (Counted by vmcnt like any vector
-// memory load; no output registers.  The host pass of the single-source compile never runs these.)
-__device__ __forceinline__ uint32_t lds_address(const void* lds_ptr) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds_ptr);
-#else
-  return 0;
-#endif
-}
-// 16 bytes from every lane's own address
-__device__ __forceinline__ void lds_transfer16(const void* gptr, uint32_t lds_addr) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory", "m0");
-#endif
-}
-__device__ __forceinline__ void wait_transfers() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#endif
-}
 // Rows of K or V (or row limits) as a raw buffer of `bytes` bytes: reads beyond its end give zero, and a row is a scalar offset
 // beside a lane's own, where addresses per row would take two registers and vector arithmetic each.
 struct RowBuffer {
