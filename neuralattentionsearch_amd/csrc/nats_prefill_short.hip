@@ -81,13 +81,24 @@ __global__ __launch_bounds__(kShortWaves * kWave, 2) void prefill_short_kernel(S
 #pragma unroll
     for (int s = 0; s < DSTEPS; ++s) kreg[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(rp + s * 16));
   };
+  // (From assembly, with one buffer per tile: the builtin's transfers were waited for, next tile's and all, before this tile's first V
+  // fragment.  32 / 8 heads of 128, 1000 / 1700 tokens 27.4 / 30.1 -> 25.7 / 28.5 us, even roles 39.7 -> 36.8; 8 heads of 64 13.2 / 17.4 ->
+  // 12.1 / 16.0.)
+  const uint32_t v_lds = lds_address(&sm.v[wave][0][0]);
   auto load_v = [&](int t, int buf) {
+    const int row0 = t * kShortRows;
+    const RowBuffer rows(vp + (int64_t)row0 * a.vs_l, (uint32_t)((min(kShortRows, a.L - row0) - 1) * (int)a.vs_l + D) * 2);  // (rows past the end are zeros)
+    int ln = lane;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(ln));
+#endif
+    const int row = ln / OCT, chunk = (ln % OCT) ^ v_swizzle(ln / OCT);
 #pragma unroll
     for (int j = 0; j < NDMA; ++j) {
-      const int i = j * kWave + lane;
-      const int row = i / OCT, chunk = (i % OCT) ^ v_swizzle(row);
-      __builtin_amdgcn_global_load_lds(vp + (int64_t)min(t * kShortRows + row, a.L - 1) * a.vs_l + chunk * 8,
-                                       (uint32_t __attribute__((address_space(3)))*)(&sm.v[wave][buf][j * kWave * 8]), 16, 0, 0);
+      constexpr int kRows = kWave / OCT;  // of one transfer
+      // (the permutation of the rows repeats within a transfer, or the lane's own row says)
+      const int c = kRows % 4 == 0 ? chunk : (ln % OCT) ^ v_swizzle(j * kRows + row);
+      rows.template to_lds<16>(v_lds + (buf * kShortRows * D + j * kWave * 8) * 2, (row * (int)a.vs_l + c * 8) * 2, (uint32_t)(j * kRows * (int)a.vs_l * 2));
     }
   };
 
@@ -185,7 +196,7 @@ __global__ __launch_bounds__(kShortWaves * kWave, 2) void prefill_short_kernel(S
   while (t >= 0) {
     mine &= ~(uint64_t(1) << t);
     const int t_next = mine ? 63 - __builtin_clzll(mine) : -1;
-    __builtin_amdgcn_s_waitcnt(0);  // K in registers, V in LDS
+    wait_transfers();  // K in registers, V in LDS
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
@@ -249,7 +260,7 @@ __global__ __launch_bounds__(kShortWaves * kWave, 2) void prefill_short_kernel(S
     auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     l_run = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   }
-  __builtin_amdgcn_s_waitcnt(0);  // (a guess that was dropped has arrived: its buffer is about to be reused)
+  wait_transfers();  // (a guess that was dropped has arrived: its buffer is about to be reused)
   if (hl == 0) sm.m[wave][l32] = m_run;
   __syncthreads();
   float m_all = sm.m[0][l32];
