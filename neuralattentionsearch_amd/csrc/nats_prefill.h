@@ -83,6 +83,20 @@ struct RowBuffer {
         : "memory", "m0", "scc");
 #endif
   }
+  // four transfers of 16 bytes to consecutive KiB of LDS, their rows `step` bytes apart
+  __device__ __forceinline__ void to_lds_quad(uint32_t lds_addr, int off0, int off1, int off2, int off3, uint32_t row_off, uint32_t step) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    uint32_t row;
+    asm volatile(
+        "s_mov_b32 m0, %6\n\ts_mov_b32 %0, %7\n\tbuffer_load_dwordx4 %1, %5, %0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_add_u32 %0, %0, %8\n\tbuffer_load_dwordx4 %2, %5, %0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_add_u32 %0, %0, %8\n\tbuffer_load_dwordx4 %3, %5, %0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_add_u32 %0, %0, %8\n\tbuffer_load_dwordx4 %4, %5, %0 offen lds"
+        : "=&s"(row)
+        : "v"(off0), "v"(off1), "v"(off2), "v"(off3), "s"(desc), "s"(lds_addr), "s"(row_off), "s"(step)
+        : "memory", "m0", "scc");
+#endif
+  }
 };
 
 // fp32 kernel on the fp32 matrix instruction (nats_prefill_f32.hip)

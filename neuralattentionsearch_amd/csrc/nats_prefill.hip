@@ -1253,14 +1253,6 @@ struct WideSmem {
   int limk[4][kTile];          // row limits of tile j in limk[j & 3]
 };
 
-// A 16-byte transfer with the global address as a uniform base (scalar registers) plus a byte offset per lane (no 64-bit
-// vector arithmetic) and the LDS address as a number.
-__device__ __forceinline__ void lds_transfer16_base(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(lds_addr)
-               : "memory", "m0");
-#endif
-}
 constexpr int kWideWaves = 4;
 
 __global__ __launch_bounds__(kWideWaves * kWave) void prefill_mfma_wide_kernel(PrefillArgs a) {
@@ -1352,38 +1344,39 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_mfma_wide_kernel(P
   // wave * 16 + 2 j + hl, chunk l32 of each.  The row part of the address is uniform (scalar arithmetic); the lane adds
   // hl rows and its swizzled chunk, which differs from transfer to transfer by an XOR with a constant: row % 32 =
   // (wave & 1) * 16 + 2 j + hl has its three parts in separate bits, and so has (row & 3) << 2 = (j & 1) << 3 | hl << 2.
-  // Rows beyond N repeat row N-1 (they are later than every query, so the mask removes their scores).
-  const uint32_t k_lane = (uint32_t)(hl * a.ks_l * 2), v_lane = (uint32_t)(hl * a.vs_l * 2);  // bytes
-  const uint32_t k_chunk0 = (uint32_t)(l32 ^ (((wave & 1) << 4) | hl)), v_chunk0 = (uint32_t)(l32 ^ (hl << 2));
-  const uint32_t lds_k0 = lds_address(&sm.k[0][0]), lds_v0 = lds_address(&sm.v[0][0]);
-  auto issue_rows = [&](const uint16_t* base, int64_t stride, uint16_t* dst, int kt, bool is_v) {
-    if (kt * kTile + kTile <= a.N) {
-      const uint16_t* tb = base + ((int64_t)kt * kTile + wave * (2 * DMA_PER_WAVE)) * stride;  // uniform
-      const uint32_t lds = (is_v ? lds_v0 + (uint32_t)((dst - &sm.v[0][0]) * 2) : lds_k0 + (uint32_t)((dst - &sm.k[0][0]) * 2)) +
-                           (uint32_t)(wave * DMA_PER_WAVE * kWave * 16);
+  // (One wavefront per SIMD: the transfers' instructions are time in which its matrix pipe idles.  Four to an assembly block, with the
+  // row as a running scalar offset, they are three instructions each instead of eleven: 16384 tokens of 32 / 8 heads, chunk 64,
+  // 606 -> 593 us, 2 x 3001 at chunk 32 102 -> 99, 4000 at chunk 1 342 -> 335.)
+  // The wavefront's 16 rows are a buffer of their own; rows beyond N are zeros (they are later than every query, so the mask
+  // removes their scores).
+  int k_off[DMA_PER_WAVE], v_off[2];  // bytes
 #pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) {
-        const uint32_t off = is_v ? v_lane + ((v_chunk0 ^ (uint32_t)((j & 1) << 3)) << 4) : k_lane + ((k_chunk0 ^ (uint32_t)(2 * j)) << 4);
-        lds_transfer16_base(tb + (int64_t)(2 * j) * stride, off, lds + (uint32_t)(j * kWave * 16));
-      }
-    } else {
+  for (int j = 0; j < DMA_PER_WAVE; ++j) k_off[j] = (int)(hl * a.ks_l) * 2 + ((l32 ^ (((wave & 1) << 4) | hl)) ^ (2 * j)) * 16;
 #pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) {
-        const int row = wave * (2 * DMA_PER_WAVE) + 2 * j + hl;
-        const int chunk = is_v ? l32 ^ v_swizzle(row) : l32 ^ (row % OCT);
-        const int n = min(kt * kTile + row, a.N - 1);
-        lds_transfer16(base + (int64_t)n * stride + chunk * 8, lds_address(dst + (wave * DMA_PER_WAVE + j) * kWave * 8));
-      }
-    }
+  for (int j = 0; j < 2; ++j) v_off[j] = (int)(hl * a.vs_l) * 2 + ((l32 ^ (hl << 2)) ^ (j << 3)) * 16;
+  const uint32_t lds_k0 = lds_address(&sm.k[0][0]) + wave * DMA_PER_WAVE * kWave * 16, lds_v0 = lds_k0 + 2 * kTile * D * 2;
+  auto wave_rows = [&](const uint16_t* base, int64_t stride, int kt) {
+    const int row0 = kt * kTile + wave * (2 * DMA_PER_WAVE);
+    const int rows = min(2 * DMA_PER_WAVE, a.N - row0);
+    return RowBuffer(base + (int64_t)row0 * stride, rows > 0 ? ((rows - 1) * (int)stride + D) * 2 : 0);
   };
+  static_assert(DMA_PER_WAVE == 8, "two groups of four transfers");
   auto issue_lim = [&](int kt, int slot) {
     if (wave == 0) RowBuffer(lim + kt * kTile, min(kTile, a.N - kt * kTile) * 4).to_lds<4>(lds_address(&sm.limk[slot][0]), lane * 4, 0);
   };
   auto issue_k = [&](int kt, int buf, int slot) {
-    issue_rows(kp, a.ks_l, sm.k[buf], kt, false);
+    const RowBuffer rows = wave_rows(kp, a.ks_l, kt);
+    const uint32_t dst = lds_k0 + buf * (kTile * D * 2), step = (uint32_t)a.ks_l * 4;
+    rows.to_lds_quad(dst, k_off[0], k_off[1], k_off[2], k_off[3], 0, step);
+    rows.to_lds_quad(dst + 4 * kWave * 16, k_off[4], k_off[5], k_off[6], k_off[7], 4 * step, step);
     issue_lim(kt, slot);
   };
-  auto issue_v = [&](int kt, int buf) { issue_rows(vp, a.vs_l, sm.v[buf], kt, true); };
+  auto issue_v = [&](int kt, int buf) {
+    const RowBuffer rows = wave_rows(vp, a.vs_l, kt);
+    const uint32_t dst = lds_v0 + buf * (kTile * D * 2), step = (uint32_t)a.vs_l * 4;
+    rows.to_lds_quad(dst, v_off[0], v_off[1], v_off[0], v_off[1], 0, step);
+    rows.to_lds_quad(dst + 4 * kWave * 16, v_off[0], v_off[1], v_off[0], v_off[1], 4 * step, step);
+  };
 
   // ---- operand fragments -------------------------------------------------------------------------------
   auto k_frag = [&](const uint16_t* Kt, int kb, int s) {
