@@ -18,6 +18,7 @@ import math
 import torch
 from torch import nn
 
+from . import cache as cache_module
 from . import ops
 from .cache import ChunkMergeType, NAtSCache, NAtSChunkLayerCache, NAtSLayerCache
 
@@ -320,9 +321,48 @@ class BaseNAtSChunkAttentionLayer(BaseNAtSAttentionLayer):
         if pre_fill + x_len < self.chunk_size:
             cache.update_nats_cached_x_in_chunk(x, self.layer_id, self.chunk_merge_method)
             return self.one_hot_values.to(x).reshape(1, 1, 1, -1).expand(x.shape[0], self.n_kv_heads, 1, -1)
+        if (roles := self._segment_roles(x, pre_fill, start_pos, cache)) is not None:
+            return roles
         x_pooled, pad_size = cache.update_nats_cached_x_across_chunk(x, pre_fill, self.layer_id, self.chunk_merge_method)
         return super()._sample_for_token_info_values_inference(x_pooled, start_pos, sink_token_end=self.chunk_size,
                                                                force_last_global=pad_size != 0)
+
+    def _segment_roles(self, x, pre_fill: int, start_pos: int, cache):
+        """The pooling, the role projection and the roles of a segment that completes a chunk, in one launch where the torch
+        ops and the library product they stand in for are up to eleven (a turn of 301 tokens at dim 4096 waits for all of
+        them).  None where something of it is replaced, watched or not what the kernel computes: a mean over a chunk size
+        that is a power of two (dividing by it is exact, so the statistics are those of the torch ops; the fp32 sums of the
+        projection run in another order).  From chunks of 8 on: below, the product over all chunks is the library's work."""
+        C, H = self.chunk_size, self.n_msks
+        proj = self._modules.get("proj_layer")
+        if (type(cache) is not NAtSCache or cache.chunk_size != C or C < 8 or C & (C - 1)
+                or self.chunk_merge_method is not ChunkMergeType.MEAN or x.dim() != 3 or proj is None or not _plain_linear(proj)):
+            return None
+        w = proj._parameters["weight"]
+        B, _, dim = x.shape
+        if (not _plain_execution(x, (w,)) or not x.is_cuda or x.device != w.device or x.dtype != w.dtype
+                or x.dtype not in (torch.bfloat16, torch.float32) or x.stride(-1) != 1 or not w.is_contiguous() or w.shape != (3 * H, dim)
+                or H > 256 or (dim + 3 * H) * 4 > 160 * 1024 or not 0 < B <= 65535 or not self._segment_as_defined(cache)):
+            return None
+        carry = None
+        if pre_fill:
+            carry = cache.get_nats_cached_x_in_chunk(self.layer_id)
+            if carry is None or carry.shape != (B, 1, dim) or carry.dtype != x.dtype or carry.device != x.device:
+                return None
+        step = ops.role_step(x, w, C, 0, pre_fill=pre_fill, carry_in=carry, global_bias=self.global_token_enhanced_value,
+                             force_first_global=start_pos < C)
+        cache._update_cache_x(step["carry"], self.layer_id)
+        return step["token_states_info"]
+
+    def _segment_as_defined(self, cache) -> bool:
+        """Whether everything `_segment_roles` stands in for is what this package (and torch) defines."""
+        return (type(self).role_logits is _ROLE_LOGITS and super()._sample_for_token_info_values_inference.__func__ is _SAMPLE
+                and ops.roles_from_logits is _ROLES_FROM_LOGITS and cache_module.pool_chunks is _POOL_CHUNKS
+                and NAtSCache.merge_new_x_values_in_chunk is _MERGE and NAtSCache.update_nats_cached_x_across_chunk is _ACROSS_CHUNK
+                and NAtSCache._update_cache_x is _UPDATE_X and NAtSCache.get_nats_cached_x_in_chunk is _CACHED_X
+                and NAtSCache.get_nats_chunk_fill_size is _FILL_SIZE
+                and nn.Linear.forward is _LINEAR_FORWARD and nn.functional.linear is _LINEAR and nn.Module.__call__ is _CALL
+                and "role_logits" not in self.__dict__ and cache.__dict__.keys().isdisjoint(_SEGMENT_CACHE_METHODS))
 
 
 
@@ -357,3 +397,6 @@ _IN_CHUNK, _ACROSS_CHUNK = NAtSCache.update_nats_cached_x_in_chunk, NAtSCache.up
 _LAYER_UPDATES = (NAtSChunkLayerCache.update, NAtSLayerCache.update)
 _VALID_TOKENS = (NAtSChunkLayerCache.valid_tokens, NAtSLayerCache.valid_tokens)
 _LINEAR_FORWARD, _LINEAR, _CALL = nn.Linear.forward, nn.functional.linear, nn.Module.__call__
+_POOL_CHUNKS = cache_module.pool_chunks
+_UPDATE_X, _CACHED_X, _FILL_SIZE = NAtSCache._update_cache_x, NAtSCache.get_nats_cached_x_in_chunk, NAtSCache.get_nats_chunk_fill_size
+_SEGMENT_CACHE_METHODS = _CACHE_METHODS | {"_update_cache_x", "get_nats_cached_x_in_chunk", "get_nats_chunk_fill_size"}

@@ -56,9 +56,13 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float v) {
 // chunk while decoding, every token of a per-token cache) the role streams are spread over workgroups, each of which
 // pools the chunk for itself and projects it onto its own streams' three weight rows: the 24 dot products of a
 // Llama-3-8B layer then run side by side instead of six per wavefront one after the other.  VEC consecutive columns
-// per thread (16-byte loads when the rows allow it, else 1).
-template <bool kBf16, int VEC>
-__global__ __launch_bounds__(256) void role_step_kernel(RoleStepArgs a) {
+// per thread (16-byte loads when the rows allow it, else 1).  Few chunks of many columns are bound by the trips to memory
+// behind one another (THREADS = 512): twice the threads, sixteen rows to a trip, and the weights of a wavefront's first output
+// requested before the rows (bf16, dim 4096: five chunks of 64 rows 18.5 -> 15.4 us, the token that closes a chunk 7.6 -> 6.1, a role
+// per token 6.0 -> 5.3; fp32, five chunks 30.2 -> 20.1).  With 256 threads, many chunks or 2048 columns, both lose (32768 tokens
+// 62.2 -> 63.7, 4 x 300 tokens of 2048 at chunk 32 13.9 -> 15.3).
+template <bool kBf16, int VEC, int THREADS>
+__global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
   extern __shared__ float pooled[];  // [dim] statistic of this chunk, then [Hkv * 3] logits behind it
   float* logit_s = pooled + a.dim;
   const int s = blockIdx.x, b = blockIdx.y;
@@ -72,7 +76,20 @@ __global__ __launch_bounds__(256) void role_step_kernel(RoleStepArgs a) {
   const bool padded = a.S > 0 && s == a.S - 1 && a.pad != 0;  // zero rows take part in the statistic
   const char* xb = static_cast<const char*>(a.x);
   constexpr int esz = kBf16 ? 2 : 4;
-  for (int d = tid * VEC; d < a.dim; d += 256 * VEC) {
+  // this workgroup's outputs h0 * 3 + wave, + n_waves, ...
+  constexpr int n_waves = THREADS / kWave;
+  const int h0 = blockIdx.z * a.hpb, h1 = min(h0 + a.hpb, a.Hkv);
+  const int n_out = h1 * 3;
+  constexpr bool kFew = THREADS > 256;
+  constexpr int kPieces = kFew ? 8 : 1;  // of 64 lanes, 16 bytes each: the weights that are requested ahead
+  uint4 w_first[kPieces];
+  const bool w_ahead = kFew && a.S > 0 && h0 * 3 + wave < n_out;
+  if (w_ahead) {
+    const char* wrow = static_cast<const char*>(a.weight) + (int64_t)(h0 * 3 + wave) * a.dim * esz;
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) w_first[i] = *reinterpret_cast<const uint4*>(wrow + min((i * 64 + lane) * VEC, a.dim - VEC) * esz);
+  }
+  for (int d = tid * VEC; d < a.dim; d += THREADS * VEC) {
     float acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? -INFINITY : 0.f;
@@ -93,7 +110,7 @@ __global__ __launch_bounds__(256) void role_step_kernel(RoleStepArgs a) {
         for (int v = 0; v < VEC; ++v) e[v] = w[v];
       }
     };
-    constexpr int kAhead = 8;
+    constexpr int kAhead = kFew ? 16 : 8;
     int t = t0;
     for (; t + kAhead <= t1; t += kAhead) {
       float e[kAhead][VEC];
@@ -131,30 +148,28 @@ __global__ __launch_bounds__(256) void role_step_kernel(RoleStepArgs a) {
   if (a.S == 0) return;
   __syncthreads();
 
-  // logits[o] = sum_d pooled[d] * W[o][d]; wavefront w takes this workgroup's outputs w, w + 4, ...
-  const int h0 = blockIdx.z * a.hpb, h1 = min(h0 + a.hpb, a.Hkv);
-  const int n_out = h1 * 3;
-  for (int o = h0 * 3 + wave; o < n_out; o += 4) {
+  // logits[o] = sum_d pooled[d] * W[o][d]; wavefront w takes this workgroup's outputs w, w + n_waves, ...
+  for (int o = h0 * 3 + wave; o < n_out; o += n_waves) {
     float acc = 0.f;
     if (VEC > 1) {
       // VEC consecutive weights per lane and step (one 16-byte load)
       const char* wrow = static_cast<const char*>(a.weight) + (int64_t)o * a.dim * esz;
-      for (int d = lane * VEC; d < a.dim; d += 64 * VEC) {
-        float w[VEC];
-        if (kBf16) {
-          const uint4 raw = *reinterpret_cast<const uint4*>(wrow + d * 2);
-          const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
+      auto add_piece = [&](const uint4& raw, int d) {
+        const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
-          for (int v = 0; v < VEC; ++v) w[v] = bf16_bits_to_f32(uint16_t(u[(v >> 1) & 3] >> ((v & 1) * 16)));
-        } else {
-          const float4 raw = *reinterpret_cast<const float4*>(wrow + d * 4);
-          const float f[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) w[v] = f[v & 3];
+        for (int v = 0; v < VEC; ++v) {
+          const float w = kBf16 ? bf16_bits_to_f32(uint16_t(u[(v >> 1) & 3] >> ((v & 1) * 16))) : __uint_as_float(u[v & 3]);
+          acc = fmaf(pooled[d + v], w, acc);
         }
+      };
+      int d = lane * VEC;
+      if (kFew && o == h0 * 3 + wave) {
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) acc = fmaf(pooled[d + v], w[v], acc);
+        for (int i = 0; i < kPieces; ++i, d += 64 * VEC)
+          if (d < a.dim) add_piece(w_first[i], d);
       }
+#pragma unroll 4
+      for (; d < a.dim; d += 64 * VEC) add_piece(*reinterpret_cast<const uint4*>(wrow + d * esz), d);
     } else {
       for (int d = lane; d < a.dim; d += 64) acc = fmaf(pooled[d], load_elem<kBf16>(a.weight, (int64_t)o * a.dim + d), acc);
     }
@@ -237,23 +252,24 @@ extern "C" int nats_role_step(const void* x, const void* carry_in, const void* w
   // few chunks: a workgroup per role stream, so that the projection's rows are read side by side
   a.hpb = (S > 0 && S * B <= 32) ? 1 : (int)H_kv;
   dim3 grid((unsigned)(S > 0 ? S : 1), (unsigned)B, (unsigned)((H_kv + a.hpb - 1) / a.hpb));
-  auto launch = [&](auto kernel) -> int {
+  auto launch = [&](auto kernel, int threads) -> int {
     if (smem > 64 * 1024) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
       if (e != hipSuccess) return fail(NATS_ERR_LAUNCH, "%s: hipFuncSetAttribute(%zu bytes of LDS): %s", who, smem, hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(kernel, grid, dim3(256), smem, st, a);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, st, a);
     return NATS_OK;
   };
-  // 16-byte loads of x and of the projection weights when every row allows them
+  // 16-byte loads of x and of the projection weights when every row allows them; twice the threads for few chunks of many columns
   const int vec = dtype == NATS_DTYPE_BF16 ? 8 : 4;
   const bool wide = dim % vec == 0 && x_strides[0] % vec == 0 && x_strides[1] % vec == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(weight) % 16 == 0;
+  const bool many = a.hpb == 1 && dim > 256 * vec;
   int rc;
   if (dtype == NATS_DTYPE_BF16) {
-    rc = wide ? launch(role_step_kernel<true, 8>) : launch(role_step_kernel<true, 1>);
+    rc = !wide ? launch(role_step_kernel<true, 1, 256>, 256) : many ? launch(role_step_kernel<true, 8, 512>, 512) : launch(role_step_kernel<true, 8, 256>, 256);
   } else {
-    rc = wide ? launch(role_step_kernel<false, 4>) : launch(role_step_kernel<false, 1>);
+    rc = !wide ? launch(role_step_kernel<false, 1, 256>, 256) : many ? launch(role_step_kernel<false, 4, 512>, 512) : launch(role_step_kernel<false, 4, 256>, 256);
   }
   if (rc) return rc;
   NATS_CHECK_LAUNCH("role_step_kernel");
