@@ -280,8 +280,8 @@ class BaseNAtSAttentionLayer(AttentionLayer):
             cache._update_cache_x(carry, layer_id)
         if layer_id == 0:
             cache.cache_model[-1].settle()  # (as `NAtSCache.update` does)
-        qkv = qkv.view(B, 1, Hq + 2 * Hkv, D).transpose(1, 2)
-        output = layer.step_attention(qkv[:, :Hq], qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:], cos, sin, None, roles, self.sm_scale)
+        q, k, v = qkv.view(B, 1, Hq + 2 * Hkv, D).transpose(1, 2).split_with_sizes((Hq, Hkv, Hkv), 1)
+        output = layer.step_attention(q, k, v, cos, sin, None, roles, self.sm_scale)
         self._post_update(cache, 1)
         return ops.matvec(output.view(B, 1, Hq * D), wo)
 

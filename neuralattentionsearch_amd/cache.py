@@ -83,7 +83,7 @@ class NAtSChunkLayerCache:
         self._kept_share = None  # logical rows after the last first eviction / rows of the uncompacted cache
         self._append_call = None  # ops.CacheAppendCall / ops.EvictInplaceCall prepared for the present buffers
         self._inplace_call = None
-        self._inplace_params = None
+        self._inplace_params = self._inplace_facts = None
         self._planned = None  # (sequence number, roles, facts) of an eviction whose plan rode with the append of its rows
         self.reset_cache()
 
@@ -311,7 +311,8 @@ class NAtSChunkLayerCache:
             if wide is not None:
                 self._clean = None
                 self._buf_k, self._buf_v, self._buf_valid, self._buf_pos = wide
-                self._rows = max(self._rows, rows)
+                self._resolve()
+                self._n_rows = max(self._n_rows, rows)
                 return
         if self._clean is not None and rows > self._clean:
             # the cache extends into spare rows: the ones it takes now (all of them before the buffers are copied)
@@ -332,7 +333,8 @@ class NAtSChunkLayerCache:
             self._buf_valid = widen(self._buf_valid, 0)
             if self._buf_pos is not None:
                 self._buf_pos = widen(self._buf_pos, -1)
-        self._rows = max(self._rows, rows)
+        self._resolve()
+        self._n_rows = max(self._n_rows, rows)
 
     def _materialize_pending(self):
         """Writes [W zeros | K | pad] (nats_chunk_layer_cache.py:215-236) if the first prefill is still raw."""
@@ -382,19 +384,23 @@ class NAtSChunkLayerCache:
         end = start + x_len
         self._grow(math.ceil(end / self.chunk_size) * self.chunk_size)
         self._write_rows(key_states, value_states, start, end, plan_ahead=True)
-        return self._buf_k[:, :, :end], self._buf_v[:, :, :end]
+        return self._buf_k.narrow(2, 0, end), self._buf_v.narrow(2, 0, end)
 
     def _inplace_prepare(self, x_len: int, seen_after: int):
         """Parameter struct and prepared call of the in-place eviction that follows an update of x_len tokens, from the
         state as it stands between that update and its post_update; also the facts the struct was filled from."""
-        C, W = self.chunk_size, self.sliding_window_size
         roles, fill = self._roles, self.chunk_fill_size
         S, D = roles.shape[-1], self._buf_k.shape[3]
         params = self._inplace_params
         if params is None or params.D != D:
-            params = self._inplace_params = ops.evict_params(self.bsz, self.n_msks, D, C, W, S, 0, 0, 0, 0, 0, False, 0)
-        facts = (S, x_len, fill, int(seen_after == x_len), self.n_ctx_data, self._n_global_min, self.sliding_queue_tail, self._rows)
-        (params.S, params.x_len, params.fill, params.first, params.n_ctx_data, params.gmin, params.tail, params.n_alloc) = facts
+            params = self._inplace_params = ops.evict_params(self.bsz, self.n_msks, D, self.chunk_size, self.sliding_window_size, S,
+                                                             0, 0, 0, 0, 0, False, 0)
+            self._inplace_facts = None
+        self._resolve()  # (once: the names below are the numbers themselves)
+        facts = (S, x_len, fill, int(seen_after == x_len), self._n_ctx, self._gmin, self.sliding_queue_tail, self._n_rows)
+        if facts != self._inplace_facts:  # (a post_update finds what its update filled in)
+            (params.S, params.x_len, params.fill, params.first, params.n_ctx_data, params.gmin, params.tail, params.n_alloc) = facts
+            self._inplace_facts = facts
         call = self._inplace_call
         if call is None or not call.matches(self._buf_k, self._buf_v, self._buf_valid, self._buf_pos, S):
             if self._evict is None:
