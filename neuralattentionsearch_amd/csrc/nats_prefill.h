@@ -52,6 +52,9 @@ struct PrefillArgs {
 
 // Rows of K or V (or row limits) as a raw buffer of `bytes` bytes: reads beyond its end give zero, and a row is a scalar offset
 // beside a lane's own, where addresses per row would take two registers and vector arithmetic each.
+// A vector memory instruction may read a scalar register five wait states after a vector instruction wrote it at the earliest (the
+// v_readlane that brings a spilled scalar back, for one).  The compiler keeps that distance for its own instructions only, so every
+// assembly block has it inside, in front of its first transfer.
 struct RowBuffer {
   typedef int Words __attribute__((ext_vector_type(4)));
   static constexpr int kFlags = 0x00027000;  // last word of a raw buffer's descriptor
@@ -65,10 +68,10 @@ struct RowBuffer {
     static_assert(kBytes == 16 || kBytes == 4, "sizes a transfer can have here");
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (kBytes == 16) {
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds" ::"v"(lane_off), "s"(desc), "s"(lds_addr), "s"(row_off)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds" ::"v"(lane_off), "s"(desc), "s"(lds_addr), "s"(row_off)
                    : "memory", "m0");
     } else {
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, %3 offen lds" ::"v"(lane_off), "s"(desc), "s"(lds_addr), "s"(row_off)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dword %0, %1, %3 offen lds" ::"v"(lane_off), "s"(desc), "s"(lds_addr), "s"(row_off)
                    : "memory", "m0");
     }
 #endif
@@ -77,7 +80,7 @@ struct RowBuffer {
   __device__ __forceinline__ void to_lds_pair(uint32_t lds_addr, int lane_off0, int lane_off1, uint32_t row_off) const {
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile(
-        "s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %2, %4 offen lds\n\t"
+        "s_mov_b32 m0, %3\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %2, %4 offen lds\n\t"
         "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %4 offen lds" ::"v"(lane_off0), "v"(lane_off1), "s"(desc), "s"(lds_addr),
         "s"(row_off)
         : "memory", "m0", "scc");
@@ -88,7 +91,7 @@ struct RowBuffer {
 #if defined(__HIP_DEVICE_COMPILE__)
     uint32_t row;
     asm volatile(
-        "s_mov_b32 m0, %6\n\ts_mov_b32 %0, %7\n\tbuffer_load_dwordx4 %1, %5, %0 offen lds\n\t"
+        "s_mov_b32 m0, %6\n\ts_mov_b32 %0, %7\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %5, %0 offen lds\n\t"
         "s_add_u32 m0, m0, 0x400\n\ts_add_u32 %0, %0, %8\n\tbuffer_load_dwordx4 %2, %5, %0 offen lds\n\t"
         "s_add_u32 m0, m0, 0x400\n\ts_add_u32 %0, %0, %8\n\tbuffer_load_dwordx4 %3, %5, %0 offen lds\n\t"
         "s_add_u32 m0, m0, 0x400\n\ts_add_u32 %0, %0, %8\n\tbuffer_load_dwordx4 %4, %5, %0 offen lds"

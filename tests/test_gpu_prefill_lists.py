@@ -49,3 +49,26 @@ def test_rows_beyond_32_bit_offsets(C):
     got = ops.prefill_attention(q, spread[0], spread[1], roles, C, W)
     # (a role per token: the far rows are walked by granules there, in another order)
     assert torch.equal(got, want) if C > 1 else (got.float() - want.float()).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("dtype,D,C,L", [
+    (torch.bfloat16, 128, 64, 3073), (torch.bfloat16, 128, 64, 3135), (torch.bfloat16, 128, 32, 3001), (torch.bfloat16, 128, 1, 3001),
+    (torch.bfloat16, 64, 64, 3100), (torch.bfloat16, 32, 64, 4097), (torch.bfloat16, 64, 8, 3001),
+    (torch.bfloat16, 256, 64, 65), (torch.bfloat16, 256, 64, 111), (torch.bfloat16, 256, 8, 273),
+    (torch.bfloat16, 128, 64, 33), (torch.bfloat16, 64, 64, 173), (torch.bfloat16, 32, 16, 70),
+    (torch.float32, 32, 64, 33), (torch.float32, 64, 64, 173), (torch.float32, 128, 8, 1001),
+])
+def test_rows_behind_the_last_one_are_not_read(dtype, D, C, L):
+    """K and V as the first L rows of longer streams: whatever lies behind them (here: NaN, which a probability of zero would
+    pass on) is the same to the result as zeros."""
+    from neuralattentionsearch_amd import ops
+    say("rows behind the last one", dtype, D, C, L)
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q = torch.randn(1, 8, L, D, generator=g, device="cuda", dtype=dtype)
+    longer = torch.randn(2, 1, 2, L + 128, D, generator=g, device="cuda", dtype=dtype)
+    roles = to_dev(draw_roles(C, 1, 2, math.ceil(L / C)))
+    outs = []
+    for tail in (0.0, float("nan")):
+        longer[:, :, :, L:] = tail
+        outs.append(ops.prefill_attention(q, longer[0, :, :, :L], longer[1, :, :, :L], roles, C, 256))
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
