@@ -285,14 +285,15 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   // ---- wavefront 0 asks for the tile summaries of the first kEarly * 64 key tiles before anything else is requested:
   // memory operations complete in the order of their issue, so the wait for these (a trip to L2) does not include
   // the Q rows (a trip to HBM), which stay in flight while the visit list is built and the first tiles are requested.
-  // Packed tiles: the same with the granule summaries, where the granules [near_g0, g_end_group] and the gathered tiles fit one
-  // early list; wavefront 1 asks for the cache rows of the first gathered tiles.
+  // Packed tiles: the same with the granule summaries, a lane per tile that the granules [near_g0, g_end_group] lie in, where those
+  // are at most 64 and the gathered tiles fit the same list; wavefront 1 asks for the cache rows of the first gathered tiles.
   constexpr int kEarly = kPacked ? 4 : 8;
   constexpr int kIdsAhead = 5;  // gathered tiles whose cache rows are known before the first step
   const int near_g0 = near_row0 / kGranule;
   const int g_end_group = (a.base + rlast_group) / kGranule;
   const int n_near = g_end_group - near_g0 + 1;
-  const bool early_list = kPacked && n_near <= kEarly * kWave && (!kFar || n_far_tiles + (n_near + kGranPerTile - 1) / kGranPerTile + 1 <= kWin - 1);
+  const int near_t0 = near_g0 / kGranPerTile, near_t1 = g_end_group / kGranPerTile;
+  const bool early_list = kPacked && near_t1 - near_t0 < kWave && (!kFar || n_far_tiles + (n_near + kGranPerTile - 1) / kGranPerTile + 1 <= kWin - 1);
   const bool early_ids = kFar && early_list && a.n_split == 1 && n_far_tiles > 0;
   int2 tl_early[kEarly];
   if (!kPacked && wave == 0) {
@@ -300,10 +301,10 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
     for (int j = 0; j < kEarly; ++j) tl_early[j] = tl[min(j * kWave + lane, kt_end_group)];
   }
   if (early_list && wave == 0) {
-    const int2* gl = a.gran_lim + (int64_t)ks * a.Tk * kGranPerTile;
+    const int2* gl = a.gran_lim + ((int64_t)ks * a.Tk + min(near_t0 + lane, near_t1)) * kGranPerTile;
+    static_assert(!kPacked || kEarly == kGranPerTile, "the granules of a lane's tile");
 #pragma unroll
-    for (int j = 0; j < kEarly; ++j)
-      if (j * kWave < n_near) tl_early[j] = gl[min(near_g0 + j * kWave + lane, g_end_group)];
+    for (int u = 0; u < kEarly; ++u) tl_early[u] = gl[u];
   }
   // (gathered tile t of the list: its first entry in the lists of long-lived rows)
   auto far_start = [&](int t) { return t < n_far_ta ? t * kTile : a.long_cap + b_lo + (t - n_far_ta) * kTile; };
@@ -735,12 +736,15 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   };
   if (early_list && wave == 0) {
     // (one trip to memory between the start of the workgroup and its list; in the windows below two, one after the other, and both
-    // behind the Q rows)
+    // behind the Q rows.  Both list the granules in one order, the first ones of up to 64 visible tiles, then their second ones and
+    // so on: the order of the keys is the order of the sums, so a query's result does not depend on which of them built its list.)
     if (kFar) list_far(0, n_far_tiles);
     int n_plain = 0, n_mask = 0;
 #pragma unroll
-    for (int j = 0; j < kEarly; ++j)
-      if (j * kWave < n_near) sort_granule(near_g0 + j * kWave + lane, j * kWave + lane < n_near, tl_early[j], n_plain, n_mask);
+    for (int u = 0; u < kEarly; ++u) {
+      const int g = (near_t0 + lane) * kGranPerTile + u;
+      sort_granule(g, g >= near_g0 && g <= g_end_group, tl_early[u], n_plain, n_mask);
+    }
     list_granules(kFar ? n_far_tiles : 0, n_plain, n_mask);
   }
   if (early_ids && wave == 1) {

@@ -29,6 +29,26 @@ def test_list_edges(monkeypatch, heads, L, D, C, W, p):
     run_case(1, heads[0], heads[1], L, D, C, W, torch.bfloat16, seed=L, p=p)
 
 
+@pytest.mark.parametrize("D,C,W,Hq,Hkv", [(128, 32, 256, 4, 1), (64, 16, 64, 8, 2), (32, 32, 64, 2, 1), (128, 64, 128, 1, 1)])
+def test_lists_of_either_kind_hold_the_same_order(monkeypatch, D, C, W, Hq, Hkv):
+    """A prompt alone (its granules are listed in one trip) and behind 4096 tokens that slide out of the window (they are not:
+    tile summaries first): the same keys in the same order, so the same bytes, for the queries that no longer see the others."""
+    from neuralattentionsearch_amd import ops
+    say("lists of either kind", D, C, W, Hq, Hkv)
+    monkeypatch.setenv("NATS_PREFILL_SPLIT", "0")
+    monkeypatch.setenv("NATS_PREFILL_SHORT", "0")
+    L, P = 3000, 4096
+    g = torch.Generator(device="cuda").manual_seed(D + C)
+    q = torch.randn(1, Hq, P + L, D, generator=g, device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.randn(1, Hkv, P + L, D, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    roles = to_dev(draw_roles(C, 1, Hkv, math.ceil((P + L) / C)))
+    roles[:, :, :P // C] = 2  # sliding window
+    both = ops.prefill_attention(q, k, v, roles, C, W)
+    alone = ops.prefill_attention(q[:, :, P:], k[:, :, P:], v[:, :, P:], roles[:, :, P // C:].contiguous(), C, W)
+    first = -(-(W + C) // 256) * 256  # (a workgroup's query tiles share one list)
+    assert torch.equal(both[:, :, P + first:], alone[:, :, first:])
+
+
 @pytest.mark.parametrize("C", [64, 32, 1])
 def test_rows_beyond_32_bit_offsets(C):
     """K and V as every 720000th element group of a 4.3 GB buffer: row 2983 on lies beyond 2^32 bytes."""
