@@ -10,12 +10,15 @@
 // input dtype, the logits are accumulated in fp32 and rounded to the input dtype, the bias is added in that
 // dtype.  (fp32 summation order differs from a library GEMM, so logits agree with it to rounding, not bit
 // for bit; the roles are the exact argmax of the logits this kernel writes.)
+#include <type_traits>
+
 #include "nats_common.h"
 
 namespace nats {
 
 int launch_role_scan(const uint8_t* roles, int64_t n_streams, int64_t S, int64_t W, int64_t C, int64_t* end_idx,
                      int32_t* vis_lim, int32_t* first_global, hipStream_t st);
+int device_cu_count();
 
 struct RoleStepArgs {
   const void* x;        // [B, L, dim]
@@ -93,7 +96,7 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
     float acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? -INFINITY : 0.f;
-    // kAhead rows are requested before the first of them is used (the sums keep the order of the rows)
+    // sixteen or eight rows are requested before the first of them is used (the sums keep the order of the rows)
     auto load_row = [&](int t, float (&e)[VEC]) {
       const char* row = xb + (b * a.xs_b + t * a.xs_l + d) * esz;
       if (VEC == 1) {
@@ -110,17 +113,21 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
         for (int v = 0; v < VEC; ++v) e[v] = w[v];
       }
     };
-    constexpr int kAhead = kFew ? 16 : 8;
     int t = t0;
-    for (; t + kAhead <= t1; t += kAhead) {
-      float e[kAhead][VEC];
+    auto take_rows = [&](auto ahead) {
+      constexpr int kAhead = decltype(ahead)::value;
+      for (; t + kAhead <= t1; t += kAhead) {
+        float e[kAhead][VEC];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) load_row(t + u, e[u]);
+        for (int u = 0; u < kAhead; ++u) load_row(t + u, e[u]);
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u)
+        for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf(acc[v], e[u][v]) : acc[v] + e[u][v];
-    }
+          for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf(acc[v], e[u][v]) : acc[v] + e[u][v];
+      }
+    };
+    if (kFew) take_rows(std::integral_constant<int, 16>{});
+    take_rows(std::integral_constant<int, 8>{});
     for (; t < t1; ++t) {
       float e[VEC];
       load_row(t, e);
@@ -168,7 +175,9 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
         for (int i = 0; i < kPieces; ++i, d += 64 * VEC)
           if (d < a.dim) add_piece(w_first[i], d);
       }
-#pragma unroll 4
+      // (unrolled for fp32 only, whose rows are twice as many pieces: 1024 chunks of eight rows at dim 2048 26.1 -> 22.6 us, bf16 7.8 -> 8.3)
+      constexpr int kTogether = kBf16 ? 1 : 4;
+#pragma unroll kTogether
       for (; d < a.dim; d += 64 * VEC) add_piece(*reinterpret_cast<const uint4*>(wrow + d * esz), d);
     } else {
       for (int d = lane; d < a.dim; d += 64) acc = fmaf(pooled[d], load_elem<kBf16>(a.weight, (int64_t)o * a.dim + d), acc);
@@ -260,16 +269,20 @@ extern "C" int nats_role_step(const void* x, const void* carry_in, const void* w
     hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, st, a);
     return NATS_OK;
   };
-  // 16-byte loads of x and of the projection weights when every row allows them; twice the threads for few chunks of many columns
+  // 16-byte loads of x and of the projection weights when every row allows them; twice the threads for few workgroups with many columns
   const int vec = dtype == NATS_DTYPE_BF16 ? 8 : 4;
   const bool wide = dim % vec == 0 && x_strides[0] % vec == 0 && x_strides[1] % vec == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(weight) % 16 == 0;
-  const bool many = a.hpb == 1 && dim > 256 * vec;
+  // (up to a workgroup per compute unit: beyond, two of 256 threads on one cover each other's trips and fewer threads idle.  256 / 512
+  // threads, us, bf16 at dim 4096 by workgroups: chunks of 64 rows 17.6 / 14.1 (33), 22.4 / 17.1 (128), 24.2 / 25.5 (256), 35.1 / 40.3
+  // (384), 44.8 / 56.7 (1024, 32 streams); of 8 rows 7.1 / 6.2, 7.2 / 6.3, 8.3 / 6.6, 10.3 / 14.8, 13.4 / 22.5.  fp32 at dim 2560: 14.4 /
+  // 10.1, 20.9 / 15.7, 27.2 / 25.6, 38.6 / 37.5, 31.4 / 31.3; of 8 rows 5.5 / 4.7, 5.7 / 4.9, 5.8 / 5.1, 7.4 / 8.7, 8.2 / 12.1.)
+  const bool few_wide = S > 0 && a.hpb == 1 && dim > 256 * vec && S * B * H_kv <= device_cu_count();
   int rc;
   if (dtype == NATS_DTYPE_BF16) {
-    rc = !wide ? launch(role_step_kernel<true, 1, 256>, 256) : many ? launch(role_step_kernel<true, 8, 512>, 512) : launch(role_step_kernel<true, 8, 256>, 256);
+    rc = !wide ? launch(role_step_kernel<true, 1, 256>, 256) : few_wide ? launch(role_step_kernel<true, 8, 512>, 512) : launch(role_step_kernel<true, 8, 256>, 256);
   } else {
-    rc = !wide ? launch(role_step_kernel<false, 1, 256>, 256) : many ? launch(role_step_kernel<false, 4, 512>, 512) : launch(role_step_kernel<false, 4, 256>, 256);
+    rc = !wide ? launch(role_step_kernel<false, 1, 256>, 256) : few_wide ? launch(role_step_kernel<false, 4, 512>, 512) : launch(role_step_kernel<false, 4, 256>, 256);
   }
   if (rc) return rc;
   NATS_CHECK_LAUNCH("role_step_kernel");

@@ -74,6 +74,24 @@ def test_role_step_streams(dtype, merge_max, C, dim, H, lens):
         pre, seen = total % C, seen + n
 
 
+@pytest.mark.parametrize("dtype,C,dim,H,B,lens", [
+    # 512 threads: the last of the eight weight pieces partial, missing, or with more behind it; rows in sixteens, eights and ones
+    (torch.bfloat16, 64, 2056, 8, 1, [301, 40]), (torch.bfloat16, 8, 2560, 3, 2, [29, 3, 1]), (torch.bfloat16, 32, 5120, 2, 1, [95]),
+    (torch.float32, 16, 1028, 8, 1, [100, 13]), (torch.float32, 64, 2056, 1, 2, [190]), (torch.float32, 8, 2560, 4, 1, [50]),
+    # more workgroups than compute units: one stream with many chunks, many streams with few
+    (torch.bfloat16, 8, 2560, 1, 1, [2403]), (torch.bfloat16, 16, 2056, 32, 1, [16 * 12]), (torch.float32, 8, 1028, 1, 2, [1203]),
+])
+def test_role_step_wide_rows(dtype, C, dim, H, B, lens):
+    say("role step wide", dtype, C, dim, H, B, lens)
+    g = torch.Generator().manual_seed(C + dim)
+    w = (torch.randn(H * 3, dim, generator=g) * (4.0 / dim ** 0.5)).to(dtype)
+    pre, carry, seen = 0, None, 0
+    for n in lens:
+        x = torch.randn(B, n, dim, generator=g).to(dtype)
+        carry = check_call(x, w, C, 4 * C, pre, carry, False, 0.1, seen < C, dtype)
+        pre, seen = (pre + n) % C, seen + n
+
+
 def test_role_step_strided_input_and_errors():
     from neuralattentionsearch_amd import ops
     say("role step strided")
