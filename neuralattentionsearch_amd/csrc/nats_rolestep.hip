@@ -62,7 +62,7 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float v) {
 // per thread (16-byte loads when the rows allow it, else 1).  Few chunks of many columns are bound by the trips to memory
 // behind one another (THREADS = 512): twice the threads, sixteen rows to a trip, and the weights of a wavefront's first output
 // requested before the rows (bf16, dim 4096: five chunks of 64 rows 18.5 -> 15.4 us, the token that closes a chunk 7.6 -> 6.1, a role
-// per token 6.0 -> 5.3; fp32, five chunks 30.2 -> 20.1).  With 256 threads, many chunks or 2048 columns, both lose (32768 tokens
+// per token 6.0 -> 5.3; fp32, five chunks 25.5 -> 14.5).  With 256 threads, many chunks or 2048 columns, both lose (32768 tokens
 // 62.2 -> 63.7, 4 x 300 tokens of 2048 at chunk 32 13.9 -> 15.3).
 template <bool kBf16, int VEC, int THREADS>
 __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
@@ -93,10 +93,13 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
     for (int i = 0; i < kPieces; ++i) w_first[i] = *reinterpret_cast<const uint4*>(wrow + min((i * 64 + lane) * VEC, a.dim - VEC) * esz);
   }
   for (int d = tid * VEC; d < a.dim; d += THREADS * VEC) {
-    float acc[VEC];
+    // (fp32 rows are summed in a tree per trip and the trips in fp64: rows added one after the other in fp32 end further from the exact
+    // mean than torch's sum in blocks, chunks of 64 twice as far, of 1024 five times.  All rows in fp64 take 17 us where this takes 10.)
+    typedef std::conditional_t<kBf16, float, double> Sum;
+    Sum acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? -INFINITY : 0.f;
-    // sixteen or eight rows are requested before the first of them is used (the sums keep the order of the rows)
+    // sixteen or eight rows are requested before the first of them is used (the sums of bf16 rows keep the order of the rows)
     auto load_row = [&](int t, float (&e)[VEC]) {
       const char* row = xb + (b * a.xs_b + t * a.xs_l + d) * esz;
       if (VEC == 1) {
@@ -120,10 +123,21 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
         float e[kAhead][VEC];
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) load_row(t + u, e[u]);
+        if (kBf16 || a.merge_max) {
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u)
+          for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-          for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf(acc[v], e[u][v]) : acc[v] + e[u][v];
+            for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf((float)acc[v], e[u][v]) : acc[v] + e[u][v];
+        } else {
+#pragma unroll
+          for (int w = kAhead / 2; w >= 1; w /= 2)
+#pragma unroll
+            for (int u = 0; u < w; ++u)
+#pragma unroll
+              for (int v = 0; v < VEC; ++v) e[u][v] += e[u + w][v];
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) acc[v] += e[0][v];
+        }
       }
     };
     if (kFew) take_rows(std::integral_constant<int, 16>{});
@@ -132,16 +146,16 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
       float e[VEC];
       load_row(t, e);
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf(acc[v], e[v]) : acc[v] + e[v];
+      for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf((float)acc[v], e[v]) : acc[v] + e[v];
     }
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
-      float stat, tail_max = acc[v];
+      float stat, tail_max = (float)acc[v];
       if (!a.merge_max) {
-        stat = round_elem<kBf16>(acc[v] * inv_c);  // power-of-two C: x / C is exact, so both torch forms agree
+        stat = round_elem<kBf16>((float)(acc[v] * inv_c));  // power-of-two C: x / C is exact, so both torch forms agree
         if (with_carry) stat = round_elem<kBf16>(load_elem<kBf16>(a.carry_in, (int64_t)b * a.dim + d + v) + stat);
       } else {
-        stat = acc[v];
+        stat = (float)acc[v];
         if (with_carry) stat = fmaxf(stat, load_elem<kBf16>(a.carry_in, (int64_t)b * a.dim + d + v));
         if (padded) stat = fmaxf(stat, 0.f);
       }
@@ -276,7 +290,7 @@ extern "C" int nats_role_step(const void* x, const void* carry_in, const void* w
   // (up to a workgroup per compute unit: beyond, two of 256 threads on one cover each other's trips and fewer threads idle.  256 / 512
   // threads, us, bf16 at dim 4096 by workgroups: chunks of 64 rows 17.6 / 14.1 (33), 22.4 / 17.1 (128), 24.2 / 25.5 (256), 35.1 / 40.3
   // (384), 44.8 / 56.7 (1024, 32 streams); of 8 rows 7.1 / 6.2, 7.2 / 6.3, 8.3 / 6.6, 10.3 / 14.8, 13.4 / 22.5.  fp32 at dim 2560: 14.4 /
-  // 10.1, 20.9 / 15.7, 27.2 / 25.6, 38.6 / 37.5, 31.4 / 31.3; of 8 rows 5.5 / 4.7, 5.7 / 4.9, 5.8 / 5.1, 7.4 / 8.7, 8.2 / 12.1.)
+  // 9.9, 20.9 / 16.0, 27.2 / 26.1, 38.6 / 37.5, 31.4 / 31.3; of 8 rows 5.5 / 4.8, 5.7 / 4.9, 5.8 / 5.1, 7.4 / 8.7, 8.2 / 12.1.)
   const bool few_wide = S > 0 && a.hpb == 1 && dim > 256 * vec && S * B * H_kv <= device_cu_count();
   int rc;
   if (dtype == NATS_DTYPE_BF16) {
