@@ -189,10 +189,18 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
         for (int i = 0; i < kPieces; ++i, d += 64 * VEC)
           if (d < a.dim) add_piece(w_first[i], d);
       }
-      // (unrolled for fp32 only, whose rows are twice as many pieces: 1024 chunks of eight rows at dim 2048 26.1 -> 22.6 us, bf16 7.8 -> 8.3)
-      constexpr int kTogether = kBf16 ? 1 : 4;
+      // (Four pieces at a time where a wavefront has several outputs, and for fp32, whose rows are twice as many pieces.  bf16, 32 streams, 128
+      // chunks of 64 rows at dim 4096 91 -> 69 us, fp32, 8 streams, 1024 chunks of eight at dim 2048 26.1 -> 22.6; bf16, one stream 7.8 -> 8.3.)
+      auto add_rest = [&](auto together) {
+        constexpr int kTogether = decltype(together)::value;
 #pragma unroll kTogether
-      for (; d < a.dim; d += 64 * VEC) add_piece(*reinterpret_cast<const uint4*>(wrow + d * esz), d);
+        for (; d < a.dim; d += 64 * VEC) add_piece(*reinterpret_cast<const uint4*>(wrow + d * esz), d);
+      };
+      if (kBf16 && a.hpb == 1) {
+        add_rest(std::integral_constant<int, 1>{});
+      } else {
+        add_rest(std::integral_constant<int, 4>{});
+      }
     } else {
       for (int d = lane; d < a.dim; d += 64) acc = fmaf(pooled[d], load_elem<kBf16>(a.weight, (int64_t)o * a.dim + d), acc);
     }
