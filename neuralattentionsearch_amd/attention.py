@@ -56,6 +56,24 @@ def _plain_execution(x: torch.Tensor, weights) -> bool:
             and not torch.compiler.is_compiling() and not nn.modules.module._has_any_global_hook())
 
 
+def _segment_roles_pay(chunks: int, streams: int, chunk_size: int, dim: int, dtype: torch.dtype) -> bool:
+    """Whether pooling and projecting `chunks` chunks (of all sequences) in the role kernel takes no longer on the GPU than the
+    torch ops and the library's product.  Up to 32 chunks the kernel pools every chunk once per stream, with more every workgroup
+    reads the whole weight for one chunk's dot products; the ops copy and pad the hidden states.
+
+    GPU us, kernel / ops, bf16, dim 4096: 5 chunks of 64, 8 streams 15 / 33; 33 of 8, 8 streams 18 / 27, 16 streams 30 / 27, 32 streams
+    54 / 28; 128 of 64, 32 streams 70 / 78; 512 of 8, 32 streams 99 / 51; 1024 of 8, 8 streams 56 / 71; 1024 of 64, 32 streams 246 / 436; fp32 34 / 29
+    (33 of 8, 32 streams), 255 / 821.  Over 1770 sizes (4 to 64 streams, chunks of 8 to 128, 3 to 4096 of them, dims 1024 to 4096) the kernel
+    is 5 % slower in two that this takes, and 15 % faster in 44 that it leaves."""
+    if chunks <= 32:
+        return chunks * streams * (16 + chunk_size) * dim <= 150_000_000
+    if dtype == torch.bfloat16:
+        kernel, most = streams * max(320, 160 + 1.05 * chunks), 13_500_000
+    else:
+        kernel, most = streams * max(110, 80 + 0.45 * chunks), 6_400_000
+    return (kernel - (chunks - 20) * chunk_size) * dim <= most
+
+
 class AttentionLayer(nn.Module):
     """Projections and head bookkeeping (base_attention.py:13-137)."""
 
@@ -332,7 +350,8 @@ class BaseNAtSChunkAttentionLayer(BaseNAtSAttentionLayer):
         ops and the library product they stand in for are up to eleven (a turn of 301 tokens at dim 4096 waits for all of
         them).  None where something of it is replaced, watched or not what the kernel computes: a mean over a chunk size
         that is a power of two (dividing by it is exact, so the statistics are those of the torch ops; the fp32 sums of the
-        projection run in another order).  From chunks of 8 on: below, the product over all chunks is the library's work."""
+        projection run in another order) from 8 on, in sizes at which the kernel is no slower (`_segment_roles_pay`), rows of whole 16
+        bytes."""
         C, H = self.chunk_size, self.n_msks
         proj = self._modules.get("proj_layer")
         if (type(cache) is not NAtSCache or cache.chunk_size != C or C < 8 or C & (C - 1)
@@ -342,7 +361,9 @@ class BaseNAtSChunkAttentionLayer(BaseNAtSAttentionLayer):
         B, _, dim = x.shape
         if (not _plain_execution(x, (w,)) or not x.is_cuda or x.device != w.device or x.dtype != w.dtype
                 or x.dtype not in (torch.bfloat16, torch.float32) or x.stride(-1) != 1 or not w.is_contiguous() or w.shape != (3 * H, dim)
-                or H > 256 or (dim + 3 * H) * 4 > 160 * 1024 or not 0 < B <= 65535 or not self._segment_as_defined(cache)):
+                or H > 256 or (dim + 3 * H) * 4 > 160 * 1024 or not 0 < B <= 65535 or not self._segment_as_defined(cache)
+                or not _segment_roles_pay(B * -(-(pre_fill + x.shape[1]) // C), H, C, dim, x.dtype)
+                or (dim * x.element_size() | x.stride(0) * x.element_size() | x.stride(1) * x.element_size() | x.data_ptr() | w.data_ptr()) % 16):
             return None
         carry = None
         if pre_fill:

@@ -22,7 +22,7 @@ def build(dtype, dim, C, seed=0):
     return m.to(dtype).eval().requires_grad_(False)
 
 
-def roles_of(m, x, fill, general, monkeypatch):
+def roles_of(m, x, fill, general, monkeypatch, heads=4):
     """One hot roles and carry of a segment behind `fill` tokens of an open chunk; which way it went."""
     C = m.chunk_size
     cache = NAtSCache(2 * C, C)
@@ -34,9 +34,9 @@ def roles_of(m, x, fill, general, monkeypatch):
             mp.setattr(LlamaNAtSChunkAttentionLayer, "_segment_roles", lambda *a: None)
         with torch.no_grad():
             if fill:
-                k = torch.zeros(x.shape[0], 4, fill, m.head_dim, device="cuda", dtype=x.dtype)
+                k = torch.zeros(x.shape[0], heads, fill, m.head_dim, device="cuda", dtype=x.dtype)
                 m._sample_for_token_info_values_inference(x[:, :fill], 0, cache)
-                cache.update(k, k, 0, {"token_states_info": m.one_hot_values.to(x).reshape(1, 1, 1, -1).expand(x.shape[0], 4, 1, -1)})
+                cache.update(k, k, 0, {"token_states_info": m.one_hot_values.to(x).reshape(1, 1, 1, -1).expand(x.shape[0], heads, 1, -1)})
                 cache.post_update(0, fill)
             out = m._sample_for_token_info_values_inference(x[:, fill:], fill, cache)
     return out, cache.get_nats_cached_x_in_chunk(0), bool(calls)
@@ -65,6 +65,24 @@ def test_agrees_with_the_torch_ops(monkeypatch, dtype, dim, C, B, fill, L):
         assert carry.shape == carry_want.shape
         tol = 2 ** -8 if dtype == torch.bfloat16 else 64 * 6e-8
         assert ((carry.float() - carry_want.float()).abs() <= tol * carry_want.float().abs().clamp_min(2 ** -6)).all()
+
+
+@pytest.mark.parametrize("dtype,dim,heads,C,B,L,shift,fused", [
+    (torch.bfloat16, 1024, 32, 8, 1, 8 * 32, 0, True), (torch.bfloat16, 4096, 32, 32, 1, 32 * 30, 0, False),    # up to 32 chunks
+    (torch.bfloat16, 4096, 8, 8, 3, 8 * 11, 0, True), (torch.bfloat16, 4096, 32, 8, 3, 8 * 11, 0, False),       # 33 chunks
+    (torch.bfloat16, 4096, 8, 8, 1, 8 * 600, 0, True), (torch.bfloat16, 4096, 32, 8, 1, 8 * 600, 0, False),     # many
+    (torch.float32, 4096, 16, 8, 1, 8 * 300, 0, True), (torch.float32, 4096, 32, 8, 1, 8 * 300, 0, False),
+    (torch.bfloat16, 1024, 8, 8, 1, 100, 1, False), (torch.float32, 1024, 8, 8, 1, 100, 1, False),              # rows off 16 bytes
+    (torch.bfloat16, 1028, 4, 8, 1, 100, 0, False),
+])
+def test_where_the_kernel_pays(monkeypatch, dtype, dim, heads, C, B, L, shift, fused):
+    say("segment roles pay", dtype, dim, heads, C, B, L, shift)
+    with torch.device("cuda"):
+        m = LlamaNAtSChunkAttentionLayer(dim=dim, n_heads=heads, n_kv_heads=heads, layer_id=0, local_seq_max_length=2 * C, chunk_size=C)
+    m = m.to(dtype).eval().requires_grad_(False)
+    x = torch.randn(B * L * dim + shift, device="cuda", dtype=dtype)[shift:].view(B, L, dim)
+    got, _, went = roles_of(m, x, 0, False, monkeypatch, heads)
+    assert went == fused and got.shape == (B, heads, -(-L // C), 3)
 
 
 @pytest.mark.parametrize("C", [8, 64, 512])
