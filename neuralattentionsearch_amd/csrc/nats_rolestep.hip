@@ -64,7 +64,8 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float v) {
 // requested before the rows (bf16, dim 4096: five chunks of 64 rows 18.5 -> 15.4 us, the token that closes a chunk 7.6 -> 6.1, a role
 // per token 6.0 -> 5.3; fp32, five chunks 25.5 -> 14.5).  With 256 threads, many chunks or 2048 columns, both lose (32768 tokens
 // 62.2 -> 63.7, 4 x 300 tokens of 2048 at chunk 32 13.9 -> 15.3).
-template <bool kBf16, int VEC, int THREADS>
+// TOGETHER: the pieces of a weight row that a wavefront requests before it uses the first (see nats_role_step).
+template <bool kBf16, int VEC, int THREADS, int TOGETHER>
 __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
   extern __shared__ float pooled[];  // [dim] statistic of this chunk, then [Hkv * 3] logits behind it
   float* logit_s = pooled + a.dim;
@@ -99,7 +100,8 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
     Sum acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? -INFINITY : 0.f;
-    // sixteen or eight rows are requested before the first of them is used (the sums of bf16 rows keep the order of the rows)
+    // sixteen or eight rows are requested before the first of them is used, of the last few four, two and one (the sums of bf16 rows
+    // keep the order of the rows)
     auto load_row = [&](int t, float (&e)[VEC]) {
       const char* row = xb + (b * a.xs_b + t * a.xs_l + d) * esz;
       if (VEC == 1) {
@@ -142,11 +144,10 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
     };
     if (kFew) take_rows(std::integral_constant<int, 16>{});
     take_rows(std::integral_constant<int, 8>{});
-    for (; t < t1; ++t) {
-      float e[VEC];
-      load_row(t, e);
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) acc[v] = a.merge_max ? fmaxf((float)acc[v], e[v]) : acc[v] + e[v];
+    if (t < t1) {
+      take_rows(std::integral_constant<int, 4>{});
+      take_rows(std::integral_constant<int, 2>{});
+      take_rows(std::integral_constant<int, 1>{});
     }
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
@@ -189,18 +190,8 @@ __global__ __launch_bounds__(THREADS) void role_step_kernel(RoleStepArgs a) {
         for (int i = 0; i < kPieces; ++i, d += 64 * VEC)
           if (d < a.dim) add_piece(w_first[i], d);
       }
-      // (Four pieces at a time where a wavefront has several outputs, and for fp32, whose rows are twice as many pieces.  bf16, 32 streams, 128
-      // chunks of 64 rows at dim 4096 91 -> 69 us, fp32, 8 streams, 1024 chunks of eight at dim 2048 26.1 -> 22.6; bf16, one stream 7.8 -> 8.3.)
-      auto add_rest = [&](auto together) {
-        constexpr int kTogether = decltype(together)::value;
-#pragma unroll kTogether
-        for (; d < a.dim; d += 64 * VEC) add_piece(*reinterpret_cast<const uint4*>(wrow + d * esz), d);
-      };
-      if (kBf16 && a.hpb == 1) {
-        add_rest(std::integral_constant<int, 1>{});
-      } else {
-        add_rest(std::integral_constant<int, 4>{});
-      }
+#pragma unroll TOGETHER
+      for (; d < a.dim; d += 64 * VEC) add_piece(*reinterpret_cast<const uint4*>(wrow + d * esz), d);
     } else {
       for (int d = lane; d < a.dim; d += 64) acc = fmaf(pooled[d], load_elem<kBf16>(a.weight, (int64_t)o * a.dim + d), acc);
     }
@@ -300,11 +291,17 @@ extern "C" int nats_role_step(const void* x, const void* carry_in, const void* w
   // (384), 44.8 / 56.7 (1024, 32 streams); of 8 rows 7.1 / 6.2, 7.2 / 6.3, 8.3 / 6.6, 10.3 / 14.8, 13.4 / 22.5.  fp32 at dim 2560: 14.4 /
   // 9.9, 20.9 / 16.0, 27.2 / 26.1, 38.6 / 37.5, 31.4 / 31.3; of 8 rows 5.5 / 4.8, 5.7 / 4.9, 5.8 / 5.1, 7.4 / 8.7, 8.2 / 12.1.)
   const bool few_wide = S > 0 && a.hpb == 1 && dim > 256 * vec && S * B * H_kv <= device_cu_count();
+  // four pieces of a weight row together for rows of more than four pieces (a loop over fewer only gets longer by it), of bf16 where a
+  // wavefront has several outputs.  One / four, us: bf16, 32 streams, 128 chunks of 64 rows at dim 4096 91 / 69, one stream 7.8 / 8.3; fp32, 8
+  // streams, 1024 chunks of eight at dim 2048 26.1 / 22.6; a role per token of 8 x 26, 32 streams, bf16 at dim 72 13.6 / 15.2, 1024 19.9 / 20.9.
+  const bool four = dim > 4 * 64 * vec && !(dtype == NATS_DTYPE_BF16 && a.hpb == 1);
   int rc;
   if (dtype == NATS_DTYPE_BF16) {
-    rc = !wide ? launch(role_step_kernel<true, 1, 256>, 256) : few_wide ? launch(role_step_kernel<true, 8, 512>, 512) : launch(role_step_kernel<true, 8, 256>, 256);
+    rc = !wide ? launch(role_step_kernel<true, 1, 256, 1>, 256) : few_wide ? launch(role_step_kernel<true, 8, 512, 1>, 512)
+         : four ? launch(role_step_kernel<true, 8, 256, 4>, 256) : launch(role_step_kernel<true, 8, 256, 1>, 256);
   } else {
-    rc = !wide ? launch(role_step_kernel<false, 1, 256>, 256) : few_wide ? launch(role_step_kernel<false, 4, 512>, 512) : launch(role_step_kernel<false, 4, 256>, 256);
+    rc = !wide ? launch(role_step_kernel<false, 1, 256, 1>, 256) : few_wide ? launch(role_step_kernel<false, 4, 512, 4>, 512)
+         : four ? launch(role_step_kernel<false, 4, 256, 4>, 256) : launch(role_step_kernel<false, 4, 256, 1>, 256);
   }
   if (rc) return rc;
   NATS_CHECK_LAUNCH("role_step_kernel");
