@@ -28,18 +28,18 @@ namespace nats {
 constexpr int kF32Rows = 32;      // query rows of a workgroup, keys of a tile
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// In LDS: Q (one copy per workgroup), and per wavefront one K tile and its row limits.
-template <int D>
+// In LDS: Q (one copy per workgroup), and per wavefront one K tile and its row limits.  Four wavefronts at head dim 128 have 80 KiB to
+// the byte, half of a compute unit's: their Q rows are permuted like K's instead of padded, and the row limits stay in registers.
+template <int D, int kWaves>
 struct F32Layout {
-  static constexpr int kQPitch = D + 4;   // floats; rows of the 16-byte reads fall into different banks
-  static constexpr int kOPitch = D + 1;   // floats per query row of a wavefront's partial result
-  static constexpr int kWaveFloats = kF32Rows * D + kWave;  // K tile, row limits
-  static size_t smem_bytes(int n_waves) {
-    const size_t q = sizeof(float) * (kF32Rows * kQPitch + n_waves * kWaveFloats);
-    const size_t merge = sizeof(float) * n_waves * kF32Rows * (kOPitch + 2);
-    return q > merge ? q : merge;  // (the partial results take their place)
-  }
+  static constexpr bool kTight = D == 128 && kWaves == 4;
+  static constexpr int kQPitch = kTight ? D : D + 4;  // floats; rows of the 16-byte reads fall into different banks
+  static constexpr int kOPitch = D + 1;               // floats per query row of a wavefront's partial result
+  static constexpr int kWaveFloats = kF32Rows * D + (kTight ? 0 : kWave);  // K tile, row limits
+  static constexpr int kOperands = kF32Rows * kQPitch + kWaves * kWaveFloats, kMerge = kWaves * kF32Rows * (kOPitch + 2);
+  static constexpr int kBytes = (int)sizeof(float) * (kOperands > kMerge ? kOperands : kMerge);  // (the partial results take their place)
 };
+static_assert(2 * F32Layout<128, 4>::kBytes <= 160 * 1024, "two workgroups of four wavefronts on a compute unit");
 
 template <int DT>
 struct F32Vec;
@@ -72,7 +72,7 @@ __device__ __forceinline__ typename F32Vec<DT>::type row_part(const RowBuffer& b
 
 template <int D, int kWaves>
 __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_kernel(PrefillArgs a, int blk_first, int n_blk, int paired) {
-  using Lay = F32Layout<D>;
+  using Lay = F32Layout<D, kWaves>;
   constexpr int HD = D / 2;   // head dimensions per half wavefront
   constexpr int DT = D / 32;  // 32-row tiles of O^T
   typedef typename F32Vec<DT>::type VecV;
@@ -106,7 +106,6 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
   float* k_lds = smem + kF32Rows * Lay::kQPitch + wave * Lay::kWaveFloats;
   int* lim_lds = reinterpret_cast<int*>(k_lds + kF32Rows * D);
   const uint32_t k_addr = lds_address(k_lds);
-  const float* q_lds = smem + l32 * Lay::kQPitch + hl * 4;
 
   f32x16 oacc[DT];
 #pragma unroll
@@ -172,6 +171,10 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
     }
   };
   auto k_frag = [&](int i) { return *reinterpret_cast<const f32x4*>(k_lds + l32 * D + ((2 * i + hl) ^ swz(l32)) * 4); };
+  auto q_frag = [&](int i) {
+    const int chunk = 2 * i + hl;
+    return *reinterpret_cast<const f32x4*>(smem + l32 * Lay::kQPitch + (Lay::kTight ? chunk ^ swz(l32) : chunk) * 4);
+  };
   const int voff = (hl * 4 * (int)a.vs_l + l32 * DT) * 4;  // bytes
 
   // ---- Q goes to LDS (the B operand of the scores); the first tile summaries are requested before it and the first K tile
@@ -193,34 +196,39 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
 #pragma unroll
   for (int j = 0; j < kQSteps; ++j) {
     const int i = min(j * n_waves * kWave + (int)threadIdx.x, kQPieces - 1);
-    *reinterpret_cast<f32x4*>(smem + i / (D / 4) * Lay::kQPitch + i % (D / 4) * 4) = qp_reg[j];
+    const int row = i / (D / 4), chunk = i % (D / 4);
+    *reinterpret_cast<f32x4*>(smem + row * Lay::kQPitch + (Lay::kTight ? chunk ^ swz(row) : chunk) * 4) = qp_reg[j];
   }
   __syncthreads();
   while (t >= 0) {
     const int k0 = t * kF32Rows;
     wait_transfers();  // K of this tile has landed in LDS
     __builtin_amdgcn_sched_barrier(0);
-    // V rows of this tile (rows past the end repeat the last one: their probabilities are 0) and the row limits
+    // V rows of this tile (rows past the end are zeros, and so are their probabilities) and the row limits
     VecV vreg[16];
     {
       const RowBuffer buf = tile_buffer(vp, a.vs_l, k0);
 #pragma unroll
       for (int i = 0; i < 16; ++i) vreg[i] = row_part<DT>(buf, voff, (8 * (i / 4) + i % 4) * (int)a.vs_l * 4);
     }
-    if (masked) lim_lds[lane] = lim[min(k0 + l32, a.N - 1)];
+    int lim_reg = 0;
+    if (masked) {
+      lim_reg = lim[min(k0 + l32, a.N - 1)];
+      if (!Lay::kTight) lim_lds[lane] = lim_reg;
+    }
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- S^T = K Q^T ----
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
-    f32x4 kn = k_frag(0), qn = *reinterpret_cast<const f32x4*>(q_lds);
+    f32x4 kn = k_frag(0), qn = q_frag(0);
 #pragma unroll
     for (int i = 0; i < HD / 4; ++i) {
       const f32x4 kv = kn, qv = qn;
       if (i + 1 < HD / 4) {
         kn = k_frag(i + 1);
-        qn = *reinterpret_cast<const f32x4*>(q_lds + (i + 1) * 8);
+        qn = q_frag(i + 1);
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qv[e], s, 0, 0, 0);
@@ -238,8 +246,14 @@ __global__ __launch_bounds__(kWaves * kWave, D <= 64 ? 4 : 2) void prefill_f32_k
       const int key0 = k0 - a.base;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int4 l4 = *reinterpret_cast<const int4*>(lim_lds + 8 * g + 4 * hl);
-        const int lv[4] = {l4.x, l4.y, l4.z, l4.w};
+        int lv[4];
+        if (Lay::kTight) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) lv[e] = __shfl(lim_reg, 8 * g + 4 * hl + e);
+        } else {
+          const int4 l4 = *reinterpret_cast<const int4*>(lim_lds + 8 * g + 4 * hl);
+          lv[0] = l4.x, lv[1] = l4.y, lv[2] = l4.z, lv[3] = l4.w;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = key0 + 8 * g + 4 * hl + e;  // (rows past the end are later than every query)
@@ -331,35 +345,39 @@ static int launch_d(const PrefillArgs& a, hipStream_t st) {
   const int blk_first = a.r_begin / kF32Rows, n_blk = (a.r_end - 1) / kF32Rows - blk_first + 1;
   const int64_t n_wg = (int64_t)a.B * a.Hq * n_blk;
   NATS_REQUIRE(n_wg < (int64_t(1) << 31), NATS_ERR_BAD_SHAPE, "prefill: grid too large");
-  // How many wavefronts share a block's tiles.  Eight (two workgroups per compute unit at head dims 32 and 64, one at 128) make
-  // the heaviest block, which ends the launch, short; four (three workgroups or more) waste less on the ends of a workgroup.
-  // 8 / 4 wavefronts, even and sparse roles, by workgroups per compute unit:
-  //   D = 64   up to 2: 27 / 28, 24 / 24 us (1.4), 36 / 38, 30 / 30 (2).  2.75: 44 / 42, 39 / 34.  3.25: 73 / 70, 54 / 50.  4: 63 / 69, 50 / 55.
-  //            5.3: 94 / 100, 67 / 69.  6.5: 126 / 127, 87 / 84.  11: 125 / 117, 107 / 101.  26: 456 / 442, 302 / 282.
-  //   D = 32   1.4: 20 / 21, 18 / 18.  2: 23 / 24, 20 / 20.  2.66: 33 / 33, 28 / 25.  4: 36 / 34, 30 / 27.  13: 150 / 139, 97 / 83.
-  //   D = 128  eight always: four are one workgroup per compute unit as well (105 / 111, 75 / 81 at 2.66).
+  // How many wavefronts share a block's tiles.  Eight make the heaviest block, which ends the launch, short; four waste less on the
+  // ends of a workgroup, more of them the shorter the lists.  LDS holds two workgroups of eight or three of four on a compute unit at
+  // head dim 64 (42 KB each; registers would allow a fourth), so just above two per compute unit and between three and six four leave more
+  // of a round empty than eight do, around three less.  At head dim 128 it holds one of eight or two of four.  Four / eight, by workgroups
+  // per compute unit, for lists of up to 24 and of more blocks (even and sparse roles):
+  //   D = 64   up to 2: 0.98 to 1.06 / 1.00 to 1.09.  2.2: - / 1.05 to 1.12.  2.5 to 2.75: 0.76 to 0.92 / -.  3: - / 0.86 to 1.12.  4 to 4.4: 0.97 /
+  //            0.99 to 1.09.  5 to 6: 0.88 to 1.00 / 0.99 to 1.08.  8 and more: 0.86 to 0.91 / 0.91 to 1.02.
+  //   D = 32   four / eight in us: 1.4: 21 / 20, 18 / 18.  2: 24 / 23, 20 / 20.  2.66: 33 / 33, 25 / 28.  4: 34 / 36, 27 / 30.  13: 139 / 150, 83 / 97.
+  //   D = 128  up to 2: 0.81 to 1.06 / 0.89 to 1.17.  2.1 to 2.75: 0.86 to 1.03 / 0.90, of more than 64 blocks 1.10 to 1.13.  3: - / 0.97 to 1.07, of more
+  //            than 64 0.99 to 1.04.  4 to 6: 0.75 to 0.87 / 0.86 to 0.98.  8 and more: 0.74 to 0.82 / 0.80 to 0.94 (64 heads, 1024 tokens 162 -> 141 us).
   const int n_cu = device_cu_count();
-  const bool few = D == 128 || n_wg <= 2 * (int64_t)n_cu || (D == 64 && 2 * n_wg > 7 * (int64_t)n_cu && n_wg <= 6 * (int64_t)n_cu);
+  auto up_to = [&](int half_rounds) { return 2 * n_wg <= half_rounds * (int64_t)n_cu; };  // (halves of a workgroup per compute unit)
+  const bool few = up_to(4) || (D == 64 && n_blk > 24 && (up_to(5) || (!up_to(7) && up_to(12)))) || (D == 128 && n_blk > 64 && up_to(6));
   // Between one and two workgroups per compute unit: workgroups i and i + n_cu share one, so the lightest blocks come last, in
   // falling order, beside the lightest of the others, and the heaviest have a compute unit to themselves (8 heads of 64, 2048
   // tokens 39.0 -> 35.8 us, 1400 31.6 -> 26.1, 4 heads, 3000 tokens 41.4 -> 34.0).
   const int per_round = (int)(n_cu / ((int64_t)a.B * a.Hq));  // blocks of a head that take every compute unit once
   const int paired = per_round > 0 && n_blk > per_round && n_blk <= 2 * per_round ? per_round : 0;
-  constexpr int kMany = D == 128 ? 8 : 4;
+  constexpr int kBytes8 = F32Layout<D, 8>::kBytes, kBytes4 = F32Layout<D, 4>::kBytes;
   if (!configured[dev]) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)F32Layout<D>::smem_bytes(8));
+                                       kBytes8);
     if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, kMany>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)F32Layout<D>::smem_bytes(kMany));
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_f32_kernel<D, 4>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kBytes4);
     if (e != hipSuccess) return fail(NATS_ERR_LAUNCH, "prefill_f32_kernel: LDS: %s", hipGetErrorString(e));
     configured[dev] = true;
   }
   const dim3 grid((unsigned)n_wg);
   if (few) {
-    hipLaunchKernelGGL((prefill_f32_kernel<D, 8>), grid, dim3(8 * kWave), F32Layout<D>::smem_bytes(8), st, a, blk_first, n_blk, paired);
+    hipLaunchKernelGGL((prefill_f32_kernel<D, 8>), grid, dim3(8 * kWave), kBytes8, st, a, blk_first, n_blk, paired);
   } else {
-    hipLaunchKernelGGL((prefill_f32_kernel<D, kMany>), grid, dim3(kMany * kWave), F32Layout<D>::smem_bytes(kMany), st, a, blk_first, n_blk, paired);
+    hipLaunchKernelGGL((prefill_f32_kernel<D, 4>), grid, dim3(4 * kWave), kBytes4, st, a, blk_first, n_blk, paired);
   }
   NATS_CHECK_LAUNCH("prefill_f32_kernel");
   return NATS_OK;

@@ -62,6 +62,37 @@ def test_segments_over_a_filled_cache(C, W, lens):
         st.post_update(n)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,Hkv,C,W,first,n", [
+    (96, 12, 64, 128, 0, 130), (96, 12, 5, 10, 0, 161), (96, 12, 64, 128, 200, 97), (128, 4, 8, 16, 67, 98),  # four wavefronts: 3.75, 4.5, 3, 4 per compute unit
+    (6, 3, 64, 128, 0, 2400), (6, 3, 64, 128, 0, 2049),   # long lists, 1.76 and 1.52: eight
+])
+def test_wavefronts_of_a_workgroup(Hq, Hkv, C, W, first, n, D):
+    """Both forms of the kernel, from empty and over cached rows, with tiles that are masked row by row."""
+    from neuralattentionsearch_amd import ops
+    from neuralattentionsearch_amd.cache import NAtSChunkLayerCache
+    say("f32 wavefronts", Hq, Hkv, C, W, first, n, D)
+    B = 2
+    if not first:
+        run_case(B, Hq, Hkv, n, D, C, W, torch.float32, seed=n)
+        return
+    g = torch.Generator().manual_seed(n)
+    cache = NAtSChunkLayerCache(B, Hkv, W, chunk_size=C, device="cuda")
+    st = orc.ChunkCacheOracle(B=B, H=Hkv, W=W, C=C)
+    for si, m in enumerate((first, n)):
+        q, k, v = (torch.randn(B, h, m, D, generator=g) for h in (Hq, Hkv, Hkv))
+        roles = draw_roles(si, B, Hkv, math.ceil((cache.chunk_fill_size + m) / C), p=(0.3, 0.3, 0.4), first_global=si == 0)
+        if (cache.chunk_fill_size + m) % C:
+            roles[:, :, -1] = 0
+        cache.update(k.cuda(), v.cuda(), orc.one_hot_roles(roles).cuda())
+        ko, vo = st.update(k, v, roles)
+        if si:
+            want = orc.masked_attention(q, ko, vo, st.generate_mask(m))
+            assert np.abs(cache.segment_attention(q.cuda()).cpu().numpy() - want.numpy()).max() <= 1e-5
+        cache.post_update(m)
+        st.post_update(m)
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.3])
 def test_scales_that_are_not_positive(scale):
     from neuralattentionsearch_amd import ops
