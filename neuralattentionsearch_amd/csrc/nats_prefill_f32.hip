@@ -347,17 +347,17 @@ static int launch_d(const PrefillArgs& a, hipStream_t st) {
   NATS_REQUIRE(n_wg < (int64_t(1) << 31), NATS_ERR_BAD_SHAPE, "prefill: grid too large");
   // How many wavefronts share a block's tiles.  Eight make the heaviest block, which ends the launch, short; four waste less on the
   // ends of a workgroup, more of them the shorter the lists.  LDS holds two workgroups of eight or three of four on a compute unit at
-  // head dim 64 (42 KB each; registers would allow a fourth), so just above two per compute unit and between three and six four leave more
+  // head dim 64 (76 and 42 KB; registers would allow a fourth), so just above two per compute unit and between three and six four leave more
   // of a round empty than eight do, around three less.  At head dim 128 it holds one of eight or two of four.  Four / eight, by workgroups
-  // per compute unit, for lists of up to 24 and of more blocks (even and sparse roles):
-  //   D = 64   up to 2: 0.98 to 1.06 / 1.00 to 1.09.  2.2: - / 1.05 to 1.12.  2.5 to 2.75: 0.76 to 0.92 / -.  3: - / 0.86 to 1.12.  4 to 4.4: 0.97 /
-  //            0.99 to 1.09.  5 to 6: 0.88 to 1.00 / 0.99 to 1.08.  8 and more: 0.86 to 0.91 / 0.91 to 1.02.
+  // per compute unit, for heads of up to 20 and of more blocks (even and sparse roles):
+  //   D = 64   up to 2: 0.98 to 1.06 / 1.00 to 1.09.  2.2: - / 1.05 to 1.12.  2.5 to 2.75: 0.76 to 0.84 / 0.90 to 0.92.  3: - / 0.86 to 1.12.  4 to 4.4:
+  //            0.97 / 0.99 to 1.09.  5 to 6: 0.88 to 0.91 / 0.98 to 1.08.  8 and more: 0.86 to 0.91 / 0.91 to 1.02.
   //   D = 32   four / eight in us: 1.4: 21 / 20, 18 / 18.  2: 24 / 23, 20 / 20.  2.66: 33 / 33, 25 / 28.  4: 34 / 36, 27 / 30.  13: 139 / 150, 83 / 97.
-  //   D = 128  up to 2: 0.81 to 1.06 / 0.89 to 1.17.  2.1 to 2.75: 0.86 to 1.03 / 0.90, of more than 64 blocks 1.10 to 1.13.  3: - / 0.97 to 1.07, of more
-  //            than 64 0.99 to 1.04.  4 to 6: 0.75 to 0.87 / 0.86 to 0.98.  8 and more: 0.74 to 0.82 / 0.80 to 0.94 (64 heads, 1024 tokens 162 -> 141 us).
+  //   D = 128  up to 2: 0.81 to 1.06 / 0.89 to 1.17.  2.1 to 2.6: 0.86 to 0.91 / 0.89 to 1.13.  3: - / 0.97 to 1.07.  4 to 6: 0.75 to 0.85 / 0.86 to
+  //            0.98.  8 and more: 0.74 to 0.82 / 0.80 to 0.94 (64 heads, 1024 tokens 165 -> 141 us).
   const int n_cu = device_cu_count();
   auto up_to = [&](int half_rounds) { return 2 * n_wg <= half_rounds * (int64_t)n_cu; };  // (halves of a workgroup per compute unit)
-  const bool few = up_to(4) || (D == 64 && n_blk > 24 && (up_to(5) || (!up_to(7) && up_to(12)))) || (D == 128 && n_blk > 64 && up_to(6));
+  const bool few = up_to(4) || (n_blk > 20 && (D == 64 ? up_to(5) || (!up_to(7) && up_to(12)) : D == 128 && up_to(6)));
   // Between one and two workgroups per compute unit: workgroups i and i + n_cu share one, so the lightest blocks come last, in
   // falling order, beside the lightest of the others, and the heaviest have a compute unit to themselves (8 heads of 64, 2048
   // tokens 39.0 -> 35.8 us, 1400 31.6 -> 26.1, 4 heads, 3000 tokens 41.4 -> 34.0).
