@@ -47,7 +47,6 @@ struct PrefillArgs {
   const int32_t* long_before;  // [streams, 2, n_gran + 1] entries of A / of B before every granule
   const int32_t* long_alive;   // [streams, n_rtile] first entry of B that a query of the 64-token region tile may see
   int long_cap, n_gran, n_rtile, t_long;
-  int rows64;  // a stream's rows of K or V reach beyond 32-bit byte offsets
 };
 
 // Rows of K or V (or row limits) as a raw buffer of `bytes` bytes: reads beyond its end give zero, and a row is a scalar offset

@@ -209,8 +209,8 @@ constexpr int kFarTileFlag = 1 << 29;     // ... the entry is a tile of long-liv
 // first kind, padding) into tiles that go through the element mask.  The softmax does not care about the order
 // of the keys, so nothing else changes; without it a tile with one visible 16- or 32-row chunk costs a whole tile.
 // (kMode: 0 whole tiles, 1 packed tiles, 2 packed tiles with the rows far behind a query gathered from the lists of
-// long-lived rows)
-template <int D, bool kUniform, int kMode>
+// long-lived rows; kRows64: a stream's rows of K or V reach beyond 32-bit byte offsets)
+template <int D, bool kUniform, int kMode, bool kRows64>
 __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned char* smem_raw, int bid, int split, int ks,
                                                   int hg, int rank) {
   constexpr bool kPacked = kMode != 0;
@@ -362,18 +362,23 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
   const RowBuffer kbuf(kp, (uint32_t)((int64_t)(a.N - 1) * a.ks_l + D) * 2), vbuf(vp, (uint32_t)((int64_t)(a.N - 1) * a.vs_l + D) * 2);
   // This wavefront's share of the tile whose rows begin at row0 (a granule: of its own rows), to the tile buffer at byte `tile`.
   // A step's transfers stand in front of its matrix instructions, so they are kept short: one offset from the stream's first
-  // row (where a stream's rows do not reach beyond 32 bits of it) and the LDS address, both scalar.
+  // row (kRows64: the address of these) and the LDS address, both scalar.
+  constexpr int kRowGroup = kPacked ? kGranule : kTile;
   auto issue_rows = [&](const RowBuffer& buf, int64_t stride, const int (&off)[DMA_PER_WAVE], uint32_t tile, int row0) {
     if (N_INST < kPrefillWaves && wave >= N_INST) return;
     uint32_t row_off = (uint32_t)row0 * ((uint32_t)stride * 2);
-    if (!kFar && __builtin_expect(a.rows64, 0)) {
-      const RowBuffer near(static_cast<const uint16_t*>(buf.base) + (int64_t)row0 * stride, ((min(kTile, a.N - row0) - 1) * (int)stride + D) * 2);
-#pragma unroll
-      for (int j = 0; j < DMA_PER_WAVE; ++j) near.template to_lds<16>(lds_wave + tile + j * kWave * 16, off[j], 0);
-    } else if (DMA_PER_WAVE == 2) {
-      buf.to_lds_pair(lds_wave + tile, off[0], off[DMA_PER_WAVE - 1], row_off);
+    RowBuffer rows = buf;
+    if (kRows64) {
+      // a buffer that begins with these rows; only the last ones of a stream are fewer than a transfer takes
+      const int last0 = (a.N - 1) & ~(kRowGroup - 1);
+      rows = RowBuffer(static_cast<const uint16_t*>(buf.base) + (int64_t)row0 * stride,
+                       (uint32_t)((row0 < last0 ? kRowGroup - 1 : a.N - 1 - last0) * (int)stride + D) * 2);
+      row_off = 0;
+    }
+    if (DMA_PER_WAVE == 2) {
+      rows.to_lds_pair(lds_wave + tile, off[0], off[DMA_PER_WAVE - 1], row_off);
     } else {
-      buf.template to_lds<16>(lds_wave + tile, off[0], row_off);
+      rows.template to_lds<16>(lds_wave + tile, off[0], row_off);
     }
   };
   static_assert(DMA_PER_WAVE <= 2, "two transfers of a wavefront at most");
@@ -397,7 +402,11 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
       const int n = max(0, min(sm.posk[slot][row], a.N - 1));  // (padding entries hold INT_MAX and the limit -1)
       const int chunk = is_v ? pos ^ v_swizzle(row) : pos ^ (row % OCT);
       const uint32_t dst = lds_wave + tile + j * kWave * 16;
-      buf.template to_lds<16>(dst, (int)((uint32_t)n * ((uint32_t)stride * 2) + chunk * 16), 0);
+      if (kRows64) {
+        lds_transfer16(static_cast<const uint16_t*>(buf.base) + (int64_t)n * stride + chunk * 8, dst);
+      } else {
+        buf.template to_lds<16>(dst, (int)((uint32_t)n * ((uint32_t)stride * 2) + chunk * 16), 0);
+      }
     }
   };
   // (packed tiles; id0: the first field of the list entry, with its flags; mine: this wavefront's granule of the tile -- its eight
@@ -1104,14 +1113,14 @@ __device__ __forceinline__ void map_balanced(const PrefillArgs& a, int* counts, 
 // earlier take more of it.  The tile loop exists twice in the code, once for each kind of workgroup, so that the
 // loop around the pooled one costs the other nothing.
 // (kBalance: an instantiation of its own, since the map's code before the tile loop costs the loop 5 % in the plain one)
-template <int D, bool kUniform, int kMode, bool kBalance>
+template <int D, bool kUniform, int kMode, bool kBalance, bool kRows64>
 __global__ __launch_bounds__(kPrefillWaves * kWave) void prefill_mfma_kernel(PrefillArgs args) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   int bid = blockIdx.x;
   if constexpr (kBalance) {
     int ks, hg, rank;
     map_balanced(args, reinterpret_cast<int*>(smem_raw), bid, ks, hg, rank);
-    prefill_mfma_item<D, kUniform, kMode>(args, smem_raw, bid, 0, ks, hg, rank);
+    prefill_mfma_item<D, kUniform, kMode, kRows64>(args, smem_raw, bid, 0, ks, hg, rank);
     return;
   }
   int split = 0;  // which share of the tile list (n_split > 1)
@@ -1122,7 +1131,7 @@ __global__ __launch_bounds__(kPrefillWaves * kWave) void prefill_mfma_kernel(Pre
   if (args.pool_ranks == 0 || bid < (args.n_qg - args.pool_ranks) * args.B * args.Hkv * args.n_hg) {
     int ks, hg, rank;
     map_workgroup(args, bid, ks, hg, rank);
-    prefill_mfma_item<D, kUniform, kMode>(args, smem_raw, bid, split, ks, hg, rank);
+    prefill_mfma_item<D, kUniform, kMode, kRows64>(args, smem_raw, bid, split, ks, hg, rank);
     return;
   }
   // Pooled query groups wait in one queue per XCD (that of their stream, heaviest first; every counter in a 128-byte
@@ -1172,7 +1181,7 @@ __global__ __launch_bounds__(kPrefillWaves * kWave) void prefill_mfma_kernel(Pre
     q = q_now;
     const int sl = t % n_x;
     const int ks = a.xcd_mode ? q + 8 * (sl / a.n_hg) : sl / a.n_hg;
-    prefill_mfma_item<D, kUniform, kMode>(a, smem_raw, bid, split, ks, sl % a.n_hg, a.n_qg - a.pool_ranks + t / n_x);
+    prefill_mfma_item<D, kUniform, kMode, kRows64>(a, smem_raw, bid, split, ks, sl % a.n_hg, a.n_qg - a.pool_ranks + t / n_x);
     __syncthreads();  // the output staging of this item and the ticket are read before the next item writes LDS
   }
 }
@@ -1616,21 +1625,29 @@ static int launch_prefill_wide(const PrefillArgs& a, int64_t n_wg, hipStream_t s
   return NATS_OK;
 }
 
-template <int D, bool kUniform, int kMode, bool kBalance = false>
-static int launch_prefill_mfma(const PrefillArgs& a, int64_t n_wg, hipStream_t st) {
+template <int D, bool kUniform, int kMode, bool kBalance, bool kRows64>
+static int launch_prefill_rows(const PrefillArgs& a, int64_t n_wg, hipStream_t st) {
   static bool configured[kMaxDevices] = {};  // per instantiation; the attribute is set once per device
   const size_t smem = sizeof(PrefillSmem<D>);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return fail(NATS_ERR_LAUNCH, "prefill: no current device");
   if (!configured[dev]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma_kernel<D, kUniform, kMode, kBalance>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma_kernel<D, kUniform, kMode, kBalance, kRows64>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return fail(NATS_ERR_LAUNCH, "hipFuncSetAttribute(%zu bytes of LDS): %s", smem, hipGetErrorString(e));
     configured[dev] = true;
   }
-  hipLaunchKernelGGL((prefill_mfma_kernel<D, kUniform, kMode, kBalance>), dim3((unsigned)n_wg), dim3(kPrefillWaves * kWave), smem, st, a);
+  hipLaunchKernelGGL((prefill_mfma_kernel<D, kUniform, kMode, kBalance, kRows64>), dim3((unsigned)n_wg), dim3(kPrefillWaves * kWave), smem, st, a);
   NATS_CHECK_LAUNCH("prefill_mfma_kernel");
   return NATS_OK;
+}
+
+// (Rows beyond 32-bit byte offsets have instantiations of their own: as a branch in every transfer their addresses put 150 scalars of the
+// packed kernels into vector lanes, 16384 tokens at chunk 32, 32 / 8 heads of 64 219 -> 214 us without.  Far rows cost them little: the same
+// call over rows 300000 apart 223 us, at chunk 1 and head dim 128 368 beside 362.)
+template <int D, bool kUniform, int kMode, bool kBalance = false>
+static int launch_prefill_mfma(const PrefillArgs& a, bool rows64, int64_t n_wg, hipStream_t st) {
+  return rows64 ? launch_prefill_rows<D, kUniform, kMode, kBalance, true>(a, n_wg, st) : launch_prefill_rows<D, kUniform, kMode, kBalance, false>(a, n_wg, st);
 }
 
 int device_cu_count() {
@@ -1780,7 +1797,7 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   a.qt_first = a.r_begin / kTile; a.qt_last = (a.r_end - 1) / kTile;
   const int64_t n_qt = a.qt_last - a.qt_first + 1;
   a.scale = sm_scale;
-  a.rows64 = ((g.N - 1) * std::max(a.ks_l, a.vs_l) + g.D) * 2 >= (int64_t(1) << 32);
+  const bool rows64 = ((g.N - 1) * std::max(a.ks_l, a.vs_l) + g.D) * 2 >= (int64_t(1) << 32);
   a.hpw = 1; a.qpw = 1; a.n_hg = 1; a.n_qg = (int)n_qt; a.xcd_mode = 0;
 
   // bf16 at head dim 256 (rows that 16-byte transfers can take; other layouts go to the plain kernel)
@@ -1852,7 +1869,7 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   // long-lived rows instead, row by row (NATS_PREFILL_FAR=0 in the environment walks every granule, for comparison).
   // (Chunks of a granule and more: a visible granule is visible as a whole there, and its transfer from one base
   // address is cheaper than a gathered one; measured 10 % slower at chunk 32.)
-  if (packed && g.C < kGranule && use_far_rows() && !a.rows64) {
+  if (packed && g.C < kGranule && use_far_rows()) {
     a.t_long = (int)long_row_threshold(g.W);
     if (int rc = launch_long_rows(w, g.B * g.H_kv, g.N, g.base, g.W, st)) return rc;
     a.long_rows = w.long_rows; a.long_lim = w.long_lim; a.long_before = w.long_before; a.long_alive = w.long_alive;
@@ -1860,8 +1877,8 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
   }
   // (head dim -> instantiation)
 #define NATS_PREFILL_BY_D(UNI, MODE, PA, NWG)                                                  \
-  (g.D == 32 ? launch_prefill_mfma<32, UNI, MODE>(PA, NWG, st)                                 \
-             : g.D == 64 ? launch_prefill_mfma<64, UNI, MODE>(PA, NWG, st) : launch_prefill_mfma<128, UNI, MODE>(PA, NWG, st))
+  (g.D == 32 ? launch_prefill_mfma<32, UNI, MODE>(PA, rows64, NWG, st)                                 \
+             : g.D == 64 ? launch_prefill_mfma<64, UNI, MODE>(PA, rows64, NWG, st) : launch_prefill_mfma<128, UNI, MODE>(PA, rows64, NWG, st))
   auto launch_packed = [&](const PrefillArgs& pa, int64_t n) {
     if (pa.long_rows) return NATS_PREFILL_BY_D(true, 2, pa, n);
     return NATS_PREFILL_BY_D(true, 1, pa, n);
@@ -1900,8 +1917,8 @@ int launch_segment(const char* who, const SegmentShape& g, const void* q, const 
       hpw == 4 && n_cu > 0 && n_wg > n_cu && n_wg < 4 * n_cu && ns > 1 && ns <= kBalanceStreams && ns * a.Tk <= kBalanceTiles &&
       (a.heavy_first = balance_threshold(g.D, ns, g.base, g.x_len, n_wg, n_cu, packed)) > 0) {
 #define NATS_PREFILL_BALANCED(MODE)                                                                  \
-  (g.D == 32 ? launch_prefill_mfma<32, true, MODE, true>(a, n_wg, st)                                \
-             : g.D == 64 ? launch_prefill_mfma<64, true, MODE, true>(a, n_wg, st) : launch_prefill_mfma<128, true, MODE, true>(a, n_wg, st))
+  (g.D == 32 ? launch_prefill_mfma<32, true, MODE, true>(a, rows64, n_wg, st)                                \
+             : g.D == 64 ? launch_prefill_mfma<64, true, MODE, true>(a, rows64, n_wg, st) : launch_prefill_mfma<128, true, MODE, true>(a, rows64, n_wg, st))
     if (!packed) return NATS_PREFILL_BALANCED(0);
     return a.long_rows ? NATS_PREFILL_BALANCED(2) : NATS_PREFILL_BALANCED(1);
 #undef NATS_PREFILL_BALANCED
