@@ -4,9 +4,11 @@
 Tolerance 2e-2 as for every bf16 prefill; the two layouts of one input hold the same rows, so their outputs are the same bytes."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
+from oracle import nats_oracle as orc
 from tests.gpu_util import draw_roles, say, to_dev
 from tests.test_gpu_prefill import run_case
 
@@ -14,12 +16,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("L,D,C,W,p", [
-    (4095, 128, 64, 256, (0.96, 0.02, 0.02)),   # 64 entries, of which a step opens the second group for nothing
-    (4161, 128, 64, 256, (0.96, 0.02, 0.02)),   # 66
-    (8300, 64, 64, 128, (0.97, 0.01, 0.02)),    # three groups
+    (4095, 128, 64, 256, (0.96, 0.02, 0.02)),   # 61 entries of whole tiles
+    (4161, 128, 64, 256, (0.96, 0.02, 0.02)),   # 65
+    (8300, 64, 64, 128, (0.97, 0.01, 0.02)),    # 126
     (4096, 128, 32, 256, (0.4, 0.3, 0.3)),      # the last query group walks 256 granules: the early list
     (4112, 128, 32, 256, (0.4, 0.3, 0.3)),      # 257: tile summaries first
-    (4300, 32, 16, 32, (0.9, 0.05, 0.05)),      # four groups of packed entries
+    (4300, 32, 16, 32, (0.9, 0.05, 0.05)),      # 62 and 63 packed entries
     (4200, 128, 1, 16, (0.5, 0.25, 0.25)),      # gathered tiles, more than the five known ahead
     (700, 128, 1, 256, (0.1, 0.5, 0.4)),        # fewer
 ])
@@ -27,6 +29,44 @@ pytestmark = pytest.mark.gpu
 def test_list_edges(monkeypatch, heads, L, D, C, W, p):
     monkeypatch.setenv("NATS_PREFILL_SPLIT", "0")  # one workgroup walks a whole list
     run_case(1, heads[0], heads[1], L, D, C, W, torch.bfloat16, seed=L, p=p)
+
+
+def list_entries(rows, packed):
+    """Entries of the list of a query group, from its rows of the mask [queries, keys]: whole tiles somebody sees, or 16-row granules in
+    fours, those that nobody masks among themselves."""
+    step = 16 if packed else 64
+    parts = np.pad(rows, ((0, 0), (0, -rows.shape[1] % step))).reshape(len(rows), -1, step)
+    seen = parts.any((0, 2))
+    if not packed:
+        return int(seen.sum())
+    plain = int(parts.all((0, 2)).sum())
+    return plain // 4 + -(-(int(seen.sum()) - plain // 4 * 4) // 4)
+
+
+@pytest.mark.parametrize("L,D,C,heads,p,entries", [
+    (64 * 64, 128, 64, (4, 1), (1.0, 0.0, 0.0), 64), (64 * 66, 64, 64, (4, 1), (1.0, 0.0, 0.0), 66),  # the second group of 64 opened for nothing, for two
+    (8711, 32, 64, (4, 1), (0.97, 0.01, 0.02), 135),
+    (64 * 64, 128, 16, (4, 1), (1.0, 0.0, 0.0), 64), (64 * 65, 64, 16, (4, 1), (1.0, 0.0, 0.0), 65),
+    (9000, 32, 16, (4, 1), (0.96, 0.02, 0.02), 136), (9000, 128, 16, (4, 1), (0.96, 0.02, 0.02), 136),
+    (4800, 128, 32, (4, 1), (0.95, 0.03, 0.02), 72), (9000, 64, 64, (1, 1), (0.97, 0.01, 0.02), 138),
+])
+def test_long_lists(monkeypatch, L, D, C, heads, p, entries):
+    """The last query group walks a list of a known length, on both sides of 64 and 128 entries (fp32 reference of its rows)."""
+    from neuralattentionsearch_amd import ops
+    say("long lists", L, D, C, heads, entries)
+    monkeypatch.setenv("NATS_PREFILL_SPLIT", "0")
+    roles = draw_roles(L, 1, 1, -(-L // C), p=p)
+    tiles = 4 if heads == (1, 1) else 1  # query tiles of a group
+    first = (L - 1) // 64 // tiles * tiles * 64
+    rows = orc.prefill_mask(roles, L, C, 2 * C)[0, 0, first:]
+    assert list_entries(rows, C < 64 or tiles > 1) == entries
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q = torch.randn(1, heads[0], L, D, generator=g, device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.randn(1, 1, L, D, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    got = ops.prefill_attention(q, k, v, to_dev(roles), C, 2 * C)[:, :, first:].float()
+    scores = (q[:, :, first:].float() @ k.float().transpose(-1, -2)) / math.sqrt(D)
+    want = scores.masked_fill(~to_dev(rows), float("-inf")).softmax(-1) @ v.float()
+    assert (got - want).abs().max().item() <= 2e-2
 
 
 @pytest.mark.parametrize("D,C,W,Hq,Hkv", [(128, 32, 256, 4, 1), (64, 16, 64, 8, 2), (32, 32, 64, 2, 1), (128, 64, 128, 1, 1)])
