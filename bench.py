@@ -706,7 +706,7 @@ def main():
         line["roofline"] = {"bound": "mfma", "achieved": pre["tflops_visited"], "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                             "frac": pre["tflops_visited"] / PEAK_BF16_TFLOPS,
                             "kernel": "prefill_mfma_wide_kernel" if args.head_dim == 256
-                                      else f"prefill_mfma_kernel<{args.head_dim}, true, {0 if args.chunk_size >= 64 else 1 if args.chunk_size >= 16 else 2}, false>"}
+                                      else f"prefill_mfma_kernel<{args.head_dim}, true, {0 if args.chunk_size >= 64 else 1 if args.chunk_size >= 16 else 2}, false, false>"}
         line["roofline"]["traffic"], line["roofline"]["traffic_source"] = (
             measured_traffic("prefill") if (args.prefill_len, args.chunk_size, args.head_dim) == (32768, 64, 128)
             else (None, "not the profiled workload"))

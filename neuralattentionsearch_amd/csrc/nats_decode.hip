@@ -54,9 +54,8 @@ __device__ __forceinline__ float exp2_guard(float x) { return __builtin_amdgcn_e
 // tile's first valid row instead (a cache hit), whose score is masked and whose probability is exactly 0.
 // ---------------------------------------------------------------------------------------------------
 constexpr float kDecodeRescaleSlack = 8.0f;
-// K and V rows are read once per step: their loads carry the streaming hint (no retention in the caches)
 constexpr int kDecTile = 32;
-constexpr int kAuxStream = 2;  // ... as the "nt" bit of a global_load_lds
+constexpr int kAuxStream = 2;  // K and V rows are read once per step: the "nt" bit of their loads (no retention in the caches)
 
 constexpr int kMaxBalancedHeads = 1024;  // (b, kv head) streams whose tile prefix sums fit in LDS
 

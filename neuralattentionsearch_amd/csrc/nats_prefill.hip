@@ -966,9 +966,10 @@ __device__ __forceinline__ void prefill_mfma_item(const PrefillArgs& a, unsigned
       // fragments and transfers are constants of the instructions.  Two wavefronts share a SIMD and either issues one instruction in
       // four cycles at most, scalar ones among them, so a step's time follows its instructions: with run-time buffer numbers, generic
       // pointers, a branch for the last tile's rows and entries read from LDS one by one it had 266 scalar and 25 vector
-      // instructions more than the matrix instructions and the softmax need, now 155 and none.  32768 tokens at chunk 64, 32 / 8 heads of 128
-      // 762 -> 721 us, 4 x 3001 at chunk 32 150.7 -> 148.1, 8192 at chunk 1 137.5 -> 128.4.  A second copy of the transfers for
-      // steps far from the list's end, without their conditions, was slower: its scalars did not fit the registers.)
+      // instructions more than the matrix instructions and the softmax need, then 155 and none (about 140 since the width of the rows'
+      // offsets is a template argument).  32768 tokens at chunk 64, 32 / 8 heads of 128 762 -> 721 us, 4 x 3001 at chunk 32 150.7 -> 148.1,
+      // 8192 at chunk 1 137.5 -> 128.4.  A second copy of the transfers for steps far from the list's end, without their conditions, was
+      // slower: its scalars did not fit the registers.)
       auto step = [&](int t, auto phase) {
         constexpr uint32_t P = decltype(phase)::value;  // t & 3
         constexpr uint32_t b0 = P * kTileBytes, b1 = (P + 1) * kTileBytes, b2 = ((P + 2) & 3) * kTileBytes, b3 = ((P + 3) & 3) * kTileBytes;

@@ -61,7 +61,7 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float v) {
 // Llama-3-8B layer then run side by side instead of six per wavefront one after the other.  VEC consecutive columns
 // per thread (16-byte loads when the rows allow it, else 1).  Few chunks of many columns are bound by the trips to memory
 // behind one another (THREADS = 512): twice the threads, sixteen rows to a trip, and the weights of a wavefront's first output
-// requested before the rows (bf16, dim 4096: five chunks of 64 rows 18.5 -> 15.4 us, the token that closes a chunk 7.6 -> 6.1, a role
+// requested before the rows (bf16, dim 4096: five chunks of 64 rows 17.5 -> 14.0 us, the token that closes a chunk 7.6 -> 6.1, a role
 // per token 6.0 -> 5.3; fp32, five chunks 25.5 -> 14.5).  With 256 threads, many chunks or 2048 columns, both lose (32768 tokens
 // 62.2 -> 63.7, 4 x 300 tokens of 2048 at chunk 32 13.9 -> 15.3).
 // TOGETHER: the pieces of a weight row that a wavefront requests before it uses the first (see nats_role_step).
