@@ -79,6 +79,9 @@ def test_role_step_streams(dtype, merge_max, C, dim, H, lens):
     (torch.bfloat16, 64, 2056, 8, 1, [301, 40]), (torch.bfloat16, 8, 2560, 3, 2, [29, 3, 1]), (torch.bfloat16, 32, 5120, 2, 1, [95]),
     (torch.float32, 16, 1028, 8, 1, [100, 13]), (torch.float32, 64, 2056, 1, 2, [190]), (torch.float32, 8, 2560, 4, 1, [50]),
     # more workgroups than compute units: one stream with many chunks, many streams with few
+    # 256 threads: weight rows of four pieces and of more, the last rows of a chunk in fours, twos and ones
+    (torch.bfloat16, 8, 2048, 4, 2, [167]), (torch.bfloat16, 8, 2056, 4, 2, [166, 1]), (torch.float32, 8, 1024, 4, 2, [167, 5]),
+    (torch.float32, 8, 1028, 4, 2, [163, 3]), (torch.float32, 16, 64, 2, 3, [7, 6, 2, 300]),
     (torch.bfloat16, 8, 2560, 1, 1, [2403]), (torch.bfloat16, 16, 2056, 32, 1, [16 * 12]), (torch.float32, 8, 1028, 1, 2, [1203]),
 ])
 def test_role_step_wide_rows(dtype, C, dim, H, B, lens):
